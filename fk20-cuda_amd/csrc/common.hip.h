@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "g1.hip.h"
+#include "g1q.hip.h"
 
 namespace fk20 {
 

@@ -21,6 +21,23 @@ static constexpr uint32_t FP_BETA[14] = {0x1195dfebu, 0x1b04e484u, 0x06026044u, 
 static constexpr uint32_t FP_BETA2[14] = {0x0abf79e7u, 0x194b14ebu, 0x1ceb16a6u, 0x1845cd5du, 0x0c814568u, 0x199ca109u, 0x13ee6ee1u, 0x05d123e5u, 0x0dfbdce2u, 0x010ecb54u, 0x0d9337edu, 0x1daaf4b0u, 0x146806fbu, 0x0000000cu};  // beta^2 (Montgomery)
 static constexpr uint64_t GLV_LAMBDA[2] = {0x00000000ffffffffull, 0xac45a4010001a402ull};  // z^2 - 1
 
+// ---- Fp, signed form: 13 x 30-bit digits, Montgomery radix 2^390 ----
+static constexpr int FQ_N = 13;
+static constexpr uint32_t FQ_MASK = 0x3fffffffu;
+static constexpr int32_t FQ_P[13] = {-21845, -402915328, 356515836, -352321620, -252304353, 55215067, 288093811, 316751073, -321428361, 517541167, -375082566, -91332614, 1704210};  // p
+static constexpr int32_t FQ_PT[14] = {-1, 135004164, 5054525, -327173, 12685220, -359651098, -383584983, 280525645, 202633227, -68632997, -303925084, -261624741, -58966498, -312};  // -196611 p: digit 0 is -1
+// (-p^-1 mod 2^30) << 2: a low word times this, shifted right by 2, is the signed quotient digit
+static constexpr uint32_t FQ_PINV4 = 0xfff3fff4u;
+static constexpr int64_t FQ_K0 = 6969937068335403541ll;
+static constexpr int32_t FQ_BETA[13] = {550457077, 529115271, 538425416, 540408362, 534947505, 530527195, 527739787, 553457329, 541486612, 537384151, 545225655, 547666669, 37975};  // digit offsets of a product
+static constexpr int32_t FQ_ONE[13] = {13762350, 433586176, -192935228, -301937177, 37952645, -425753694, -36732706, 162803105, -437337492, 366579475, 78814996, -442511456, 89578};  // R mod p
+static constexpr int32_t FQ_R2[13] = {84958308, 320669453, -336452545, -23350980, 68258640, -130586467, 277172093, -144228653, 171105485, -419190883, -282802362, -41659541, -694179};  // R^2 mod p
+static constexpr int32_t FQ_GLV[13] = {479228289, -54664058, -430486465, -215714323, 473873436, -101816220, 385853527, -332097025, 89177367, 348892208, 399608966, -514237961, 640725};  // beta of the endomorphism (Montgomery)
+static constexpr int32_t FQ_GLV2[13] = {-492990639, -378922118, -450320131, 517651501, -511826081, 527569914, -349120821, 169293920, 348160125, 358270141, -478423963, -116992407, -730302};  // beta^2
+static constexpr int32_t FQ_4P[13] = {1073654444, 535822335, 352321518, 738197169, 64524410, 220860267, 78633420, 193262469, 861770205, 996422842, 647153385, 708411366, 6816839};  // 4 p, non-negative digits
+static constexpr uint32_t FQ_FROM_FP[14] = {0x00d1ff2eu, 0x13b00000u, 0x12002b11u, 0x10066f36u, 0x0431c84bu, 0x13f07441u, 0x13e03766u, 0x1a16d07bu, 0x0ec26c26u, 0x131e252fu, 0x0a7c515du, 0x1e7d0096u, 0x15de9967u, 0x00000000u};  // 2^390 mod p: x 2^406 -> x 2^390
+static constexpr uint32_t FP_FROM_FQ[14] = {0x1a7f6bafu, 0x1e281d51u, 0x19fe47cbu, 0x16b3408eu, 0x136783f9u, 0x0d3c8407u, 0x1e61f415u, 0x15deb981u, 0x10c53570u, 0x0067aa9du, 0x0256511cu, 0x08eb4399u, 0x004f0125u, 0x00000002u};  // 2^422 mod p: x 2^390 -> x 2^406
+
 // p as 12 x 32-bit limbs (packed storage form)
 static constexpr uint32_t FP_P_PACKED[12] = {0xffffaaabu, 0xb9feffffu, 0xb153ffffu, 0x1eabfffeu, 0xf6b0f624u, 0x6730d2a0u, 0xf38512bfu, 0x64774b84u, 0x434bacd7u, 0x4b1ba7b6u, 0x397fe69au, 0x1a0111eau};
 static constexpr uint32_t FP_HALF_PACKED[12] = {0xffffd555u, 0xdcff7fffu, 0x58a9ffffu, 0x0f55ffffu, 0x7b587b12u, 0xb3986950u, 0x79c2895fu, 0xb23ba5c2u, 0x21a5d66bu, 0x258dd3dbu, 0x1cbff34du, 0x0d0088f5u};  // (p - 1) / 2: y above it is the larger root

@@ -54,11 +54,12 @@ std::vector<int> wnaf(u128 k, int W) {
     return d;
 }
 
-// Ladder cost of a program over digit strings d1, d2, in 32 x 32-bit multiply-adds of the
-// 14 x 29-bit field arithmetic (a product 392, a square 301, a sum of two products sharing
-// one reduction 588): one Jacobian doubling (3 squares, 2 products, 1 pair: 2275) per position
-// below the top, one mixed addition (4 squares, 5 products, 1 pair: 3752) per non-zero digit
-// after the first, and one product (x times beta or beta^2) per digit on phi(P) or phi^2(P).
+// Ladder cost of a program over digit strings d1, d2, in 32 x 32-bit multiply-adds of
+// fq.hip.h (a product 338, a square 260, a pair with one reduction 507): one Jacobian doubling
+// (g1h_dbl: 1924 with its linear combinations) per position below the top, one mixed addition
+// (g1h_madd: 3393) per non-zero digit after the first, and one product (x times beta or beta^2)
+// per digit on phi(P) or phi^2(P).
+static constexpr int COST_DBL = 1924, COST_MADD = 3393, COST_PHI = 338;
 int program_cost(const std::vector<int> &d1, const std::vector<int> &d2, int t) {
     const int L = (int)std::max(d1.size(), d2.size());
     int nz = 0, nphi = 0;
@@ -67,7 +68,7 @@ int program_cost(const std::vector<int> &d1, const std::vector<int> &d2, int t) 
     for (int part = 0; part < 2; part++)
         if ((t + part) % 3 != 0)
             for (int x : part ? d2 : d1) nphi += x != 0;
-    return std::max(L - 1, 0) * 2275 + std::max(nz - 1, 0) * 3752 + nphi * 392;
+    return std::max(L - 1, 0) * COST_DBL + std::max(nz - 1, 0) * COST_MADD + nphi * COST_PHI;
 }
 
 // lambda (the eigenvalue of phi on G1) in Montgomery form
@@ -254,7 +255,7 @@ int ops_cost(const uint32_t *ops) {
         add++;
         phi += (ops[k] & (TWOP_PHI | TWOP_PHI2)) != 0;
     }
-    return dbl * 2275 + std::max(add - 1, 0) * 3752 + phi * 392;
+    return dbl * COST_DBL + std::max(add - 1, 0) * COST_MADD + phi * COST_PHI;
 }
 
 // The twiddle layers' item tables (index[TW_LAYER ..]): every (q, e) of layer_twiddle, per

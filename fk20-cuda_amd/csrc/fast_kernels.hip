@@ -31,16 +31,16 @@ namespace fk20 {
 
 // ---------------------------------------------------------------- setup: scaled bases
 
-__device__ __noinline__ void g1_mul_std(g1p &r, const g1p &p, const uint32_t *k) {
-    g1p q;
-    g1_inf(q);
+__device__ __noinline__ void g1_mul_std(g1q &r, const g1q &p, const uint32_t *k) {
+    g1q q;
+    g1q_inf(q);
 #pragma unroll 1
     for (int w = 7; w >= 0; w--) {
         const uint32_t kw = k[w];
 #pragma unroll 1
         for (int b = 31; b >= 0; b--) {
-            g1_dbl(q, q);
-            if ((kw >> b) & 1) g1_add(q, q, p);
+            g1q_dbl(q, q);
+            if ((kw >> b) & 1) g1q_add(q, q, p);
         }
     }
     r = q;
@@ -53,11 +53,9 @@ __global__ void __launch_bounds__(64) k_scale_bases(uint32_t *xs, uint32_t *inf,
     if (b >= count) return;
     uint32_t w[36];
     ld_words(w, xext + b * G1P_WORDS, 9);
-    g1p p;
-    g1_load_std(p, w);
-    fe zc;
-    fe_canonical(zc, p.z);
-    inf[b] = fe_is_zero_canonical(zc) ? 1u : 0u;
+    g1q p;
+    g1q_load_std(p, w);
+    inf[b] = g1q_is_inf(p) ? 1u : 0u;
     uint32_t k[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) k[i] = scale[i];
@@ -75,17 +73,17 @@ __global__ void k_fill_u32(uint32_t *p, size_t n, uint32_t v) {
 // A lane's point in LDS, packed (36 words, stride 37 to spread the lanes over the banks).
 struct LdsSlot {
     uint32_t *w;
-    __device__ void put(const g1p &p) {
+    __device__ void put(const g1q &p) {
         uint32_t t[36];
-        g1_store_packed(t, p);
+        g1q_store_packed(t, p);
 #pragma unroll
         for (int k = 0; k < 36; k++) w[k] = t[k];
     }
-    __device__ void get(g1p &p) const {
+    __device__ void get(g1q &p) const {
         uint32_t t[36];
 #pragma unroll
         for (int k = 0; k < 36; k++) t[k] = w[k];
-        g1_load_packed(p, t);
+        g1q_load_packed(p, t);
     }
 };
 
@@ -98,8 +96,8 @@ __global__ void __launch_bounds__(64, 2) k_subgroup_groups(uint32_t *flags, cons
     if (i >= count) return;
     uint32_t w[36];
     ld_words(w, pts + i * G1P_WORDS, 9);
-    g1p p;
-    g1_load_std(p, w);
+    g1q p;
+    g1q_load_std(p, w);
     LdsSlot orig{slots[0] + threadIdx.x * 37}, base{slots[1] + threadIdx.x * 37};
     if (!g1_in_subgroup(p, orig, base)) atomicOr(flags + i / per_group, 1u);
 }
@@ -118,19 +116,28 @@ __global__ void __launch_bounds__(64, 2) k_subgroup_groups(uint32_t *flags, cons
 // formulas (g1_mul_std, as g1p_mul.cu:18).  One workgroup of 256 threads per row; the row's n
 // points live in `work` (n * 36 words per row, row-contiguous); barriers order the stages.
 
+// (a, b) <- (a + b, a - b)
+__device__ __forceinline__ void addsub(g1q &a, g1q &b) {
+    g1q s;
+    g1q_add(s, a, b);
+    g1q_neg(b, b);
+    g1q_add(b, a, b);
+    a = s;
+}
+
 __device__ __forceinline__ void ref_butterfly(uint32_t *Wr, unsigned s, unsigned t, bool inverse, unsigned logn,
                                               const DevTables *T) {
     const unsigned h = 1u << s, j = t & (h - 1);
     const unsigned l = ((t >> s) << (s + 1)) + j, r = l + h;
     const unsigned e = j << (8 - s);  // twiddle w^e of the order-512 root w
-    g1p a, b;
+    g1q a, b;
     pt_load(a, Wr + (size_t)l * 36);
     pt_load(b, Wr + (size_t)r * 36);
     if (!inverse) {
         if (e) g1_mul_std(b, b, T->tw_std[e]);
-        g1_addsub(a, b);
+        addsub(a, b);
     } else {
-        g1_addsub(a, b);
+        addsub(a, b);
         if (s == 1) {
             g1_mul_std(a, a, T->inv2k_std[logn]);
             g1_mul_std(b, b, j ? T->inv2k_w384_std[logn] : T->inv2k_std[logn]);
@@ -153,13 +160,13 @@ __global__ void __launch_bounds__(256) k_ref_rows(unsigned kind, uint32_t *out, 
     const unsigned n = 1u << logn, t = threadIdx.x;
     uint32_t *Wr = work + (size_t)row * n * 36;
     for (unsigned j = t; j < n; j += 256) {
-        g1p p;
+        g1q p;
         if (in_D) {
             pt_load(p, in_D + ((size_t)bitrev(j, logn) * rows + row) * 36);
         } else {
             uint32_t w[36];
             ld_words(w, in + ((size_t)row * n + j) * G1P_WORDS, 9);
-            g1_load_std(p, w);
+            g1q_load_std(p, w);
         }
         pt_store(Wr + (size_t)(kind == 0 ? bitrev(j, logn) : j) * 36, p);
     }
@@ -173,8 +180,8 @@ __global__ void __launch_bounds__(256) k_ref_rows(unsigned kind, uint32_t *out, 
         if (kind == 2) {
             // the upper half of the inverse's natural-order output sits at the odd positions
             for (unsigned j = 2 * t + 1; j < n; j += 512) {
-                g1p z;
-                g1_inf(z);
+                g1q z;
+                g1q_inf(z);
                 pt_store(Wr + (size_t)j * 36, z);
             }
             __syncthreads();
@@ -188,10 +195,10 @@ __global__ void __launch_bounds__(256) k_ref_rows(unsigned kind, uint32_t *out, 
         }
     }
     for (unsigned j = t; j < n; j += 256) {
-        g1p p;
+        g1q p;
         pt_load(p, Wr + (size_t)(kind == 1 ? bitrev(j, logn) : j) * 36);
         uint32_t w[36];
-        g1_store_std(w, p);
+        g1q_store_std(w, p);
         st_words(out + ((size_t)row * n + j) * G1P_WORDS, w, 9);
     }
 }
@@ -223,54 +230,53 @@ __global__ void __launch_bounds__(64, 3) k_table_build(uint32_t *table, uint32_t
     // B' = 2^(w win) B in affine form, so each entry is one mixed addition of B' (B' is not
     // infinity: the base is not, and E(Fp) has odd order).  An entry d B' is infinity only
     // for a base of small order outside G1; the block's inversion then fails and *err says so.
-    g1p E;
-    fe bx, by;
+    g1q E;
+    fq bx, by;
     {
-        g1p B;
+        g1q B;
         pt_load(B, xs + (size_t)b * 36);
 #pragma unroll 1
-        for (unsigned d = 0; d < win_bits * win; d++) g1_dbl(B, B);
-        g1_to_affine(bx, by, B);
+        for (unsigned d = 0; d < win_bits * win; d++) g1q_dbl(B, B);
+        g1q_to_affine(bx, by, B);
     }
     E.x = bx;
     E.y = by;
-    fe_one(E.z);
+    fq_one(E.z);
 #pragma unroll 1
     for (unsigned e0 = 0; e0 < H; e0 += blk) {
-        fe prefix;
-        fe_one(prefix);
+        fq prefix;
+        fq_one(prefix);
 #pragma unroll 1
         for (unsigned i = 0; i < blk; i++) {
             const unsigned e = e0 + i;
-            if (e) g1_add_aff(E, E, bx, by);
+            if (e) g1q_add_aff(E, E, bx, by);
             uint32_t *z = zt + ((size_t)i * nthreads + t) * 24;
-            fe_store(tab + (size_t)e * TABLE_ENTRY_WORDS, E.x);
-            fe_store(tab + (size_t)e * TABLE_ENTRY_WORDS + 12, E.y);
-            fe_store(z, E.z);
-            fe_store(z + 12, prefix);  // prefix of z_e0 .. z_{e-1}
-            fe_mul(prefix, prefix, E.z);
+            fq_store(tab + (size_t)e * TABLE_ENTRY_WORDS, E.x);
+            fq_store(tab + (size_t)e * TABLE_ENTRY_WORDS + 12, E.y);
+            fq_store(z, E.z);
+            fq_store(z + 12, prefix);  // prefix of z_e0 .. z_{e-1}
+            fq_mul(prefix, prefix, E.z);
         }
-        fe inv;
-        fe_canonical(prefix, prefix);
-        if (fe_is_zero_canonical(prefix)) atomicOr(err, 1u);
-        fe_inv(inv, prefix);
+        fq inv;
+        if (fq_is_zero(prefix)) atomicOr(err, 1u);
+        fq_inv(inv, prefix);
 #pragma unroll 1
         for (int i = (int)blk - 1; i >= 0; i--) {
             const unsigned e = e0 + (unsigned)i;
             const uint32_t *z = zt + ((size_t)i * nthreads + t) * 24;
-            fe ze, pe, zinv, x, y;
-            fe_load(ze, z);
-            fe_load(pe, z + 12);
-            fe_mul(zinv, inv, pe);
-            fe_mul(inv, inv, ze);
-            fe_load(x, tab + (size_t)e * TABLE_ENTRY_WORDS);
-            fe_load(y, tab + (size_t)e * TABLE_ENTRY_WORDS + 12);
-            fe_mul(x, x, zinv);
-            fe_mul(y, y, zinv);
-            fe_canonical(x, x);
-            fe_canonical(y, y);
-            fe_store(tab + (size_t)e * TABLE_ENTRY_WORDS, x);
-            fe_store(tab + (size_t)e * TABLE_ENTRY_WORDS + 12, y);
+            fq ze, pe, zinv, x, y;
+            fq_load(ze, z);
+            fq_load(pe, z + 12);
+            fq_mul(zinv, inv, pe);
+            fq_mul(inv, inv, ze);
+            fq_load(x, tab + (size_t)e * TABLE_ENTRY_WORDS);
+            fq_load(y, tab + (size_t)e * TABLE_ENTRY_WORDS + 12);
+            fq_mul(x, x, zinv);
+            fq_mul(y, y, zinv);
+            uint32_t w[24];
+            fq_canon_words(w, x);
+            fq_canon_words(w + 12, y);
+            st_words(tab + (size_t)e * TABLE_ENTRY_WORDS, w, 6);
         }
     }
 }
@@ -341,7 +347,7 @@ __global__ void __launch_bounds__(256) k_toeplitz_fft_multi(Launch L, const DevT
 // of WIN bits over B's table tb[win][d - 1] = d * 2^(WIN*win) * B (affine): one mixed
 // addition per non-zero digit, no doublings.  k < r < 2^255 keeps the last window's carry
 // inside the ceil(256/WIN) windows for every WIN in 8..13.
-__device__ __forceinline__ void window_term(g1p &acc, uint32_t *k, const uint32_t *tb, unsigned WIN) {
+__device__ __forceinline__ void window_term(g1q &acc, uint32_t *k, const uint32_t *tb, unsigned WIN) {
     const unsigned NWIN = (256 + WIN - 1) / WIN, H = 1u << (WIN - 1), MASK = (1u << WIN) - 1;
     uint32_t carry = 0;
 #pragma unroll 1
@@ -356,11 +362,11 @@ __device__ __forceinline__ void window_term(g1p &acc, uint32_t *k, const uint32_
         if (d != 0) {
             const unsigned e = (unsigned)(d < 0 ? -d : d) - 1;
             const uint32_t *ent = tb + ((size_t)win * H + e) * TABLE_ENTRY_WORDS;
-            fe x, y;
-            fe_load(x, ent);
-            fe_load(y, ent + 12);
-            if (d < 0) fe_neg<2>(y, y);
-            g1_add_aff(acc, acc, x, y);
+            fq x, y;
+            fq_load_raw(x, ent);
+            fq_load_raw(y, ent + 12);
+            if (d < 0) fq_neg(y, y);
+            g1q_add_aff(acc, acc, x, y);
         }
     }
 }
@@ -374,8 +380,8 @@ __global__ void __launch_bounds__(64) k_msm_multi(Launch L) {
     const unsigned WIN = it.win, NWIN = (256 + WIN - 1) / WIN, H = 1u << (WIN - 1);
     const unsigned j = local / rg;
     const unsigned row = min((local % rg) * 64 + threadIdx.x, rows - 1);  // spare lanes repeat the last row
-    g1p acc;
-    g1_inf(acc);
+    g1q acc;
+    g1q_inf(acc);
 #pragma unroll 1
     for (unsigned i = 0; i < 16; i++) {
         const unsigned b = i * n2 + j;
@@ -402,8 +408,8 @@ __global__ void __launch_bounds__(64) k_msm_multi_small(Launch L) {
     const unsigned j = local / rg4, t = threadIdx.x, i = t % 16, r = t / 16;
     const unsigned row0 = (local % rg4) * 4 + r, row = min(row0, rows - 1);  // spare lanes repeat a row
     const unsigned b = i * n2 + j;
-    g1p acc;
-    g1_inf(acc);
+    g1q acc;
+    g1q_inf(acc);
     if (!it.inf[b]) {
         uint32_t k[8];
         ld_words(k, it.tcT + (((size_t)j * 16 + i) * rows + row) * FR_WORDS, 2);
@@ -413,10 +419,10 @@ __global__ void __launch_bounds__(64) k_msm_multi_small(Launch L) {
 #pragma unroll 1
     for (unsigned h = 8; h >= 1; h /= 2) {
         __syncthreads();
-        g1p o;
+        g1q o;
         if (i < h) {
             pt_load(o, lds + (t + h) * 36);
-            g1_add(acc, acc, o);
+            g1q_add(acc, acc, o);
         }
         __syncthreads();
         if (i < h) pt_store(lds + t * 36, acc);
@@ -438,8 +444,8 @@ __global__ void __launch_bounds__(64) k_commit_partial(const uint32_t *poly, con
     const unsigned row = min((blockIdx.x % rg) * 64 + threadIdx.x, rows - 1);  // spare lanes repeat the last row
     const unsigned NWIN = (256 + win_bits - 1) / win_bits, H = 1u << (win_bits - 1);
     const unsigned i0 = c * chunk, i1 = min(i0 + chunk, N);
-    g1p acc;
-    g1_inf(acc);
+    g1q acc;
+    g1q_inf(acc);
 #pragma unroll 1
     for (unsigned i = i0; i < i1; i++) {
         if (inf[i]) continue;
@@ -463,16 +469,16 @@ __global__ void __launch_bounds__(64) k_commit_reduce(const uint32_t *in, uint32
     if (t >= (size_t)rows * nout) return;
     const unsigned row = (unsigned)(t % rows), q = (unsigned)(t / rows);
     const unsigned p0 = q * group, p1 = min(p0 + group, nparts);
-    g1p acc, x;
-    g1_inf(acc);
+    g1q acc, x;
+    g1q_inf(acc);
 #pragma unroll 1
     for (unsigned p = p0; p < p1; p++) {
         pt_load(x, in + ((size_t)p * rows + row) * 36);
-        g1_add(acc, acc, x);
+        g1q_add(acc, acc, x);
     }
     if (std_out) {
         uint32_t w[36];
-        g1_store_std(w, acc);
+        g1q_store_std(w, acc);
         st_words(out + (size_t)row * G1P_WORDS, w, 9);
     } else {
         pt_store(out + ((size_t)q * rows + row) * 36, acc);
@@ -519,17 +525,17 @@ __global__ void __launch_bounds__(64) k_output_multi(Launch L) {
     const unsigned row = (local % rg) * 64 + threadIdx.x;
     if (row >= rows) return;
     if (it.rowflag && it.rowflag[(size_t)row * it.flag_stride]) return;  // written by k_ref_rows
-    g1p p;
+    g1q p;
     pt_load(p, it.D + ((size_t)pos * rows + row) * 36);
     const unsigned fmt = it.out_format;
     const size_t slot = (size_t)row * (1u << logn2) + ((fmt & 1u) ? pos : bitrev(pos, logn2));
     if (fmt & 2u) {
         uint32_t w[12];
-        g1_compress(w, p);
+        g1q_compress(w, p);
         st_words(it.h_fft + slot * 12, w, 3);
     } else {
         uint32_t w[36];
-        g1_store_std(w, p);
+        g1q_store_std(w, p);
         st_words(it.h_fft + slot * G1P_WORDS, w, 9);
     }
 }

@@ -16,56 +16,40 @@ __device__ __forceinline__ void words_load(uint32_t *dst, const uint32_t *src, i
     }
 }
 
-__device__ __forceinline__ void g1_lds_load(g1p &p, const uint32_t *lds) {
+__device__ __forceinline__ void g1_lds_load(g1q &p, const uint32_t *lds) {
     uint32_t w[36];
 #pragma unroll
     for (int i = 0; i < 9; i++) {
         uint4 v = reinterpret_cast<const uint4 *>(lds)[i];
         w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
     }
-    g1_load_packed(p, w);
+    g1q_load_packed(p, w);
 }
 
-__device__ __forceinline__ void g1_lds_store(uint32_t *lds, const g1p &p) {
+__device__ __forceinline__ void g1_lds_store(uint32_t *lds, const g1q &p) {
     uint32_t w[36];
-    g1_store_packed(w, p);
+    g1q_store_packed(w, p);
 #pragma unroll
     for (int i = 0; i < 9; i++)
         reinterpret_cast<uint4 *>(lds)[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
 }
 
-__device__ __forceinline__ void g1_gload_std(g1p &p, const uint32_t *g) {
+__device__ __forceinline__ void g1q_gload_std(g1q &p, const uint32_t *g) {
     uint32_t w[36];
 #pragma unroll
     for (int i = 0; i < 9; i++) {
         uint4 v = reinterpret_cast<const uint4 *>(g)[i];
         w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
     }
-    g1_load_std(p, w);
+    g1q_load_std(p, w);
 }
 
-__device__ __forceinline__ void g1_gstore_std(uint32_t *g, const g1p &p) {
+__device__ __forceinline__ void g1q_gstore_std(uint32_t *g, const g1q &p) {
     uint32_t w[36];
-    g1_store_std(w, p);
+    g1q_store_std(w, p);
 #pragma unroll
     for (int i = 0; i < 9; i++)
         reinterpret_cast<uint4 *>(g)[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
-}
-
-// Scalar multiplication with a non-unrolled bit loop (one inlined dbl and add); any 256-bit k.
-__device__ __noinline__ void g1_mul_dev(g1p &r, const g1p &p, const uint32_t *k) {
-    g1p q;
-    g1_inf(q);
-#pragma unroll 1
-    for (int w = 7; w >= 0; w--) {
-        const uint32_t kw = k[w];
-#pragma unroll 1
-        for (int b = 31; b >= 0; b--) {
-            g1_dbl(q, q);
-            if ((kw >> b) & 1) g1_add(q, q, p);
-        }
-    }
-    r = q;
 }
 
 // h[row][n/2..n) = (0, 1, 0)  (fk20_poly2h_fft.cu:27)
@@ -84,8 +68,8 @@ __global__ void k_hext2h(uint32_t *h, unsigned rows, unsigned n2) {
 __global__ void k_std_to_packed(uint32_t *packed, const uint32_t *pts, size_t count) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= count) return;
-    g1p p;
-    g1_gload_std(p, pts + e * G1P_WORDS);
+    g1q p;
+    g1q_gload_std(p, pts + e * G1P_WORDS);
     g1_lds_store(packed + e * 36, p);
 }
 
@@ -135,13 +119,13 @@ __global__ void __launch_bounds__(256) k_msm_digits(int8_t *digits, const uint32
     }
 }
 
-__device__ __forceinline__ void msm_booth_add(g1p &acc, const uint32_t *tab, int dg) {
+__device__ __forceinline__ void msm_booth_add(g1q &acc, const uint32_t *tab, int dg) {
     const unsigned a = (unsigned)(dg < 0 ? -dg : dg);
-    g1p X;
+    g1q X;
     g1_lds_load(X, tab + (a ? a - 1 : 0) * 36);
-    if (dg < 0) fe_neg<2>(X.y, X.y);
-    if (a == 0) g1_inf(X);
-    g1_add(acc, acc, X);
+    if (dg < 0) fq_neg(X.y, X.y);
+    if (a == 0) g1q_inf(X);
+    g1q_add(acc, acc, X);
 }
 
 __global__ void __launch_bounds__(256, 2) k_msm_booth(uint32_t *out, const int8_t *digits, const uint32_t *xpk,
@@ -151,13 +135,13 @@ __global__ void __launch_bounds__(256, 2) k_msm_booth(uint32_t *out, const int8_
     // entry e = 32 i + (m - 1) holds m X_i, by double-and-add over m's 6 bits
     for (unsigned e = t; e < 16 * MSM_HALF; e += blockDim.x) {
         const unsigned i = e / MSM_HALF, mult = e % MSM_HALF + 1;
-        g1p X, acc;
+        g1q X, acc;
         g1_lds_load(X, xpk + ((size_t)i * n2 + j) * 36);  // packed Montgomery points in HBM
-        g1_inf(acc);
+        g1q_inf(acc);
 #pragma unroll 1
         for (int b = 5; b >= 0; b--) {
-            g1_dbl(acc, acc);
-            if ((mult >> b) & 1) g1_add(acc, acc, X);
+            g1q_dbl(acc, acc);
+            if ((mult >> b) & 1) g1q_add(acc, acc, X);
         }
         g1_lds_store(lds + e * 36, acc);
     }
@@ -165,13 +149,13 @@ __global__ void __launch_bounds__(256, 2) k_msm_booth(uint32_t *out, const int8_
     const unsigned row0 = blockIdx.y * blockDim.x + t;
     const unsigned row = min(row0, rows - 1);  // lanes past the last row repeat it
     const int8_t *dg = digits + (size_t)j * 16 * MSM_NWIN * rows + row;
-    g1p acc;
-    g1_inf(acc);
+    g1q acc;
+    g1q_inf(acc);
 #pragma unroll 1
     for (int w = MSM_NWIN - 1; w >= 0; w--) {
         if (w != (int)MSM_NWIN - 1) {
 #pragma unroll 1
-            for (int d = 0; d < 6; d++) g1_dbl(acc, acc);
+            for (int d = 0; d < 6; d++) g1q_dbl(acc, acc);
         }
 #pragma unroll 1
         for (unsigned i = 0; i < 16; i++)
@@ -179,7 +163,7 @@ __global__ void __launch_bounds__(256, 2) k_msm_booth(uint32_t *out, const int8_
     }
     if (row0 < rows) {
         if (to_D) g1_lds_store(out + ((size_t)bitrev(j, 31 - __builtin_clz(n2)) * rows + row) * 36, acc);
-        else g1_gstore_std(out + ((size_t)row * n2 + j) * G1P_WORDS, acc);
+        else g1q_gstore_std(out + ((size_t)row * n2 + j) * G1P_WORDS, acc);
     }
 }
 
@@ -195,31 +179,31 @@ __global__ void __launch_bounds__(64) k_msm_booth_small(uint32_t *out, const int
     __shared__ __attribute__((aligned(16))) uint32_t lds[16 * MSM_HALF * 36];
     const unsigned j = blockIdx.x, t = threadIdx.x, i = t % 16, r = t / 16;
     {
-        g1p X, step, e;
+        g1q X, step, e;
         g1_lds_load(X, xpk + ((size_t)i * n2 + j) * 36);  // packed Montgomery points in HBM
-        g1_dbl(step, X);                                  // 2 X
+        g1q_dbl(step, X);                                  // 2 X
         if (r == 0) e = X;
         else if (r == 1) e = step;
-        else if (r == 2) g1_add(e, step, X);
-        else g1_dbl(e, step);
-        g1_dbl(step, step);                               // 4 X
+        else if (r == 2) g1q_add(e, step, X);
+        else g1q_dbl(e, step);
+        g1q_dbl(step, step);                               // 4 X
 #pragma unroll 1
         for (unsigned k = 0; k < MSM_HALF / 4; k++) {     // entry m - 1 holds m X_i, m = r + 1 + 4k
             g1_lds_store(lds + (i * MSM_HALF + r + 4 * k) * 36, e);
-            if (k + 1 < MSM_HALF / 4) g1_add(e, e, step);
+            if (k + 1 < MSM_HALF / 4) g1q_add(e, e, step);
         }
     }
     __syncthreads();
     const unsigned row0 = blockIdx.y * 4 + r;
     const unsigned row = min(row0, rows - 1);  // lanes past the last row repeat it
     const int8_t *dg = digits + ((size_t)j * 16 + i) * MSM_NWIN * rows + row;
-    g1p acc;
-    g1_inf(acc);
+    g1q acc;
+    g1q_inf(acc);
 #pragma unroll 1
     for (int w = MSM_NWIN - 1; w >= 0; w--) {
         if (w != (int)MSM_NWIN - 1) {
 #pragma unroll 1
-            for (int d = 0; d < 6; d++) g1_dbl(acc, acc);
+            for (int d = 0; d < 6; d++) g1q_dbl(acc, acc);
         }
         msm_booth_add(acc, lds + i * MSM_HALF * 36, dg[(size_t)w * rows]);
     }
@@ -228,17 +212,17 @@ __global__ void __launch_bounds__(64) k_msm_booth_small(uint32_t *out, const int
 #pragma unroll 1
     for (unsigned h = 8; h >= 1; h /= 2) {
         __syncthreads();
-        g1p o;
+        g1q o;
         if (i < h) {
             g1_lds_load(o, lds + (t + h) * 36);
-            g1_add(acc, acc, o);
+            g1q_add(acc, acc, o);
         }
         __syncthreads();
         if (i < h) g1_lds_store(lds + t * 36, acc);
     }
     if (i == 0 && row0 < rows) {
         if (to_D) g1_lds_store(out + ((size_t)bitrev(j, 31 - __builtin_clz(n2)) * rows + row) * 36, acc);
-        else g1_gstore_std(out + ((size_t)row * n2 + j) * G1P_WORDS, acc);
+        else g1q_gstore_std(out + ((size_t)row * n2 + j) * G1P_WORDS, acc);
     }
 }
 
@@ -368,15 +352,14 @@ __global__ void k_setup_gather(uint32_t *xext, const uint32_t *srs, unsigned N) 
 __global__ void k_to_affine(uint32_t *out, const uint32_t *in, size_t count) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= count) return;
-    g1p p;
-    g1_gload_std(p, in + e * G1P_WORDS);
-    fe x, y;
-    g1_to_affine(x, y, p);
-    fe_from_mont(x, x);
-    fe_from_mont(y, y);
-    uint32_t w[24];
-    fe_pack(w, x);
-    fe_pack(w + 12, y);
+    g1q p;
+    g1q_gload_std(p, in + e * G1P_WORDS);
+    fq x, y;
+    uint32_t w[24] = {0};
+    if (g1q_to_affine(x, y, p)) {
+        fq_to_std(w, x);
+        fq_to_std(w + 12, y);
+    }
     uint4 *q = reinterpret_cast<uint4 *>(out + e * G1A_WORDS);
 #pragma unroll
     for (int i = 0; i < 6; i++) q[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
@@ -385,16 +368,50 @@ __global__ void k_to_affine(uint32_t *out, const uint32_t *in, size_t count) {
 __global__ void k_compress(uint32_t *out, const uint32_t *in, size_t count) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= count) return;
-    g1p p;
-    g1_gload_std(p, in + e * G1P_WORDS);
+    g1q p;
+    g1q_gload_std(p, in + e * G1P_WORDS);
     uint32_t w[12];
-    g1_compress(w, p);
+    g1q_compress(w, p);
     uint4 *q = reinterpret_cast<uint4 *>(out + e * 12);
 #pragma unroll
     for (int i = 0; i < 3; i++) q[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
 }
 
 // ---------------------------------------------------------------- element-wise ops
+
+// Scalar multiplication with a non-unrolled bit loop (one inlined dbl and add); any 256-bit k.
+__device__ __noinline__ void g1_mul_dev(g1p &r, const g1p &p, const uint32_t *k) {
+    g1p q;
+    g1_inf(q);
+#pragma unroll 1
+    for (int w = 7; w >= 0; w--) {
+        const uint32_t kw = k[w];
+#pragma unroll 1
+        for (int b = 31; b >= 0; b--) {
+            g1_dbl(q, q);
+            if ((kw >> b) & 1) g1_add(q, q, p);
+        }
+    }
+    r = q;
+}
+
+__device__ __forceinline__ void g1_gload_std(g1p &p, const uint32_t *g) {
+    uint32_t w[36];
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+        uint4 v = reinterpret_cast<const uint4 *>(g)[i];
+        w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
+    }
+    g1_load_std(p, w);
+}
+
+__device__ __forceinline__ void g1_gstore_std(uint32_t *g, const g1p &p) {
+    uint32_t w[36];
+    g1_store_std(w, p);
+#pragma unroll
+    for (int i = 0; i < 9; i++)
+        reinterpret_cast<uint4 *>(g)[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
+}
 
 __device__ __forceinline__ void fe_gload_std(fe &a, const uint32_t *g) {
     uint32_t w[12];

@@ -22,28 +22,35 @@ __device__ __forceinline__ void st_words(uint32_t *g, const uint32_t *w, int n4)
         reinterpret_cast<uint4 *>(g)[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
 }
 
-__device__ __forceinline__ void pt_load(g1p &p, const uint32_t *g) {
+__device__ __forceinline__ void pt_load(g1q &p, const uint32_t *g) {
     uint32_t w[36];
     ld_words(w, g, 9);
-    g1_load_packed(p, w);
+    g1q_load_packed(p, w);
 }
 
-__device__ __forceinline__ void pt_store(uint32_t *g, const g1p &p) {
+__device__ __forceinline__ void pt_store(uint32_t *g, const g1q &p) {
     uint32_t w[36];
-    g1_store_packed(w, p);
+    g1q_store_packed(w, p);
     st_words(g, w, 9);
 }
 
-__device__ __forceinline__ void fe_load(fe &a, const uint32_t *g) {
+__device__ __forceinline__ void fq_load(fq &a, const uint32_t *g) {
     uint32_t w[12];
     ld_words(w, g, 3);
-    fe_unpack(a, w);
+    fq_unpack(a, w);
 }
 
-__device__ __forceinline__ void fe_store(uint32_t *g, const fe &a) {
+__device__ __forceinline__ void fq_store(uint32_t *g, const fq &a) {
     uint32_t w[12];
-    fe_pack(w, a);
+    fq_pack(w, a);
     st_words(g, w, 3);
+}
+
+// a coordinate of a window-table entry: canonical Montgomery, no offset
+__device__ __forceinline__ void fq_load_raw(fq &a, const uint32_t *g) {
+    uint32_t w[12];
+    ld_words(w, g, 3);
+    fq_unpack_raw(a, w);
 }
 
 // ---------------------------------------------------------------- multi-item decoding

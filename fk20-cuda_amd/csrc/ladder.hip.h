@@ -13,13 +13,14 @@
 //   bit  12     negate
 //   bit  31     END
 //
-// Arithmetic.  The input is converted to Jacobian coordinates and its odd multiples
+// Arithmetic (g1q.hip.h).  The input is converted to Jacobian coordinates and its odd multiples
 // P, 3P, .., (2^(W-1) - 1) P are built with one common Z (doubling with update, then co-Z
 // additions 2P + (2i - 1)P, then each entry rescaled to the last Z): on the isomorphic curve
-// y^2 = x^3 + b Z^6 they are affine points, so the ladder runs Jacobian doublings (3S + 2M +
-// a shared-reduction product pair) and mixed additions (4S + 5M + a pair) instead of complete
-// projective formulas, and the table holds x and y only.  At the end the accumulator's Z is
-// multiplied by the table's Z and the point converted back to homogeneous coordinates.
+// y^2 = x^3 + b Z^6 they are affine points, so the ladder runs Jacobian doublings (3 squares, 2
+// products, a product minus square) and mixed additions (3 squares, 6 products, a pair) instead
+// of complete projective formulas, and the table holds x and 2 y only.  At the end the
+// accumulator's Z is multiplied by the table's Z and the point converted back to homogeneous
+// coordinates.
 //
 // The formulas are incomplete.  For an input of prime order r that is not infinity, the
 // accumulator before each addition is a P and the entry b P with a, b known scalars; the host
@@ -29,6 +30,7 @@
 // transforms find such rows with g1_in_subgroup below and recompute them on another path.
 #pragma once
 #include "g1.hip.h"
+#include "g1q.hip.h"
 
 #ifndef FK20_UNIFORM
 #define FK20_UNIFORM(x) __builtin_amdgcn_readfirstlane(x)
@@ -51,76 +53,77 @@ static constexpr uint32_t TWOP_END = 1u << 31;
 static constexpr int TW_WNAF = FK20_TW_WNAF;
 
 // x <- k * x for the wave-uniform scalar whose program starts at ops[0].  x: homogeneous
-// projective, coordinates < 10 p; out: x < 2 p, y < 4 p, z < 2 p.
+// projective, coordinates < 8 p; out: < 2 p.
 template <int W>
-FK20_HD void tw_mul(g1p &x, const uint32_t *ops) {
+FK20_HD void tw_mul(g1q &x, const uint32_t *ops) {
     constexpr int NT = 1 << (W - 2);
     static_assert(NT >= 2, "table of at least P and 3P");
     // The table lives in the lane's private memory, not in registers: each addition reads
     // one entry chosen by a wave-uniform index, so the loads are coalesced per dword and the
     // ladder's register footprint leaves room for several waves per SIMD.
-    fe TX[NT], TY[NT], MU[NT - 1];
-    fe zc;
-    fe_canonical(zc, x.z);
-    const bool inf = fe_is_zero_canonical(zc);
+    fq TX[NT], TY[NT], MU[NT - 1];
+    const bool inf = g1q_is_inf(x);
     // homogeneous (X : Y : Z) -> Jacobian (X Z, Y Z^2, Z)
-    g1j P;
-    fe_sqr(zc, x.z);                // < 2p
-    fe_mul(P.x, x.x, x.z);          // < 2p
-    fe_mul(P.y, x.y, zc);           // < 2p
-    P.z = x.z;                      // < 10p
-    g1j Q;                          // 2P, re-scaled by every co-Z addition
-    g1j_dblu(Q, TX[0], TY[0], P);
-    fe x1 = Q.x, y1 = Q.y;
-#pragma unroll
-    for (int k = 1; k < NT; k++) g1j_zaddu(TX[k], TY[k], MU[k - 1], x1, y1, TX[k - 1], TY[k - 1]);
+    g1j_q P, Q;                     // Q = 2P, re-scaled by every co-Z addition
+    fq t;
+    fq_sqr(t, x.z);
+    fq_mul(P.x, x.x, x.z);
+    fq_mul(P.y, x.y, t);
+    P.z = x.z;
+    g1q_dblu(Q, TX[0], TY[0], P);
+    fq x1 = Q.x, y1 = Q.y;
+#pragma unroll 1
+    for (int k = 1; k < NT; k++) g1q_zaddu(TX[k], TY[k], MU[k - 1], x1, y1, TX[k - 1], TY[k - 1]);
     // entry k has Z0 * mu_0 ... mu_{k-1}; bring it to the last entry's Z by the product of
-    // the later factors
-    fe s = MU[NT - 2], s2, s3;
-#pragma unroll
+    // the later factors, y doubled on the way
+    fq s = MU[NT - 2], s2, s3;
+    fq_add(TY[NT - 1], TY[NT - 1], TY[NT - 1]);
+#pragma unroll 1
     for (int k = NT - 2; k >= 0; k--) {
-        if (k < NT - 2) fe_mul(s, s, MU[k]);   // < 2p
-        fe_sqr(s2, s);
-        fe_mul(s3, s2, s);
-        fe_mul(TX[k], TX[k], s2);
-        fe_mul(TY[k], TY[k], s3);
+        if (k < NT - 2) fq_mul(s, s, MU[k]);   // 12 * 12 -> < 0.8
+        fq_sqr(s2, s);
+        fq_mul(s3, s2, s);
+        fq_mul(TX[k], TX[k], s2);
+        fq_addw(s3, s3, s3);                   // wide
+        fq_mul(TY[k], TY[k], s3);
     }
-    fe zt;
-    fe_mul(zt, Q.z, s);             // the table's common Z < 2p
-    fe beta, beta2;
-    fe_set(beta, FP_BETA);
-    fe_set(beta2, FP_BETA2);
-    g1j acc;
+    fq zt;
+    fq_mul(zt, Q.z, s);             // the table's common Z
+    fq beta, beta2;
+    fq_set(beta, FQ_GLV);
+    fq_set(beta2, FQ_GLV2);
+    g1h acc;
     bool started = false;
 #pragma unroll 1
     for (unsigned k = 0;; k++) {
         const uint32_t op = FK20_UNIFORM(ops[k]);
         const unsigned nd = op & TWOP_DBL_MASK;
 #pragma unroll 1
-        for (unsigned d = 0; d < nd; d++) g1j_dbl(acc, acc);
+        for (unsigned d = 0; d < nd; d++) g1h_dbl(acc, acc);
         if (op & TWOP_END) break;
         const unsigned e = (op >> TWOP_ENTRY_SHIFT) & (NT - 1);
-        fe qx = TX[e], qy = TY[e];
-        if (op & TWOP_PHI2) fe_mul(qx, qx, beta2);
-        else if (op & TWOP_PHI) fe_mul(qx, qx, beta);
-        if (op & TWOP_NEG) fe_neg<4>(qy, qy);
+        fq qx = TX[e], qy = TY[e];
+        if (op & TWOP_PHI2) fq_mul(qx, qx, beta2);
+        else if (op & TWOP_PHI) fq_mul(qx, qx, beta);
+        if (op & TWOP_NEG) fq_neg(qy, qy);
         if (started) {
-            g1j_madd(acc, acc, qx, qy);
+            g1h_madd(acc, acc, qx, qy);
         } else {
             acc.x = qx;
-            acc.y = qy;
-            fe_one(acc.z);
+            acc.h = qy;
+            fq_one(acc.z);
             started = true;
         }
     }
-    // Jacobian with Z = acc.z * zt -> homogeneous (X Z : Y : Z^3)
-    fe z, z2;
-    fe_mul(z, acc.z, zt);
-    fe_sqr(z2, z);
-    fe_mul(x.z, z2, z);
-    fe_mul(x.x, acc.x, z);
-    x.y = acc.y;
-    if (inf) g1_inf(x);
+    // Jacobian with Z = acc.z * zt -> homogeneous (2 X Z : 2 Y : 2 Z^3)
+    fq z, z2;
+    fq_mul(z, acc.z, zt);
+    fq_sqr(z2, z);
+    fq_addw(z, z, z);               // wide
+    fq_mul(x.z, z2, z);
+    fq_mul(x.x, acc.x, z);
+    x.y = acc.h;
+    if (inf) g1q_inf(x);
 }
 
 // x <- [w^384] x = [w^-128] x (w128 = false) or [w^128] x (w128 = true) for x in G1.  With
@@ -132,44 +135,44 @@ FK20_HD void tw_mul(g1p &x, const uint32_t *ops) {
 // the result's X by beta^2.  This replaces a program of two 64-bit halves, its 8-entry table
 // and about 11 additions.  No exceptional case for x in G1 \ {O}: before each addition the
 // accumulator is [m] x with m even, 2 <= m < 2^64, so m -+ 1 is not a multiple of r.
-// x: homogeneous projective, coordinates < 10 p; out: x < 2 p, y < 4 p, z < 2 p.
-FK20_HD void tw_mul_z3(g1p &x, bool w128) {
+// x: homogeneous projective, coordinates < 8 p; out: < 2 p.
+FK20_HD void tw_mul_z3(g1q &x, bool w128) {
     constexpr uint64_t ZABS = 0xd201000000010000ull;
-    fe zc;
-    fe_canonical(zc, x.z);
-    const bool inf = fe_is_zero_canonical(zc);
-    fe px, py;
-    fe_sqr(zc, x.z);                // < 2p
-    fe_mul(px, x.x, x.z);           // Jacobian X = X Z < 2p
-    fe_mul(py, x.y, zc);            // Jacobian Y = Y Z^2 < 2p
-    g1j acc;
+    const bool inf = g1q_is_inf(x);
+    fq px, ph, t;
+    fq_sqr(t, x.z);
+    fq_mul(px, x.x, x.z);           // Jacobian X = X Z
+    fq_mul(ph, x.y, t);             // Jacobian Y = Y Z^2
+    fq_add(ph, ph, ph);
+    g1h acc;
     acc.x = px;
-    acc.y = py;
-    fe_one(acc.z);
+    acc.h = ph;
+    fq_one(acc.z);
 #pragma unroll 1
     for (int b = 62; b >= 0; b--) {
-        g1j_dbl(acc, acc);
-        if ((ZABS >> b) & 1) g1j_madd(acc, acc, px, py);
+        g1h_dbl(acc, acc);
+        if ((ZABS >> b) & 1) g1h_madd(acc, acc, px, ph);
     }
-    // Jacobian with Z = acc.z * x.z -> homogeneous (X Z beta^2 : +-Y : Z^3)
-    fe z, z2, beta2;
-    fe_mul(z, acc.z, x.z);
-    fe_sqr(z2, z);
-    fe_mul(x.z, z2, z);
-    fe_set(beta2, FP_BETA2);
-    fe_mul(z, z, beta2);
-    fe_mul(x.x, acc.x, z);
-    if (w128) fe_neg<4>(x.y, acc.y);
-    else x.y = acc.y;
-    if (inf) g1_inf(x);
+    // Jacobian with Z = acc.z * x.z -> homogeneous (2 X Z beta^2 : +-2 Y : 2 Z^3)
+    fq z, z2, beta2;
+    fq_mul(z, acc.z, x.z);
+    fq_sqr(z2, z);
+    fq_addw(z, z, z);               // wide
+    fq_mul(x.z, z2, z);
+    fq_set(beta2, FQ_GLV2);
+    fq_mul(z, z, beta2);
+    fq_mul(x.x, acc.x, z);
+    if (w128) fq_neg(x.y, acc.h);
+    else x.y = acc.h;
+    if (inf) g1q_inf(x);
 }
 
 // A point held in registers (the host build; the kernel keeps its copies in LDS instead, to
 // leave the registers to the formulas).
 struct RegSlot {
-    g1p v;
-    FK20_HD void put(const g1p &p) { v = p; }
-    FK20_HD void get(g1p &p) const { p = v; }
+    g1q v;
+    FK20_HD void put(const g1q &p) { v = p; }
+    FK20_HD void get(g1q &p) const { p = v; }
 };
 
 // Whether p lies in the order-r subgroup G1 (infinity included): phi^2(p) = (beta^2 x, y)
@@ -179,37 +182,130 @@ struct RegSlot {
 // |z| = 0xd201000000010000 (63 doublings and 5 additions per round), complete formulas.
 // `orig` and `base` hold p and each round's base while the doublings run.
 template <class Slot>
-FK20_HD bool g1_in_subgroup(const g1p &p, Slot &orig, Slot &base) {
+FK20_HD bool g1_in_subgroup(const g1q &p, Slot &orig, Slot &base) {
     constexpr uint64_t ZABS = 0xd201000000010000ull;
     orig.put(p);
-    g1p q = p;
+    g1q q = p;
 #pragma unroll 1
     for (int round = 0; round < 2; round++) {
         base.put(q);
 #pragma unroll 1
         for (int b = 62; b >= 0; b--) {
-            g1_dbl(q, q);
+            g1q_dbl(q, q);
             if ((ZABS >> b) & 1) {
-                g1p t;
+                g1q t;
                 base.get(t);
-                g1_add(q, q, t);
+                g1q_add(q, q, t);
             }
         }
     }
-    g1p f;
+    g1q f;
     orig.get(f);
-    fe beta2;
-    fe_set(beta2, FP_BETA2);
-    fe_mul(f.x, f.x, beta2);
-    g1_add(q, q, f);
-    fe zc;
-    fe_canonical(zc, q.z);
-    return fe_is_zero_canonical(zc);
+    fq beta2;
+    fq_set(beta2, FQ_GLV2);
+    fq_mul(f.x, f.x, beta2);
+    g1q_add(q, q, f);
+    return g1q_is_inf(q);
+}
+
+// ---------------------------------------------------------------- points over fp.hip.h
+//
+// The same operations on points in the unsigned Fp form, by conversion: the element-wise entry
+// points and the CPU tests use that form.
+
+FK20_HD void fq_from_fe(fq &z, const fe &a) {
+    fe t, c;
+    fe_set(c, FQ_FROM_FP);
+    fe_mul(t, a, c);
+    uint32_t w[12];
+    fe_pack(w, t);
+    fq_unpack_raw(z, w);
+}
+
+FK20_HD void fe_from_fq(fe &z, const fq &a) {  // |a| < 4 p
+    uint32_t w[12];
+    fq_pack(w, a);
+    fe t, c;
+    fe_unpack(t, w);
+    fe_set(c, FP_FROM_FQ);
+    fe_mul(z, t, c);
+}
+
+FK20_HD void g1q_from_g1p(g1q &r, const g1p &p) {
+    fq_from_fe(r.x, p.x);
+    fq_from_fe(r.y, p.y);
+    fq_from_fe(r.z, p.z);
+}
+
+FK20_HD void g1p_from_g1q(g1p &r, const g1q &p) {
+    fe_from_fq(r.x, p.x);
+    fe_from_fq(r.y, p.y);
+    fe_from_fq(r.z, p.z);
+}
+
+template <int W>
+FK20_HD void tw_mul(g1p &x, const uint32_t *ops) {
+    g1q q;
+    g1q_from_g1p(q, x);
+    tw_mul<W>(q, ops);
+    g1p_from_g1q(x, q);
+}
+
+FK20_HD void tw_mul_z3(g1p &x, bool w128) {
+    g1q q;
+    g1q_from_g1p(q, x);
+    tw_mul_z3(q, w128);
+    g1p_from_g1q(x, q);
 }
 
 FK20_HD bool g1_in_subgroup(const g1p &p) {
     RegSlot orig, base;
-    return g1_in_subgroup(p, orig, base);
+    g1q q;
+    g1q_from_g1p(q, p);
+    return g1_in_subgroup(q, orig, base);
+}
+
+// Jacobian (X, Y, Z) with the plain Y; results as the representative (4 X, 8 Y, 2 Z).
+struct g1j {
+    fe x, y, z;
+};
+
+FK20_HD void g1h_from_g1j(g1h &r, const g1j &p) {
+    fq_from_fe(r.x, p.x);
+    fq_from_fe(r.h, p.y);
+    fq_add(r.h, r.h, r.h);
+    fq_from_fe(r.z, p.z);
+}
+
+FK20_HD void g1j_from_g1h(g1j &r, const g1h &p) {
+    fq one;
+    fq_one(one);
+    fq t;
+    fq_mul(t, p.x, one);
+    fe_from_fq(r.x, t);
+    fe_mul_small<4>(r.x, r.x);
+    fe_from_fq(r.y, p.h);
+    fe_mul_small<4>(r.y, r.y);
+    fe_from_fq(r.z, p.z);
+    fe_mul_small<2>(r.z, r.z);
+}
+
+FK20_HD void g1j_dbl(g1j &r, const g1j &p) {
+    g1h t;
+    g1h_from_g1j(t, p);
+    g1h_dbl(t, t);
+    g1j_from_g1h(r, t);
+}
+
+FK20_HD void g1j_madd(g1j &r, const g1j &p, const fe &x2, const fe &y2) {
+    g1h t;
+    fq x, h;
+    g1h_from_g1j(t, p);
+    fq_from_fe(x, x2);
+    fq_from_fe(h, y2);
+    fq_add(h, h, h);
+    g1h_madd(t, t, x, h);
+    g1j_from_g1h(r, t);
 }
 
 }  // namespace fk20

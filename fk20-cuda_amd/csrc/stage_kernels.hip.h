@@ -20,17 +20,17 @@ namespace fk20 {
 // of w^-e for TW_INV): w^+-128 by tw_mul_z3, w^256 = -1 by a negation, any other exponent by
 // its program.  The exponent is wave-uniform, so is the branch.
 template <int W>
-__device__ __forceinline__ void twiddle(g1p &x, const uint32_t *ops, const uint32_t *index, unsigned dir,
+__device__ __forceinline__ void twiddle(g1q &x, const uint32_t *ops, const uint32_t *index, unsigned dir,
                                         unsigned e) {
     const unsigned E = (dir == TW_FWD ? e : 512u - e) & 511u;  // x <- w^E x
     if (E == 128 || E == 384) tw_mul_z3(x, E == 128);
-    else if (E == 256) fe_neg<4>(x.y, x.y);  // stored points have y < 4p
+    else if (E == 256) fq_neg(x.y, x.y);
     else if (E) tw_mul<W>(x, ops + index[dir * 512 + e]);
 }
 
 // The butterflies' twiddle: in the radix-2^2 schedule always w^+-128 (idx 128), else any.
 template <int W, bool R22>
-__device__ __forceinline__ void bf_twiddle(g1p &x, const uint32_t *ops, const uint32_t *index, unsigned dir,
+__device__ __forceinline__ void bf_twiddle(g1q &x, const uint32_t *ops, const uint32_t *index, unsigned dir,
                                            unsigned idx) {
     if constexpr (R22) tw_mul_z3(x, dir == TW_FWD);
     else twiddle<W>(x, ops, index, dir, idx);
@@ -40,14 +40,14 @@ __device__ __forceinline__ void bf_twiddle(g1p &x, const uint32_t *ops, const ui
 template <int W, bool R22>
 __device__ __forceinline__ void dit_butterfly(uint32_t *D, unsigned rows, unsigned row, const Butterfly &f,
                                               const uint32_t *ops, const uint32_t *index) {
-    g1p x, y, a;
+    g1q x, y, a;
     pt_load(x, D + ((size_t)f.p1 * rows + row) * 36);
     if (f.idx) bf_twiddle<W, R22>(x, ops, index, TW_INV, f.idx);
     pt_load(y, D + ((size_t)f.p0 * rows + row) * 36);
-    g1_add(a, y, x);
+    g1q_add(a, y, x);
     pt_store(D + ((size_t)f.p0 * rows + row) * 36, a);  // stored first: not live in the next add
-    g1_neg(x, x);
-    g1_add(x, y, x);
+    g1q_neg(x, x);
+    g1q_add(x, y, x);
     pt_store(D + ((size_t)f.p1 * rows + row) * 36, x);
 }
 
@@ -56,11 +56,11 @@ __device__ __forceinline__ void dit_butterfly(uint32_t *D, unsigned rows, unsign
 template <int W, bool R22>
 __device__ __forceinline__ void middle_butterfly(uint32_t *D, unsigned rows, unsigned row, const Butterfly &f,
                                                  const uint32_t *ops, const uint32_t *index) {
-    g1p o, e;
+    g1q o, e;
     pt_load(o, D + ((size_t)f.p1 * rows + row) * 36);
     if (f.idx) bf_twiddle<W, R22>(o, ops, index, TW_INV, f.idx);
     pt_load(e, D + ((size_t)f.p0 * rows + row) * 36);
-    g1_add(e, e, o);
+    g1q_add(e, e, o);
     pt_store(D + ((size_t)f.p0 * rows + row) * 36, e);
     if (f.idx) bf_twiddle<W, R22>(e, ops, index, TW_FWD, f.idx);
     pt_store(D + ((size_t)f.p1 * rows + row) * 36, e);
@@ -73,13 +73,13 @@ __device__ __forceinline__ void middle_butterfly(uint32_t *D, unsigned rows, uns
 template <int W, bool R22>
 __device__ __forceinline__ void dif_butterfly(uint32_t *D, unsigned rows, unsigned row, const Butterfly &f,
                                               const uint32_t *ops, const uint32_t *index) {
-    g1p u, v, a;
+    g1q u, v, a;
     pt_load(u, D + ((size_t)f.p0 * rows + row) * 36);
     pt_load(v, D + ((size_t)f.p1 * rows + row) * 36);
-    g1_add(a, u, v);
+    g1q_add(a, u, v);
     pt_store(D + ((size_t)f.p0 * rows + row) * 36, a);  // stored first: not live across tw_mul
-    g1_neg(v, v);
-    g1_add(v, u, v);
+    g1q_neg(v, v);
+    g1q_add(v, u, v);
     if (!R22 && f.idx) bf_twiddle<W, R22>(v, ops, index, TW_FWD, f.idx);
     pt_store(D + ((size_t)f.p1 * rows + row) * 36, v);
 }
@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(64, OCC) k_twiddle_multi(Launch L, const uint3
     const unsigned row = min((local % rg) * 64 + threadIdx.x, it.rows - 1);
     const uint32_t item = index[TW_LAYER + layer_table_offset(it.logn2, (unsigned)it.stage, dir) + local / rg];
     uint32_t *p = it.D + ((size_t)(item & 0xffffu) * it.rows + row) * 36;
-    g1p x;
+    g1q x;
     pt_load(x, p);
     twiddle<W>(x, ops, index, dir, item >> 16);
     pt_store(p, x);
@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(64, OCC) k_quarter_multi(Launch L) {
     const unsigned b = (1u << (it.logn2 - 2)) + local / rg;
     const Butterfly f = stage_positions<true>(it.logn2 - 1 + (unsigned)it.stage, it.logn2, b);
     uint32_t *p = it.D + ((size_t)f.p1 * it.rows + row) * 36;
-    g1p x;
+    g1q x;
     pt_load(x, p);
     tw_mul_z3(x, true);
     pt_store(p, x);
@@ -233,8 +233,8 @@ __global__ void __launch_bounds__(64, OCC) k_plain_load(uint32_t *D, const uint3
     const unsigned row = min((blockIdx.x % rg) * 64 + threadIdx.x, rows - 1);  // spare lanes repeat the last row
     uint32_t w[36];
     ld_words(w, in + ((size_t)row * (1u << logn) + j) * G1P_WORDS, 9);
-    g1p p;
-    g1_load_std(p, w);
+    g1q p;
+    g1q_load_std(p, w);
     if (scale_ops) tw_mul<W>(p, scale_ops);
     pt_store(D + ((size_t)(brev ? bitrev(j, logn) : j) * rows + row) * 36, p);
 }
