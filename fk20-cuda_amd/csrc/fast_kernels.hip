@@ -343,15 +343,27 @@ __global__ void __launch_bounds__(256) k_toeplitz_fft_multi(Launch L, const DevT
 
 // ---------------------------------------------------------------- window-table MSM
 
-// acc += k * B for a standard-form scalar k < r (8 words, consumed) by signed fixed windows
-// of WIN bits over B's table tb[win][d - 1] = d * 2^(WIN*win) * B (affine): one mixed
-// addition per non-zero digit, no doublings.  k < r < 2^255 keeps the last window's carry
-// inside the ceil(256/WIN) windows for every WIN in 8..13.
-__device__ __forceinline__ void window_term(g1q &acc, uint32_t *k, const uint32_t *tb, unsigned WIN) {
-    const unsigned NWIN = (256 + WIN - 1) / WIN, H = 1u << (WIN - 1), MASK = (1u << WIN) - 1;
-    uint32_t carry = 0;
-#pragma unroll 1
-    for (unsigned win = 0; win < NWIN; win++) {
+// A standard-form scalar k < r as signed fixed windows of WIN bits over a base's table
+// tb[win][d - 1] = d * 2^(WIN*win) * B (affine): one mixed addition per non-zero digit, no
+// doublings.  k < r < 2^255 keeps the last window's carry inside the ceil(256/WIN) windows for
+// every WIN in 8..13.
+//
+// The entry of the next window is fetched while the current one is added: a gathered entry is a
+// 128-byte line somewhere in gigabytes of tables, several microseconds away under load, and at
+// two waves per SIMD (the addition's registers) nothing else covers it.
+struct WindowStream {
+    const uint32_t *tb;
+    uint32_t k[8];
+    uint32_t carry;
+    unsigned win;
+    __device__ void start(const uint32_t *table) {
+        tb = table;
+        carry = 0;
+        win = 0;
+    }
+    // the next digit; fetches its entry (the first one for digit 0)
+    __device__ int next(uint32_t *ent, unsigned WIN) {
+        const unsigned H = 1u << (WIN - 1), MASK = (1u << WIN) - 1;
         const uint32_t bits = (k[0] & MASK) + carry;
         carry = bits > H ? 1u : 0u;
         const int d = (int)bits - (int)(carry << WIN);
@@ -359,15 +371,42 @@ __device__ __forceinline__ void window_term(g1q &acc, uint32_t *k, const uint32_
 #pragma unroll
         for (int q = 0; q < 7; q++) k[q] = (k[q] >> WIN) | (k[q + 1] << (32 - WIN));
         k[7] >>= WIN;
-        if (d != 0) {
-            const unsigned e = (unsigned)(d < 0 ? -d : d) - 1;
-            const uint32_t *ent = tb + ((size_t)win * H + e) * TABLE_ENTRY_WORDS;
-            fq x, y;
-            fq_load_raw(x, ent);
-            fq_load_raw(y, ent + 12);
-            if (d < 0) fq_neg(y, y);
-            g1q_add_aff(acc, acc, x, y);
+        const unsigned e = (unsigned)(d < 0 ? -d : d);
+        ld_words(ent, tb + ((size_t)win * H + (e ? e - 1 : 0)) * TABLE_ENTRY_WORDS, 6);
+        win++;
+        return d;
+    }
+};
+
+// acc += sum of the scalars that `fetch(t, k)` gives (t = 0 .. nterms - 1, false: skip the term)
+// times their bases, term t's table at tables + t * stride words.
+template <class Fetch>
+__device__ __forceinline__ void window_sum(g1q &acc, const uint32_t *tables, size_t stride, unsigned nterms,
+                                           unsigned WIN, const Fetch &fetch) {
+    const unsigned NWIN = (256 + WIN - 1) / WIN;
+    unsigned t = 0;
+    WindowStream w;
+    while (t < nterms && !fetch(t, w.k)) t++;
+    if (t == nterms) return;
+    w.start(tables + t * stride);
+    uint32_t ent[24];
+    int d = w.next(ent, WIN);
+#pragma unroll 1
+    while (true) {
+        fq x, y;
+        fq_unpack_raw(x, ent);
+        fq_unpack_raw(y, ent + 12);
+        if (d < 0) fq_neg(y, y);
+        const bool add = d != 0;
+        if (w.win == NWIN) {
+            t++;
+            while (t < nterms && !fetch(t, w.k)) t++;
+            if (t < nterms) w.start(tables + t * stride);
         }
+        const bool more = t < nterms;
+        if (more) d = w.next(ent, WIN);
+        if (add) g1q_add_aff(acc, acc, x, y);
+        if (!more) break;
     }
 }
 
@@ -382,14 +421,13 @@ __global__ void __launch_bounds__(64) k_msm_multi(Launch L) {
     const unsigned row = min((local % rg) * 64 + threadIdx.x, rows - 1);  // spare lanes repeat the last row
     g1q acc;
     g1q_inf(acc);
-#pragma unroll 1
-    for (unsigned i = 0; i < 16; i++) {
-        const unsigned b = i * n2 + j;
-        if (it.inf[b]) continue;
-        uint32_t k[8];
-        ld_words(k, it.tcT + (((size_t)j * 16 + i) * rows + row) * FR_WORDS, 2);
-        window_term(acc, k, it.table + (size_t)b * NWIN * H * TABLE_ENTRY_WORDS, WIN);
-    }
+    const size_t per_base = (size_t)NWIN * H * TABLE_ENTRY_WORDS;
+    const uint32_t *tc = it.tcT + ((size_t)j * 16 * rows + row) * FR_WORDS, *inf = it.inf + j;
+    window_sum(acc, it.table + j * per_base, n2 * per_base, 16, WIN, [&](unsigned i, uint32_t *k) {
+        if (inf[i * n2]) return false;
+        ld_words(k, tc + (size_t)i * rows * FR_WORDS, 2);
+        return true;
+    });
     pt_store(it.D + ((size_t)bitrev(j, it.logn2) * rows + row) * 36, acc);
 }
 
@@ -410,11 +448,13 @@ __global__ void __launch_bounds__(64) k_msm_multi_small(Launch L) {
     const unsigned b = i * n2 + j;
     g1q acc;
     g1q_inf(acc);
-    if (!it.inf[b]) {
-        uint32_t k[8];
-        ld_words(k, it.tcT + (((size_t)j * 16 + i) * rows + row) * FR_WORDS, 2);
-        window_term(acc, k, it.table + (size_t)b * NWIN * H * TABLE_ENTRY_WORDS, WIN);
-    }
+    const uint32_t *tc = it.tcT + (((size_t)j * 16 + i) * rows + row) * FR_WORDS;
+    const bool skip = it.inf[b] != 0;
+    window_sum(acc, it.table + (size_t)b * NWIN * H * TABLE_ENTRY_WORDS, 0, 1, WIN, [&](unsigned, uint32_t *k) {
+        if (skip) return false;
+        ld_words(k, tc, 2);
+        return true;
+    });
     pt_store(lds + t * 36, acc);
 #pragma unroll 1
     for (unsigned h = 8; h >= 1; h /= 2) {
@@ -446,17 +486,20 @@ __global__ void __launch_bounds__(64) k_commit_partial(const uint32_t *poly, con
     const unsigned i0 = c * chunk, i1 = min(i0 + chunk, N);
     g1q acc;
     g1q_inf(acc);
-#pragma unroll 1
-    for (unsigned i = i0; i < i1; i++) {
-        if (inf[i]) continue;
+    const size_t per_base = (size_t)NWIN * H * TABLE_ENTRY_WORDS;
+    const uint32_t *coeff = poly + ((size_t)row * N + i0) * FR_WORDS;
+    window_sum(acc, table + i0 * per_base, per_base, i1 - i0, win_bits, [&](unsigned t, uint32_t *k) {
+        if (inf[i0 + t]) return false;
         // the caller's coefficient may be any 256-bit representative: reduce it below r, so
         // the top signed window's carry stays inside the ceil(256/w) windows (at w = 8 the
         // windows end exactly at bit 256, and a value >= 2^255 would carry out of them)
-        fs k;
-        ld_words(k.l, poly + ((size_t)row * N + i) * FR_WORDS, 2);
-        fs_reduce_std(k);
-        window_term(acc, k.l, table + (size_t)i * NWIN * H * TABLE_ENTRY_WORDS, win_bits);
-    }
+        fs c;
+        ld_words(c.l, coeff + (size_t)t * FR_WORDS, 2);
+        fs_reduce_std(c);
+#pragma unroll
+        for (int q = 0; q < 8; q++) k[q] = c.l[q];
+        return true;
+    });
     pt_store(partial + ((size_t)c * rows + row) * 36, acc);
 }
 
