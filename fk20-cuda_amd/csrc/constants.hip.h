@@ -32,6 +32,7 @@ static constexpr int64_t FQ_K0 = 6969937068335403541ll;
 static constexpr int32_t FQ_BETA[13] = {550457077, 529115271, 538425416, 540408362, 534947505, 530527195, 527739787, 553457329, 541486612, 537384151, 545225655, 547666669, 37975};  // digit offsets of a product
 static constexpr int32_t FQ_ONE[13] = {13762350, 433586176, -192935228, -301937177, 37952645, -425753694, -36732706, 162803105, -437337492, 366579475, 78814996, -442511456, 89578};  // R mod p
 static constexpr int32_t FQ_R2[13] = {84958308, 320669453, -336452545, -23350980, 68258640, -130586467, 277172093, -144228653, 171105485, -419190883, -282802362, -41659541, -694179};  // R^2 mod p
+static constexpr int32_t FQ_R3[13] = {323471757, -333343540, 453147883, -343099995, 303348703, 190774532, -101855041, 455817637, -223343770, 488336821, -74511473, 315118520, 446639};  // R^3 mod p
 static constexpr int32_t FQ_GLV[13] = {479228289, -54664058, -430486465, -215714323, 473873436, -101816220, 385853527, -332097025, 89177367, 348892208, 399608966, -514237961, 640725};  // beta of the endomorphism (Montgomery)
 static constexpr int32_t FQ_GLV2[13] = {-492990639, -378922118, -450320131, 517651501, -511826081, 527569914, -349120821, 169293920, 348160125, 358270141, -478423963, -116992407, -730302};  // beta^2
 static constexpr int32_t FQ_4P[13] = {1073654444, 535822335, 352321518, 738197169, 64524410, 220860267, 78633420, 193262469, 861770205, 996422842, 647153385, 708411366, 6816839};  // 4 p, non-negative digits

@@ -322,22 +322,6 @@ FK20_HD void fq_unpack_raw(fq &z, const uint32_t *w) {
 
 // ---------------------------------------------------------------- conversions
 
-// Inverse by Fermat (a^(p-2)); 0 gives 0.  Montgomery in and out.
-FK20_HD void fq_inv(fq &z, const fq &a) {
-    fq acc, base = a;
-    fq_one(acc);
-#pragma unroll 1
-    for (int w = 11; w >= 0; w--) {
-        const uint32_t e = FP_PM2[w];
-#pragma unroll 1
-        for (int b = 31; b >= 0; b--) {
-            fq_sqr(acc, acc);
-            if ((e >> b) & 1) fq_mul(acc, acc, base);
-        }
-    }
-    z = acc;
-}
-
 // |a| < p -> non-negative digits of a mod p in [0, p)
 FK20_HD void fq_canon_digits(fq &z, const fq &a) {
     fq t, u;
@@ -389,6 +373,109 @@ FK20_HD bool fq_is_zero(const fq &a) {
 #pragma unroll
     for (int i = 0; i < FQ_N; i++) acc |= (uint32_t)t.l[i];
     return acc == 0;
+}
+
+// ---------------------------------------------------------------- inversion
+//
+// 1 / a by divsteps (Bernstein and Yang, "Fast constant-time gcd computation and modular
+// inversion", TCHES 2019), 30 of them per pass over the digits, starting from delta = 1/2.  A
+// division step needs only the low bits of f and g, so a pass runs 30 on one word of each with
+// 32-bit adds and masks (the instructions that issue at twice the rate of a multiply-add),
+// collects them in a 2 x 2 matrix and applies it to f, g and to the cofactors d, e (whose
+// division by 2^30 mod p takes one quotient digit).  |d|, |e| grow by at most p / 2 a pass,
+// which the digits hold without reduction.  About 30 passes of 900 instructions, the lanes of a
+// wave together until the last is done, against 610 products by Fermat's theorem: 262 144
+// affine points in 0.24 ms instead of 1.35, 512 in 0.066 instead of 0.47.
+
+#ifdef __HIP_DEVICE_COMPILE__
+#define FQ_ANY(x) __any(x)
+#else
+#define FQ_ANY(x) (x)
+#endif
+
+// 30 division steps on the low words: 2^30 (f', g') = (u f + v g, q f + r g).  D = 2 delta.
+struct fq_divsteps {
+    int32_t u, v, q, r;
+    FK20_HD void run(int32_t &D, uint32_t f, uint32_t g) {
+        u = 1, v = 0, q = 0, r = 1;
+#pragma unroll 6
+        for (int i = 0; i < 30; i++) {
+            const int32_t odd = -(int32_t)(g & 1);
+            int32_t pos = (-D) >> 31;  // delta > 0: subtract f (and swap if g is odd), else add
+            g += (((uint32_t)f ^ (uint32_t)pos) - (uint32_t)pos) & (uint32_t)odd;
+            q += ((u ^ pos) - pos) & odd;
+            r += ((v ^ pos) - pos) & odd;
+            pos &= odd;
+            D = (D ^ pos) - pos + 2;
+            f += g & (uint32_t)pos;
+            u += q & pos;
+            v += r & pos;
+            g >>= 1;
+            u = (int32_t)((uint32_t)u << 1);
+            v = (int32_t)((uint32_t)v << 1);
+        }
+    }
+};
+
+// Inverse of a Montgomery value (balanced, |a| < 200 p), Montgomery; 0 gives 0.
+FK20_HD void fq_inv(fq &z, const fq &a) {
+    // non-negative 30-bit digits below a signed top digit
+    fq f, g, d, e;
+    fq_one(e);
+    fq_mul(g, a, e);
+    fq_canon_digits(g, g);
+    fq_set(f, FQ_P);
+    fq_ripple(f, f);
+    fq_zero(d);
+    fq_zero(e);
+    e.l[0] = 1;
+    int32_t D = 1;
+    // 381-bit values are done after at most 37 passes (1102 steps); the bound only ends the loop
+#pragma unroll 1
+    for (int pass = 0; pass < 40; pass++) {
+        uint32_t nz = 0;
+#pragma unroll
+        for (int i = 0; i < FQ_N; i++) nz |= (uint32_t)g.l[i];
+        if (!FQ_ANY(nz != 0)) break;
+        fq_divsteps t;
+        t.run(D, (uint32_t)f.l[0] | (uint32_t)f.l[1] << 30, (uint32_t)g.l[0] | (uint32_t)g.l[1] << 30);
+        int64_t cf = (int64_t)t.u * f.l[0] + (int64_t)t.v * g.l[0];
+        int64_t cg = (int64_t)t.q * f.l[0] + (int64_t)t.r * g.l[0];
+        int64_t cd = (int64_t)t.u * d.l[0] + (int64_t)t.v * e.l[0];
+        int64_t ce = (int64_t)t.q * d.l[0] + (int64_t)t.r * e.l[0];
+        const int32_t md = (int32_t)((uint32_t)cd * FQ_PINV4) >> 2, me = (int32_t)((uint32_t)ce * FQ_PINV4) >> 2;
+        cd += (int64_t)md * FQ_P[0];
+        ce += (int64_t)me * FQ_P[0];
+        cf >>= 30, cg >>= 30, cd >>= 30, ce >>= 30;
+#pragma unroll
+        for (int i = 1; i < FQ_N; i++) {
+            const int32_t fi = f.l[i], gi = g.l[i], di = d.l[i], ei = e.l[i];
+            cf += (int64_t)t.u * fi + (int64_t)t.v * gi;
+            cg += (int64_t)t.q * fi + (int64_t)t.r * gi;
+            cd += (int64_t)t.u * di + (int64_t)t.v * ei + (int64_t)md * FQ_P[i];
+            ce += (int64_t)t.q * di + (int64_t)t.r * ei + (int64_t)me * FQ_P[i];
+            f.l[i - 1] = (int32_t)((uint32_t)cf & FQ_MASK);
+            g.l[i - 1] = (int32_t)((uint32_t)cg & FQ_MASK);
+            d.l[i - 1] = (int32_t)((uint32_t)cd & FQ_MASK);
+            e.l[i - 1] = (int32_t)((uint32_t)ce & FQ_MASK);
+            FQ_OPAQUE_V(f.l[i - 1]);
+            FQ_OPAQUE_V(g.l[i - 1]);
+            FQ_OPAQUE_V(d.l[i - 1]);
+            FQ_OPAQUE_V(e.l[i - 1]);
+            cf >>= 30, cg >>= 30, cd >>= 30, ce >>= 30;
+        }
+        f.l[FQ_N - 1] = (int32_t)cf;
+        g.l[FQ_N - 1] = (int32_t)cg;
+        d.l[FQ_N - 1] = (int32_t)cd;
+        e.l[FQ_N - 1] = (int32_t)ce;
+    }
+    // f = +-1 (or p for a = 0, where d = 0): 1 / (x R) = f d, times R^3 / R
+    const int32_t s = f.l[FQ_N - 1] >> 31;
+    fq_norm(d, d);
+#pragma unroll
+    for (int i = 0; i < FQ_N; i++) d.l[i] = (d.l[i] ^ s) - s;
+    fq_set(e, FQ_R3);
+    fq_mul(z, d, e);
 }
 
 }  // namespace fk20

@@ -65,7 +65,7 @@ __global__ void k_hext2h(uint32_t *h, unsigned rows, unsigned n2) {
 }
 
 // Standard-form points -> packed Montgomery points (internal operand form).
-__global__ void k_std_to_packed(uint32_t *packed, const uint32_t *pts, size_t count) {
+__global__ void __launch_bounds__(64) k_std_to_packed(uint32_t *packed, const uint32_t *pts, size_t count) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= count) return;
     g1q p;
@@ -349,7 +349,7 @@ __global__ void k_setup_gather(uint32_t *xext, const uint32_t *srs, unsigned N) 
 }
 
 // Canonical affine (x, y); infinity -> (0, 0) as g1a_fromG1p (g1a.cu:48-56) gives.
-__global__ void k_to_affine(uint32_t *out, const uint32_t *in, size_t count) {
+__global__ void __launch_bounds__(64) k_to_affine(uint32_t *out, const uint32_t *in, size_t count) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= count) return;
     g1q p;
@@ -365,7 +365,7 @@ __global__ void k_to_affine(uint32_t *out, const uint32_t *in, size_t count) {
     for (int i = 0; i < 6; i++) q[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
 }
 
-__global__ void k_compress(uint32_t *out, const uint32_t *in, size_t count) {
+__global__ void __launch_bounds__(64) k_compress(uint32_t *out, const uint32_t *in, size_t count) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= count) return;
     g1q p;

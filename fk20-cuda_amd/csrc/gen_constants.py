@@ -84,7 +84,8 @@ def fq_constants():
            "static constexpr int64_t FQ_K0 = %dll;" % FQ_K0,
            iarr("FQ_BETA", FQ_BETA) + "  // digit offsets of a product",
            iarr("FQ_ONE", balanced(centred(R))) + "  // R mod p",
-           iarr("FQ_R2", balanced(centred(R * R))) + "  // R^2 mod p"]
+           iarr("FQ_R2", balanced(centred(R * R))) + "  // R^2 mod p",
+           iarr("FQ_R3", balanced(centred(R * R * R))) + "  // R^3 mod p"]
     beta = 0x1A0111EA397FE699EC02408663D4DE85AA0D857D89759AD4897D29650FB85F9B409427EB4F49FFFD8BFD00000000AAAC
     out += [iarr("FQ_GLV", balanced(centred(beta * R))) + "  // beta of the endomorphism (Montgomery)",
             iarr("FQ_GLV2", balanced(centred(beta * beta * R))) + "  // beta^2",

@@ -137,9 +137,18 @@ def test_forms_round_trip(L):
             assert val(u) == val(d) and all(abs(int(x)) <= (1 << 29) + 1 for x in u[:12])
             L.fq_host_to_std(ptr(w), ptr(d))
             assert unwords(w) == v % P
-    for v in [0, 1, P - 1] + [int.from_bytes(rng.bytes(48), "little") % P for _ in range(40)]:
-        z = raw(L, 11, digits(v * 2**390 % P))
+
+
+def test_inverse(L):
+    """Zero, units, values with long runs of equal bits (long and short division chains), and
+    random ones, as any representative a product can leave."""
+    rng = np.random.default_rng(104)
+    vals = [0, 1, 2, 3, P - 1, P - 2, (P + 1) // 2, 2**380, 2**380 - 1, 2**190, P >> 1, 0x30003]
+    vals += [pow(2, k, P) for k in range(1, 781, 30)] + [int.from_bytes(rng.bytes(48), "little") % P for _ in range(400)]
+    for n, v in enumerate(vals):
+        z = raw(L, 11, digits(v * 2**390 % P + (n % 5 - 2) * P))
         assert val(z) % P == pow(v, P - 2, P) * 2**390 % P
+        assert abs(val(z)) < 0.6 * P and all(abs(int(x)) <= BAL for x in z[:12])
 
 
 def test_points_against_oracle(L):
