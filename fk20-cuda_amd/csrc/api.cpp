@@ -24,6 +24,8 @@ static __device__ DevTables g_tables_dev;
 static constexpr size_t PROG_OPS_CAP = (size_t)1 << 16;  // words; the programs take about 48 K
 static __device__ uint32_t g_prog_ops[PROG_OPS_CAP];
 static __device__ uint32_t g_prog_index[TW_INDEX_SIZE];
+static constexpr size_t DIRECT_WORDS_CAP = (size_t)1 << 19;  // the plans take 498 822
+static __device__ uint32_t g_direct_words[DIRECT_WORDS_CAP];
 
 // Workspace of fk20_poly2h_fft_noalloc, the entry point for callers that cannot allocate:
 // a fixed array per device, held until the process ends.  Host code uses only the address
@@ -62,6 +64,7 @@ struct DeviceState {
     void *scratch = nullptr;                // workspace of the drop-in entry points
     size_t scratch_bytes = 0;
     unsigned char *noalloc = nullptr;       // this device's address of `scratch`
+    DirectPlan direct;                      // plans of the direct schedule (g_direct_words)
 };
 
 std::mutex g_mu;
@@ -157,6 +160,15 @@ int device_state(DeviceState **out) {
         FK20_TRY(load_programs(st.prog, reinterpret_cast<uint32_t *>(ops), PROG_OPS_CAP,
                                reinterpret_cast<uint32_t *>(index)));
     }
+    if (!st.direct.words) {
+        const std::vector<uint32_t> &words = direct_plan_words();
+        if (words.empty() || words.size() > DIRECT_WORDS_CAP) return hip_status(hipErrorInvalidValue);
+        void *d = nullptr;
+        FK20_TRY(hipGetSymbolAddress(&d, HIP_SYMBOL(g_direct_words)));
+        FK20_TRY(hipMemcpy(d, words.data(), words.size() * 4, hipMemcpyHostToDevice));
+        st.direct.words = reinterpret_cast<const uint32_t *>(d);
+        st.direct.rec = reinterpret_cast<const DirectStep *>(words.data());
+    }
     *out = &st;
     return FK20_OK;
 }
@@ -194,6 +206,16 @@ const DevTables *current_device_tables(hipError_t *err) {
         return nullptr;
     }
     return st->tables;
+}
+
+DirectPlan current_direct_plan(hipError_t *err) {
+    DeviceState *st;
+    *err = hipSuccess;
+    if (device_state(&st) != FK20_OK) {
+        *err = (hipError_t)(g_last_hip_error ? g_last_hip_error : (int)hipErrorUnknown);
+        return DirectPlan();
+    }
+    return st->direct;
 }
 }  // namespace fk20
 
@@ -248,6 +270,13 @@ int fr_ift(fk20_fr_t *output, const fk20_fr_t *input, unsigned count, unsigned n
     return fr_transform(output, input, count, n, true, stream);
 }
 
+// Scratch of the drop-in transforms besides the points: one flag per row, padded, and the direct
+// schedule's products when the batch is small enough for it.
+static size_t flag_bytes(unsigned rows) { return ((size_t)rows * 4 + 255) & ~(size_t)255; }
+static size_t transform_product_bytes(const DeviceState *st, unsigned rows, unsigned logn) {
+    return rows <= DIRECT_MAX_ROWS ? direct_product_bytes(st->direct, rows, logn, 2) : 0;
+}
+
 // The G1 transforms run column-batched (lanes = transforms) through D in scratch, so the
 // output may alias the input as in the reference (g1p_fft.cu:17).
 static int g1_transform(fk20_g1p_t *out, const fk20_g1p_t *in, unsigned count, unsigned n, bool inv,
@@ -258,13 +287,14 @@ static int g1_transform(fk20_g1p_t *out, const fk20_g1p_t *in, unsigned count, u
     int rc = device_state(&st);
     if (rc) return rc;
     void *D;
-    const size_t d_bytes = (size_t)count * n * 144;
-    rc = device_scratch(st, d_bytes + (size_t)count * 4, &D);
+    const size_t d_bytes = (size_t)count * n * 144, f_bytes = flag_bytes(count);
+    const size_t p_bytes = transform_product_bytes(st, count, log2u(n));
+    rc = device_scratch(st, d_bytes + f_bytes + p_bytes, &D);
     if (rc) return rc;
-    uint32_t *flags = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(D) + d_bytes);
+    char *base = reinterpret_cast<char *>(D);
     return hip_status(launch_plain(inv ? PLAIN_G1_IFT : PLAIN_G1_FFT, W(out), W(in), nullptr, count, log2u(n),
-                                   reinterpret_cast<uint32_t *>(D), nullptr, nullptr, flags, st->tables, st->prog,
-                                   S(stream)));
+                                   W(base), nullptr, nullptr, W(base + d_bytes), st->tables, st->prog, S(stream),
+                                   st->direct, W(base + d_bytes + f_bytes), p_bytes));
 }
 
 int g1p_fft(fk20_g1p_t *output, const fk20_g1p_t *input, unsigned count, unsigned n, fk20_stream_t stream) {
@@ -308,20 +338,22 @@ int fk20_hext_fft2h_fft(fk20_g1p_t *h_fft, const fk20_g1p_t *hext_fft, unsigned 
     int rc = device_state(&st);
     if (rc) return rc;
     void *D;
-    const size_t d_bytes = (size_t)rows * n2 * 144;
-    rc = device_scratch(st, d_bytes + (size_t)rows * 4, &D);
+    const size_t d_bytes = (size_t)rows * n2 * 144, f_bytes = flag_bytes(rows);
+    const size_t p_bytes = transform_product_bytes(st, rows, log2u(n2));
+    rc = device_scratch(st, d_bytes + f_bytes + p_bytes, &D);
     if (rc) return rc;
-    uint32_t *flags = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(D) + d_bytes);
-    return hip_status(launch_plain(PLAIN_HEXT_FFT2H_FFT, W(h_fft), W(hext_fft), nullptr, rows, log2u(n2),
-                                   reinterpret_cast<uint32_t *>(D), nullptr, nullptr, flags, st->tables, st->prog,
-                                   S(stream)));
+    char *base = reinterpret_cast<char *>(D);
+    return hip_status(launch_plain(PLAIN_HEXT_FFT2H_FFT, W(h_fft), W(hext_fft), nullptr, rows, log2u(n2), W(base),
+                                   nullptr, nullptr, W(base + d_bytes), st->tables, st->prog, S(stream), st->direct,
+                                   W(base + d_bytes + f_bytes), p_bytes));
 }
 
 // fk20_poly2h_fft.cu:47-80: toeplitz -> NTT (16 per row) -> MSM -> IFFT -> zero -> FFT, with
 // the 1/n2 of the IFFT moved onto the NTT output (a field multiplication instead of a
 // scalar multiplication per point) and the transforms column-batched over the rows.
-// Workspace: tcT, D, the packed bases, the subgroup flag of the bases (one 256-byte slot)
-// and the MSM digits, in that order.
+// Workspace: D, the packed bases, the subgroup flag of the bases (one 256-byte slot), tcT and the
+// MSM digits, in that order; tcT and the digits are dead after the MSM, and a small batch's
+// transforms keep their products there.
 static size_t poly2h_scratch_bytes(unsigned rows, unsigned n2) {
     return (size_t)rows * 16 * n2 * 32 + (size_t)rows * n2 * 144 + (size_t)16 * n2 * 144 + 256 +
            msm_plain_digit_bytes(rows, n2);
@@ -333,17 +365,16 @@ static int poly2h_fft_in(void *scratch, DeviceState *st, fk20_g1p_t *h_fft, cons
     const size_t d_bytes = (size_t)rows * n2 * 144;
     const size_t x_bytes = (size_t)16 * n2 * 144;
     char *base = reinterpret_cast<char *>(scratch);
-    uint32_t *tcT = reinterpret_cast<uint32_t *>(base);
-    uint32_t *D = reinterpret_cast<uint32_t *>(base + tc_bytes);
-    uint32_t *xpk = reinterpret_cast<uint32_t *>(base + tc_bytes + d_bytes);
-    uint32_t *flag = reinterpret_cast<uint32_t *>(base + tc_bytes + d_bytes + x_bytes);
-    int8_t *digits = reinterpret_cast<int8_t *>(base + tc_bytes + d_bytes + x_bytes + 256);
+    uint32_t *D = W(base), *xpk = W(base + d_bytes), *flag = W(base + d_bytes + x_bytes);
+    uint32_t *tcT = W(base + d_bytes + x_bytes + 256);
+    int8_t *digits = reinterpret_cast<int8_t *>(base + d_bytes + x_bytes + 256 + tc_bytes);
     hipStream_t s = S(stream);
     // one flag for all rows: a base outside G1 can put every row's MSM output outside it
     FK20_TRY(launch_subgroup_groups(flag, W(xext_fft), (size_t)16 * n2, (size_t)16 * n2, s));
     FK20_TRY(launch_std_to_packed(xpk, W(xext_fft), (size_t)16 * n2, s));
     return hip_status(launch_plain(PLAIN_POLY2H_FFT, W(h_fft), W(poly), xpk, rows, log2u(n2), D, tcT, digits,
-                                   flag, st->tables, st->prog, s));
+                                   flag, st->tables, st->prog, s, st->direct, tcT,
+                                   tc_bytes + msm_plain_digit_bytes(rows, n2)));
 }
 
 int fk20_poly2h_fft(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20_g1p_t *xext_fft, unsigned rows,
@@ -382,15 +413,16 @@ int fk20_setup2xext_fft(fk20_g1p_t *xext_fft, const fk20_g1p_t *setup, unsigned 
     int rc = device_state(&st);
     if (rc) return rc;
     void *D;
-    const size_t d_bytes = (size_t)16 * (N / 8) * 144;
-    rc = device_scratch(st, d_bytes + 16 * 4, &D);
+    const size_t d_bytes = (size_t)16 * (N / 8) * 144, f_bytes = flag_bytes(16);
+    const size_t p_bytes = transform_product_bytes(st, 16, log2u(N / 8));
+    rc = device_scratch(st, d_bytes + f_bytes + p_bytes, &D);
     if (rc) return rc;
-    uint32_t *flags = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(D) + d_bytes);
+    char *base = reinterpret_cast<char *>(D);
     hipStream_t s = S(stream);
     FK20_TRY(launch_setup_gather(W(xext_fft), W(setup), N, s));
-    return hip_status(launch_plain(PLAIN_G1_FFT, W(xext_fft), W(xext_fft), nullptr, 16, log2u(N / 8),
-                                   reinterpret_cast<uint32_t *>(D), nullptr, nullptr, flags, st->tables, st->prog,
-                                   s));
+    return hip_status(launch_plain(PLAIN_G1_FFT, W(xext_fft), W(xext_fft), nullptr, 16, log2u(N / 8), W(base), nullptr,
+                                   nullptr, W(base + d_bytes), st->tables, st->prog, s, st->direct,
+                                   W(base + d_bytes + f_bytes), p_bytes));
 }
 
 // ---------------------------------------------------------------- helpers

@@ -233,6 +233,7 @@ struct Setup {
     unsigned N = 0, n2 = 0, win = 0, nwin = 0;
     uint32_t *table = nullptr;
     uint32_t *inf = nullptr;
+    unsigned logn2() const { return n2 == 128 ? 7 : n2 == 256 ? 8 : 9; }
 };
 
 bool valid_N(unsigned N) { return N == 1024 || N == 2048 || N == 4096; }
@@ -332,9 +333,23 @@ void fk20::free_programs(Programs &P) {
     P.ops = P.index = nullptr;
 }
 
+const std::vector<uint32_t> &fk20::direct_plan_words() {
+    static const std::vector<uint32_t> words = [] {
+        std::vector<uint32_t> w, ops, index;
+        uint32_t scale_off[10];
+        int cost[256] = {};
+        if (!all_programs_host(ops, index, scale_off)) return w;
+        for (int e = 1; e < 256; e++) cost[e] = e == 128 ? 63 * COST_DBL : ops_cost(ops.data() + index[TW_FWD * 512 + e]);
+        direct_build(w, cost);
+        return w;
+    }();
+    return words;
+}
+
 struct fk20_ctx {
     int device = 0;
     const DevTables *T = nullptr;
+    DirectPlan direct;
     Programs prog;
     std::vector<Setup> setups;
     void *work = nullptr;
@@ -402,6 +417,7 @@ int fk20_ctx_create(fk20_ctx_t **out) {
     fk20_ctx *c = new fk20_ctx();
     hipError_t e = hipGetDevice(&c->device);
     if (e == hipSuccess) c->T = current_device_tables(&e);
+    if (e == hipSuccess) c->direct = current_direct_plan(&e);
     if (e == hipSuccess) e = build_programs(c->prog, c->sch_wnaf);
     if (e != hipSuccess) {
         fk20_ctx_destroy(c);
@@ -535,6 +551,7 @@ int fk20_ctx_set_graph(fk20_ctx_t *c, int enable) {
 }
 
 static hipError_t grow_work(fk20_ctx *c, size_t bytes);
+static size_t direct_extra_bytes(const fk20_ctx *c, unsigned rows, unsigned logn);
 
 // Window tables of nbases points (standard-form g1p_t, device), each first multiplied by the
 // standard-form scalar `scale` (device, 8 words).  Fills st.table / st.inf.  *outside: some
@@ -693,6 +710,11 @@ int fk20_setup_unload(fk20_ctx_t *c, int id) {
     return FK20_OK;
 }
 
+static size_t direct_extra_bytes(const fk20_ctx *c, unsigned rows, unsigned logn) {
+    const size_t need = direct_product_bytes(c->direct, rows, logn, 2), tc = ((size_t)rows << logn) * 16 * 32;
+    return need > tc ? need : 0;
+}
+
 static hipError_t grow_work(fk20_ctx *c, size_t bytes) {
     if (c->work_bytes >= bytes) return hipSuccess;
     if (c->work) {
@@ -714,7 +736,20 @@ static hipError_t grow_work(fk20_ctx *c, size_t bytes) {
 int fk20_ctx_reserve(fk20_ctx_t *c, unsigned rows, unsigned N) {
     if (!c || !valid_N(N)) return FK20_EINVAL;
     std::lock_guard<std::mutex> lk(c->mu);
-    return status_of(grow_work(c, fk20_rows_workspace_bytes(rows, N)));
+    const size_t bytes = fk20_rows_workspace_bytes(rows, N);
+    const unsigned logn = N == 1024 ? 7 : N == 2048 ? 8 : 9;
+    return status_of(grow_work(c, bytes + (rows <= DIRECT_MAX_ROWS ? direct_extra_bytes(c, rows, logn) : 0)));
+}
+
+// Extra workspace of a batch's items in the two-level direct schedule: the products of an item
+// that its tcT cannot hold (three levels' always fit there).
+static size_t items_direct_bytes(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n) {
+    size_t total = 0;
+    for (unsigned k = 0; k < n; k++) {
+        if (items[k].rows > DIRECT_MAX_ROWS) return 0;
+        total += direct_extra_bytes(c, items[k].rows, c->setups[items[k].setup_id].logn2());
+    }
+    return total;
 }
 
 static size_t items_workspace_bytes(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n) {
@@ -735,7 +770,7 @@ static bool same_items(const std::vector<fk20_batch_item_t> &a, const fk20_batch
 // Carves each item's workspace (tcT, D, chain flags, control block) from w and launches the
 // batch on s.
 static hipError_t enqueue_launch(fk20_ctx *c, const fk20_batch_item_t *items, unsigned n, hipStream_t s,
-                                 LaunchHook hook, char *w, bool chain) {
+                                 LaunchHook hook, char *w, bool chain, bool direct = false, char *extra = nullptr) {
     Launch L;
     memset(&L, 0, sizeof L);
     L.nitems = n;
@@ -758,7 +793,7 @@ static hipError_t enqueue_launch(fk20_ctx *c, const fk20_batch_item_t *items, un
         it.inf = st.inf;
         it.rows = items[k].rows;
         it.N = st.N;
-        it.logn2 = st.n2 == 128 ? 7 : st.n2 == 256 ? 8 : 9;
+        it.logn2 = st.logn2();
         it.win = st.win;
         it.out_format = (uint32_t)c->out_format;
         it.stage = -1;
@@ -767,7 +802,28 @@ static hipError_t enqueue_launch(fk20_ctx *c, const fk20_batch_item_t *items, un
     // the persistent form runs radix-2 stages: the schedule's width and occupancy, radix 2
     const StageKernels *K = stage_kernels(c->sch_wnaf, chain ? false : c->sch_r22, c->sch_occ);
     if (!K) return hipErrorInvalidValue;
-    return launch_batch(L, c->T, c->prog.ops, c->prog.index, *K, s, hook, chain ? ctl : nullptr, c->chain_wait);
+    // small batches: the direct schedule, its products in tcT (dead after the MSM) or in `extra`
+    const bool two = extra != nullptr || !items_direct_bytes(c, items, n);
+    const unsigned levels = direct && K->direct ? direct_choose(L, c->direct, true, two) : 0;
+    for (unsigned k = 0; levels && k < n; k++) {
+        Item &it = L.item[k];
+        const size_t more = levels == 2 ? direct_extra_bytes(c, it.rows, it.logn2) : 0;
+        it.P = more ? reinterpret_cast<uint32_t *>(extra) : it.tcT;
+        extra += more;
+    }
+    return launch_batch(L, c->T, c->prog.ops, c->prog.index, *K, s, hook, chain ? ctl : nullptr, c->chain_wait,
+                        c->direct, levels);
+}
+
+// Whether the batch's transforms take the direct schedule.
+static bool direct_items(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n, bool two) {
+    Launch L;
+    L.nitems = n;
+    for (unsigned k = 0; k < n; k++) {
+        L.item[k].rows = items[k].rows;
+        L.item[k].logn2 = c->setups[items[k].setup_id].logn2();
+    }
+    return direct_choose(L, c->direct, true, two) != 0;
 }
 
 static hipError_t enqueue_items(fk20_ctx *c, const fk20_batch_item_t *items, unsigned n, hipStream_t s,
@@ -779,7 +835,17 @@ static hipError_t enqueue_items(fk20_ctx *c, const fk20_batch_item_t *items, uns
     unsigned groups = 0;
     for (unsigned k = 0; k < n; k++) groups += (items[k].rows + 63) / 64;
     // the context path with at least two 64-row groups, launches not timed one by one
-    if (workspace || c->nsub < 2 || groups < 2 || hook.fn) return enqueue_launch(c, items, n, s, hook, w, chain);
+    // small batches run unsplit in the direct schedule (their halves would not be faster)
+    char *extra = nullptr;
+    bool direct = false;
+    if (!chain && c->sch_r22) {
+        const size_t base = items_workspace_bytes(c, items, n);
+        const size_t more = items_direct_bytes(c, items, n);
+        if (!workspace && more && c->work_bytes >= base + more) extra = w + base;
+        direct = direct_items(c, items, n, extra || !more);
+    }
+    if (workspace || c->nsub < 2 || groups < 2 || hook.fn || direct)
+        return enqueue_launch(c, items, n, s, hook, w, chain, direct, extra);
     // halves: each item's rows split at a 64-row boundary (items of one group go to the first)
     fk20_batch_item_t half[2][MAX_ITEMS];
     unsigned nh[2] = {0, 0};
@@ -839,7 +905,11 @@ int fk20_prove_batch(fk20_ctx_t *c, const fk20_batch_item_t *items, unsigned nit
     if (v.empty()) return FK20_OK;
     const unsigned n = (unsigned)v.size();
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    hipError_t e = grow_work(c, items_workspace_bytes(c, v.data(), n));
+    // what is reserved is not grown for the direct schedule's extra products (three levels do
+    // without); a workspace that has to grow anyway takes them along
+    hipError_t e = hipSuccess;
+    const size_t base = items_workspace_bytes(c, v.data(), n);
+    if (c->work_bytes < base) e = grow_work(c, base + items_direct_bytes(c, v.data(), n));
     if (e == hipSuccess) e = order_before(c, s);
     if (e != hipSuccess) return status_of(e);
     if (c->timing) {

@@ -1,0 +1,195 @@
+// The direct schedule of the column-batched G1 transforms, for batches too small to fill the
+// chip: fewer ladders in a row, more of them side by side.
+//
+// A twiddle ladder takes about as long on an idle chip as on a busy one, so a small batch's
+// transform lasts the number of ladders on its longest path: four generic and four w^128 ones
+// per transform of 512 in the radix-2^2 schedule (schedule.hip.h).  Here a transform is two or
+// three mixed-radix steps, each of them one round of ladders.  A step of radix a on blocks of
+// N = a b points computes
+//     Y[j][m] = sum_t w_N^(j (m + b t)) X[m + b t],     j, t < a, m < b,
+// (the twiddles of the next step included), in three launches:
+//  * k_direct_split, in place: for every m the a points become the sum of all, the difference of
+//    the two halves' sums, .., the a/2 differences X[t] - X[t + a/2]: log2(a) additions by a
+//    lanes at once.  Output j with j = 2^v odd only needs the a / 2^(v+1) differences of level v.
+//  * k_direct_products: one ladder per distinct (point, exponent) into P[slot][row]; exponents
+//    are taken below 256 (w^256 = -1), and all products of one exponent are next to each other,
+//    so a wave runs one program over several points times the batch's rows.
+//  * k_direct_sums: every output adds its a / 2^(v+1) products.
+// The blocks' size-b transforms follow with root w_N^a.  Radix 16 takes 5.3 ladders per point,
+// a last step of radix 32 3.5 (radix-2^2: 2.3 and 1.2 short ones per point, in eight rounds).
+//
+// Shared by the kernels, the launchers and, compiled by g++, the CPU tests.
+#pragma once
+#include <stdint.h>
+
+#ifndef FK20_HD
+#define FK20_HD __host__ __device__ __forceinline__
+#endif
+
+namespace fk20 {
+
+// Which transform: the batched path's halves (hext_fft in bit-reversed order -> h, its n/2
+// coefficients in natural order; h -> h_fft at bit-reversed positions) and the whole transforms
+// of the drop-ins (in the positions their load and output kernels use).
+enum DirectKind { DIRECT_IFFT_HALF = 0, DIRECT_FFT_HALF = 1, DIRECT_FFT = 2, DIRECT_IFFT = 3 };
+static constexpr unsigned DIRECT_KINDS = 4;
+// levels 2: [16, 32], [16, 16], [8, 16] for n = 512, 256, 128; levels 3: [8, 8, 8], [4, 8, 8],
+// [4, 4, 8]
+static constexpr unsigned DIRECT_MAX_STEPS = 3;
+
+// log2 of the lanes a product's rows take in k_direct_products
+FK20_HD unsigned direct_row_lanes(unsigned rows) {
+    unsigned lr = 0;
+    while (lr < 6 && (1u << lr) < rows) lr++;
+    return lr;
+}
+
+FK20_HD unsigned direct_radix_log(unsigned logn, unsigned levels, unsigned step) {
+    if (levels == 2) return step == 0 ? (logn == 7 ? 3u : 4u) : (logn == 9 ? 5u : 4u);
+    return step == 0 ? (logn == 9 ? 3u : 2u) : step == 1 ? (logn == 7 ? 2u : 3u) : 3u;
+}
+
+// A step's record in the plan words: counts, then offsets (from the plan words' start).
+struct DirectStep {
+    uint32_t loga, logb, logblocks;  // radix, stride, number of blocks (log2)
+    uint32_t in_map;                 // bit 0: position of index i is bitrev(i); bit 1: upper half zero
+    uint32_t nprod, prod;            // products: position | exponent << 16, in slot order
+    uint32_t nout, sums;             // outputs: DIRECT_SUM_WORDS each
+    uint32_t nwaves[7], waves[7];    // for 2^k products per wave: first slot | count << 16 (k = 0..6)
+};
+static constexpr unsigned DIRECT_STEP_WORDS = sizeof(DirectStep) / 4;
+// an output: its position, then up to 16 terms: slot | sign << 31, DIRECT_NONE past the last
+static constexpr unsigned DIRECT_SUM_WORDS = 20, DIRECT_SUM_FIRST = 4;
+static constexpr uint32_t DIRECT_NONE = 0xffffffffu;
+// index of the step record of (logn, kind, levels, step) in the record table at the words' start
+FK20_HD unsigned direct_record(unsigned logn, unsigned kind, unsigned levels, unsigned step) {
+    return (((logn - 7) * DIRECT_KINDS + kind) * 2 + (levels - 2)) * DIRECT_MAX_STEPS + step;
+}
+static constexpr unsigned DIRECT_RECORDS = 3 * DIRECT_KINDS * 2 * DIRECT_MAX_STEPS;
+
+}  // namespace fk20
+
+// ---------------------------------------------------------------- host: the plans
+
+#include <algorithm>
+#include <cstring>
+#include <map>
+#include <vector>
+
+namespace fk20 {
+
+inline unsigned direct_bitrev(unsigned x, unsigned bits) {
+    unsigned r = 0;
+    for (unsigned i = 0; i < bits; i++) r |= ((x >> i) & 1u) << (bits - 1 - i);
+    return r;
+}
+
+// Appends one step's tables to `words` and returns its record.  cost[e]: ladder cost of w^e
+// (e < 256; 0 for e = 0), the order in which exponents are handed out.
+inline DirectStep direct_build_step(std::vector<uint32_t> &words, unsigned logn, unsigned kind, unsigned levels,
+                                    unsigned step, const int *cost) {
+    const unsigned steps = levels, n = 1u << logn;
+    const bool inverse = kind == DIRECT_IFFT_HALF || kind == DIRECT_IFFT;
+    unsigned logdone = 0;
+    for (unsigned s = 0; s < step; s++) logdone += direct_radix_log(logn, levels, s);
+    DirectStep r;
+    memset(&r, 0, sizeof r);
+    r.loga = direct_radix_log(logn, levels, step);
+    r.logb = logn - logdone - r.loga;
+    r.logblocks = logdone;
+    const bool last = step + 1 == steps;
+    r.in_map = step == 0 ? (inverse ? 1u : 0u) | (kind == DIRECT_FFT_HALF ? 2u : 0u) : 0u;
+    const unsigned a = 1u << r.loga, b = 1u << r.logb, N = a * b;
+    auto position = [&](unsigned i) { return (r.in_map & 1u) ? direct_bitrev(i, logn) : i; };
+
+    struct Out {
+        unsigned pos;
+        std::vector<std::pair<unsigned, unsigned>> terms;  // (position << 8 | exponent, sign)
+    };
+    std::vector<Out> outs;
+    std::map<unsigned, unsigned> slot;  // position << 8 | exponent -> slot
+    for (unsigned blk = 0; blk < (1u << r.logblocks); blk++)
+        for (unsigned j = 0; j < a; j++) {
+            // output index of this block's Y[j][0]: the digits so far, least significant first
+            unsigned k = 0, shift = 0;
+            for (unsigned s = 0, rem = blk, left = logdone; s < step; s++) {
+                const unsigned ls = direct_radix_log(logn, levels, s);
+                left -= ls;
+                k |= (rem >> left) << shift;
+                rem &= (1u << left) - 1;
+                shift += ls;
+            }
+            k |= j << shift;
+            if (last && kind == DIRECT_IFFT_HALF && k >= n / 2) continue;
+            for (unsigned m = 0; m < b; m++) {
+                Out o;
+                if (!last) o.pos = ((blk << r.loga | j) << r.logb) | m;
+                else o.pos = kind == DIRECT_FFT || kind == DIRECT_FFT_HALF ? direct_bitrev(k, logn) : k;
+                // level v differences: positions t in [a >> (v+1), a >> v) of the split array;
+                // j = 0: the total at t = 0
+                unsigned lo = 0, hi = 1;
+                if (j) {
+                    const unsigned v = (unsigned)__builtin_ctz(j);
+                    lo = a >> (v + 1);
+                    hi = a >> v;
+                }
+                for (unsigned t = lo; t < hi; t++) {
+                    unsigned e = (j * (m + b * (t - lo))) % N * (512 / N);
+                    if (inverse) e = (512 - e) % 512;
+                    const unsigned p = position(blk * N + m + b * t);
+                    o.terms.push_back({p << 8 | (e & 255u), e >> 8});
+                    slot[p << 8 | (e & 255u)] = 0;
+                }
+                outs.push_back(o);
+            }
+        }
+    // slots: exponents by decreasing cost, all products of one exponent together
+    std::vector<unsigned> keys;
+    for (const auto &s : slot) keys.push_back(s.first);
+    std::stable_sort(keys.begin(), keys.end(), [&](unsigned x, unsigned y) {
+        const unsigned ex = x & 255u, ey = y & 255u;
+        return cost[ex] != cost[ey] ? cost[ex] > cost[ey] : ex < ey;
+    });
+    r.nprod = (uint32_t)keys.size();
+    r.prod = (uint32_t)words.size();
+    for (unsigned i = 0; i < keys.size(); i++) {
+        slot[keys[i]] = i;
+        words.push_back(keys[i] >> 8 | (keys[i] & 255u) << 16);
+    }
+    for (unsigned lk = 0; lk < 7; lk++) {
+        r.waves[lk] = (uint32_t)words.size();
+        for (unsigned i = 0; i < keys.size();) {
+            unsigned c = 1;
+            while (i + c < keys.size() && c < (1u << lk) && (keys[i + c] & 255u) == (keys[i] & 255u)) c++;
+            words.push_back(i | c << 16);
+            i += c;
+        }
+        r.nwaves[lk] = (uint32_t)words.size() - r.waves[lk];
+    }
+    r.nout = (uint32_t)outs.size();
+    r.sums = (uint32_t)words.size();
+    // longest sums first
+    std::stable_sort(outs.begin(), outs.end(), [](const Out &x, const Out &y) { return x.terms.size() > y.terms.size(); });
+    for (const Out &o : outs) {
+        const size_t at = words.size();
+        words.resize(at + DIRECT_SUM_WORDS, DIRECT_NONE);
+        words[at] = o.pos;
+        for (size_t t = 0; t < o.terms.size(); t++)
+            words[at + DIRECT_SUM_FIRST + t] = slot[o.terms[t].first] | o.terms[t].second << 31;
+    }
+    return r;
+}
+
+// Every plan: the record table (DIRECT_RECORDS records), then the records' tables.
+inline void direct_build(std::vector<uint32_t> &words, const int *cost) {
+    words.assign((size_t)DIRECT_RECORDS * DIRECT_STEP_WORDS, 0);
+    for (unsigned logn = 7; logn <= 9; logn++)
+        for (unsigned kind = 0; kind < DIRECT_KINDS; kind++)
+            for (unsigned levels = 2; levels <= 3; levels++)
+                for (unsigned s = 0; s < levels; s++) {
+                    const DirectStep r = direct_build_step(words, logn, kind, levels, s, cost);
+                    memcpy(&words[(size_t)direct_record(logn, kind, levels, s) * DIRECT_STEP_WORDS], &r, sizeof r);
+                }
+}
+
+}  // namespace fk20

@@ -1,6 +1,7 @@
 // Batched FK20 path: twiddle-program encoding and launchers (fast_kernels.hip, ctx.cpp).
 #pragma once
 #include "common.hip.h"
+#include "direct.hip.h"
 #include "ladder.hip.h"
 #include "schedule.hip.h"
 
@@ -94,6 +95,7 @@ struct Item {
     // is recomputed by launch_ref_rows, so the output kernel leaves it alone (nullptr: none)
     const uint32_t *rowflag;
     uint32_t flag_stride;
+    uint32_t *P;            // products of the direct schedule [slot][rows], dead data before
 };
 struct Launch {
     Item item[MAX_ITEMS];
@@ -141,6 +143,7 @@ struct StageKernels {
     // radix-2^2 only: the w^128 twiddles of a DIF stage, after its butterflies (k_quarter_multi)
     void (*quarter)(Launch) = nullptr;
     void (*chain)(Chain, const uint32_t *, const uint32_t *) = nullptr;
+    void (*direct)(Launch, const uint32_t *, const uint32_t *, const uint32_t *) = nullptr;
     void (*plain_load)(uint32_t *, const uint32_t *, unsigned, unsigned, unsigned, const uint32_t *) = nullptr;
     int wnaf = 0;
     bool r22 = false;
@@ -152,6 +155,25 @@ const StageKernels *stage_kernels(unsigned wnaf, bool r22, unsigned occupancy);
 static constexpr unsigned DEFAULT_OCCUPANCY = 2;
 inline const StageKernels &default_stage_kernels() { return *stage_kernels(TW_WNAF, true, DEFAULT_OCCUPANCY); }
 
+// The direct schedule's plans on the current device: the words the kernels read, and the records
+// on the host, for the launchers.
+struct DirectPlan {
+    const uint32_t *words = nullptr;
+    const DirectStep *rec = nullptr;
+};
+// The plans' words (host; built once per process) and records.
+const std::vector<uint32_t> &direct_plan_words();
+// The plans of the current device (api.cpp), or nullptr words on failure.
+DirectPlan current_direct_plan(hipError_t *err);
+// Levels of the direct schedule that transform the items of L fastest (2 or 3), or 0 for the
+// radix-2^2 launches.  both: IFFT and FFT halves (the batched path), else one whole transform;
+// two: whether the workspace holds the products of two levels (three levels' always fit).
+unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, bool two);
+// Bytes of P an item of `rows` transforms of 2^logn points needs at `levels`.
+size_t direct_product_bytes(const DirectPlan &P, unsigned rows, unsigned logn, unsigned levels);
+// Largest batch the direct schedule is used for, in rows of one size: workspaces are sized by it.
+static constexpr unsigned DIRECT_MAX_ROWS = 256;
+
 // The whole batched path for the items of `L`: Toeplitz + NTT, MSM, 2*Lmax - 1 transform
 // stages, output -- one launch per stage covering every item.
 // chain != nullptr: the transform stages run as one persistent k_chain launch whose work
@@ -159,10 +181,11 @@ inline const StageKernels &default_stage_kernels() { return *stage_kernels(TW_WN
 // of its waits gives up after chain_wait ticks and then sets chain[1].
 static constexpr uint64_t CHAIN_WAIT_TICKS = 1ull << 27;  // ~1.3 s at the 100 MHz wall clock
 // K: the transform kernels (K.chain must be set when chain is); ops / index: programs built
-// for K.wnaf.
+// for K.wnaf.  levels != 0: the transforms run in the direct schedule (the items' P set).
 hipError_t launch_batch(const Launch &L, const DevTables *T, const uint32_t *ops, const uint32_t *index,
                         const StageKernels &K, hipStream_t s, LaunchHook hook, uint32_t *chain = nullptr,
-                        uint64_t chain_wait = CHAIN_WAIT_TICKS);
+                        uint64_t chain_wait = CHAIN_WAIT_TICKS, const DirectPlan &direct = DirectPlan(),
+                        unsigned levels = 0);
 
 // The drop-in entry points on the same column-batched transform kernels, for `rows`
 // transforms of n = 2^logn points (n2 = n for the FK20 kinds), with D = rows * n * 144
@@ -175,11 +198,14 @@ hipError_t launch_batch(const Launch &L, const DevTables *T, const uint32_t *ops
 //                         Montgomery bases), then as above            (fk20_poly2h_fft)
 // out may alias in: every input is read into D before the first output is written.
 enum PlainKind { PLAIN_G1_FFT = 0, PLAIN_G1_IFT = 1, PLAIN_HEXT_FFT2H_FFT = 2, PLAIN_POLY2H_FFT = 3 };
+// products: product_bytes of workspace for the direct schedule (it is not used when they are too
+// few); it may overlap tcT and digits.
 // flags: `rows` words of workspace (one word for PLAIN_POLY2H_FFT, set by the caller with
 // launch_subgroup_groups over the bases).  Rows holding a point outside G1 are recomputed in
 // the reference's order of operations (launch_ref_rows).
 hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const uint32_t *xpk, unsigned rows,
                         unsigned logn, uint32_t *D, uint32_t *tcT, int8_t *digits, uint32_t *flags,
-                        const DevTables *T, const Programs &P, hipStream_t s);
+                        const DevTables *T, const Programs &P, hipStream_t s, const DirectPlan &direct, uint32_t *products,
+                        size_t product_bytes);
 
 }  // namespace fk20

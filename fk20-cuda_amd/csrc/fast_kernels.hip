@@ -555,10 +555,82 @@ __global__ void k_chain_reset(Chain C) {
     for (unsigned e = threadIdx.x; e < n; e += blockDim.x) it.flags[e] = 0;
 }
 
+// ---------------------------------------------------------------- direct schedule (direct.hip.h)
+
+__device__ __forceinline__ void shfl_point(g1q &r, const g1q &p, int lane) {
+#pragma unroll
+    for (int i = 0; i < FQ_N; i++) {
+        r.x.l[i] = __shfl(p.x.l[i], lane);
+        r.y.l[i] = __shfl(p.y.l[i], lane);
+        r.z.l[i] = __shfl(p.z.l[i], lane);
+    }
+}
+
+// The split of a direct step, in place: a lanes per (block, m, row), lane t holding point t; after
+// level h the upper half [h, 2h) keeps differences and the lower one goes on with sums.
+__global__ void __launch_bounds__(64) k_direct_split(Launch L, const uint32_t *plan) {
+    unsigned local;
+    const Item &it = L.item[find_item(L, blockIdx.x, local)];
+    const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
+    const unsigned rows = it.rows, logn = it.logn2, lane = threadIdx.x, t = lane & ((1u << st.loga) - 1);
+    const unsigned total = (rows << logn) >> st.loga;
+    // spare lane groups repeat the last one's work
+    const unsigned id = min((local * 64 + lane) >> st.loga, total - 1), row = id % rows, g = id / rows;
+    const unsigned i = ((g >> st.logb) << (st.loga + st.logb)) + (g & ((1u << st.logb) - 1)) + (t << st.logb);
+    const unsigned pos = (st.in_map & 1u) ? bitrev(i, logn) : i;
+    uint32_t *p = it.D + ((size_t)pos * rows + row) * 36;
+    g1q x, o, u;
+    g1q_inf(x);
+    if (!(st.in_map & 2u) || i < (1u << (logn - 1))) pt_load(x, p);
+#pragma unroll 1
+    for (unsigned h = 1u << (st.loga - 1); h; h >>= 1) {
+        shfl_point(o, x, (int)(t < h ? lane + h : t < 2 * h ? lane - h : lane));
+        u = x;
+        if (t >= h) g1q_neg(u, x);
+        g1q_add(o, o, u);
+        if (t < 2 * h) x = o;
+    }
+    pt_store(p, x);
+}
+
+// The sums of a direct step: 4 lanes per (output, row), each adding every fourth term, then
+// across the lanes; D is free to be overwritten, every term is in P.
+__global__ void __launch_bounds__(64) k_direct_sums(Launch L, const uint32_t *plan) {
+    unsigned local;
+    const Item &it = L.item[find_item(L, blockIdx.x, local)];
+    const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
+    const unsigned rows = it.rows, lane = threadIdx.x, part = lane & 3;
+    const unsigned id = min(local * 16 + (lane >> 2), st.nout * rows - 1), row = id % rows;
+    const uint32_t *o = plan + st.sums + (size_t)(id / rows) * DIRECT_SUM_WORDS, *terms = o + DIRECT_SUM_FIRST + part;
+    g1q acc, x;
+    auto term = [&](g1q &p, uint32_t c) {
+        g1q_inf(p);
+        if (c == DIRECT_NONE) return;
+        pt_load(p, it.P + ((size_t)(c & 0x7fffffffu) * rows + row) * 36);
+        if (c >> 31) g1q_neg(p, p);
+    };
+    term(acc, terms[0]);
+#pragma unroll 1
+    for (unsigned k = 4; k < 16; k += 4) {
+        const uint32_t c = terms[k];
+        if (!__any(c != DIRECT_NONE)) break;  // outputs come longest first
+        term(x, c);
+        g1q_add(acc, acc, x);
+    }
+#pragma unroll 1
+    for (int d = 1; d <= 2; d *= 2) {
+        shfl_point(x, acc, (int)lane ^ d);
+        g1q_add(acc, acc, x);
+    }
+    if (part == 0) pt_store(it.D + ((size_t)o[0] * rows + row) * 36, acc);
+}
+
 // D[pos][row] -> the item's output format.  D is in bit-reversed order, so the natural
 // index of pos is bitrev(pos) and the data-availability order (FK20Py
 // list_to_reverse_bit_order of the natural list) is pos itself.
-//   FK20_OUT_G1P / _DA:               g1p_t, canonical standard projective (144 bytes)
+//   FK20_OUT_G1P / _DA:               g1p_t, canonical standard projective (144 bytes) with z = 1
+//                                     (infinity (0 : 1 : 0)): a row's proofs are the same words
+//                                     whatever batch and schedule they were computed in
 //   FK20_OUT_COMPRESSED / _DA:        48-byte compressed G1 (g1_compress)
 __global__ void __launch_bounds__(64) k_output_multi(Launch L) {
     unsigned local;
@@ -577,8 +649,15 @@ __global__ void __launch_bounds__(64) k_output_multi(Launch L) {
         g1q_compress(w, p);
         st_words(it.h_fft + slot * 12, w, 3);
     } else {
-        uint32_t w[36];
-        g1q_store_std(w, p);
+        uint32_t w[36] = {0};
+        fq x, y;
+        if (g1q_to_affine(x, y, p)) {
+            fq_to_std(w, x);
+            fq_to_std(w + 12, y);
+            w[24] = 1;
+        } else {
+            w[12] = 1;
+        }
         st_words(it.h_fft + slot * G1P_WORDS, w, 9);
     }
 }
@@ -647,12 +726,92 @@ static unsigned set_blocks(Launch &L, const unsigned *per_item) {
     return total;
 }
 
+// ---- direct schedule
+
+size_t direct_product_bytes(const DirectPlan &P, unsigned rows, unsigned logn, unsigned levels) {
+    size_t most = 0;
+    for (unsigned kind = 0; kind < DIRECT_KINDS; kind++)
+        for (unsigned s = 0; s < levels; s++)
+            most = std::max<size_t>(most, P.rec[direct_record(logn, kind, levels, s)].nprod);
+    return most * rows * 144;
+}
+
+// Estimated microseconds of the transforms of L's items, measured on MI355X: a round of generic
+// ladders takes 1100 when each SIMD has at most one wave and about 950 more per further wave,
+// one of w^128 ladders 360 and 300; a launch of additions 55 (a direct step has two), a
+// butterfly launch 25.  The choice only depends on the items' sizes and rows.
+unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, bool two) {
+    if (!P.rec) return 0;
+    unsigned lmax = 0;
+    for (unsigned k = 0; k < L.nitems; k++) {
+        lmax = std::max(lmax, L.item[k].logn2);
+        if (L.item[k].rows > DIRECT_MAX_ROWS) return 0;
+    }
+    auto rounds = [](unsigned waves, unsigned first, unsigned more) {
+        return waves ? first + ((waves + 1023) / 1024 - 1) * more : 0;
+    };
+    // radix 2^2: per transform, the layers (odd stages) and the w^128 of the even ones
+    unsigned best = 0, time = 0;
+    for (unsigned sd = 0; sd < lmax; sd++) {
+        unsigned layer = 0, quarter = 0;
+        for (unsigned k = 0; k < L.nitems; k++) {
+            const unsigned logn = L.item[k].logn2, rg = (L.item[k].rows + 63) / 64;
+            if ((sd & 1) && sd < logn) layer += layer_count(sd, logn) * rg;
+            if (!(sd & 1) && sd + 1 < logn) quarter += (1u << (logn - 2)) * rg;
+        }
+        time += 25 + rounds(layer, 1100, 950) + rounds(quarter, 360, 300);
+    }
+    if (both) time *= 2;
+    for (unsigned levels = two ? 2 : 3; levels <= 3; levels++) {
+        unsigned t = 0;
+        for (unsigned half = 0; half < (both ? 2u : 1u); half++)
+            for (unsigned s = 0; s < levels; s++) {
+                unsigned waves = 0;
+                for (unsigned k = 0; k < L.nitems; k++) {
+                    const DirectStep &st = P.rec[direct_record(L.item[k].logn2, both ? half : (unsigned)DIRECT_FFT, levels, s)];
+                    waves += st.nwaves[6 - direct_row_lanes(L.item[k].rows)] * ((L.item[k].rows + 63) / 64);
+                }
+                t += 110 + rounds(waves, 1100, 950);
+            }
+        if (t < time) time = t, best = levels;
+    }
+    return best;
+}
+
+// One transform of every item in the direct schedule.
+static void launch_direct(Launch &L, const DirectPlan &P, unsigned levels, unsigned kind, const uint32_t *ops,
+                          const uint32_t *index, const StageKernels &K, hipStream_t s, const LaunchHook &hook) {
+    unsigned per[MAX_ITEMS];
+    const int add = kind == DIRECT_FFT_HALF || kind == DIRECT_FFT ? LK_DIF : LK_DIT;
+    for (unsigned step = 0; step < levels; step++) {
+        auto blocks = [&](auto &&count) {
+            for (unsigned k = 0; k < L.nitems; k++) {
+                const unsigned rec = direct_record(L.item[k].logn2, kind, levels, step);
+                L.item[k].stage = (int)rec;
+                per[k] = count(L.item[k], P.rec[rec]);
+            }
+            return set_blocks(L, per);
+        };
+        unsigned total = blocks([](const Item &it, const DirectStep &) { return ((it.rows << it.logn2) + 63) / 64; });
+        hipLaunchKernelGGL(k_direct_split, dim3(total), dim3(64), 0, s, L, P.words);
+        hook(add);
+        total = blocks([](const Item &it, const DirectStep &st) {
+            return st.nwaves[6 - direct_row_lanes(it.rows)] * ((it.rows + 63) / 64);
+        });
+        hipLaunchKernelGGL(K.direct, dim3(total), dim3(64), 0, s, L, P.words, ops, index);
+        hook(LK_TWIDDLE);
+        total = blocks([](const Item &it, const DirectStep &st) { return (st.nout * it.rows + 15) / 16; });
+        hipLaunchKernelGGL(k_direct_sums, dim3(total), dim3(64), 0, s, L, P.words);
+        hook(add);
+    }
+}
+
 // Resident waves of k_chain: two per SIMD on 256 CUs.
 static constexpr unsigned CHAIN_WAVES = 2048;
 
 hipError_t launch_batch(const Launch &base, const DevTables *T, const uint32_t *ops, const uint32_t *index,
                         const StageKernels &K, hipStream_t s, LaunchHook hook, uint32_t *chain,
-                        uint64_t chain_wait) {
+                        uint64_t chain_wait, const DirectPlan &direct, unsigned levels) {
     if (chain && !K.chain) return hipErrorInvalidValue;
     Launch L = base;
     unsigned per[MAX_ITEMS], lmax = 0;
@@ -707,6 +866,9 @@ hipError_t launch_batch(const Launch &base, const DevTables *T, const uint32_t *
         C.total = acc;
         if (acc) hipLaunchKernelGGL(K.chain, dim3(std::min(acc, CHAIN_WAVES)), dim3(64), 0, s, C, ops, index);
         hook(LK_CHAIN);
+    } else if (levels) {
+        launch_direct(L, direct, levels, DIRECT_IFFT_HALF, ops, index, K, s, hook);
+        launch_direct(L, direct, levels, DIRECT_FFT_HALF, ops, index, K, s, hook);
     } else {
         // one launch per stage; IFFT DIT stages right-aligned to the middle launch.  In the
         // radix-2^2 schedule a DIT stage whose transposed DIF stage is odd is preceded by that
@@ -791,7 +953,8 @@ hipError_t launch_batch(const Launch &base, const DevTables *T, const uint32_t *
 // DIF's bit-reversed positions (format 0) or position by position (format 1).
 hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const uint32_t *xpk, unsigned rows,
                         unsigned logn, uint32_t *D, uint32_t *tcT, int8_t *digits, uint32_t *flags,
-                        const DevTables *T, const Programs &P, hipStream_t s) {
+                        const DevTables *T, const Programs &P, hipStream_t s, const DirectPlan &direct, uint32_t *products,
+                        size_t product_bytes) {
     if (!rows) return hipSuccess;
     // rows holding a point outside G1 are recomputed by k_ref_rows: the transform kinds check
     // their inputs here, one flag per row; PLAIN_POLY2H_FFT's caller has set flags[0] from the
@@ -818,6 +981,17 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
     unsigned per[MAX_ITEMS] = {};
     const uint32_t *scale = P.ops + P.scale_off[logn];
     const StageKernels &K = default_stage_kernels();  // radix-2^2, built for P's width
+    // small batches: the direct schedule, as many levels as the workspace holds products for
+    it.P = products;
+    const bool both = kind == PLAIN_HEXT_FFT2H_FFT || kind == PLAIN_POLY2H_FFT;
+    unsigned levels = 0;
+    if (rows <= DIRECT_MAX_ROWS) {
+        levels = direct_choose(L, direct, both, direct_product_bytes(direct, rows, logn, 2) <= product_bytes);
+        if (levels && direct_product_bytes(direct, rows, logn, levels) > product_bytes) levels = 0;
+    }
+    auto run_direct = [&](unsigned k) {
+        launch_direct(L, direct, levels, k, P.ops, P.index, K, s, LaunchHook{nullptr, nullptr});
+    };
     // radix-2^2 twiddle layers (see stage_positions): DIF stage t's after its butterflies,
     // the transposed DIF stage's before DIT stage t
     auto layer = [&](unsigned sd, unsigned dir) {
@@ -844,11 +1018,13 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
     case PLAIN_G1_FFT:
         hipLaunchKernelGGL(K.plain_load, dim3(n * rg), dim3(64), 0, s, D, in, rows, logn, 0u,
                            (const uint32_t *)nullptr);
-        for (unsigned t = 0; t < logn; t++) stage(K.dif, (int)t);
+        if (levels) run_direct(DIRECT_FFT);
+        else for (unsigned t = 0; t < logn; t++) stage(K.dif, (int)t);
         break;
     case PLAIN_G1_IFT:
         hipLaunchKernelGGL(K.plain_load, dim3(n * rg), dim3(64), 0, s, D, in, rows, logn, 1u, scale);
-        for (unsigned t = 0; t < logn; t++) stage(K.dit, (int)t);
+        if (levels) run_direct(DIRECT_IFFT);
+        else for (unsigned t = 0; t < logn; t++) stage(K.dit, (int)t);
         it.out_format = 1;
         break;
     case PLAIN_HEXT_FFT2H_FFT:
@@ -864,6 +1040,11 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
             // with tcT (no longer read) as their workspace
             hipLaunchKernelGGL(k_ref_rows, dim3(rows), dim3(256), 0, s, 2u, out, (const uint32_t *)nullptr,
                                (const uint32_t *)D, rows, logn, tcT, (const uint32_t *)flags, 0u, T);
+        }
+        if (levels) {
+            run_direct(DIRECT_IFFT_HALF);
+            run_direct(DIRECT_FFT_HALF);
+            break;
         }
         for (unsigned t = 0; t + 1 < logn; t++) stage(K.dit, (int)t);
         stage(K.middle, 0);

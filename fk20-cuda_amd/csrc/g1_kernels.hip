@@ -44,6 +44,16 @@ __device__ __forceinline__ void g1q_gload_std(g1q &p, const uint32_t *g) {
     g1q_load_std(p, w);
 }
 
+// whether a standard-form point's z is 1
+__device__ __forceinline__ bool g1_z_is_one(const uint32_t *g) {
+    uint32_t w[12];
+    words_load(w, g + 24, 12);
+    uint32_t rest = 0;
+#pragma unroll
+    for (int i = 1; i < 12; i++) rest |= w[i];
+    return w[0] == 1 && rest == 0;
+}
+
 __device__ __forceinline__ void g1q_gstore_std(uint32_t *g, const g1q &p) {
     uint32_t w[36];
     g1q_store_std(w, p);
@@ -356,7 +366,7 @@ __global__ void __launch_bounds__(64) k_to_affine(uint32_t *out, const uint32_t 
     g1q_gload_std(p, in + e * G1P_WORDS);
     fq x, y;
     uint32_t w[24] = {0};
-    if (g1q_to_affine(x, y, p)) {
+    if (g1q_to_affine(x, y, p, g1_z_is_one(in + e * G1P_WORDS))) {
         fq_to_std(w, x);
         fq_to_std(w + 12, y);
     }
@@ -371,7 +381,7 @@ __global__ void __launch_bounds__(64) k_compress(uint32_t *out, const uint32_t *
     g1q p;
     g1q_gload_std(p, in + e * G1P_WORDS);
     uint32_t w[12];
-    g1q_compress(w, p);
+    g1q_compress(w, p, g1_z_is_one(in + e * G1P_WORDS));
     uint4 *q = reinterpret_cast<uint4 *>(out + e * 12);
 #pragma unroll
     for (int i = 0; i < 3; i++) q[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);

@@ -205,8 +205,14 @@ FK20_HD void g1q_zaddu(fq &x3, fq &y3, fq &mu, fq &x1, fq &y1, const fq &x2, con
     x1 = W1;
 }
 
-// (x, y) = (X / Z, Y / Z); false when Z = 0.
-FK20_HD bool g1q_to_affine(fq &x, fq &y, const g1q &p) {
+// (x, y) = (X / Z, Y / Z); false when Z = 0.  z_one: Z is known to be 1 (the transforms' own
+// outputs are); a wave whose lanes all say so has nothing to invert.
+FK20_HD bool g1q_to_affine(fq &x, fq &y, const g1q &p, bool z_one = false) {
+    if (!FQ_ANY(!z_one)) {
+        x = p.x;
+        y = p.y;
+        return true;
+    }
     if (g1q_is_inf(p)) return false;
     fq zi;
     fq_inv(zi, p.z);
@@ -218,9 +224,9 @@ FK20_HD bool g1q_to_affine(fq &x, fq &y, const g1q &p) {
 // 48-byte compressed serialisation, as 12 words in memory order: big-endian canonical x, top
 // byte flags 0x80 (compressed), 0x40 (infinity: 0xc0 then zeros), 0x20 (y is the larger of
 // y and p - y).
-FK20_HD void g1q_compress(uint32_t *w, const g1q &p) {
+FK20_HD void g1q_compress(uint32_t *w, const g1q &p, bool z_one = false) {
     fq x, y;
-    if (!g1q_to_affine(x, y, p)) {
+    if (!g1q_to_affine(x, y, p, z_one)) {
 #pragma unroll
         for (int i = 0; i < 12; i++) w[i] = 0;
         w[0] = 0xc0u;

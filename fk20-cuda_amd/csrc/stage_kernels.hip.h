@@ -159,6 +159,29 @@ __global__ void __launch_bounds__(64, OCC) k_quarter_multi(Launch L) {
     pt_store(p, x);
 }
 
+// The ladders of a direct step (direct.hip.h), record it.stage: a wave takes up to 64 >> lr
+// products of one exponent, 2^lr >= rows lanes each (more than 32 rows: one product and 64 rows).
+// One round of the chip's 1024 SIMDs lasts a ladder, 1.1 ms, however few of them work.
+template <int W, int OCC>
+__global__ void __launch_bounds__(64, OCC) k_direct_products(Launch L, const uint32_t *plan, const uint32_t *ops,
+                                                            const uint32_t *index) {
+    unsigned local;
+    const Item &it = L.item[find_item(L, blockIdx.x, local)];
+    const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
+    const unsigned rows = it.rows, rg = (rows + 63) / 64, lr = direct_row_lanes(rows);
+    const uint32_t w = plan[st.waves[6 - lr] + local / rg];
+    const unsigned sub = threadIdx.x >> lr, count = w >> 16;
+    const unsigned row = min((local % rg) * 64 + (threadIdx.x & ((1u << lr) - 1)), rows - 1);
+    const unsigned slot = (w & 0xffffu) + min(sub, count - 1);  // spare lanes repeat a product
+    const uint32_t pe = plan[st.prod + slot];
+    const unsigned e = FK20_UNIFORM(pe >> 16);
+    g1q x;
+    pt_load(x, it.D + ((size_t)(pe & 0xffffu) * rows + row) * 36);
+    if (e == 128) tw_mul_z3(x, true);
+    else if (e) tw_mul<W>(x, ops + index[TW_FWD * 512 + e]);
+    pt_store(it.P + ((size_t)slot * rows + row) * 36, x);
+}
+
 // ---------------------------------------------------------------- persistent transform chain
 //
 // All 2*Lmax - 1 stages in one launch of resident waves.  Work items (one butterfly of one
@@ -250,6 +273,7 @@ constexpr StageKernels make_stage_kernels() {
     K.twiddle = k_twiddle_multi<W, R22, OCC>;
     if constexpr (!R22) K.chain = k_chain<W, R22, OCC>;
     if constexpr (R22) K.quarter = k_quarter_multi<W, R22, OCC>;
+    if constexpr (R22) K.direct = k_direct_products<W, OCC>;
     K.plain_load = k_plain_load<W, R22, OCC>;
     K.wnaf = W;
     K.r22 = R22;

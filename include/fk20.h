@@ -12,8 +12,10 @@
  *   fk20_g1p_t = g1p_t  (g1.cuh:27)   x, y, z, each 6 x u64, homogeneous projective
  *   fk20_g1a_t = g1a_t  (g1.cuh:20)   x, y affine, infinity = (0, 0) (g1a.cu:91)
  * Inputs may be any representative (fr: any 256-bit value, fp: any 384-bit value).
- * Outputs are standard form with every coordinate canonical (< p or < r); projective
- * outputs are not normalised (use fk20_g1p_to_affine for canonical affine points).
+ * Outputs are standard form with every coordinate canonical (< p or < r); projective outputs
+ * may have any z (use fk20_g1p_to_affine for canonical affine points).  Proofs of rows and the G1
+ * transforms of points in G1 have z = 1 (infinity (0 : 1 : 0)), so they are the same words
+ * whatever batch they were computed in.
  * G1 inputs may be any point of E(Fp), as in the reference.  On the order-r subgroup G1 (all
  * FK20 data lie in it) a transform is a linear map mod r; on a point outside it [a]P and [b]P
  * differ for a = b (mod r), so the transforms check their inputs and recompute a row holding

@@ -1,0 +1,24 @@
+// Host build of the direct schedule's plans (direct.hip.h) for CPU tests.
+#define FK20_HD inline
+#define __host__
+#define __device__
+#include "../../fk20-cuda_amd/csrc/direct.hip.h"
+
+using namespace fk20;
+
+static std::vector<uint32_t> g_words;
+
+extern "C" {
+// Builds every plan with all exponents of one cost but w^128; returns the number of words.
+unsigned direct_host_build(void) {
+    int cost[256];
+    for (int e = 0; e < 256; e++) cost[e] = e == 0 ? 0 : e == 128 ? 1 : 2;
+    direct_build(g_words, cost);
+    return (unsigned)g_words.size();
+}
+const uint32_t *direct_host_words(void) { return g_words.data(); }
+unsigned direct_host_record(unsigned logn, unsigned kind, unsigned levels, unsigned step) {
+    return direct_record(logn, kind, levels, step) * DIRECT_STEP_WORDS;
+}
+unsigned direct_host_row_lanes(unsigned rows) { return direct_row_lanes(rows); }
+}
