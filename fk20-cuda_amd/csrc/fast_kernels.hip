@@ -410,85 +410,74 @@ __device__ __forceinline__ void window_sum(g1q &acc, const uint32_t *tables, siz
     }
 }
 
-// hext_fft[j] for 64 rows of one column j: sum over 16 terms of ceil(256/w) signed-window
-// digits, one mixed addition each.  Output to D[bitrev(j)][row].
+__device__ __forceinline__ void shfl_point(g1q &r, const g1q &p, int lane) {
+#pragma unroll
+    for (int i = 0; i < FQ_N; i++) {
+        r.x.l[i] = __shfl(p.x.l[i], lane);
+        r.y.l[i] = __shfl(p.y.l[i], lane);
+        r.z.l[i] = __shfl(p.z.l[i], lane);
+    }
+}
+
+// the sum of the points of the lanes t, t ^ 1, .., t ^ (span - 1) in each of them (span a power of two)
+__device__ __forceinline__ void lane_sum(g1q &acc, unsigned span) {
+    g1q o;
+#pragma unroll 1
+    for (unsigned d = 1; d < span; d *= 2) {
+        shfl_point(o, acc, (int)(threadIdx.x ^ d));
+        g1q_add(acc, acc, o);
+    }
+}
+
+// hext_fft[j] of one column j: sum over 16 terms of ceil(256/w) signed-window digits, one mixed
+// addition each; output to D[bitrev(j)][row].  LP lanes share a row, each with 16 / LP of the
+// terms, and add up across the wave: an addition takes 9 us in a wave alone on its SIMD and 8.3
+// per wave beside others, so LP = 1 (no closing additions) is best where its waves fill the
+// chip, and 4 or 16 shorten a small or ragged launch (msm_lanes picks by waves and additions:
+// 64 rows of 4096 at window 8 take 4.6 ms with LP = 1 and 2.7 with 16; 512 rows 17.2 and 19.9).
+template <unsigned LP>
 __global__ void __launch_bounds__(64) k_msm_multi(Launch L) {
     unsigned local;
     const Item &it = L.item[find_item(L, blockIdx.x, local)];
-    const unsigned rows = it.rows, n2 = 1u << it.logn2, rg = (rows + 63) / 64;
+    const unsigned rows = it.rows, n2 = 1u << it.logn2, per_wave = 64 / LP, rg = (rows + per_wave - 1) / per_wave;
     const unsigned WIN = it.win, NWIN = (256 + WIN - 1) / WIN, H = 1u << (WIN - 1);
-    const unsigned j = local / rg;
-    const unsigned row = min((local % rg) * 64 + threadIdx.x, rows - 1);  // spare lanes repeat the last row
-    g1q acc;
-    g1q_inf(acc);
+    const unsigned j = local / rg, i0 = threadIdx.x % LP;
+    const unsigned row0 = (local % rg) * per_wave + threadIdx.x / LP;
+    const unsigned row = min(row0, rows - 1);  // spare lanes repeat the last row
     const size_t per_base = (size_t)NWIN * H * TABLE_ENTRY_WORDS;
-    const uint32_t *tc = it.tcT + ((size_t)j * 16 * rows + row) * FR_WORDS, *inf = it.inf + j;
-    window_sum(acc, it.table + j * per_base, n2 * per_base, 16, WIN, [&](unsigned i, uint32_t *k) {
-        if (inf[i * n2]) return false;
-        ld_words(k, tc + (size_t)i * rows * FR_WORDS, 2);
-        return true;
-    });
-    pt_store(it.D + ((size_t)bitrev(j, it.logn2) * rows + row) * 36, acc);
-}
-
-// The same MSM for launches whose items all have at most MSM_SMALL_ROWS rows, where the
-// 16 x ceil(256/w) mixed additions of a lane are latency: lanes are (term i, row) pairs, 16
-// terms x 4 rows per wave, each lane sums one term's windows, and the 16 partial sums of a
-// row are added in LDS (4 levels).  Output to D[bitrev(j)][row] like k_msm_multi.
-static constexpr unsigned MSM_SMALL_ROWS = 16;
-
-__global__ void __launch_bounds__(64) k_msm_multi_small(Launch L) {
-    __shared__ __attribute__((aligned(16))) uint32_t lds[64 * 36];
-    unsigned local;
-    const Item &it = L.item[find_item(L, blockIdx.x, local)];
-    const unsigned rows = it.rows, n2 = 1u << it.logn2, rg4 = (rows + 3) / 4;
-    const unsigned WIN = it.win, NWIN = (256 + WIN - 1) / WIN, H = 1u << (WIN - 1);
-    const unsigned j = local / rg4, t = threadIdx.x, i = t % 16, r = t / 16;
-    const unsigned row0 = (local % rg4) * 4 + r, row = min(row0, rows - 1);  // spare lanes repeat a row
-    const unsigned b = i * n2 + j;
+    const uint32_t *tc = it.tcT + (((size_t)j * 16 + i0) * rows + row) * FR_WORDS, *inf = it.inf + i0 * n2 + j;
     g1q acc;
     g1q_inf(acc);
-    const uint32_t *tc = it.tcT + (((size_t)j * 16 + i) * rows + row) * FR_WORDS;
-    const bool skip = it.inf[b] != 0;
-    window_sum(acc, it.table + (size_t)b * NWIN * H * TABLE_ENTRY_WORDS, 0, 1, WIN, [&](unsigned, uint32_t *k) {
-        if (skip) return false;
-        ld_words(k, tc, 2);
+    window_sum(acc, it.table + (i0 * n2 + j) * per_base, LP * n2 * per_base, 16 / LP, WIN, [&](unsigned t, uint32_t *k) {
+        if (inf[t * LP * n2]) return false;
+        ld_words(k, tc + (size_t)t * LP * rows * FR_WORDS, 2);
         return true;
     });
-    pt_store(lds + t * 36, acc);
-#pragma unroll 1
-    for (unsigned h = 8; h >= 1; h /= 2) {
-        __syncthreads();
-        g1q o;
-        if (i < h) {
-            pt_load(o, lds + (t + h) * 36);
-            g1q_add(acc, acc, o);
-        }
-        __syncthreads();
-        if (i < h) pt_store(lds + t * 36, acc);
-    }
-    if (i == 0 && row0 < rows) pt_store(it.D + ((size_t)bitrev(j, it.logn2) * rows + row) * 36, acc);
+    lane_sum(acc, LP);
+    if (i0 == 0 && (LP == 1 || row0 < rows)) pt_store(it.D + ((size_t)bitrev(j, it.logn2) * rows + row) * 36, acc);
 }
 
 // ---------------------------------------------------------------- KZG commitments
 //
 // commit[row] = sum_i poly[row][i] * srs[i] (FK20Py kzg_proofs.py:159 commit_to_poly) over
-// window tables of the SRS points built like the FK20 setup's.  Lanes are rows; a block sums
-// one chunk of consecutive coefficients into partial[chunk][row], then two reduction passes
-// add the chunks.
+// window tables of the SRS points built like the FK20 setup's.  A lane sums `chunk` consecutive
+// coefficients of one row; lp lanes share a row (a power of two: 64 / rows for small batches, so
+// that no lane is idle) and add up across the wave into partial[chunk][row]; one wave per row
+// then adds the row's partial sums (commit_shape picks lp and chunk).
 
 __global__ void __launch_bounds__(64) k_commit_partial(const uint32_t *poly, const uint32_t *table,
                                                        const uint32_t *inf, uint32_t *partial, unsigned rows,
-                                                       unsigned N, unsigned win_bits, unsigned chunk) {
-    const unsigned rg = (rows + 63) / 64, c = blockIdx.x / rg;
-    const unsigned row = min((blockIdx.x % rg) * 64 + threadIdx.x, rows - 1);  // spare lanes repeat the last row
+                                                       unsigned N, unsigned win_bits, unsigned chunk, unsigned lp) {
+    const unsigned per_wave = 64 / lp, rg = (rows + per_wave - 1) / per_wave, c = blockIdx.x / rg;
+    const unsigned row0 = (blockIdx.x % rg) * per_wave + threadIdx.x / lp;
+    const unsigned row = min(row0, rows - 1);  // spare lanes repeat the last row
     const unsigned NWIN = (256 + win_bits - 1) / win_bits, H = 1u << (win_bits - 1);
-    const unsigned i0 = c * chunk, i1 = min(i0 + chunk, N);
-    g1q acc;
-    g1q_inf(acc);
+    const unsigned i0 = (c * lp + threadIdx.x % lp) * chunk;  // chunk * lp divides N
     const size_t per_base = (size_t)NWIN * H * TABLE_ENTRY_WORDS;
     const uint32_t *coeff = poly + ((size_t)row * N + i0) * FR_WORDS;
-    window_sum(acc, table + i0 * per_base, per_base, i1 - i0, win_bits, [&](unsigned t, uint32_t *k) {
+    g1q acc;
+    g1q_inf(acc);
+    window_sum(acc, table + i0 * per_base, per_base, chunk, win_bits, [&](unsigned t, uint32_t *k) {
         if (inf[i0 + t]) return false;
         // the caller's coefficient may be any 256-bit representative: reduce it below r, so
         // the top signed window's carry stays inside the ceil(256/w) windows (at w = 8 the
@@ -500,31 +489,27 @@ __global__ void __launch_bounds__(64) k_commit_partial(const uint32_t *poly, con
         for (int q = 0; q < 8; q++) k[q] = c.l[q];
         return true;
     });
-    pt_store(partial + ((size_t)c * rows + row) * 36, acc);
+    lane_sum(acc, lp);
+    if (threadIdx.x % lp == 0 && row0 < rows) pt_store(partial + ((size_t)c * rows + row) * 36, acc);
 }
 
-// out[q][row] = sum of in[q*group .. min((q+1)*group, nparts)][row]; with std_out the single
-// group's sum goes to out[row] as a canonical standard-form g1p_t.
-__global__ void __launch_bounds__(64) k_commit_reduce(const uint32_t *in, uint32_t *out, unsigned rows,
-                                                      unsigned nparts, unsigned group, unsigned nout,
-                                                      unsigned std_out) {
-    const size_t t = (size_t)blockIdx.x * 64 + threadIdx.x;
-    if (t >= (size_t)rows * nout) return;
-    const unsigned row = (unsigned)(t % rows), q = (unsigned)(t / rows);
-    const unsigned p0 = q * group, p1 = min(p0 + group, nparts);
+// out[row] = the sum of partial[0 .. nparts)[row], as a canonical standard-form g1p_t: a wave per row.
+__global__ void __launch_bounds__(64) k_commit_reduce(const uint32_t *partial, uint32_t *out, unsigned rows,
+                                                      unsigned nparts) {
+    const unsigned row = blockIdx.x;
     g1q acc, x;
     g1q_inf(acc);
+    if (threadIdx.x < nparts) pt_load(acc, partial + ((size_t)threadIdx.x * rows + row) * 36);
 #pragma unroll 1
-    for (unsigned p = p0; p < p1; p++) {
-        pt_load(x, in + ((size_t)p * rows + row) * 36);
+    for (unsigned p = threadIdx.x + 64; p < nparts; p += 64) {
+        pt_load(x, partial + ((size_t)p * rows + row) * 36);
         g1q_add(acc, acc, x);
     }
-    if (std_out) {
+    lane_sum(acc, 64);
+    if (threadIdx.x == 0) {
         uint32_t w[36];
         g1q_store_std(w, acc);
         st_words(out + (size_t)row * G1P_WORDS, w, 9);
-    } else {
-        pt_store(out + ((size_t)q * rows + row) * 36, acc);
     }
 }
 
@@ -556,15 +541,6 @@ __global__ void k_chain_reset(Chain C) {
 }
 
 // ---------------------------------------------------------------- direct schedule (direct.hip.h)
-
-__device__ __forceinline__ void shfl_point(g1q &r, const g1q &p, int lane) {
-#pragma unroll
-    for (int i = 0; i < FQ_N; i++) {
-        r.x.l[i] = __shfl(p.x.l[i], lane);
-        r.y.l[i] = __shfl(p.y.l[i], lane);
-        r.z.l[i] = __shfl(p.z.l[i], lane);
-    }
-}
 
 // The split of a direct step, in place: a lanes per (block, m, row), lane t holding point t; after
 // level h the upper half [h, 2h) keeps differences and the lower one goes on with sums.
@@ -691,29 +667,63 @@ hipError_t launch_table_build(uint32_t *table, uint32_t *zt, const uint32_t *xs,
     return hipGetLastError();
 }
 
-// Commitment chunking: coefficients per partial sum, partials per first reduction group.
-static constexpr unsigned COMMIT_CHUNK = 16, COMMIT_GROUP = 16;
-
-size_t commit_workspace_bytes(unsigned rows, unsigned N) {
-    const size_t nparts = (N + COMMIT_CHUNK - 1) / COMMIT_CHUNK;
-    const size_t nmid = (nparts + COMMIT_GROUP - 1) / COMMIT_GROUP;
-    return (nparts + nmid) * rows * 144;
+// Additions one after the other that `waves` waves of `adds` additions take on 1024 SIMDs: a wave
+// alone on its SIMD needs about 1.1 times an addition's share of a busy SIMD.
+static unsigned add_rounds(size_t waves, unsigned adds) {
+    const unsigned rounds = (unsigned)((waves + 1023) / 1024);
+    return rounds <= 1 ? adds + adds / 8 : rounds * adds;
 }
+
+// Lanes per row and coefficients per lane of k_commit_partial: no idle lanes below 64 rows, then
+// the chunk with the fewest additions one after the other (20 windows per coefficient; larger
+// chunks where it does not matter, for fewer partial sums).
+struct CommitShape {
+    unsigned lp, chunk, nparts;
+};
+static CommitShape commit_shape(unsigned rows, unsigned N) {
+    CommitShape best{1, 16, N / 16};
+    unsigned lp = 1, time = ~0u;
+    while (lp < 64 && rows * lp * 2 <= 64) lp *= 2;
+    for (unsigned chunk = 16; chunk * lp >= 4 && chunk >= 1; chunk /= 2) {
+        const unsigned nparts = N / (chunk * lp), per_wave = 64 / lp;
+        const size_t waves = (size_t)((rows + per_wave - 1) / per_wave) * nparts;
+        unsigned close = (nparts + 63) / 64 + 6;
+        for (unsigned l = lp; l > 1; l /= 2) close++;
+        const unsigned t = add_rounds(waves, chunk * 20) + close;
+        if (t < time) time = t, best = CommitShape{lp, chunk, nparts};
+    }
+    return best;
+}
+
+size_t commit_workspace_bytes(unsigned rows, unsigned N) { return (size_t)commit_shape(rows, N).nparts * rows * 144; }
 
 hipError_t launch_commit(uint32_t *out, const uint32_t *poly, const uint32_t *table, const uint32_t *inf,
                          uint32_t *work, unsigned rows, unsigned N, unsigned win_bits, hipStream_t s) {
     if (!rows) return hipSuccess;
-    const unsigned nparts = (N + COMMIT_CHUNK - 1) / COMMIT_CHUNK;
-    const unsigned nmid = (nparts + COMMIT_GROUP - 1) / COMMIT_GROUP;
-    const unsigned rg = (rows + 63) / 64;
-    uint32_t *partial = work, *mid = work + (size_t)nparts * rows * 36;
-    hipLaunchKernelGGL(k_commit_partial, dim3(nparts * rg), dim3(64), 0, s, poly, table, inf, partial, rows, N,
-                       win_bits, COMMIT_CHUNK);
-    const size_t t1 = (size_t)rows * nmid;
-    hipLaunchKernelGGL(k_commit_reduce, dim3((unsigned)((t1 + 63) / 64)), dim3(64), 0, s, partial, mid, rows, nparts,
-                       COMMIT_GROUP, nmid, 0u);
-    hipLaunchKernelGGL(k_commit_reduce, dim3((rows + 63) / 64), dim3(64), 0, s, mid, out, rows, nmid, nmid, 1u, 1u);
+    const CommitShape c = commit_shape(rows, N);
+    const unsigned per_wave = 64 / c.lp, rg = (rows + per_wave - 1) / per_wave;
+    hipLaunchKernelGGL(k_commit_partial, dim3(c.nparts * rg), dim3(64), 0, s, poly, table, inf, work, rows, N, win_bits,
+                       c.chunk, c.lp);
+    hipLaunchKernelGGL(k_commit_reduce, dim3(rows), dim3(64), 0, s, work, out, rows, c.nparts);
     return hipGetLastError();
+}
+
+// Lanes per row of the MSM over the items of L (k_msm_multi): the fewest additions one after the
+// other, the closing additions across the lanes included.
+static unsigned msm_lanes(const Launch &L) {
+    unsigned best = 1, time = ~0u;
+    for (unsigned lp = 1, close = 0; lp <= 16; lp *= 4, close += 2) {
+        size_t waves = 0;
+        unsigned adds = 0;
+        for (unsigned k = 0; k < L.nitems; k++) {
+            const unsigned nwin = (256 + L.item[k].win - 1) / L.item[k].win;
+            waves += ((size_t)L.item[k].rows * lp + 63) / 64 << L.item[k].logn2;
+            adds = std::max(adds, 16 / lp * nwin + close + close / 4);
+        }
+        const unsigned t = add_rounds(waves, adds);
+        if (t < time) time = t, best = lp;
+    }
+    return best;
 }
 
 // Fills L.blk_end from per-item block counts; returns the total.
@@ -829,13 +839,11 @@ hipError_t launch_batch(const Launch &base, const DevTables *T, const uint32_t *
     if (total) hipLaunchKernelGGL(k_toeplitz_fft_multi, dim3(total), dim3(256), 0, s, L, T);
     hook(LK_TOEPLITZ_FFT);
     // MSM
-    bool small = true;
-    for (unsigned k = 0; k < L.nitems; k++) small = small && L.item[k].rows <= MSM_SMALL_ROWS;
-    for (unsigned k = 0; k < L.nitems; k++)
-        per[k] = (1u << L.item[k].logn2) * (small ? (L.item[k].rows + 3) / 4 : (L.item[k].rows + 63) / 64);
+    const unsigned lp = msm_lanes(L);
+    for (unsigned k = 0; k < L.nitems; k++) per[k] = ((L.item[k].rows * lp + 63) / 64) << L.item[k].logn2;
     total = set_blocks(L, per);
-    if (total && small) hipLaunchKernelGGL(k_msm_multi_small, dim3(total), dim3(64), 0, s, L);
-    else if (total) hipLaunchKernelGGL(k_msm_multi, dim3(total), dim3(64), 0, s, L);
+    if (total) hipLaunchKernelGGL((lp == 1 ? k_msm_multi<1> : lp == 4 ? k_msm_multi<4> : k_msm_multi<16>), dim3(total),
+                                  dim3(64), 0, s, L);
     hook(LK_MSM);
     // transform stages: global stage t = 0 .. 2*lmax - 2; item k (L = logn2) runs local stage
     // u = t - (lmax - L) while 0 <= u <= 2L - 2 (DIT right-aligned to the middle at t = lmax-1,
