@@ -369,9 +369,10 @@ struct fk20_ctx {
     // schedule of the transform kernels (fk20_ctx_set_schedule); prog is built for sch_wnaf
     unsigned sch_wnaf = TW_WNAF, sch_occ = DEFAULT_OCCUPANCY;
     bool sch_r22 = true;
-    // fk20_prove_batch splits its rows into `nsub` halves at 64-row boundaries and runs each
+    // fk20_prove_batch may split its rows into `nsub` halves at 64-row boundaries and run each
     // half's launch sequence on its own stream, forked from and joined back to the caller's
     // stream, so one half's stage launches fill the SIMDs the other half's idle at a boundary
+    // (worth_splitting)
     unsigned nsub = 2;
     hipStream_t sub[2] = {nullptr, nullptr};
     hipEvent_t fork = nullptr, join[2] = {nullptr, nullptr};
@@ -815,6 +816,17 @@ static hipError_t enqueue_launch(fk20_ctx *c, const fk20_batch_item_t *items, un
                         c->direct, levels);
 }
 
+// Whether two halves on two streams beat one sequence.  The layers hand their ladders to the
+// SIMDs in decreasing cost, which two concurrent launches disturb: batches of one size are faster
+// in one sequence (rows x N: 100 x 4096 17.3 against 22.9 ms, 512 x 4096 43.9 against 46.1,
+// 200 x 2048 15.0 against 19.3, 512 x 1024 14.7 against 19.0), and so are small mixed ones
+// (150 + 75 + 301 rows 39.4 against 39.6); 512 rows of each size take 74.8 in one and 74.2 in two.
+static bool worth_splitting(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n, unsigned groups) {
+    bool mixed = false;
+    for (unsigned k = 1; k < n; k++) mixed = mixed || c->setups[items[k].setup_id].N != c->setups[items[0].setup_id].N;
+    return mixed && groups >= 16;
+}
+
 // Whether the batch's transforms take the direct schedule.
 static bool direct_items(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n, bool two) {
     Launch L;
@@ -844,7 +856,7 @@ static hipError_t enqueue_items(fk20_ctx *c, const fk20_batch_item_t *items, uns
         if (!workspace && more && c->work_bytes >= base + more) extra = w + base;
         direct = direct_items(c, items, n, extra || !more);
     }
-    if (workspace || c->nsub < 2 || groups < 2 || hook.fn || direct)
+    if (workspace || c->nsub < 2 || groups < 2 || hook.fn || direct || !worth_splitting(c, items, n, groups))
         return enqueue_launch(c, items, n, s, hook, w, chain, direct, extra);
     // halves: each item's rows split at a 64-row boundary (items of one group go to the first)
     fk20_batch_item_t half[2][MAX_ITEMS];

@@ -169,10 +169,11 @@ int fk20_ctx_set_chain(fk20_ctx_t *ctx, int enable);
  * pass, tens of ms).  0 makes every wait that finds its inputs unfinished give up at once:
  * a test of the FK20_ETIMEDOUT path in which every kernel still exits normally. */
 int fk20_ctx_set_chain_wait(fk20_ctx_t *ctx, uint64_t ticks);
-/* 2 (default): fk20_prove_rows / fk20_prove_batch split the rows into two halves at a 64-row
+/* 2 (default): fk20_prove_rows / fk20_prove_batch may split the rows into two halves at a 64-row
  * boundary and run the halves' launch sequences on two internal streams forked from and
  * joined back to the caller's stream (captured as such in a hipGraph), so that one half's
- * stage launches fill the SIMDs the other half's leave idle at a launch boundary;
+ * stage launches fill the SIMDs the other half's leave idle at a launch boundary; they do so
+ * for large batches of several sizes, where it is faster;
  * 1: a single sequence on the caller's stream.  Results are identical.  fk20_prove_batch_ws
  * (the serving loop's, which overlaps batches itself) always uses the caller's stream. */
 int fk20_ctx_set_streams(fk20_ctx_t *ctx, unsigned n);
