@@ -70,20 +70,22 @@ __global__ void k_fill_u32(uint32_t *p, size_t n, uint32_t v) {
     if (i < n) p[i] = v;
 }
 
-// A lane's point in LDS, packed (36 words, stride 37 to spread the lanes over the banks).
+// A lane's (x, 2 y) in LDS, packed (24 words, stride 25 to spread the lanes over the banks).
 struct LdsSlot {
     uint32_t *w;
-    __device__ void put(const g1q &p) {
-        uint32_t t[36];
-        g1q_store_packed(t, p);
+    __device__ void put(const fq &x, const fq &h) {
+        uint32_t t[24];
+        fq_pack(t, x);
+        fq_pack(t + 12, h);
 #pragma unroll
-        for (int k = 0; k < 36; k++) w[k] = t[k];
+        for (int k = 0; k < 24; k++) w[k] = t[k];
     }
-    __device__ void get(g1q &p) const {
-        uint32_t t[36];
+    __device__ void get(fq &x, fq &h) const {
+        uint32_t t[24];
 #pragma unroll
-        for (int k = 0; k < 36; k++) t[k] = w[k];
-        g1q_load_packed(p, t);
+        for (int k = 0; k < 24; k++) t[k] = w[k];
+        fq_unpack(x, t);
+        fq_unpack(h, t + 12);
     }
 };
 
@@ -91,14 +93,14 @@ struct LdsSlot {
 // saved points sit in LDS, which leaves room for two waves per SIMD without spills.
 __global__ void __launch_bounds__(64, 2) k_subgroup_groups(uint32_t *flags, const uint32_t *pts, size_t count,
                                                            size_t per_group) {
-    __shared__ uint32_t slots[2][64 * 37];
+    __shared__ uint32_t slots[2][64 * 25];
     const size_t i = (size_t)blockIdx.x * 64 + threadIdx.x;
     if (i >= count) return;
     uint32_t w[36];
     ld_words(w, pts + i * G1P_WORDS, 9);
     g1q p;
     g1q_load_std(p, w);
-    LdsSlot orig{slots[0] + threadIdx.x * 37}, base{slots[1] + threadIdx.x * 37};
+    LdsSlot orig{slots[0] + threadIdx.x * 25}, base{slots[1] + threadIdx.x * 25};
     if (!g1_in_subgroup(p, orig, base)) atomicOr(flags + i / per_group, 1u);
 }
 
