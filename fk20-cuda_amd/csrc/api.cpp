@@ -126,6 +126,16 @@ void fk20::build_host_tables(DevTables &T) {
         memcpy(T.inv2k_w384_std[j], std.l, 32);
         fs_mul(acc, acc, half);
     }
+    // x 2^261 from the Montgomery form x 2^256: five doublings
+    auto digits29 = [](int32_t *z, const uint32_t *mont) {
+        fs v;
+        fs_set(v, mont);
+        for (int i = 0; i < 5; i++) fs_add(v, v, v);
+        memset(z, 0, 12 * 4);
+        fn_from_words(z, v.l);
+    };
+    for (int i = 0; i <= 512; i++) digits29(T.tw29[i], T.tw_mont[i]);
+    for (int j = 0; j < 10; j++) digits29(T.scale29[j], T.inv2k_mont[j]);
 }
 
 namespace {

@@ -16,6 +16,9 @@ struct DevTables {
     uint32_t inv2k_mont[10][8];   // 2^-j mod r, Montgomery form, j = 0..9
     uint32_t inv2k_std[10][8];    // 2^-j mod r, standard form
     uint32_t inv2k_w384_std[10][8];  // 2^-j w^384 = 2^-j w^-128 mod r, standard form
+    // the factors of the scalar transforms (fr.hip.h fn): w^i and 2^-j times 2^261, 9 balanced digits
+    int32_t tw29[513][12];
+    int32_t scale29[10][12];
 };
 
 // Reference ABI element sizes in 32-bit words

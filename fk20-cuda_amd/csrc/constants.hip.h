@@ -52,6 +52,8 @@ static constexpr uint32_t FR_RINV = 0xffffffffu;  // -r^-1 mod 2^32
 static constexpr uint32_t FR_R2[8] = {0xf3f29c6du, 0xc999e990u, 0x87925c23u, 0x2b6cedcbu, 0x7254398fu, 0x05d31496u, 0x9f59ff11u, 0x0748d9d9u};  // 2^512 mod r
 static constexpr uint32_t FR_ONE[8] = {0xfffffffeu, 0x00000001u, 0x00034802u, 0x5884b7fau, 0xecbc4ff5u, 0x998c4fefu, 0xacc5056fu, 0x1824b159u};  // 2^256 mod r
 static constexpr uint32_t FR_RM2[8] = {0xffffffffu, 0xfffffffeu, 0xfffe5bfeu, 0x53bda402u, 0x09a1d805u, 0x3339d808u, 0x299d7d48u, 0x73eda753u};  // r - 2 (Fermat inverse exponent)
+// Fr of the transforms: 9 x 29-bit digits, Montgomery radix 2^261
+static constexpr int32_t FN_RT[9] = {-1, 8, 6881344, 79165952, 41921220, -201589969, 182399769, -174404528, -7597479};  // -r: digit 0 is -1
 static constexpr uint32_t FP_PM2[12] = {0xffffaaa9u, 0xb9feffffu, 0xb153ffffu, 0x1eabfffeu, 0xf6b0f624u, 0x6730d2a0u, 0xf38512bfu, 0x64774b84u, 0x434bacd7u, 0x4b1ba7b6u, 0x397fe69au, 0x1a0111eau};  // p - 2 (Fermat inverse exponent)
 
 }  // namespace fk20

@@ -26,6 +26,7 @@
 #include "common.hip.h"
 #include "fast.hip.h"
 #include "kutil.hip.h"
+#include "ntt.hip.h"
 
 namespace fk20 {
 
@@ -292,55 +293,39 @@ __device__ __forceinline__ int toeplitz_src_T(unsigned i, unsigned j, unsigned N
     return (int)(31 - i + 16 * (j - (k + 2)));
 }
 
-// One (row, i) NTT of size n2 <= 512 per workgroup of 256 threads (n2/2 of them active).
-__global__ void __launch_bounds__(256) k_toeplitz_fft_multi(Launch L, const DevTables *T) {
-    __shared__ fs lds[512];
+template <unsigned LOGN, bool WIDE>
+__device__ __forceinline__ void toeplitz_fft(uint32_t *lds, const Item &it, unsigned local, const DevTables *T) {
+    constexpr unsigned n = 1u << LOGN, lanes = n / 8, N = 8 * n;
+    const unsigned sub = threadIdx.x / lanes, t = threadIdx.x % lanes;
+    const unsigned id = WIDE ? local : local * (64 / lanes) + sub, i = id % 16;  // 16 divides into whole waves
+    const size_t row = id / 16;
+    const uint32_t *poly = it.poly + row * N * FR_WORDS;
+    uint32_t *out = it.tcT + ((size_t)i * it.rows + row) * FR_WORDS;
+    // the reference's order (k_ref_rows) applies 1/n2 inside the inverse transform
+    const bool scaled = it.scale_tc && !(it.rowflag && it.rowflag[row * it.flag_stride]);
+    const auto load = [&](unsigned e, fn &x) {
+        const int src = toeplitz_src_T(i, e, N);
+        uint32_t w[8] = {0};
+        if (src >= 0) ld_words(w, poly + (size_t)src * FR_WORDS, 2);
+        fn_unpack(x, w);
+    };
+    const auto store = [&](unsigned k, const uint32_t *w) {
+        st_words(out + (size_t)k * 16 * it.rows * FR_WORDS, w, 2);
+    };
+    if constexpr (!WIDE) ntt<LOGN, false>(lds + sub * n * 9, t, scaled ? LOGN : 0, T, load, store);
+    else if (threadIdx.x < n / 2) ntt_wide<LOGN, false>(lds, scaled ? LOGN : 0, T, load, store);
+}
+
+// The (row, i) transforms of the items, 512 / n2 per wave; WIDE: one per workgroup of 256 threads
+// (whole waves of which leave before the first barrier where n2 is smaller).
+template <bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 256 : 64, 2) k_toeplitz_fft_multi(Launch L, const DevTables *T) {
+    __shared__ uint32_t lds[WIDE ? 512 * 9 : NTT_LDS_WORDS];
     unsigned local;
     const Item &it = L.item[find_item(L, blockIdx.x, local)];
-    const unsigned logn = it.logn2, n = 1u << logn, half = n / 2, N = it.N;
-    const unsigned t = threadIdx.x;
-    const unsigned i = local % 16;
-    const size_t row = local / 16;
-    const uint32_t *poly = it.poly + row * N * FR_WORDS;
-    if (t < half) {
-        for (unsigned e = t; e < n; e += half) {
-            const int src = toeplitz_src_T(i, e, N);
-            fs a;
-            fs_zero(a);
-            if (src >= 0) {
-                uint32_t w[8];
-                ld_words(w, poly + (size_t)src * FR_WORDS, 2);
-#pragma unroll
-                for (int q = 0; q < 8; q++) a.l[q] = w[q];
-                fs_to_mont(a, a);
-            }
-            lds[bitrev(e, logn)] = a;
-        }
-    }
-    __syncthreads();
-    for (unsigned s = 0; s < logn; s++) {
-        if (t < half) {
-            const unsigned h = 1u << s, j = t & (h - 1);
-            const unsigned l = ((t >> s) << (s + 1)) + j, r = l + h;
-            fs x = lds[r], y = lds[l], w;
-            fs_set(w, T->tw_mont[j << (8 - s)]);
-            fs_mul(x, x, w);
-            fs_add(lds[l], y, x);
-            fs_sub(lds[r], y, x);
-        }
-        __syncthreads();
-    }
-    fs scale;
-    fs_set(scale, T->inv2k_mont[logn]);
-    if (t < half) {
-        for (unsigned e = t; e < n; e += half) {
-            fs a = lds[e];
-            // the reference's order (k_ref_rows) applies 1/n2 inside the inverse transform
-            if (it.scale_tc && !(it.rowflag && it.rowflag[(size_t)row * it.flag_stride])) fs_mul(a, a, scale);
-            fs_from_mont(a, a);
-            st_words(it.tcT + (((size_t)e * 16 + i) * it.rows + row) * FR_WORDS, a.l, 2);
-        }
-    }
+    if (it.logn2 == 9) toeplitz_fft<9, WIDE>(lds, it, local, T);
+    else if (it.logn2 == 8) toeplitz_fft<8, WIDE>(lds, it, local, T);
+    else toeplitz_fft<7, WIDE>(lds, it, local, T);
 }
 
 // ---------------------------------------------------------------- window-table MSM
@@ -737,6 +722,20 @@ static unsigned set_blocks(Launch &L, const unsigned *per_item) {
     }
     return total;
 }
+// Toeplitz coefficients and their transforms, of every item
+static void launch_toeplitz_multi(Launch &L, const DevTables *T, hipStream_t s) {
+    unsigned per[MAX_ITEMS];
+    for (unsigned k = 0; k < L.nitems; k++) per[k] = L.item[k].rows * 16 >> (9 - L.item[k].logn2);
+    unsigned total = set_blocks(L, per);
+    if (total > NTT_WIDE_WAVES) {
+        hipLaunchKernelGGL(k_toeplitz_fft_multi<false>, dim3(total), dim3(64), 0, s, L, T);
+        return;
+    }
+    for (unsigned k = 0; k < L.nitems; k++) per[k] = L.item[k].rows * 16;
+    total = set_blocks(L, per);
+    if (total) hipLaunchKernelGGL(k_toeplitz_fft_multi<true>, dim3(total), dim3(256), 0, s, L, T);
+}
+
 
 // ---- direct schedule
 
@@ -826,7 +825,7 @@ hipError_t launch_batch(const Launch &base, const DevTables *T, const uint32_t *
                         uint64_t chain_wait, const DirectPlan &direct, unsigned levels) {
     if (chain && !K.chain) return hipErrorInvalidValue;
     Launch L = base;
-    unsigned per[MAX_ITEMS], lmax = 0;
+    unsigned per[MAX_ITEMS], lmax = 0, total;
     for (unsigned k = 0; k < L.nitems; k++) lmax = std::max(lmax, L.item[k].logn2);
     if (chain) {
         Chain C;
@@ -836,9 +835,7 @@ hipError_t launch_batch(const Launch &base, const DevTables *T, const uint32_t *
         hipLaunchKernelGGL(k_chain_reset, dim3(L.nitems), dim3(256), 0, s, C);
     }
     // Toeplitz + NTT
-    for (unsigned k = 0; k < L.nitems; k++) per[k] = L.item[k].rows * 16;
-    unsigned total = set_blocks(L, per);
-    if (total) hipLaunchKernelGGL(k_toeplitz_fft_multi, dim3(total), dim3(256), 0, s, L, T);
+    launch_toeplitz_multi(L, T, s);
     hook(LK_TOEPLITZ_FFT);
     // MSM
     const unsigned lp = msm_lanes(L);
@@ -1042,8 +1039,7 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
         if (kind == PLAIN_HEXT_FFT2H_FFT) {
             hipLaunchKernelGGL(K.plain_load, dim3(n * rg), dim3(64), 0, s, D, in, rows, logn, 1u, scale);
         } else {
-            per[0] = rows * 16;
-            hipLaunchKernelGGL(k_toeplitz_fft_multi, dim3(set_blocks(L, per)), dim3(256), 0, s, L, T);
+            launch_toeplitz_multi(L, T, s);
             hipError_t e = launch_msm_plain_T(D, tcT, xpk, digits, rows, n, s);
             if (e != hipSuccess) return e;
             // rows of a setup outside G1 take the reference's order from the MSM output on,

@@ -1,11 +1,10 @@
 // Fr kernels: Toeplitz coefficient layout, Fr NTT of size 128/256/512, fused Toeplitz+NTT,
 // and element-wise Fr arithmetic.
 //
-// NTT: one transform per workgroup of n/2 threads (one radix-2 butterfly per thread and
-// stage), data staged in LDS in Montgomery form, decimation in time from a bit-reversed
-// load to a natural-order result -- the same natural-order DFT as fr_fft.cu:28-168
-// (forward) and fr_fft.cu:172-300 (inverse, scaled by 1/n).
+// NTT (ntt.hip.h): the same natural-order DFT as fr_fft.cu:28-168 (forward) and
+// fr_fft.cu:172-300 (inverse, scaled by 1/n).
 #include "common.hip.h"
+#include "ntt.hip.h"
 
 namespace fk20 {
 
@@ -37,7 +36,7 @@ __global__ void __launch_bounds__(256) k_toeplitz(uint4 *tc, const uint4 *poly, 
     tc[2 * e + 1] = hi;
 }
 
-// ---------------------------------------------------------------- NTT core
+// ---------------------------------------------------------------- transforms
 
 __device__ __forceinline__ void fs_load(fs &a, const uint32_t *p) {
     const uint4 *q = reinterpret_cast<const uint4 *>(p);
@@ -52,82 +51,56 @@ __device__ __forceinline__ void fs_store(uint32_t *p, const fs &a) {
     q[1] = make_uint4(a.l[4], a.l[5], a.l[6], a.l[7]);
 }
 
-// In-place radix-2 DIT over LDS holding n = 2^logn Montgomery values in bit-reversed
-// order; leaves the natural-order transform.  Stage s uses w_{2^(s+1)}^j = w_512^(j << (8-s)).
-template <bool INV>
-__device__ __forceinline__ void ntt_dit(fs *lds, unsigned logn, const DevTables *T) {
-    const unsigned t = threadIdx.x;
-    for (unsigned s = 0; s < logn; s++) {
-        const unsigned h = 1u << s;
-        const unsigned j = t & (h - 1);
-        const unsigned l = ((t >> s) << (s + 1)) + j, r = l + h;
-        const unsigned idx = j << (8 - s);
-        fs x = lds[r], y = lds[l], w;
-        fs_load(w, T->tw_mont[INV ? 512 - idx : idx]);
-        fs_mul(x, x, w);
-        fs_add(lds[l], y, x);
-        fs_sub(lds[r], y, x);
-        __syncthreads();
-    }
-}
-
-template <unsigned LOGN, bool INV>
-__global__ void __launch_bounds__(256) k_fr_ntt(uint32_t *out, const uint32_t *in, const DevTables *T) {
-    constexpr unsigned n = 1u << LOGN, half = n / 2;
-    __shared__ fs lds[n];
-    const unsigned t = threadIdx.x;
-    in += (size_t)blockIdx.x * n * FR_WORDS;
-    out += (size_t)blockIdx.x * n * FR_WORDS;
-#pragma unroll
-    for (unsigned e = t; e < n; e += half) {
+// count transforms; the spare lanes of the last wave repeat the last one (same loads, same stores).
+// A transform is read before any of it is written, so out may alias in.
+template <unsigned LOGN, bool INV, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? (1u << LOGN) / 2 : 64) k_fr_ntt(uint32_t *out, const uint32_t *in,
+                                                                        unsigned count, const DevTables *T) {
+    constexpr unsigned n = 1u << LOGN, lanes = n / 8;
+    __shared__ uint32_t lds[WIDE ? n * 9 : NTT_LDS_WORDS];
+    const unsigned sub = threadIdx.x / lanes, t = threadIdx.x % lanes;
+    const size_t id = WIDE ? blockIdx.x : min(blockIdx.x * (64 / lanes) + sub, count - 1);
+    const uint32_t *src = in + id * n * FR_WORDS;
+    uint32_t *dst = out + id * n * FR_WORDS;
+    const auto load = [&](unsigned i, fn &x) {
         fs a;
-        fs_load(a, in + (size_t)e * FR_WORDS);
-        fs_to_mont(a, a);
-        lds[bitrev(e, LOGN)] = a;
-    }
-    __syncthreads();
-    ntt_dit<INV>(lds, LOGN, T);
-    fs sc;
-    if (INV) fs_load(sc, T->inv2k_mont[LOGN]);
-#pragma unroll
-    for (unsigned e = t; e < n; e += half) {
-        fs a = lds[e];
-        if (INV) fs_mul(a, a, sc);
-        fs_from_mont(a, a);
-        fs_store(out + (size_t)e * FR_WORDS, a);
-    }
+        fs_load(a, src + (size_t)i * FR_WORDS);
+        fn_unpack(x, a.l);
+    };
+    const auto store = [&](unsigned k, const uint32_t *w) {
+        fs a;
+        fs_set(a, w);
+        fs_store(dst + (size_t)k * FR_WORDS, a);
+    };
+    if constexpr (WIDE) ntt_wide<LOGN, INV>(lds, INV ? LOGN : 0, T, load, store);
+    else ntt<LOGN, INV>(lds + sub * n * 9, t, INV ? LOGN : 0, T, load, store);
 }
 
-// Toeplitz coefficients of one (row, i) built straight into LDS, then the NTT.
-template <unsigned LOGN>
-__global__ void __launch_bounds__(256) k_toeplitz_fft(uint32_t *tc_fft, const uint32_t *poly, unsigned N,
-                                                      const DevTables *T) {
-    constexpr unsigned n = 1u << LOGN, half = n / 2;
-    __shared__ fs lds[n];
-    const unsigned t = threadIdx.x;
-    const unsigned i = blockIdx.x % 16;
-    const size_t row = blockIdx.x / 16;
-    poly += row * N * FR_WORDS;
-    tc_fft += (size_t)blockIdx.x * n * FR_WORDS;
-#pragma unroll
-    for (unsigned e = t; e < n; e += half) {
-        const int src = toeplitz_src(i, e, N);
+// The Toeplitz coefficients of (row, i) straight into the transform.
+template <unsigned LOGN, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? (1u << LOGN) / 2 : 64) k_toeplitz_fft(uint32_t *tc_fft, const uint32_t *poly,
+                                                                              unsigned count, const DevTables *T) {
+    constexpr unsigned n = 1u << LOGN, lanes = n / 8, N = 8 * n;
+    __shared__ uint32_t lds[WIDE ? n * 9 : NTT_LDS_WORDS];
+    const unsigned sub = threadIdx.x / lanes, t = threadIdx.x % lanes;
+    const size_t id = WIDE ? blockIdx.x : min(blockIdx.x * (64 / lanes) + sub, count - 1);
+    const unsigned i = (unsigned)(id % 16);
+    const uint32_t *src = poly + id / 16 * N * FR_WORDS;
+    uint32_t *dst = tc_fft + id * n * FR_WORDS;
+    const auto load = [&](unsigned e, fn &x) {
+        const int c = toeplitz_src(i, e, N);
         fs a;
         fs_zero(a);
-        if (src >= 0) {
-            fs_load(a, poly + (size_t)src * FR_WORDS);
-            fs_to_mont(a, a);
-        }
-        lds[bitrev(e, LOGN)] = a;
-    }
-    __syncthreads();
-    ntt_dit<false>(lds, LOGN, T);
-#pragma unroll
-    for (unsigned e = t; e < n; e += half) {
-        fs a = lds[e];
-        fs_from_mont(a, a);
-        fs_store(tc_fft + (size_t)e * FR_WORDS, a);
-    }
+        if (c >= 0) fs_load(a, src + (size_t)c * FR_WORDS);
+        fn_unpack(x, a.l);
+    };
+    const auto store = [&](unsigned k, const uint32_t *w) {
+        fs a;
+        fs_set(a, w);
+        fs_store(dst + (size_t)k * FR_WORDS, a);
+    };
+    if constexpr (WIDE) ntt_wide<LOGN, false>(lds, 0, T, load, store);
+    else ntt<LOGN, false>(lds + sub * n * 9, t, 0, T, load, store);
 }
 
 // ---------------------------------------------------------------- element-wise Fr ops
@@ -178,13 +151,22 @@ hipError_t launch_toeplitz(uint32_t *tc, const uint32_t *poly, unsigned rows, un
     return hipGetLastError();
 }
 
+template <unsigned LOGN, bool INV>
+static void ntt_launch(uint32_t *out, const uint32_t *in, unsigned count, const DevTables *T, hipStream_t s) {
+    constexpr unsigned n = 1u << LOGN, per = 512 / n;
+    if ((count + per - 1) / per <= NTT_WIDE_WAVES)
+        hipLaunchKernelGGL((k_fr_ntt<LOGN, INV, true>), dim3(count), dim3(n / 2), 0, s, out, in, count, T);
+    else
+        hipLaunchKernelGGL((k_fr_ntt<LOGN, INV, false>), dim3((count + per - 1) / per), dim3(64), 0, s, out, in, count, T);
+}
+
 template <bool INV>
 static hipError_t ntt_dispatch(uint32_t *out, const uint32_t *in, unsigned count, unsigned n,
                                const DevTables *T, hipStream_t s) {
     switch (n) {
-    case 128: hipLaunchKernelGGL((k_fr_ntt<7, INV>), dim3(count), dim3(64), 0, s, out, in, T); break;
-    case 256: hipLaunchKernelGGL((k_fr_ntt<8, INV>), dim3(count), dim3(128), 0, s, out, in, T); break;
-    case 512: hipLaunchKernelGGL((k_fr_ntt<9, INV>), dim3(count), dim3(256), 0, s, out, in, T); break;
+    case 128: ntt_launch<7, INV>(out, in, count, T, s); break;
+    case 256: ntt_launch<8, INV>(out, in, count, T, s); break;
+    case 512: ntt_launch<9, INV>(out, in, count, T, s); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -196,14 +178,23 @@ hipError_t launch_fr_ntt(uint32_t *out, const uint32_t *in, unsigned count, unsi
     return inverse ? ntt_dispatch<true>(out, in, count, n, T, s) : ntt_dispatch<false>(out, in, count, n, T, s);
 }
 
+template <unsigned LOGN>
+static void toeplitz_fft_launch(uint32_t *tc_fft, const uint32_t *poly, unsigned rows, const DevTables *T, hipStream_t s) {
+    constexpr unsigned n = 1u << LOGN, per = 512 / n;
+    const unsigned count = rows * 16;  // a multiple of the transforms per wave
+    if (count / per <= NTT_WIDE_WAVES)
+        hipLaunchKernelGGL((k_toeplitz_fft<LOGN, true>), dim3(count), dim3(n / 2), 0, s, tc_fft, poly, count, T);
+    else
+        hipLaunchKernelGGL((k_toeplitz_fft<LOGN, false>), dim3(count / per), dim3(64), 0, s, tc_fft, poly, count, T);
+}
+
 hipError_t launch_toeplitz_fft(uint32_t *tc_fft, const uint32_t *poly, unsigned rows, unsigned N,
                                const DevTables *T, hipStream_t s) {
     if (!rows) return hipSuccess;
-    const unsigned blocks = rows * 16;
     switch (N) {
-    case 1024: hipLaunchKernelGGL(k_toeplitz_fft<7>, dim3(blocks), dim3(64), 0, s, tc_fft, poly, N, T); break;
-    case 2048: hipLaunchKernelGGL(k_toeplitz_fft<8>, dim3(blocks), dim3(128), 0, s, tc_fft, poly, N, T); break;
-    case 4096: hipLaunchKernelGGL(k_toeplitz_fft<9>, dim3(blocks), dim3(256), 0, s, tc_fft, poly, N, T); break;
+    case 1024: toeplitz_fft_launch<7>(tc_fft, poly, rows, T, s); break;
+    case 2048: toeplitz_fft_launch<8>(tc_fft, poly, rows, T, s); break;
+    case 4096: toeplitz_fft_launch<9>(tc_fft, poly, rows, T, s); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -140,6 +140,11 @@ def main():
     out.append(carr("FR_R2", limbs(rr * rr % R, 32, FR_N)) + "  // 2^512 mod r")
     out.append(carr("FR_ONE", limbs(rr, 32, FR_N)) + "  // 2^256 mod r")
     out.append(carr("FR_RM2", limbs(R - 2, 32, FR_N)) + "  // r - 2 (Fermat inverse exponent)")
+    # Fr of the transforms: 9 signed digits of 29 bits, radix 2^261
+    rt = balanced(-R, 9, 29)
+    assert rt[0] == -1
+    out.append("// Fr of the transforms: 9 x 29-bit digits, Montgomery radix 2^261")
+    out.append(iarr("FN_RT", rt) + "  // -r: digit 0 is -1")
     out.append(carr("FP_PM2", limbs(P - 2, 32, 12)) + "  // p - 2 (Fermat inverse exponent)")
     out.append("")
     out.append("}  // namespace fk20")
