@@ -24,7 +24,7 @@ static __device__ DevTables g_tables_dev;
 static constexpr size_t PROG_OPS_CAP = (size_t)1 << 16;  // words; the programs take about 48 K
 static __device__ uint32_t g_prog_ops[PROG_OPS_CAP];
 static __device__ uint32_t g_prog_index[TW_INDEX_SIZE];
-static constexpr size_t DIRECT_WORDS_CAP = (size_t)1 << 19;  // the plans take 498 822
+static constexpr size_t DIRECT_WORDS_CAP = (size_t)1 << 21;  // the plans take 1 406 473
 static __device__ uint32_t g_direct_words[DIRECT_WORDS_CAP];
 
 // Workspace of fk20_poly2h_fft_noalloc, the entry point for callers that cannot allocate:
@@ -283,8 +283,13 @@ int fr_ift(fk20_fr_t *output, const fk20_fr_t *input, unsigned count, unsigned n
 // Scratch of the drop-in transforms besides the points: one flag per row, padded, and the direct
 // schedule's products when the batch is small enough for it.
 static size_t flag_bytes(unsigned rows) { return ((size_t)rows * 4 + 255) & ~(size_t)255; }
-static size_t transform_product_bytes(const DeviceState *st, unsigned rows, unsigned logn) {
-    return rows <= DIRECT_MAX_ROWS ? direct_product_bytes(st->direct, rows, logn, 2) : 0;
+static size_t transform_product_bytes(const DeviceState *st, unsigned rows, unsigned logn, bool both = false) {
+    Launch L;
+    L.nitems = 1;
+    L.item[0].rows = rows;
+    L.item[0].logn2 = logn;
+    const unsigned levels = direct_choose(L, st->direct, both, DIRECT_ANY);
+    return levels ? direct_product_bytes(st->direct, rows, logn, levels) : 0;
 }
 
 // The G1 transforms run column-batched (lanes = transforms) through D in scratch, so the
@@ -349,7 +354,7 @@ int fk20_hext_fft2h_fft(fk20_g1p_t *h_fft, const fk20_g1p_t *hext_fft, unsigned 
     if (rc) return rc;
     void *D;
     const size_t d_bytes = (size_t)rows * n2 * 144, f_bytes = flag_bytes(rows);
-    const size_t p_bytes = transform_product_bytes(st, rows, log2u(n2));
+    const size_t p_bytes = transform_product_bytes(st, rows, log2u(n2), true);
     rc = device_scratch(st, d_bytes + f_bytes + p_bytes, &D);
     if (rc) return rc;
     char *base = reinterpret_cast<char *>(D);
@@ -363,13 +368,14 @@ int fk20_hext_fft2h_fft(fk20_g1p_t *h_fft, const fk20_g1p_t *hext_fft, unsigned 
 // scalar multiplication per point) and the transforms column-batched over the rows.
 // Workspace: D, the packed bases, the subgroup flag of the bases (one 256-byte slot), tcT and the
 // MSM digits, in that order; tcT and the digits are dead after the MSM, and a small batch's
-// transforms keep their products there.
+// transforms keep their products there and past their end.
 static size_t poly2h_scratch_bytes(unsigned rows, unsigned n2) {
     return (size_t)rows * 16 * n2 * 32 + (size_t)rows * n2 * 144 + (size_t)16 * n2 * 144 + 256 +
            msm_plain_digit_bytes(rows, n2);
 }
 
-static int poly2h_fft_in(void *scratch, DeviceState *st, fk20_g1p_t *h_fft, const fk20_fr_t *poly,
+// more: bytes of scratch past poly2h_scratch_bytes, for a small batch's products
+static int poly2h_fft_in(void *scratch, size_t more, DeviceState *st, fk20_g1p_t *h_fft, const fk20_fr_t *poly,
                          const fk20_g1p_t *xext_fft, unsigned rows, unsigned n2, fk20_stream_t stream) {
     const size_t tc_bytes = (size_t)rows * 16 * n2 * 32;
     const size_t d_bytes = (size_t)rows * n2 * 144;
@@ -384,7 +390,7 @@ static int poly2h_fft_in(void *scratch, DeviceState *st, fk20_g1p_t *h_fft, cons
     FK20_TRY(launch_std_to_packed(xpk, W(xext_fft), (size_t)16 * n2, s));
     return hip_status(launch_plain(PLAIN_POLY2H_FFT, W(h_fft), W(poly), xpk, rows, log2u(n2), D, tcT, digits,
                                    flag, st->tables, st->prog, s, st->direct, tcT,
-                                   tc_bytes + msm_plain_digit_bytes(rows, n2)));
+                                   tc_bytes + msm_plain_digit_bytes(rows, n2) + more));
 }
 
 int fk20_poly2h_fft(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20_g1p_t *xext_fft, unsigned rows,
@@ -396,9 +402,11 @@ int fk20_poly2h_fft(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20_g1p_t *
     int rc = device_state(&st);
     if (rc) return rc;
     void *scr;
-    rc = device_scratch(st, poly2h_scratch_bytes(rows, n2), &scr);
+    const size_t bytes = poly2h_scratch_bytes(rows, n2), dead = (size_t)rows * 16 * n2 * 32 + msm_plain_digit_bytes(rows, n2);
+    const size_t products = transform_product_bytes(st, rows, log2u(n2), true), more = products > dead ? products - dead : 0;
+    rc = device_scratch(st, bytes + more, &scr);
     if (rc) return rc;
-    return poly2h_fft_in(scr, st, h_fft, poly, xext_fft, rows, n2, stream);
+    return poly2h_fft_in(scr, more, st, h_fft, poly, xext_fft, rows, n2, stream);
 }
 
 // The same launch sequence with its workspace in this device's fixed `scratch` array: no
@@ -414,7 +422,8 @@ int fk20_poly2h_fft_noalloc(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20
     DeviceState *st;
     int rc = device_state(&st);
     if (rc) return rc;
-    return poly2h_fft_in(st->noalloc, st, h_fft, poly, xext_fft, rows, n2, stream);
+    const size_t more = NOALLOC_SCRATCH_BYTES - poly2h_scratch_bytes(rows, n2);
+    return poly2h_fft_in(st->noalloc, more, st, h_fft, poly, xext_fft, rows, n2, stream);
 }
 
 int fk20_setup2xext_fft(fk20_g1p_t *xext_fft, const fk20_g1p_t *setup, unsigned N, fk20_stream_t stream) {

@@ -552,7 +552,6 @@ int fk20_ctx_set_graph(fk20_ctx_t *c, int enable) {
 }
 
 static hipError_t grow_work(fk20_ctx *c, size_t bytes);
-static size_t direct_extra_bytes(const fk20_ctx *c, unsigned rows, unsigned logn);
 
 // Window tables of nbases points (standard-form g1p_t, device), each first multiplied by the
 // standard-form scalar `scale` (device, 8 words).  Fills st.table / st.inf.  *outside: some
@@ -711,9 +710,35 @@ int fk20_setup_unload(fk20_ctx_t *c, int id) {
     return FK20_OK;
 }
 
-static size_t direct_extra_bytes(const fk20_ctx *c, unsigned rows, unsigned logn) {
-    const size_t need = direct_product_bytes(c->direct, rows, logn, 2), tc = ((size_t)rows << logn) * 16 * 32;
+// Workspace besides tcT that an item's products need at `levels` (three levels' always fit in tcT,
+// which is dead after the MSM).
+static size_t direct_extra_bytes(const fk20_ctx *c, unsigned rows, unsigned logn, unsigned levels) {
+    const size_t need = direct_product_bytes(c->direct, rows, logn, levels), tc = ((size_t)rows << logn) * 16 * 32;
     return need > tc ? need : 0;
+}
+
+// Levels of the direct schedule for a batch whose workspace has `spare` bytes beyond the items' own
+// (0: the radix-2^2 launches), and the bytes of it that they take.
+static unsigned direct_levels(const fk20_ctx *c, const Launch &L, size_t spare, size_t *bytes) {
+    unsigned allowed = DIRECT_ANY;
+    while (true) {
+        const unsigned levels = direct_choose(L, c->direct, true, allowed);
+        *bytes = 0;
+        for (unsigned k = 0; levels && k < L.nitems; k++)
+            *bytes += direct_extra_bytes(c, L.item[k].rows, L.item[k].logn2, levels);
+        if (*bytes <= spare) return levels;
+        allowed &= ~(1u << levels);
+    }
+}
+
+static Launch items_launch(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n) {
+    Launch L;
+    L.nitems = n;
+    for (unsigned k = 0; k < n; k++) {
+        L.item[k].rows = items[k].rows;
+        L.item[k].logn2 = c->setups[items[k].setup_id].logn2();
+    }
+    return L;
 }
 
 static hipError_t grow_work(fk20_ctx *c, size_t bytes) {
@@ -737,20 +762,13 @@ static hipError_t grow_work(fk20_ctx *c, size_t bytes) {
 int fk20_ctx_reserve(fk20_ctx_t *c, unsigned rows, unsigned N) {
     if (!c || !valid_N(N)) return FK20_EINVAL;
     std::lock_guard<std::mutex> lk(c->mu);
-    const size_t bytes = fk20_rows_workspace_bytes(rows, N);
-    const unsigned logn = N == 1024 ? 7 : N == 2048 ? 8 : 9;
-    return status_of(grow_work(c, bytes + (rows <= DIRECT_MAX_ROWS ? direct_extra_bytes(c, rows, logn) : 0)));
-}
-
-// Extra workspace of a batch's items in the two-level direct schedule: the products of an item
-// that its tcT cannot hold (three levels' always fit there).
-static size_t items_direct_bytes(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n) {
-    size_t total = 0;
-    for (unsigned k = 0; k < n; k++) {
-        if (items[k].rows > DIRECT_MAX_ROWS) return 0;
-        total += direct_extra_bytes(c, items[k].rows, c->setups[items[k].setup_id].logn2());
-    }
-    return total;
+    Launch L;
+    L.nitems = rows ? 1 : 0;
+    L.item[0].rows = rows;
+    L.item[0].logn2 = N == 1024 ? 7 : N == 2048 ? 8 : 9;
+    size_t more = 0;
+    if (rows) (void)direct_levels(c, L, ~(size_t)0, &more);
+    return status_of(grow_work(c, fk20_rows_workspace_bytes(rows, N) + more));
 }
 
 static size_t items_workspace_bytes(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n) {
@@ -771,7 +789,7 @@ static bool same_items(const std::vector<fk20_batch_item_t> &a, const fk20_batch
 // Carves each item's workspace (tcT, D, chain flags, control block) from w and launches the
 // batch on s.
 static hipError_t enqueue_launch(fk20_ctx *c, const fk20_batch_item_t *items, unsigned n, hipStream_t s,
-                                 LaunchHook hook, char *w, bool chain, bool direct = false, char *extra = nullptr) {
+                                 LaunchHook hook, char *w, bool chain, unsigned levels = 0, char *extra = nullptr) {
     Launch L;
     memset(&L, 0, sizeof L);
     L.nitems = n;
@@ -803,12 +821,10 @@ static hipError_t enqueue_launch(fk20_ctx *c, const fk20_batch_item_t *items, un
     // the persistent form runs radix-2 stages: the schedule's width and occupancy, radix 2
     const StageKernels *K = stage_kernels(c->sch_wnaf, chain ? false : c->sch_r22, c->sch_occ);
     if (!K) return hipErrorInvalidValue;
-    // small batches: the direct schedule, its products in tcT (dead after the MSM) or in `extra`
-    const bool two = extra != nullptr || !items_direct_bytes(c, items, n);
-    const unsigned levels = direct && K->direct ? direct_choose(L, c->direct, true, two) : 0;
+    // small batches: the direct schedule, its products in tcT or in `extra`
     for (unsigned k = 0; levels && k < n; k++) {
         Item &it = L.item[k];
-        const size_t more = levels == 2 ? direct_extra_bytes(c, it.rows, it.logn2) : 0;
+        const size_t more = direct_extra_bytes(c, it.rows, it.logn2, levels);
         it.P = more ? reinterpret_cast<uint32_t *>(extra) : it.tcT;
         extra += more;
     }
@@ -827,17 +843,6 @@ static bool worth_splitting(const fk20_ctx *c, const fk20_batch_item_t *items, u
     return mixed && groups >= 16;
 }
 
-// Whether the batch's transforms take the direct schedule.
-static bool direct_items(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n, bool two) {
-    Launch L;
-    L.nitems = n;
-    for (unsigned k = 0; k < n; k++) {
-        L.item[k].rows = items[k].rows;
-        L.item[k].logn2 = c->setups[items[k].setup_id].logn2();
-    }
-    return direct_choose(L, c->direct, true, two) != 0;
-}
-
 static hipError_t enqueue_items(fk20_ctx *c, const fk20_batch_item_t *items, unsigned n, hipStream_t s,
                                 LaunchHook hook, void *workspace = nullptr) {
     // the persistent form only on the context's own workspace (fk20_prove_batch reads its
@@ -847,17 +852,16 @@ static hipError_t enqueue_items(fk20_ctx *c, const fk20_batch_item_t *items, uns
     unsigned groups = 0;
     for (unsigned k = 0; k < n; k++) groups += (items[k].rows + 63) / 64;
     // the context path with at least two 64-row groups, launches not timed one by one
-    // small batches run unsplit in the direct schedule (their halves would not be faster)
-    char *extra = nullptr;
-    bool direct = false;
+    // small batches run unsplit in the direct schedule, with what the context's workspace has
+    // beyond the items' own for its products
+    unsigned levels = 0;
+    const size_t base = items_workspace_bytes(c, items, n);
     if (!chain && c->sch_r22) {
-        const size_t base = items_workspace_bytes(c, items, n);
-        const size_t more = items_direct_bytes(c, items, n);
-        if (!workspace && more && c->work_bytes >= base + more) extra = w + base;
-        direct = direct_items(c, items, n, extra || !more);
+        size_t bytes;
+        levels = direct_levels(c, items_launch(c, items, n), workspace ? 0 : c->work_bytes - base, &bytes);
     }
-    if (workspace || c->nsub < 2 || groups < 2 || hook.fn || direct || !worth_splitting(c, items, n, groups))
-        return enqueue_launch(c, items, n, s, hook, w, chain, direct, extra);
+    if (workspace || c->nsub < 2 || groups < 2 || hook.fn || levels || !worth_splitting(c, items, n, groups))
+        return enqueue_launch(c, items, n, s, hook, w, chain, levels, w + base);
     // halves: each item's rows split at a 64-row boundary (items of one group go to the first)
     fk20_batch_item_t half[2][MAX_ITEMS];
     unsigned nh[2] = {0, 0};
@@ -917,11 +921,15 @@ int fk20_prove_batch(fk20_ctx_t *c, const fk20_batch_item_t *items, unsigned nit
     if (v.empty()) return FK20_OK;
     const unsigned n = (unsigned)v.size();
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    // what is reserved is not grown for the direct schedule's extra products (three levels do
-    // without); a workspace that has to grow anyway takes them along
+    // what is reserved is not grown for the direct schedule's products (three levels do without);
+    // a workspace that has to grow anyway takes them along
     hipError_t e = hipSuccess;
     const size_t base = items_workspace_bytes(c, v.data(), n);
-    if (c->work_bytes < base) e = grow_work(c, base + items_direct_bytes(c, v.data(), n));
+    if (c->work_bytes < base) {
+        size_t more = 0;
+        (void)direct_levels(c, items_launch(c, v.data(), n), ~(size_t)0, &more);
+        e = grow_work(c, base + more);
+    }
     if (e == hipSuccess) e = order_before(c, s);
     if (e != hipSuccess) return status_of(e);
     if (c->timing) {

@@ -3,20 +3,21 @@
 //
 // A twiddle ladder takes about as long on an idle chip as on a busy one, so a small batch's
 // transform lasts the number of ladders on its longest path: four generic and four w^128 ones
-// per transform of 512 in the radix-2^2 schedule (schedule.hip.h).  Here a transform is two or
+// per transform of 512 in the radix-2^2 schedule (schedule.hip.h).  Here a transform is one to
 // three mixed-radix steps, each of them one round of ladders.  A step of radix a on blocks of
 // N = a b points computes
 //     Y[j][m] = sum_t w_N^(j (m + b t)) X[m + b t],     j, t < a, m < b,
 // (the twiddles of the next step included), in three launches:
 //  * k_direct_split, in place: for every m the a points become the sum of all, the difference of
 //    the two halves' sums, .., the a/2 differences X[t] - X[t + a/2]: log2(a) additions by a
-//    lanes at once.  Output j with j = 2^v odd only needs the a / 2^(v+1) differences of level v.
+//    lanes at once (radix above 32: two launches, the second on the sums that are left).  Output j with j = 2^v odd only needs the a / 2^(v+1) differences of level v.
 //  * k_direct_products: one ladder per distinct (point, exponent) into P[slot][row]; exponents
 //    are taken below 256 (w^256 = -1), and all products of one exponent are next to each other,
 //    so a wave runs one program over several points times the batch's rows.
 //  * k_direct_sums: every output adds its a / 2^(v+1) products.
 // The blocks' size-b transforms follow with root w_N^a.  Radix 16 takes 5.3 ladders per point,
-// a last step of radix 32 3.5 (radix-2^2: 2.3 and 1.2 short ones per point, in eight rounds).
+// a last step of radix 32 3.5, a single step 57 for 512 points and 14 for 128 (radix-2^2: 2.3 and
+// 1.2 short ones per point, in eight rounds).
 //
 // Shared by the kernels, the launchers and, compiled by g++, the CPU tests.
 #pragma once
@@ -33,7 +34,7 @@ namespace fk20 {
 // of the drop-ins (in the positions their load and output kernels use).
 enum DirectKind { DIRECT_IFFT_HALF = 0, DIRECT_FFT_HALF = 1, DIRECT_FFT = 2, DIRECT_IFFT = 3 };
 static constexpr unsigned DIRECT_KINDS = 4;
-// levels 2: [16, 32], [16, 16], [8, 16] for n = 512, 256, 128; levels 3: [8, 8, 8], [4, 8, 8],
+// levels 1: [n]; levels 2: [16, 32], [16, 16], [8, 16] for n = 512, 256, 128; levels 3: [8, 8, 8], [4, 8, 8],
 // [4, 4, 8]
 static constexpr unsigned DIRECT_MAX_STEPS = 3;
 
@@ -45,6 +46,7 @@ FK20_HD unsigned direct_row_lanes(unsigned rows) {
 }
 
 FK20_HD unsigned direct_radix_log(unsigned logn, unsigned levels, unsigned step) {
+    if (levels == 1) return logn;
     if (levels == 2) return step == 0 ? (logn == 7 ? 3u : 4u) : (logn == 9 ? 5u : 4u);
     return step == 0 ? (logn == 9 ? 3u : 2u) : step == 1 ? (logn == 7 ? 2u : 3u) : 3u;
 }
@@ -53,19 +55,27 @@ FK20_HD unsigned direct_radix_log(unsigned logn, unsigned levels, unsigned step)
 struct DirectStep {
     uint32_t loga, logb, logblocks;  // radix, stride, number of blocks (log2)
     uint32_t in_map;                 // bit 0: position of index i is bitrev(i); bit 1: upper half zero
+    uint32_t log_lanes, sum_words;   // lanes per output of the sums (log2), words per output
     uint32_t nprod, prod;            // products: position | exponent << 16, in slot order
-    uint32_t nout, sums;             // outputs: DIRECT_SUM_WORDS each
+    uint32_t nout, sums;             // outputs
     uint32_t nwaves[7], waves[7];    // for 2^k products per wave: first slot | count << 16 (k = 0..6)
 };
 static constexpr unsigned DIRECT_STEP_WORDS = sizeof(DirectStep) / 4;
-// an output: its position, then up to 16 terms: slot | sign << 31, DIRECT_NONE past the last
-static constexpr unsigned DIRECT_SUM_WORDS = 20, DIRECT_SUM_FIRST = 4;
+// an output's words: its position, three unused, then its terms: slot | sign << 31, DIRECT_NONE
+// past the last, to the step's longest sum rounded up to a multiple of the lanes
+static constexpr unsigned DIRECT_SUM_FIRST = 4;
+// The split of radix a = 2^loga and stride 2^logb in passes of at most 32 points: pass 0 takes
+// up to 5 levels, pass 1 the rest on the sums it leaves, at the lowest 2^(loga + logb - 5) indices.
+FK20_HD unsigned direct_split_passes(unsigned loga) { return loga > 5 ? 2 : 1; }
+FK20_HD unsigned direct_split_log(unsigned loga, unsigned pass) {
+    return pass == 0 ? (loga > 5 ? 5 : loga) : loga - 5;
+}
 static constexpr uint32_t DIRECT_NONE = 0xffffffffu;
 // index of the step record of (logn, kind, levels, step) in the record table at the words' start
 FK20_HD unsigned direct_record(unsigned logn, unsigned kind, unsigned levels, unsigned step) {
-    return (((logn - 7) * DIRECT_KINDS + kind) * 2 + (levels - 2)) * DIRECT_MAX_STEPS + step;
+    return (((logn - 7) * DIRECT_KINDS + kind) * DIRECT_MAX_STEPS + (levels - 1)) * DIRECT_MAX_STEPS + step;
 }
-static constexpr unsigned DIRECT_RECORDS = 3 * DIRECT_KINDS * 2 * DIRECT_MAX_STEPS;
+static constexpr unsigned DIRECT_RECORDS = 3 * DIRECT_KINDS * DIRECT_MAX_STEPS * DIRECT_MAX_STEPS;
 
 }  // namespace fk20
 
@@ -73,7 +83,6 @@ static constexpr unsigned DIRECT_RECORDS = 3 * DIRECT_KINDS * 2 * DIRECT_MAX_STE
 
 #include <algorithm>
 #include <cstring>
-#include <map>
 #include <vector>
 
 namespace fk20 {
@@ -103,11 +112,11 @@ inline DirectStep direct_build_step(std::vector<uint32_t> &words, unsigned logn,
     auto position = [&](unsigned i) { return (r.in_map & 1u) ? direct_bitrev(i, logn) : i; };
 
     struct Out {
-        unsigned pos;
-        std::vector<std::pair<unsigned, unsigned>> terms;  // (position << 8 | exponent, sign)
+        unsigned pos, first, terms;  // terms in `terms`: position << 8 | exponent | sign << 31
     };
     std::vector<Out> outs;
-    std::map<unsigned, unsigned> slot;  // position << 8 | exponent -> slot
+    std::vector<uint32_t> terms, slot((size_t)n << 8, DIRECT_NONE);  // position << 8 | exponent -> slot
+    std::vector<unsigned> keys;
     for (unsigned blk = 0; blk < (1u << r.logblocks); blk++)
         for (unsigned j = 0; j < a; j++) {
             // output index of this block's Y[j][0]: the digits so far, least significant first
@@ -123,6 +132,7 @@ inline DirectStep direct_build_step(std::vector<uint32_t> &words, unsigned logn,
             if (last && kind == DIRECT_IFFT_HALF && k >= n / 2) continue;
             for (unsigned m = 0; m < b; m++) {
                 Out o;
+                o.first = (unsigned)terms.size();
                 if (!last) o.pos = ((blk << r.loga | j) << r.logb) | m;
                 else o.pos = kind == DIRECT_FFT || kind == DIRECT_FFT_HALF ? direct_bitrev(k, logn) : k;
                 // level v differences: positions t in [a >> (v+1), a >> v) of the split array;
@@ -137,18 +147,21 @@ inline DirectStep direct_build_step(std::vector<uint32_t> &words, unsigned logn,
                     unsigned e = (j * (m + b * (t - lo))) % N * (512 / N);
                     if (inverse) e = (512 - e) % 512;
                     const unsigned p = position(blk * N + m + b * t);
-                    o.terms.push_back({p << 8 | (e & 255u), e >> 8});
-                    slot[p << 8 | (e & 255u)] = 0;
+                    const unsigned key = p << 8 | (e & 255u);
+                    terms.push_back(key | (e >> 8) << 31);
+                    if (slot[key] == DIRECT_NONE) {
+                        slot[key] = 0;
+                        keys.push_back(key);
+                    }
                 }
+                o.terms = (unsigned)terms.size() - o.first;
                 outs.push_back(o);
             }
         }
     // slots: exponents by decreasing cost, all products of one exponent together
-    std::vector<unsigned> keys;
-    for (const auto &s : slot) keys.push_back(s.first);
-    std::stable_sort(keys.begin(), keys.end(), [&](unsigned x, unsigned y) {
+    std::sort(keys.begin(), keys.end(), [&](unsigned x, unsigned y) {
         const unsigned ex = x & 255u, ey = y & 255u;
-        return cost[ex] != cost[ey] ? cost[ex] > cost[ey] : ex < ey;
+        return cost[ex] != cost[ey] ? cost[ex] > cost[ey] : ex != ey ? ex < ey : x < y;
     });
     r.nprod = (uint32_t)keys.size();
     r.prod = (uint32_t)words.size();
@@ -169,13 +182,19 @@ inline DirectStep direct_build_step(std::vector<uint32_t> &words, unsigned logn,
     r.nout = (uint32_t)outs.size();
     r.sums = (uint32_t)words.size();
     // longest sums first
-    std::stable_sort(outs.begin(), outs.end(), [](const Out &x, const Out &y) { return x.terms.size() > y.terms.size(); });
+    std::stable_sort(outs.begin(), outs.end(), [](const Out &x, const Out &y) { return x.terms > y.terms; });
+    // 4 lanes per output for up to 16 terms, 64 for a single step's up to 256
+    r.log_lanes = a > 32 ? 6 : 2;
+    const unsigned lanes = 1u << r.log_lanes;
+    r.sum_words = DIRECT_SUM_FIRST + ((outs[0].terms + lanes - 1) & ~(lanes - 1));
     for (const Out &o : outs) {
         const size_t at = words.size();
-        words.resize(at + DIRECT_SUM_WORDS, DIRECT_NONE);
+        words.resize(at + r.sum_words, DIRECT_NONE);
         words[at] = o.pos;
-        for (size_t t = 0; t < o.terms.size(); t++)
-            words[at + DIRECT_SUM_FIRST + t] = slot[o.terms[t].first] | o.terms[t].second << 31;
+        for (unsigned t = 0; t < o.terms; t++) {
+            const uint32_t k = terms[o.first + t];
+            words[at + DIRECT_SUM_FIRST + t] = slot[k & 0x7fffffffu] | (k & 0x80000000u);
+        }
     }
     return r;
 }
@@ -185,7 +204,7 @@ inline void direct_build(std::vector<uint32_t> &words, const int *cost) {
     words.assign((size_t)DIRECT_RECORDS * DIRECT_STEP_WORDS, 0);
     for (unsigned logn = 7; logn <= 9; logn++)
         for (unsigned kind = 0; kind < DIRECT_KINDS; kind++)
-            for (unsigned levels = 2; levels <= 3; levels++)
+            for (unsigned levels = 1; levels <= DIRECT_MAX_STEPS; levels++)
                 for (unsigned s = 0; s < levels; s++) {
                     const DirectStep r = direct_build_step(words, logn, kind, levels, s, cost);
                     memcpy(&words[(size_t)direct_record(logn, kind, levels, s) * DIRECT_STEP_WORDS], &r, sizeof r);

@@ -165,10 +165,11 @@ struct DirectPlan {
 const std::vector<uint32_t> &direct_plan_words();
 // The plans of the current device (api.cpp), or nullptr words on failure.
 DirectPlan current_direct_plan(hipError_t *err);
-// Levels of the direct schedule that transform the items of L fastest (2 or 3), or 0 for the
+// Levels of the direct schedule that transform the items of L fastest (1 to 3), or 0 for the
 // radix-2^2 launches.  both: IFFT and FFT halves (the batched path), else one whole transform;
-// two: whether the workspace holds the products of two levels (three levels' always fit).
-unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, bool two);
+// allowed: bit l set if the workspace holds the products of l levels.
+static constexpr unsigned DIRECT_ANY = 0xe;
+unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned allowed);
 // Bytes of P an item of `rows` transforms of 2^logn points needs at `levels`.
 size_t direct_product_bytes(const DirectPlan &P, unsigned rows, unsigned logn, unsigned levels);
 // Largest batch the direct schedule is used for, in rows of one size: workspaces are sized by it.

@@ -529,24 +529,26 @@ __global__ void k_chain_reset(Chain C) {
 
 // ---------------------------------------------------------------- direct schedule (direct.hip.h)
 
-// The split of a direct step, in place: a lanes per (block, m, row), lane t holding point t; after
-// level h the upper half [h, 2h) keeps differences and the lower one goes on with sums.
-__global__ void __launch_bounds__(64) k_direct_split(Launch L, const uint32_t *plan) {
+// The split of a direct step, in place: 2^loga lanes per (block, m, row), lane t holding point t;
+// after level h the upper half [h, 2h) keeps differences and the lower one goes on with sums.
+__global__ void __launch_bounds__(64) k_direct_split(Launch L, const uint32_t *plan, unsigned pass) {
     unsigned local;
     const Item &it = L.item[find_item(L, blockIdx.x, local)];
     const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
-    const unsigned rows = it.rows, logn = it.logn2, lane = threadIdx.x, t = lane & ((1u << st.loga) - 1);
-    const unsigned total = (rows << logn) >> st.loga;
+    const unsigned loga = direct_split_log(st.loga, pass), logN = st.loga + st.logb;
+    const unsigned logb = pass == 0 ? logN - loga : st.logb;
+    const unsigned rows = it.rows, logn = it.logn2, lane = threadIdx.x, t = lane & ((1u << loga) - 1);
+    const unsigned total = rows << (st.logblocks + logb);
     // spare lane groups repeat the last one's work
-    const unsigned id = min((local * 64 + lane) >> st.loga, total - 1), row = id % rows, g = id / rows;
-    const unsigned i = ((g >> st.logb) << (st.loga + st.logb)) + (g & ((1u << st.logb) - 1)) + (t << st.logb);
+    const unsigned id = min((local * 64 + lane) >> loga, total - 1), row = id % rows, g = id / rows;
+    const unsigned i = ((g >> logb) << logN) + (g & ((1u << logb) - 1)) + (t << logb);
     const unsigned pos = (st.in_map & 1u) ? bitrev(i, logn) : i;
     uint32_t *p = it.D + ((size_t)pos * rows + row) * 36;
     g1q x, o, u;
     g1q_inf(x);
-    if (!(st.in_map & 2u) || i < (1u << (logn - 1))) pt_load(x, p);
+    if (pass || !(st.in_map & 2u) || i < (1u << (logn - 1))) pt_load(x, p);
 #pragma unroll 1
-    for (unsigned h = 1u << (st.loga - 1); h; h >>= 1) {
+    for (unsigned h = 1u << (loga - 1); h; h >>= 1) {
         shfl_point(o, x, (int)(t < h ? lane + h : t < 2 * h ? lane - h : lane));
         u = x;
         if (t >= h) g1q_neg(u, x);
@@ -556,15 +558,15 @@ __global__ void __launch_bounds__(64) k_direct_split(Launch L, const uint32_t *p
     pt_store(p, x);
 }
 
-// The sums of a direct step: 4 lanes per (output, row), each adding every fourth term, then
-// across the lanes; D is free to be overwritten, every term is in P.
+// The sums of a direct step: 2^log_lanes lanes per (output, row), each adding every so-manieth
+// term, then across the lanes; D is free to be overwritten, every term is in P.
 __global__ void __launch_bounds__(64) k_direct_sums(Launch L, const uint32_t *plan) {
     unsigned local;
     const Item &it = L.item[find_item(L, blockIdx.x, local)];
     const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
-    const unsigned rows = it.rows, lane = threadIdx.x, part = lane & 3;
-    const unsigned id = min(local * 16 + (lane >> 2), st.nout * rows - 1), row = id % rows;
-    const uint32_t *o = plan + st.sums + (size_t)(id / rows) * DIRECT_SUM_WORDS, *terms = o + DIRECT_SUM_FIRST + part;
+    const unsigned rows = it.rows, lanes = 1u << st.log_lanes, part = threadIdx.x & (lanes - 1);
+    const unsigned id = min((local * 64 + threadIdx.x) >> st.log_lanes, st.nout * rows - 1), row = id % rows;
+    const uint32_t *o = plan + st.sums + (size_t)(id / rows) * st.sum_words;
     g1q acc, x;
     auto term = [&](g1q &p, uint32_t c) {
         g1q_inf(p);
@@ -572,19 +574,15 @@ __global__ void __launch_bounds__(64) k_direct_sums(Launch L, const uint32_t *pl
         pt_load(p, it.P + ((size_t)(c & 0x7fffffffu) * rows + row) * 36);
         if (c >> 31) g1q_neg(p, p);
     };
-    term(acc, terms[0]);
+    term(acc, o[DIRECT_SUM_FIRST + part]);
 #pragma unroll 1
-    for (unsigned k = 4; k < 16; k += 4) {
-        const uint32_t c = terms[k];
+    for (unsigned k = DIRECT_SUM_FIRST + lanes; k < st.sum_words; k += lanes) {
+        const uint32_t c = o[k + part];
         if (!__any(c != DIRECT_NONE)) break;  // outputs come longest first
         term(x, c);
         g1q_add(acc, acc, x);
     }
-#pragma unroll 1
-    for (int d = 1; d <= 2; d *= 2) {
-        shfl_point(x, acc, (int)lane ^ d);
-        g1q_add(acc, acc, x);
-    }
+    lane_sum(acc, lanes);
     if (part == 0) pt_store(it.D + ((size_t)o[0] * rows + row) * 36, acc);
 }
 
@@ -598,10 +596,11 @@ __global__ void __launch_bounds__(64) k_direct_sums(Launch L, const uint32_t *pl
 __global__ void __launch_bounds__(64) k_output_multi(Launch L) {
     unsigned local;
     const Item &it = L.item[find_item(L, blockIdx.x, local)];
-    const unsigned rows = it.rows, rg = (rows + 63) / 64, logn2 = it.logn2;
-    const unsigned pos = local / rg;
-    const unsigned row = (local % rg) * 64 + threadIdx.x;
-    if (row >= rows) return;
+    // lanes take (position, row) pairs, rows fastest, so that few rows still fill the waves that
+    // run an inversion (one active lane took 146 us, 64 take 65)
+    const unsigned rows = it.rows, logn2 = it.logn2, id = local * 64 + threadIdx.x;
+    if (id >= rows << logn2) return;
+    const unsigned pos = id / rows, row = id % rows;
     if (it.rowflag && it.rowflag[(size_t)row * it.flag_stride]) return;  // written by k_ref_rows
     g1q p;
     pt_load(p, it.D + ((size_t)pos * rows + row) * 36);
@@ -722,6 +721,7 @@ static unsigned set_blocks(Launch &L, const unsigned *per_item) {
     }
     return total;
 }
+
 // Toeplitz coefficients and their transforms, of every item
 static void launch_toeplitz_multi(Launch &L, const DevTables *T, hipStream_t s) {
     unsigned per[MAX_ITEMS];
@@ -736,7 +736,6 @@ static void launch_toeplitz_multi(Launch &L, const DevTables *T, hipStream_t s) 
     if (total) hipLaunchKernelGGL(k_toeplitz_fft_multi<true>, dim3(total), dim3(256), 0, s, L, T);
 }
 
-
 // ---- direct schedule
 
 size_t direct_product_bytes(const DirectPlan &P, unsigned rows, unsigned logn, unsigned levels) {
@@ -750,8 +749,9 @@ size_t direct_product_bytes(const DirectPlan &P, unsigned rows, unsigned logn, u
 // Estimated microseconds of the transforms of L's items, measured on MI355X: a round of generic
 // ladders takes 1100 when each SIMD has at most one wave and about 950 more per further wave,
 // one of w^128 ladders 360 and 300; a launch of additions 55 (a direct step has two), a
-// butterfly launch 25.  The choice only depends on the items' sizes and rows.
-unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, bool two) {
+// butterfly launch 25.  The choice only depends on the items' sizes and rows, and the levels
+// whose products the workspace holds.
+unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned allowed) {
     if (!P.rec) return 0;
     unsigned lmax = 0;
     for (unsigned k = 0; k < L.nitems; k++) {
@@ -773,7 +773,8 @@ unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, bool two
         time += 25 + rounds(layer, 1100, 950) + rounds(quarter, 360, 300);
     }
     if (both) time *= 2;
-    for (unsigned levels = two ? 2 : 3; levels <= 3; levels++) {
+    for (unsigned levels = 1; levels <= DIRECT_MAX_STEPS; levels++) {
+        if (!(allowed >> levels & 1)) continue;
         unsigned t = 0;
         for (unsigned half = 0; half < (both ? 2u : 1u); half++)
             for (unsigned s = 0; s < levels; s++) {
@@ -782,7 +783,7 @@ unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, bool two
                     const DirectStep &st = P.rec[direct_record(L.item[k].logn2, both ? half : (unsigned)DIRECT_FFT, levels, s)];
                     waves += st.nwaves[6 - direct_row_lanes(L.item[k].rows)] * ((L.item[k].rows + 63) / 64);
                 }
-                t += 110 + rounds(waves, 1100, 950);
+                t += (levels == 1 ? 190 : 110) + rounds(waves, 1100, 950);
             }
         if (t < time) time = t, best = levels;
     }
@@ -803,15 +804,24 @@ static void launch_direct(Launch &L, const DirectPlan &P, unsigned levels, unsig
             }
             return set_blocks(L, per);
         };
-        unsigned total = blocks([](const Item &it, const DirectStep &) { return ((it.rows << it.logn2) + 63) / 64; });
-        hipLaunchKernelGGL(k_direct_split, dim3(total), dim3(64), 0, s, L, P.words);
-        hook(add);
+        unsigned total;
+        // the items' steps are of one kind (a single step or the same number of them), so of the
+        // same number of passes, but for a second pass that only radix 128 and up have
+        for (unsigned pass = 0; pass < (levels == 1 ? 2u : 1u); pass++) {
+            total = blocks([&](const Item &it, const DirectStep &st) {
+                const unsigned loga = direct_split_log(st.loga, pass), logN = st.loga + st.logb;
+                const unsigned groups = it.rows << (st.logblocks + (pass == 0 ? logN - loga : st.logb));
+                return ((groups << loga) + 63) / 64;
+            });
+            hipLaunchKernelGGL(k_direct_split, dim3(total), dim3(64), 0, s, L, P.words, pass);
+            hook(add);
+        }
         total = blocks([](const Item &it, const DirectStep &st) {
             return st.nwaves[6 - direct_row_lanes(it.rows)] * ((it.rows + 63) / 64);
         });
         hipLaunchKernelGGL(K.direct, dim3(total), dim3(64), 0, s, L, P.words, ops, index);
         hook(LK_TWIDDLE);
-        total = blocks([](const Item &it, const DirectStep &st) { return (st.nout * it.rows + 15) / 16; });
+        total = blocks([](const Item &it, const DirectStep &st) { return ((st.nout * it.rows << st.log_lanes) + 63) / 64; });
         hipLaunchKernelGGL(k_direct_sums, dim3(total), dim3(64), 0, s, L, P.words);
         hook(add);
     }
@@ -947,7 +957,7 @@ hipError_t launch_batch(const Launch &base, const DevTables *T, const uint32_t *
         }
     }
     // output
-    for (unsigned k = 0; k < L.nitems; k++) per[k] = (1u << L.item[k].logn2) * ((L.item[k].rows + 63) / 64);
+    for (unsigned k = 0; k < L.nitems; k++) per[k] = ((L.item[k].rows << L.item[k].logn2) + 63) / 64;
     total = set_blocks(L, per);
     if (total) hipLaunchKernelGGL(k_output_multi, dim3(total), dim3(64), 0, s, L);
     hook(LK_OUTPUT);
@@ -993,8 +1003,10 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
     const bool both = kind == PLAIN_HEXT_FFT2H_FFT || kind == PLAIN_POLY2H_FFT;
     unsigned levels = 0;
     if (rows <= DIRECT_MAX_ROWS) {
-        levels = direct_choose(L, direct, both, direct_product_bytes(direct, rows, logn, 2) <= product_bytes);
-        if (levels && direct_product_bytes(direct, rows, logn, levels) > product_bytes) levels = 0;
+        unsigned allowed = 0;
+        for (unsigned l = 1; l <= DIRECT_MAX_STEPS; l++)
+            if (direct_product_bytes(direct, rows, logn, l) <= product_bytes) allowed |= 1u << l;
+        levels = direct_choose(L, direct, both, allowed);
     }
     auto run_direct = [&](unsigned k) {
         launch_direct(L, direct, levels, k, P.ops, P.index, K, s, LaunchHook{nullptr, nullptr});
@@ -1057,7 +1069,7 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
         for (unsigned t = 1; t < logn; t++) stage(K.dif, (int)t);
         break;
     }
-    per[0] = n * rg;
+    per[0] = (n * rows + 63) / 64;
     hipLaunchKernelGGL(k_output_multi, dim3(set_blocks(L, per)), dim3(64), 0, s, L);
     // flagged rows of the transform kinds: their input rows are intact (the output kernel
     // skipped them, so an aliased output has not overwritten them) and D is free as workspace

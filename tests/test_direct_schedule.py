@@ -37,11 +37,11 @@ def rev(i, bits):
 def step(words, at, logn, D):
     """One step over Fr as the three kernels run it, in place on the list D."""
     n = 1 << logn
-    loga, logb, logblocks, in_map, nprod, prod, nout, sums = words[at:at + 8]
-    nwaves, waves = words[at + 8:at + 15], words[at + 15:at + 22]
-    a, b = 1 << loga, 1 << logb
-    assert loga + logb + logblocks == logn and 4 <= a <= 32
-    for g in range(n // a):
+    loga, logb, logblocks, in_map, log_lanes, sum_words, nprod, prod, nout, sums = words[at:at + 10]
+    nwaves, waves = words[at + 10:at + 17], words[at + 17:at + 24]
+    a, b, lanes = 1 << loga, 1 << logb, 1 << log_lanes
+    assert loga + logb + logblocks == logn and 4 <= a <= n
+    for g in range(n // a):  # the passes of a radix above 32 together
         idx = [((g >> logb) << (loga + logb)) + (g & (b - 1)) + (t << logb) for t in range(a)]
         pos = [rev(i, logn) if in_map & 1 else i for i in idx]
         x = [0 if in_map & 2 and i >= n // 2 else D[p] for i, p in zip(idx, pos)]
@@ -73,7 +73,8 @@ def step(words, at, logn, D):
         assert covered == list(range(nprod))
     out = {}
     for k in range(nout):
-        o = words[sums + 20 * k:sums + 20 * k + 20]
+        o = words[sums + sum_words * k:sums + sum_words * (k + 1)]
+        assert (len(o) - 4) % lanes == 0
         acc, ended = 0, False
         for t in o[4:]:
             if t == NONE:
@@ -100,7 +101,7 @@ def dft(x, sign):
     return [sum(v * pw[i * k % n] for i, v in enumerate(x)) % R for k in range(n)]
 
 
-@pytest.mark.parametrize("levels", [2, 3])
+@pytest.mark.parametrize("levels", [1, 2, 3])
 @pytest.mark.parametrize("logn", [7, 8, 9])
 def test_plans_compute_the_transforms(plans, logn, levels):
     n = 1 << logn
