@@ -214,7 +214,7 @@ __global__ void __launch_bounds__(256) k_ref_rows(unsigned kind, uint32_t *out, 
 // (z_e, prefix_{e-1}) of the current block per thread, laid out [entry][thread] so that the
 // 64 lanes of a wave touch consecutive words; it is sized by the launch, not by H, so every
 // (base, window) of a setup fits in one or two launches.
-__global__ void __launch_bounds__(64, 3) k_table_build(uint32_t *table, uint32_t *zt, const uint32_t *xs,
+__global__ void __launch_bounds__(64, 2) k_table_build(uint32_t *table, uint32_t *zt, const uint32_t *xs,
                                                     const uint32_t *inf, uint32_t *err, unsigned base0,
                                                     unsigned nb, unsigned win_bits, unsigned nwin) {
     const unsigned nthreads = nb * nwin;
