@@ -3,6 +3,7 @@
 // interface it replaces).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -308,7 +309,7 @@ static int g1_transform(fk20_g1p_t *out, const fk20_g1p_t *in, unsigned count, u
     if (rc) return rc;
     char *base = reinterpret_cast<char *>(D);
     return hip_status(launch_plain(inv ? PLAIN_G1_IFT : PLAIN_G1_FFT, W(out), W(in), nullptr, count, log2u(n),
-                                   W(base), nullptr, nullptr, W(base + d_bytes), st->tables, st->prog, S(stream),
+                                   W(base), nullptr, nullptr, 0, W(base + d_bytes), st->tables, st->prog, S(stream),
                                    st->direct, W(base + d_bytes + f_bytes), p_bytes));
 }
 
@@ -321,7 +322,7 @@ int g1p_ift(fk20_g1p_t *output, const fk20_g1p_t *input, unsigned count, unsigne
 }
 
 // MSM with the bases converted once per call into packed Montgomery form in scratch,
-// followed there by the scalars' Booth digits.
+// followed there by the MSM's own workspace.
 int fk20_msm(fk20_g1p_t *hext_fft, const fk20_fr_t *tc_fft, const fk20_g1p_t *xext_fft, unsigned rows,
              unsigned n2, fk20_stream_t stream) {
     if (!valid_n(n2) || (rows && (!hext_fft || !tc_fft || !xext_fft))) return FK20_EINVAL;
@@ -331,13 +332,14 @@ int fk20_msm(fk20_g1p_t *hext_fft, const fk20_fr_t *tc_fft, const fk20_g1p_t *xe
     if (rc) return rc;
     const size_t x_bytes = (size_t)16 * n2 * 144;
     void *scratch;
-    rc = device_scratch(st, x_bytes + msm_plain_digit_bytes(rows, n2), &scratch);
+    const size_t m_bytes = msm_plain_bytes(rows, n2);
+    rc = device_scratch(st, x_bytes + m_bytes, &scratch);
     if (rc) return rc;
     uint32_t *xpk = reinterpret_cast<uint32_t *>(scratch);
-    int8_t *digits = reinterpret_cast<int8_t *>(scratch) + x_bytes;
+    void *work = reinterpret_cast<char *>(scratch) + x_bytes;
     hipStream_t s = S(stream);
     FK20_TRY(launch_std_to_packed(xpk, W(xext_fft), (size_t)16 * n2, s));
-    return hip_status(launch_msm_plain(W(hext_fft), W(tc_fft), xpk, digits, rows, n2, s));
+    return hip_status(launch_msm_plain(W(hext_fft), W(tc_fft), xpk, work, m_bytes, rows, n2, s));
 }
 
 int fk20_hext2h(fk20_g1p_t *h, unsigned rows, unsigned n2, fk20_stream_t stream) {
@@ -359,7 +361,7 @@ int fk20_hext_fft2h_fft(fk20_g1p_t *h_fft, const fk20_g1p_t *hext_fft, unsigned 
     if (rc) return rc;
     char *base = reinterpret_cast<char *>(D);
     return hip_status(launch_plain(PLAIN_HEXT_FFT2H_FFT, W(h_fft), W(hext_fft), nullptr, rows, log2u(n2), W(base),
-                                   nullptr, nullptr, W(base + d_bytes), st->tables, st->prog, S(stream), st->direct,
+                                   nullptr, nullptr, 0, W(base + d_bytes), st->tables, st->prog, S(stream), st->direct,
                                    W(base + d_bytes + f_bytes), p_bytes));
 }
 
@@ -367,15 +369,14 @@ int fk20_hext_fft2h_fft(fk20_g1p_t *h_fft, const fk20_g1p_t *hext_fft, unsigned 
 // the 1/n2 of the IFFT moved onto the NTT output (a field multiplication instead of a
 // scalar multiplication per point) and the transforms column-batched over the rows.
 // Workspace: D, the packed bases, the subgroup flag of the bases (one 256-byte slot), tcT and the
-// MSM digits, in that order; tcT and the digits are dead after the MSM, and a small batch's
-// transforms keep their products there and past their end.
-static size_t poly2h_scratch_bytes(unsigned rows, unsigned n2) {
-    return (size_t)rows * 16 * n2 * 32 + (size_t)rows * n2 * 144 + (size_t)16 * n2 * 144 + 256 +
-           msm_plain_digit_bytes(rows, n2);
+// MSM's workspace, in that order; tcT and that workspace are dead after the MSM, and a small
+// batch's transforms keep their products there and past their end.
+static size_t poly2h_scratch_bytes(unsigned rows, unsigned n2, size_t msm_bytes) {
+    return (size_t)rows * 16 * n2 * 32 + (size_t)rows * n2 * 144 + (size_t)16 * n2 * 144 + 256 + msm_bytes;
 }
 
-// more: bytes of scratch past poly2h_scratch_bytes, for a small batch's products
-static int poly2h_fft_in(void *scratch, size_t more, DeviceState *st, fk20_g1p_t *h_fft, const fk20_fr_t *poly,
+// bytes: all of scratch, at least poly2h_scratch_bytes with the smallest MSM workspace
+static int poly2h_fft_in(void *scratch, size_t bytes, DeviceState *st, fk20_g1p_t *h_fft, const fk20_fr_t *poly,
                          const fk20_g1p_t *xext_fft, unsigned rows, unsigned n2, fk20_stream_t stream) {
     const size_t tc_bytes = (size_t)rows * 16 * n2 * 32;
     const size_t d_bytes = (size_t)rows * n2 * 144;
@@ -383,14 +384,14 @@ static int poly2h_fft_in(void *scratch, size_t more, DeviceState *st, fk20_g1p_t
     char *base = reinterpret_cast<char *>(scratch);
     uint32_t *D = W(base), *xpk = W(base + d_bytes), *flag = W(base + d_bytes + x_bytes);
     uint32_t *tcT = W(base + d_bytes + x_bytes + 256);
-    int8_t *digits = reinterpret_cast<int8_t *>(base + d_bytes + x_bytes + 256 + tc_bytes);
+    void *work = base + d_bytes + x_bytes + 256 + tc_bytes;
+    const size_t rest = bytes - (d_bytes + x_bytes + 256 + tc_bytes);
     hipStream_t s = S(stream);
     // one flag for all rows: a base outside G1 can put every row's MSM output outside it
     FK20_TRY(launch_subgroup_groups(flag, W(xext_fft), (size_t)16 * n2, (size_t)16 * n2, s));
     FK20_TRY(launch_std_to_packed(xpk, W(xext_fft), (size_t)16 * n2, s));
-    return hip_status(launch_plain(PLAIN_POLY2H_FFT, W(h_fft), W(poly), xpk, rows, log2u(n2), D, tcT, digits,
-                                   flag, st->tables, st->prog, s, st->direct, tcT,
-                                   tc_bytes + msm_plain_digit_bytes(rows, n2) + more));
+    return hip_status(launch_plain(PLAIN_POLY2H_FFT, W(h_fft), W(poly), xpk, rows, log2u(n2), D, tcT, work, rest,
+                                   flag, st->tables, st->prog, s, st->direct, tcT, tc_bytes + rest));
 }
 
 int fk20_poly2h_fft(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20_g1p_t *xext_fft, unsigned rows,
@@ -402,11 +403,13 @@ int fk20_poly2h_fft(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20_g1p_t *
     int rc = device_state(&st);
     if (rc) return rc;
     void *scr;
-    const size_t bytes = poly2h_scratch_bytes(rows, n2), dead = (size_t)rows * 16 * n2 * 32 + msm_plain_digit_bytes(rows, n2);
-    const size_t products = transform_product_bytes(st, rows, log2u(n2), true), more = products > dead ? products - dead : 0;
-    rc = device_scratch(st, bytes + more, &scr);
+    // the workspace past D, bases and flag holds first tcT and the MSM's, then the products
+    const size_t tc_bytes = (size_t)rows * 16 * n2 * 32, dead = tc_bytes + msm_plain_bytes(rows, n2);
+    const size_t products = transform_product_bytes(st, rows, log2u(n2), true);
+    const size_t bytes = poly2h_scratch_bytes(rows, n2, std::max(dead, products) - tc_bytes);
+    rc = device_scratch(st, bytes, &scr);
     if (rc) return rc;
-    return poly2h_fft_in(scr, more, st, h_fft, poly, xext_fft, rows, n2, stream);
+    return poly2h_fft_in(scr, bytes, st, h_fft, poly, xext_fft, rows, n2, stream);
 }
 
 // The same launch sequence with its workspace in this device's fixed `scratch` array: no
@@ -418,12 +421,11 @@ int fk20_poly2h_fft_noalloc(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20
     if (!valid_N(N) || (rows && (!h_fft || !poly || !xext_fft))) return FK20_EINVAL;
     if (!rows) return FK20_OK;
     const unsigned n2 = N / 8;
-    if (poly2h_scratch_bytes(rows, n2) > NOALLOC_SCRATCH_BYTES) return FK20_ERANGE;
+    if (poly2h_scratch_bytes(rows, n2, msm_plain_min_bytes(rows, n2)) > NOALLOC_SCRATCH_BYTES) return FK20_ERANGE;
     DeviceState *st;
     int rc = device_state(&st);
     if (rc) return rc;
-    const size_t more = NOALLOC_SCRATCH_BYTES - poly2h_scratch_bytes(rows, n2);
-    return poly2h_fft_in(st->noalloc, more, st, h_fft, poly, xext_fft, rows, n2, stream);
+    return poly2h_fft_in(st->noalloc, NOALLOC_SCRATCH_BYTES, st, h_fft, poly, xext_fft, rows, n2, stream);
 }
 
 int fk20_setup2xext_fft(fk20_g1p_t *xext_fft, const fk20_g1p_t *setup, unsigned N, fk20_stream_t stream) {
@@ -440,7 +442,7 @@ int fk20_setup2xext_fft(fk20_g1p_t *xext_fft, const fk20_g1p_t *setup, unsigned 
     hipStream_t s = S(stream);
     FK20_TRY(launch_setup_gather(W(xext_fft), W(setup), N, s));
     return hip_status(launch_plain(PLAIN_G1_FFT, W(xext_fft), W(xext_fft), nullptr, 16, log2u(N / 8), W(base), nullptr,
-                                   nullptr, W(base + d_bytes), st->tables, st->prog, s, st->direct,
+                                   nullptr, 0, W(base + d_bytes), st->tables, st->prog, s, st->direct,
                                    W(base + d_bytes + f_bytes), p_bytes));
 }
 

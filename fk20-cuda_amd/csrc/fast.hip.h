@@ -191,7 +191,7 @@ hipError_t launch_batch(const Launch &L, const DevTables *T, const uint32_t *ops
 // The drop-in entry points on the same column-batched transform kernels, for `rows`
 // transforms of n = 2^logn points (n2 = n for the FK20 kinds), with D = rows * n * 144
 // bytes of workspace (and, for PLAIN_POLY2H_FFT, tcT = rows * 16 * n * 32 bytes and
-// digits = msm_plain_digit_bytes(rows, n)):
+// msm_work = msm_bytes of launch_msm_plain's workspace):
 //   PLAIN_G1_FFT          out[r] = DFT(in[r])                         (g1p_fft)
 //   PLAIN_G1_IFT          out[r] = DFT^-1(in[r]), scaled by 1/n       (g1p_ift)
 //   PLAIN_HEXT_FFT2H_FFT  IFFT, zero upper half, FFT                  (fk20_hext_fft2h_fft)
@@ -200,12 +200,12 @@ hipError_t launch_batch(const Launch &L, const DevTables *T, const uint32_t *ops
 // out may alias in: every input is read into D before the first output is written.
 enum PlainKind { PLAIN_G1_FFT = 0, PLAIN_G1_IFT = 1, PLAIN_HEXT_FFT2H_FFT = 2, PLAIN_POLY2H_FFT = 3 };
 // products: product_bytes of workspace for the direct schedule (it is not used when they are too
-// few); it may overlap tcT and digits.
+// few); it may overlap tcT and msm_work.
 // flags: `rows` words of workspace (one word for PLAIN_POLY2H_FFT, set by the caller with
 // launch_subgroup_groups over the bases).  Rows holding a point outside G1 are recomputed in
 // the reference's order of operations (launch_ref_rows).
 hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const uint32_t *xpk, unsigned rows,
-                        unsigned logn, uint32_t *D, uint32_t *tcT, int8_t *digits, uint32_t *flags,
+                        unsigned logn, uint32_t *D, uint32_t *tcT, void *msm_work, size_t msm_bytes, uint32_t *flags,
                         const DevTables *T, const Programs &P, hipStream_t s, const DirectPlan &direct, uint32_t *products,
                         size_t product_bytes);
 

@@ -397,25 +397,6 @@ __device__ __forceinline__ void window_sum(g1q &acc, const uint32_t *tables, siz
     }
 }
 
-__device__ __forceinline__ void shfl_point(g1q &r, const g1q &p, int lane) {
-#pragma unroll
-    for (int i = 0; i < FQ_N; i++) {
-        r.x.l[i] = __shfl(p.x.l[i], lane);
-        r.y.l[i] = __shfl(p.y.l[i], lane);
-        r.z.l[i] = __shfl(p.z.l[i], lane);
-    }
-}
-
-// the sum of the points of the lanes t, t ^ 1, .., t ^ (span - 1) in each of them (span a power of two)
-__device__ __forceinline__ void lane_sum(g1q &acc, unsigned span) {
-    g1q o;
-#pragma unroll 1
-    for (unsigned d = 1; d < span; d *= 2) {
-        shfl_point(o, acc, (int)(threadIdx.x ^ d));
-        g1q_add(acc, acc, o);
-    }
-}
-
 // hext_fft[j] of one column j: sum over 16 terms of ceil(256/w) signed-window digits, one mixed
 // addition each; output to D[bitrev(j)][row].  LP lanes share a row, each with 16 / LP of the
 // terms, and add up across the wave: an addition takes 9 us in a wave alone on its SIMD and 8.3
@@ -653,13 +634,6 @@ hipError_t launch_table_build(uint32_t *table, uint32_t *zt, const uint32_t *xs,
     return hipGetLastError();
 }
 
-// Additions one after the other that `waves` waves of `adds` additions take on 1024 SIMDs: a wave
-// alone on its SIMD needs about 1.1 times an addition's share of a busy SIMD.
-static unsigned add_rounds(size_t waves, unsigned adds) {
-    const unsigned rounds = (unsigned)((waves + 1023) / 1024);
-    return rounds <= 1 ? adds + adds / 8 : rounds * adds;
-}
-
 // Lanes per row and coefficients per lane of k_commit_partial: no idle lanes below 64 rows, then
 // the chunk with the fewest additions one after the other (20 windows per coefficient; larger
 // chunks where it does not matter, for fewer partial sums).
@@ -747,8 +721,8 @@ size_t direct_product_bytes(const DirectPlan &P, unsigned rows, unsigned logn, u
 }
 
 // Estimated microseconds of the transforms of L's items, measured on MI355X: a round of generic
-// ladders takes 1100 when each SIMD has at most one wave and about 950 more per further wave,
-// one of w^128 ladders 360 and 300; a launch of additions 55 (a direct step has two), a
+// ladders takes 1100 when each SIMD has at most one wave, 2050 per pair of waves and 1250 for an odd
+// one after them, one of w^128 ladders 360, 660 and 400; a launch of additions 55 (a direct step has two), a
 // butterfly launch 25.  The choice only depends on the items' sizes and rows, and the levels
 // whose products the workspace holds.
 unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned allowed) {
@@ -758,8 +732,9 @@ unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned
         lmax = std::max(lmax, L.item[k].logn2);
         if (L.item[k].rows > DIRECT_MAX_ROWS) return 0;
     }
-    auto rounds = [](unsigned waves, unsigned first, unsigned more) {
-        return waves ? first + ((waves + 1023) / 1024 - 1) * more : 0;
+    auto rounds = [](unsigned waves, unsigned one, unsigned pair, unsigned odd) {
+        const unsigned c = (waves + 1023) / 1024;
+        return c == 1 ? one : c / 2 * pair + c % 2 * odd;
     };
     // radix 2^2: per transform, the layers (odd stages) and the w^128 of the even ones
     unsigned best = 0, time = 0;
@@ -770,7 +745,7 @@ unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned
             if ((sd & 1) && sd < logn) layer += layer_count(sd, logn) * rg;
             if (!(sd & 1) && sd + 1 < logn) quarter += (1u << (logn - 2)) * rg;
         }
-        time += 25 + rounds(layer, 1100, 950) + rounds(quarter, 360, 300);
+        time += 25 + rounds(layer, 1100, 2050, 1250) + rounds(quarter, 360, 660, 400);
     }
     if (both) time *= 2;
     for (unsigned levels = 1; levels <= DIRECT_MAX_STEPS; levels++) {
@@ -783,7 +758,7 @@ unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned
                     const DirectStep &st = P.rec[direct_record(L.item[k].logn2, both ? half : (unsigned)DIRECT_FFT, levels, s)];
                     waves += st.nwaves[6 - direct_row_lanes(L.item[k].rows)] * ((L.item[k].rows + 63) / 64);
                 }
-                t += (levels == 1 ? 190 : 110) + rounds(waves, 1100, 950);
+                t += (levels == 1 ? 190 : 110) + rounds(waves, 1100, 2050, 1250);
             }
         if (t < time) time = t, best = levels;
     }
@@ -969,7 +944,7 @@ hipError_t launch_batch(const Launch &base, const DevTables *T, const uint32_t *
 // stages 0 .. L-1 (the first likewise), and the output kernel writes natural order from the
 // DIF's bit-reversed positions (format 0) or position by position (format 1).
 hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const uint32_t *xpk, unsigned rows,
-                        unsigned logn, uint32_t *D, uint32_t *tcT, int8_t *digits, uint32_t *flags,
+                        unsigned logn, uint32_t *D, uint32_t *tcT, void *msm_work, size_t msm_bytes, uint32_t *flags,
                         const DevTables *T, const Programs &P, hipStream_t s, const DirectPlan &direct, uint32_t *products,
                         size_t product_bytes) {
     if (!rows) return hipSuccess;
@@ -1052,7 +1027,7 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
             hipLaunchKernelGGL(K.plain_load, dim3(n * rg), dim3(64), 0, s, D, in, rows, logn, 1u, scale);
         } else {
             launch_toeplitz_multi(L, T, s);
-            hipError_t e = launch_msm_plain_T(D, tcT, xpk, digits, rows, n, s);
+            hipError_t e = launch_msm_plain_T(D, tcT, xpk, msm_work, msm_bytes, rows, n, s);
             if (e != hipSuccess) return e;
             // rows of a setup outside G1 take the reference's order from the MSM output on,
             // with tcT (no longer read) as their workspace

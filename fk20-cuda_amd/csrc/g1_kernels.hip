@@ -5,6 +5,7 @@
 #include <algorithm>
 
 #include "common.hip.h"
+#include "kutil.hip.h"
 
 namespace fk20 {
 
@@ -232,6 +233,112 @@ __global__ void __launch_bounds__(64) k_msm_booth_small(uint32_t *out, const int
     }
     if (i == 0 && row0 < rows) {
         if (to_D) g1_lds_store(out + ((size_t)bitrev(j, 31 - __builtin_clz(n2)) * rows + row) * 36, acc);
+        else g1q_gstore_std(out + ((size_t)row * n2 + j) * G1P_WORDS, acc);
+    }
+}
+
+// The MSM of more rows, with the multiples 1 .. 2^(w-1) of every base in HBM: larger windows than
+// the 72 KiB of LDS hold (w = 6), so fewer additions -- 26 x 16 at w = 10 against 43 x 16 -- for a
+// table that all rows share (16 n2 2^(w-1) points, built by one addition each).  LP lanes share a
+// row, each with 16 / LP of the terms and its own doublings: with few rows more waves, with many
+// LP = 1.  msm_plan picks w and LP by the additions that a launch runs one after the other.  What
+// bounds it is the additions' instructions; the next entry is fetched during the current addition.
+// 300 rows of 512 columns: 32.8 ms from LDS, 18.6 with w = 10; 32 rows 10.1 and 3.6.
+
+// digits[j][i][win][row] (int16): signed radix-2^w Booth digits, as k_msm_digits for any w
+__global__ void __launch_bounds__(256) k_msm_digits_w(int16_t *digits, const uint32_t *tc, unsigned n2, unsigned rows,
+                                                      MsmLayout m, unsigned w, unsigned nwin) {
+    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;  // (j, i, row), row fastest
+    if (e >= (size_t)n2 * 16 * rows) return;
+    const unsigned row = (unsigned)(e % rows), i = (unsigned)((e / rows) % 16), j = (unsigned)(e / rows / 16);
+    uint32_t k[8];
+    words_load(k, tc + ((size_t)row * m.row_stride + (size_t)i * m.i_stride + (size_t)j * m.j_stride) * FR_WORDS, 8);
+    int16_t *out = digits + ((size_t)j * 16 + i) * nwin * rows + row;
+    uint32_t below = 0;  // the bit under the window
+#pragma unroll 1
+    for (unsigned q = 0; q < nwin; q++) {
+        const uint32_t f = k[0] & ((1u << w) - 1);
+        out[(size_t)q * rows] = (int16_t)((int)(f + below) - (int)(f >> (w - 1) << w));
+        below = f >> (w - 1);
+#pragma unroll
+        for (int x = 0; x < 7; x++) k[x] = (k[x] >> w) | (k[x + 1] << (32 - w));
+        k[7] >>= w;
+    }
+}
+
+// table[base][d - 1] = d X, d = 1 .. 2^(w-1), for the bases [i][j]: a thread per run of
+// MSM_RUN entries, whose first one it makes by double-and-add.
+static constexpr unsigned MSM_RUN = 32;
+
+__global__ void __launch_bounds__(64, 2) k_msm_table(uint32_t *table, const uint32_t *xpk, unsigned bases, unsigned w) {
+    const unsigned half = 1u << (w - 1), runs = half / MSM_RUN;
+    const unsigned t = blockIdx.x * 64 + threadIdx.x;
+    if (t >= bases * runs) return;
+    const unsigned base = t % bases, first = t / bases * MSM_RUN + 1;  // a wave's runs start at one multiple
+    uint32_t *out = table + ((size_t)base * half + first - 1) * 36;
+    g1q X, e;
+    pt_load(X, xpk + (size_t)base * 36);
+    e = X;
+    // one addition in the code: first the bits of `first` below its top one, then the run
+    int b = 30 - __builtin_clz(first);
+#pragma unroll 1
+    for (unsigned k = 0; k < MSM_RUN;) {
+        bool add = true;
+        if (b >= 0) {
+            g1q_dbl(e, e);
+            add = (first >> b) & 1;
+            b--;
+        } else {
+            pt_store(out + k * 36, e);
+            k++;
+        }
+        if (add) g1q_add(e, e, X);
+    }
+}
+
+template <unsigned LP>
+__global__ void __launch_bounds__(64, 2) k_msm_straus(uint32_t *out, const int16_t *digits, const uint32_t *table,
+                                                     unsigned n2, unsigned rows, unsigned to_D, unsigned w,
+                                                     unsigned nwin) {
+    constexpr unsigned per_wave = 64 / LP, terms = 16 / LP;
+    const unsigned rg = (rows + per_wave - 1) / per_wave, j = blockIdx.x / rg, i0 = threadIdx.x % LP;
+    const unsigned row0 = (blockIdx.x % rg) * per_wave + threadIdx.x / LP;
+    const unsigned row = min(row0, rows - 1);  // spare lanes repeat the last row
+    const unsigned half = 1u << (w - 1);
+    // term t of the lane: base (i0 + LP t, j)
+    const int16_t *dg = digits + ((size_t)j * 16 + i0) * nwin * rows + row;
+    const uint32_t *tab = table + ((size_t)i0 * n2 + j) * half * 36;
+    uint32_t ent[36];
+    int d = 0;
+    auto fetch = [&](unsigned q, unsigned t) {
+        d = dg[((size_t)LP * t * nwin + q) * rows];
+        const unsigned m = (unsigned)(d < 0 ? -d : d);
+        ld_words(ent, tab + ((size_t)LP * t * n2 * half + (m ? m - 1 : 0)) * 36, 9);
+    };
+    g1q acc;
+    g1q_inf(acc);
+    unsigned q = nwin - 1, t = 0;
+    fetch(q, t);
+#pragma unroll 1
+    while (true) {
+        g1q X;
+        g1q_load_packed(X, ent);
+        if (d < 0) fq_neg(X.y, X.y);
+        if (d == 0) g1q_inf(X);
+        if (++t == terms) t = 0;
+        const bool last = t == 0 && q == 0;
+        if (!last) fetch(t ? q : q - 1, t);
+        g1q_add(acc, acc, X);
+        if (last) break;
+        if (t == 0) {
+            q--;
+#pragma unroll 1
+            for (unsigned k = 0; k < w; k++) g1q_dbl(acc, acc);
+        }
+    }
+    lane_sum(acc, LP);
+    if (i0 == 0 && row0 < rows) {
+        if (to_D) pt_store(out + ((size_t)bitrev(j, 31 - __builtin_clz(n2)) * rows + row) * 36, acc);
         else g1q_gstore_std(out + ((size_t)row * n2 + j) * G1P_WORDS, acc);
     }
 }
@@ -554,12 +661,58 @@ hipError_t launch_std_to_packed(uint32_t *packed, const uint32_t *pts, size_t co
     return hipGetLastError();
 }
 
-size_t msm_plain_digit_bytes(unsigned rows, unsigned n2) { return (size_t)rows * n2 * 16 * MSM_NWIN; }
+size_t msm_plain_min_bytes(unsigned rows, unsigned n2) { return (size_t)rows * n2 * 16 * MSM_NWIN; }
 
-static hipError_t msm_plain(uint32_t *out, const uint32_t *tc, const uint32_t *xpk, int8_t *digits, unsigned rows,
-                            unsigned n2, MsmLayout m, hipStream_t s) {
+// Window and lanes per row of k_msm_straus with the fewest additions one after the other (a doubling
+// counts 2/3), or w = 0: the LDS kernels.  The LDS kernel for few rows is the same
+// sum with 16 lanes per row at w = 6, without a table launch.
+struct MsmPlan {
+    unsigned w, lp, nwin;
+    size_t digits, table;  // bytes
+};
+static MsmPlan msm_plan(unsigned rows, unsigned n2, size_t bytes) {
+    MsmPlan best{0, 1, MSM_NWIN, 0, 0};
+    auto adds = [&](unsigned w, unsigned lp, unsigned close) {
+        const unsigned nwin = 256 / w + 1;
+        return add_rounds((size_t)n2 * ((rows * lp + 63) / 64), nwin * 16 / lp + (nwin - 1) * w * 2 / 3 + close);
+    };
+    // (its 72 KiB of LDS per wave leave room for 512 waves)
+    unsigned time = adds(6, 1, 16);
+    if (rows <= MSM_SMALL_ROWS) time = (n2 * ((rows + 3) / 4) + 511) / 512 * (MSM_NWIN + 42 * 4 + 14);
+    for (unsigned w = 7; w <= 10; w++)
+        for (unsigned lp = 1, close = 0; lp <= 16; lp *= 4, close += 2) {
+            const unsigned nwin = 256 / w + 1, half = 1u << (w - 1);
+            const MsmPlan p{w, lp, nwin, ((size_t)rows * n2 * 16 * nwin * 2 + 255) & ~(size_t)255, (size_t)16 * n2 * half * 144};
+            if (p.digits + p.table > bytes) continue;
+            const unsigned t = adds(w, lp, close) + add_rounds((size_t)16 * n2 * half / MSM_RUN / 64, MSM_RUN + 14);
+            if (t < time) time = t, best = p;
+        }
+    return best;
+}
+
+size_t msm_plain_bytes(unsigned rows, unsigned n2) {
+    const MsmPlan p = msm_plan(rows, n2, ~(size_t)0);
+    return p.w ? p.digits + p.table : msm_plain_min_bytes(rows, n2);
+}
+
+static hipError_t msm_plain(uint32_t *out, const uint32_t *tc, const uint32_t *xpk, void *work, size_t work_bytes,
+                            unsigned rows, unsigned n2, MsmLayout m, hipStream_t s) {
     if (!rows) return hipSuccess;
     const size_t scalars = (size_t)rows * n2 * 16;
+    const MsmPlan p = msm_plan(rows, n2, work_bytes);
+    if (p.w) {
+        int16_t *digits = reinterpret_cast<int16_t *>(work);
+        uint32_t *table = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(work) + p.digits);
+        const unsigned threads = 16 * n2 * ((1u << (p.w - 1)) / MSM_RUN);
+        hipLaunchKernelGGL(k_msm_digits_w, dim3((unsigned)((scalars + 255) / 256)), dim3(256), 0, s, digits, tc, n2, rows,
+                           m, p.w, p.nwin);
+        hipLaunchKernelGGL(k_msm_table, dim3((threads + 63) / 64), dim3(64), 0, s, table, xpk, 16 * n2, p.w);
+        hipLaunchKernelGGL((p.lp == 1 ? k_msm_straus<1> : p.lp == 4 ? k_msm_straus<4> : k_msm_straus<16>),
+                           dim3(n2 * ((rows * p.lp + 63) / 64)), dim3(64), 0, s, out, (const int16_t *)digits,
+                           (const uint32_t *)table, n2, rows, m.to_D, p.w, p.nwin);
+        return hipGetLastError();
+    }
+    int8_t *digits = reinterpret_cast<int8_t *>(work);
     hipLaunchKernelGGL(k_msm_digits, dim3((unsigned)((scalars + 255) / 256)), dim3(256), 0, s, digits, tc, n2, rows, m);
     if (rows <= MSM_SMALL_ROWS) {
         hipLaunchKernelGGL(k_msm_booth_small, dim3(n2, (rows + 3) / 4), dim3(64), 0, s, out, (const int8_t *)digits,
@@ -572,16 +725,16 @@ static hipError_t msm_plain(uint32_t *out, const uint32_t *tc, const uint32_t *x
     return hipGetLastError();
 }
 
-hipError_t launch_msm_plain(uint32_t *hext, const uint32_t *tc_fft, const uint32_t *xpk, int8_t *digits,
+hipError_t launch_msm_plain(uint32_t *hext, const uint32_t *tc_fft, const uint32_t *xpk, void *work, size_t work_bytes,
                             unsigned rows, unsigned n2, hipStream_t s) {
     // scalars tc_fft[row][i][j], output hext_fft[row][j] (standard form)
-    return msm_plain(hext, tc_fft, xpk, digits, rows, n2, MsmLayout{16u * n2, n2, 1u, 0u}, s);
+    return msm_plain(hext, tc_fft, xpk, work, work_bytes, rows, n2, MsmLayout{16u * n2, n2, 1u, 0u}, s);
 }
 
-hipError_t launch_msm_plain_T(uint32_t *D, const uint32_t *tcT, const uint32_t *xpk, int8_t *digits, unsigned rows,
-                              unsigned n2, hipStream_t s) {
+hipError_t launch_msm_plain_T(uint32_t *D, const uint32_t *tcT, const uint32_t *xpk, void *work, size_t work_bytes,
+                              unsigned rows, unsigned n2, hipStream_t s) {
     // scalars tcT[j][i][row], output D[bitrev(j)][row] (packed Montgomery)
-    return msm_plain(D, tcT, xpk, digits, rows, n2, MsmLayout{1u, rows, 16u * rows, 1u}, s);
+    return msm_plain(D, tcT, xpk, work, work_bytes, rows, n2, MsmLayout{1u, rows, 16u * rows, 1u}, s);
 }
 
 hipError_t launch_mad_probe(uint64_t *out, unsigned blocks, unsigned iters, hipStream_t s) {

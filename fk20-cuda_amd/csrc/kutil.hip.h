@@ -53,6 +53,34 @@ __device__ __forceinline__ void fq_load_raw(fq &a, const uint32_t *g) {
     fq_unpack_raw(a, w);
 }
 
+// ---------------------------------------------------------------- sums across lanes
+
+__device__ __forceinline__ void shfl_point(g1q &r, const g1q &p, int lane) {
+#pragma unroll
+    for (int i = 0; i < FQ_N; i++) {
+        r.x.l[i] = __shfl(p.x.l[i], lane);
+        r.y.l[i] = __shfl(p.y.l[i], lane);
+        r.z.l[i] = __shfl(p.z.l[i], lane);
+    }
+}
+
+// the sum of the points of the lanes t, t ^ 1, .., t ^ (span - 1) in each of them (span a power of two)
+__device__ __forceinline__ void lane_sum(g1q &acc, unsigned span) {
+    g1q o;
+#pragma unroll 1
+    for (unsigned d = 1; d < span; d *= 2) {
+        shfl_point(o, acc, (int)(threadIdx.x ^ d));
+        g1q_add(acc, acc, o);
+    }
+}
+
+// Additions one after the other that `waves` waves of `adds` additions take on 1024 SIMDs: a wave
+// alone on its SIMD needs about 1.1 times an addition's share of a busy SIMD.
+inline unsigned add_rounds(size_t waves, unsigned adds) {
+    const unsigned rounds = (unsigned)((waves + 1023) / 1024);
+    return rounds <= 1 ? adds + adds / 8 : rounds * adds;
+}
+
 // ---------------------------------------------------------------- multi-item decoding
 //
 // Every launch below covers a list of items (row groups, each with its own setup, N and
