@@ -144,6 +144,7 @@ struct StageKernels {
     void (*quarter)(Launch) = nullptr;
     void (*chain)(Chain, const uint32_t *, const uint32_t *) = nullptr;
     void (*direct)(Launch, const uint32_t *, const uint32_t *, const uint32_t *) = nullptr;
+    void (*direct_pair)(Launch, const uint32_t *, const uint32_t *, const uint32_t *) = nullptr;
     void (*plain_load)(uint32_t *, const uint32_t *, unsigned, unsigned, unsigned, const uint32_t *) = nullptr;
     int wnaf = 0;
     bool r22 = false;

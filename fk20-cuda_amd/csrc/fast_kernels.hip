@@ -720,10 +720,17 @@ size_t direct_product_bytes(const DirectPlan &P, unsigned rows, unsigned logn, u
     return most * rows * 144;
 }
 
+// Waves that step `rec` of an item takes, one or two lanes per ladder
+static unsigned direct_waves(const DirectStep &st, unsigned rows, bool pair) {
+    if (!pair) return st.nwaves[6 - direct_row_lanes(rows)] * ((rows + 63) / 64);
+    return st.nwaves[5 - std::min(direct_row_lanes(rows), 5u)] * ((rows + 31) / 32);
+}
+
 // Estimated microseconds of the transforms of L's items, measured on MI355X: a round of generic
-// ladders takes 1100 when each SIMD has at most one wave, 2050 per pair of waves and 1250 for an odd
-// one after them, one of w^128 ladders 360, 660 and 400; a launch of additions 55 (a direct step has two), a
-// butterfly launch 25.  The choice only depends on the items' sizes and rows, and the levels
+// ladders takes 870 by pairs of lanes if these need at most one wave per SIMD, else 1100 when
+// each SIMD has at most one wave, 2050 per pair of waves and 1250 for an odd one after them, one
+// of w^128 ladders 360, 660 and 400; a launch of additions 55 (a direct step has two), a butterfly
+// launch 25.  The choice only depends on the items' sizes and rows, and the levels
 // whose products the workspace holds.
 unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned allowed) {
     if (!P.rec) return 0;
@@ -753,12 +760,14 @@ unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned
         unsigned t = 0;
         for (unsigned half = 0; half < (both ? 2u : 1u); half++)
             for (unsigned s = 0; s < levels; s++) {
-                unsigned waves = 0;
+                unsigned waves = 0, pairs = 0;
                 for (unsigned k = 0; k < L.nitems; k++) {
                     const DirectStep &st = P.rec[direct_record(L.item[k].logn2, both ? half : (unsigned)DIRECT_FFT, levels, s)];
-                    waves += st.nwaves[6 - direct_row_lanes(L.item[k].rows)] * ((L.item[k].rows + 63) / 64);
+                    waves += direct_waves(st, L.item[k].rows, false);
+                    pairs += direct_waves(st, L.item[k].rows, true);
                 }
-                t += (levels == 1 ? 190 : 110) + rounds(waves, 1100, 2050, 1250);
+                t += (levels == 1 ? 190 : 110) +
+                     (pairs <= DIRECT_PAIR_WAVES ? 870 : rounds(waves, 1100, 2050, 1250));
             }
         if (t < time) time = t, best = levels;
     }
@@ -791,10 +800,10 @@ static void launch_direct(Launch &L, const DirectPlan &P, unsigned levels, unsig
             hipLaunchKernelGGL(k_direct_split, dim3(total), dim3(64), 0, s, L, P.words, pass);
             hook(add);
         }
-        total = blocks([](const Item &it, const DirectStep &st) {
-            return st.nwaves[6 - direct_row_lanes(it.rows)] * ((it.rows + 63) / 64);
-        });
-        hipLaunchKernelGGL(K.direct, dim3(total), dim3(64), 0, s, L, P.words, ops, index);
+        total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, true); });
+        const bool pair = total <= DIRECT_PAIR_WAVES;
+        if (!pair) total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, false); });
+        hipLaunchKernelGGL(pair ? K.direct_pair : K.direct, dim3(total), dim3(64), 0, s, L, P.words, ops, index);
         hook(LK_TWIDDLE);
         total = blocks([](const Item &it, const DirectStep &st) { return ((st.nout * it.rows << st.log_lanes) + 63) / 64; });
         hipLaunchKernelGGL(k_direct_sums, dim3(total), dim3(64), 0, s, L, P.words);

@@ -52,17 +52,13 @@ static constexpr uint32_t TWOP_END = 1u << 31;
 #endif
 static constexpr int TW_WNAF = FK20_TW_WNAF;
 
-// x <- k * x for the wave-uniform scalar whose program starts at ops[0].  x: homogeneous
-// projective, coordinates < 8 p; out: < 2 p.
+// The ladder's table: x and 2 y of the odd multiples P, 3P, .., (2^(W-1) - 1) P of the homogeneous
+// point x (coordinates < 8 p, not infinity), affine on the isomorphic curve of the common Z zt.
 template <int W>
-FK20_HD void tw_mul(g1q &x, const uint32_t *ops) {
+FK20_HD void tw_table(fq *TX, fq *TY, fq &zt, const g1q &x) {
     constexpr int NT = 1 << (W - 2);
     static_assert(NT >= 2, "table of at least P and 3P");
-    // The table lives in the lane's private memory, not in registers: each addition reads
-    // one entry chosen by a wave-uniform index, so the loads are coalesced per dword and the
-    // ladder's register footprint leaves room for several waves per SIMD.
-    fq TX[NT], TY[NT], MU[NT - 1];
-    const bool inf = g1q_is_inf(x);
+    fq MU[NT - 1];
     // homogeneous (X : Y : Z) -> Jacobian (X Z, Y Z^2, Z)
     g1j_q P, Q;                     // Q = 2P, re-scaled by every co-Z addition
     fq t;
@@ -87,8 +83,20 @@ FK20_HD void tw_mul(g1q &x, const uint32_t *ops) {
         fq_addw(s3, s3, s3);                   // wide
         fq_mul(TY[k], TY[k], s3);
     }
-    fq zt;
     fq_mul(zt, Q.z, s);             // the table's common Z
+}
+
+// x <- k * x for the wave-uniform scalar whose program starts at ops[0].  x: homogeneous
+// projective, coordinates < 8 p; out: < 2 p.
+template <int W>
+FK20_HD void tw_mul(g1q &x, const uint32_t *ops) {
+    constexpr int NT = 1 << (W - 2);
+    // The table lives in the lane's private memory, not in registers: each addition reads
+    // one entry chosen by a wave-uniform index, so the loads are coalesced per dword and the
+    // ladder's register footprint leaves room for several waves per SIMD.
+    fq TX[NT], TY[NT], zt;
+    const bool inf = g1q_is_inf(x);
+    tw_table<W>(TX, TY, zt, x);
     fq beta, beta2;
     fq_set(beta, FQ_GLV);
     fq_set(beta2, FQ_GLV2);

@@ -4,6 +4,7 @@
 // StageKernels table; a context picks its variant at run time (fk20_ctx_set_schedule).
 #pragma once
 #include "kutil.hip.h"
+#include "ladder_pair.hip.h"
 
 namespace fk20 {
 
@@ -182,6 +183,28 @@ __global__ void __launch_bounds__(64, OCC) k_direct_products(Launch L, const uin
     pt_store(it.P + ((size_t)slot * rows + row) * 36, x);
 }
 
+// The same ladders by two lanes each (ladder_pair.hip.h): 2^lr rows of up to 32 >> lr products a
+// wave, both lanes of a pair storing the result they share.
+template <int W>
+__global__ void __launch_bounds__(64, 1) k_direct_products_pair(Launch L, const uint32_t *plan, const uint32_t *ops,
+                                                                const uint32_t *index) {
+    unsigned local;
+    const Item &it = L.item[find_item(L, blockIdx.x, local)];
+    const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
+    const unsigned rows = it.rows, rg = (rows + 31) / 32, lr = min(direct_row_lanes(rows), 5u);
+    const uint32_t w = plan[st.waves[5 - lr] + local / rg];
+    const unsigned pair = threadIdx.x >> 1, sub = pair >> lr, count = w >> 16;
+    const unsigned row = min((local % rg) * 32 + (pair & ((1u << lr) - 1)), rows - 1);
+    const unsigned slot = (w & 0xffffu) + min(sub, count - 1);  // spare lanes repeat a product
+    const uint32_t pe = plan[st.prod + slot];
+    const unsigned e = FK20_UNIFORM(pe >> 16);
+    g1q x;
+    pt_load(x, it.D + ((size_t)(pe & 0xffffu) * rows + row) * 36);
+    if (e == 128) tw_mul_z3_pair(x, true);
+    else if (e) tw_mul_pair<W>(x, ops + index[TW_FWD * 512 + e]);
+    pt_store(it.P + ((size_t)slot * rows + row) * 36, x);
+}
+
 // ---------------------------------------------------------------- persistent transform chain
 //
 // All 2*Lmax - 1 stages in one launch of resident waves.  Work items (one butterfly of one
@@ -273,7 +296,10 @@ constexpr StageKernels make_stage_kernels() {
     K.twiddle = k_twiddle_multi<W, R22, OCC>;
     if constexpr (!R22) K.chain = k_chain<W, R22, OCC>;
     if constexpr (R22) K.quarter = k_quarter_multi<W, R22, OCC>;
-    if constexpr (R22) K.direct = k_direct_products<W, OCC>;
+    if constexpr (R22) {
+        K.direct = k_direct_products<W, OCC>;
+        K.direct_pair = k_direct_products_pair<W>;
+    }
     K.plain_load = k_plain_load<W, R22, OCC>;
     K.wnaf = W;
     K.r22 = R22;

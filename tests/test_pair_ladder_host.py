@@ -1,0 +1,46 @@
+"""CPU check of the two-lane ladder (ladder_pair.hip.h, both lanes emulated): every twiddle program
+and the short w^128 form on random points given as non-normalised projective inputs."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import oracle as O
+from fk20_amd import prover, synthetic as S
+
+P, R = O.P_MOD, O.R_MOD
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def L(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("pair") / "libpair_host.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fsanitize=signed-integer-overflow",
+                    "-fsanitize-undefined-trap-on-error", "-o", out,
+                    os.path.join(ROOT, "tests", "native", "pair_host.cpp")], check=True)
+    return ctypes.CDLL(out)
+
+
+def ptr(a):
+    return a.ctypes.data_as(ctypes.c_void_p)
+
+
+def test_programs_and_short_form(L):
+    rng = np.random.default_rng(301)
+    w = pow(5, (R - 1) // 512, R)
+    exps = [e for e in range(1, 256) if e != 128] + [128]
+    s = S.random_fr(len(exps), 302)
+    zs = np.array([O.fp(int.from_bytes(rng.bytes(48), "little") % (P - 1) + 1) for _ in exps])
+    pts = np.ascontiguousarray(O.gen_mul_projective(s, zs))
+    want = O.gen_mul_affine(np.array([O.fr(pow(w, e, R) * O.limbs_to_int(k) % R) for e, k in zip(exps, s)]))
+    r = np.zeros((2, len(exps), 18), dtype=np.uint64)
+    for n, e in enumerate(exps):
+        if e == 128:
+            L.pair_host_z3(ptr(r[0, n]), ptr(r[1, n]), ptr(pts[n]))
+        else:
+            L.pair_host_tw_mul(ptr(r[0, n]), ptr(r[1, n]), ptr(pts[n]), ptr(prover.twiddle_program(0, e)))
+    assert np.array_equal(r[0], r[1])
+    bad, first = O.match_affine(r[0], want)
+    assert bad == 0, exps[first]
