@@ -145,7 +145,8 @@ struct StageKernels {
     void (*chain)(Chain, const uint32_t *, const uint32_t *) = nullptr;
     void (*direct)(Launch, const uint32_t *, const uint32_t *, const uint32_t *) = nullptr;
     void (*direct_pair)(Launch, const uint32_t *, const uint32_t *, const uint32_t *) = nullptr;
-    void (*plain_load)(uint32_t *, const uint32_t *, unsigned, unsigned, unsigned, const uint32_t *) = nullptr;
+    void (*plain_load)(uint32_t *, const uint32_t *, unsigned, unsigned, unsigned, const uint32_t *,
+                       uint32_t *) = nullptr;
     int wnaf = 0;
     bool r22 = false;
     int occupancy = 0;

@@ -71,38 +71,11 @@ __global__ void k_fill_u32(uint32_t *p, size_t n, uint32_t v) {
     if (i < n) p[i] = v;
 }
 
-// A lane's (x, 2 y) in LDS, packed (24 words, stride 25 to spread the lanes over the banks).
-struct LdsSlot {
-    uint32_t *w;
-    __device__ void put(const fq &x, const fq &h) {
-        uint32_t t[24];
-        fq_pack(t, x);
-        fq_pack(t + 12, h);
-#pragma unroll
-        for (int k = 0; k < 24; k++) w[k] = t[k];
-    }
-    __device__ void get(fq &x, fq &h) const {
-        uint32_t t[24];
-#pragma unroll
-        for (int k = 0; k < 24; k++) t[k] = w[k];
-        fq_unpack(x, t);
-        fq_unpack(h, t + 12);
-    }
-};
-
-// flags[i / per_group] |= 1 when pts[i] lies outside the order-r subgroup.  The test's two
-// saved points sit in LDS, which leaves room for two waves per SIMD without spills.
+// flags[i / per_group] |= 1 when pts[i] lies outside the order-r subgroup.
 __global__ void __launch_bounds__(64, 2) k_subgroup_groups(uint32_t *flags, const uint32_t *pts, size_t count,
                                                            size_t per_group) {
-    __shared__ uint32_t slots[2][64 * 25];
-    const size_t i = (size_t)blockIdx.x * 64 + threadIdx.x;
-    if (i >= count) return;
-    uint32_t w[36];
-    ld_words(w, pts + i * G1P_WORDS, 9);
-    g1q p;
-    g1q_load_std(p, w);
-    LdsSlot orig{slots[0] + threadIdx.x * 25}, base{slots[1] + threadIdx.x * 25};
-    if (!g1_in_subgroup(p, orig, base)) atomicOr(flags + i / per_group, 1u);
+    __shared__ uint32_t slots[SUBGROUP_SLOT_WORDS];
+    subgroup_test(flags, pts, (size_t)blockIdx.x * 64 + threadIdx.x, count, per_group, slots);
 }
 
 // ---------------------------------------------------------------- rows outside G1
@@ -607,12 +580,15 @@ __global__ void __launch_bounds__(64) k_output_multi(Launch L) {
 
 // ---------------------------------------------------------------- launchers
 
+// a fill kernel, not hipMemsetAsync: callers may capture these launches into a graph
+static void launch_clear_flags(uint32_t *flags, size_t groups, hipStream_t s) {
+    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, flags, groups, 0u);
+}
+
 hipError_t launch_subgroup_groups(uint32_t *flags, const uint32_t *pts, size_t count, size_t per_group,
                                   hipStream_t s) {
     if (!count || !per_group) return hipSuccess;
-    const size_t groups = (count + per_group - 1) / per_group;
-    // a fill kernel, not hipMemsetAsync: callers may capture these launches into a graph
-    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, flags, groups, 0u);
+    launch_clear_flags(flags, (count + per_group - 1) / per_group, s);
     hipLaunchKernelGGL(k_subgroup_groups, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, s, flags, pts, count,
                        per_group);
     return hipGetLastError();
@@ -957,13 +933,6 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
                         const DevTables *T, const Programs &P, hipStream_t s, const DirectPlan &direct, uint32_t *products,
                         size_t product_bytes) {
     if (!rows) return hipSuccess;
-    // rows holding a point outside G1 are recomputed by k_ref_rows: the transform kinds check
-    // their inputs here, one flag per row; PLAIN_POLY2H_FFT's caller has set flags[0] from the
-    // bases, which every row's MSM output combines
-    if (kind != PLAIN_POLY2H_FFT) {
-        hipError_t e = launch_subgroup_groups(flags, in, (size_t)rows << logn, (size_t)1 << logn, s);
-        if (e != hipSuccess) return e;
-    }
     Launch L;
     memset(&L, 0, sizeof L);
     L.nitems = 1;
@@ -992,6 +961,14 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
             if (direct_product_bytes(direct, rows, logn, l) <= product_bytes) allowed |= 1u << l;
         levels = direct_choose(L, direct, both, allowed);
     }
+    // rows holding a point outside G1 are recomputed by k_ref_rows: the transform kinds check
+    // their inputs as they load them, one flag per row; PLAIN_POLY2H_FFT's caller has set
+    // flags[0] from the bases, which every row's MSM output combines
+    auto load = [&](unsigned brev, const uint32_t *scale) {
+        launch_clear_flags(flags, rows, s);
+        hipLaunchKernelGGL(K.plain_load, dim3(n * rg + (rows * n + 63) / 64), dim3(64), 0, s, D, in, rows, logn, brev,
+                           scale, flags);
+    };
     auto run_direct = [&](unsigned k) {
         launch_direct(L, direct, levels, k, P.ops, P.index, K, s, LaunchHook{nullptr, nullptr});
     };
@@ -1019,13 +996,12 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
     };
     switch (kind) {
     case PLAIN_G1_FFT:
-        hipLaunchKernelGGL(K.plain_load, dim3(n * rg), dim3(64), 0, s, D, in, rows, logn, 0u,
-                           (const uint32_t *)nullptr);
+        load(0u, nullptr);
         if (levels) run_direct(DIRECT_FFT);
         else for (unsigned t = 0; t < logn; t++) stage(K.dif, (int)t);
         break;
     case PLAIN_G1_IFT:
-        hipLaunchKernelGGL(K.plain_load, dim3(n * rg), dim3(64), 0, s, D, in, rows, logn, 1u, scale);
+        load(1u, scale);
         if (levels) run_direct(DIRECT_IFFT);
         else for (unsigned t = 0; t < logn; t++) stage(K.dit, (int)t);
         it.out_format = 1;
@@ -1033,7 +1009,7 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
     case PLAIN_HEXT_FFT2H_FFT:
     case PLAIN_POLY2H_FFT:
         if (kind == PLAIN_HEXT_FFT2H_FFT) {
-            hipLaunchKernelGGL(K.plain_load, dim3(n * rg), dim3(64), 0, s, D, in, rows, logn, 1u, scale);
+            load(1u, scale);
         } else {
             launch_toeplitz_multi(L, T, s);
             hipError_t e = launch_msm_plain_T(D, tcT, xpk, msm_work, msm_bytes, rows, n, s);

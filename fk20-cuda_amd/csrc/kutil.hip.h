@@ -97,4 +97,40 @@ __device__ __forceinline__ unsigned find_item(const Launch &L, unsigned blk, uns
     return k;
 }
 
+// ---------------------------------------------------------------- subgroup membership
+
+// A lane's (x, 2 y) in LDS, packed (24 words, stride 25 to spread the lanes over the banks).
+struct LdsSlot {
+    uint32_t *w;
+    __device__ void put(const fq &x, const fq &h) {
+        uint32_t t[24];
+        fq_pack(t, x);
+        fq_pack(t + 12, h);
+#pragma unroll
+        for (int k = 0; k < 24; k++) w[k] = t[k];
+    }
+    __device__ void get(fq &x, fq &h) const {
+        uint32_t t[24];
+#pragma unroll
+        for (int k = 0; k < 24; k++) t[k] = w[k];
+        fq_unpack(x, t);
+        fq_unpack(h, t + 12);
+    }
+};
+
+// flags[i / per_group] |= 1 when pts[i] (i < count, 64 lanes a block) lies outside the order-r subgroup.
+// The test's two saved points sit in LDS (`slots`), which leaves room for two waves per SIMD
+// without spills.
+static constexpr unsigned SUBGROUP_SLOT_WORDS = 2 * 64 * 25;
+__device__ __forceinline__ void subgroup_test(uint32_t *flags, const uint32_t *pts, size_t i, size_t count,
+                                              size_t per_group, uint32_t *slots) {
+    if (i >= count) return;
+    uint32_t w[36];
+    ld_words(w, pts + i * G1P_WORDS, 9);
+    g1q p;
+    g1q_load_std(p, w);
+    LdsSlot orig{slots + threadIdx.x * 25}, base{slots + 64 * 25 + threadIdx.x * 25};
+    if (!g1_in_subgroup(p, orig, base)) atomicOr(flags + i / per_group, 1u);
+}
+
 }  // namespace fk20
