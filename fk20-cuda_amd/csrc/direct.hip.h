@@ -38,11 +38,26 @@ static constexpr unsigned DIRECT_KINDS = 4;
 // [4, 4, 8]
 static constexpr unsigned DIRECT_MAX_STEPS = 3;
 
-// log2 of the lanes a product's rows take in k_direct_products
+// log2 of the lanes that up to 64 rows take
 FK20_HD unsigned direct_row_lanes(unsigned rows) {
     unsigned lr = 0;
     while (lr < 6 && (1u << lr) < rows) lr++;
     return lr;
+}
+
+// How the waves of a step cover `rows` rows: `full` groups of 2^max_lr rows of one product each,
+// then waves of 2^k products whose rows are the `rest` last ones, 2^lr lanes each (max_lr = k + lr:
+// 6 with one lane per ladder, 5 with two).  Without the packing of the rest a batch of 65 rows would
+// cost as much as one of 128.
+struct DirectRows {
+    unsigned full, rest, lr;
+};
+FK20_HD DirectRows direct_rows(unsigned rows, unsigned max_lr) {
+    DirectRows d;
+    d.full = rows >> max_lr;
+    d.rest = rows - (d.full << max_lr);
+    d.lr = direct_row_lanes(d.rest);
+    return d;
 }
 
 // Two lanes per ladder (k_direct_products_pair) while such a launch gives no SIMD a second wave:
@@ -64,6 +79,34 @@ struct DirectStep {
     uint32_t nout, sums;             // outputs
     uint32_t nwaves[7], waves[7];    // for 2^k products per wave: first slot | count << 16 (k = 0..6)
 };
+// Waves of one step over `rows` rows
+FK20_HD unsigned direct_waves(const DirectStep &st, unsigned rows, unsigned max_lr) {
+    const DirectRows d = direct_rows(rows, max_lr);
+    return st.nwaves[0] * d.full + (d.rest ? st.nwaves[max_lr - d.lr] : 0);
+}
+// What wave `local` of them does: row0 + the lane's index below 2^lr, product word w
+struct DirectWave {
+    unsigned row0, last, lr;  // last: the batch's last row among them
+    uint32_t w;
+};
+FK20_HD DirectWave direct_wave(const DirectStep &st, const uint32_t *plan, unsigned rows, unsigned max_lr,
+                               unsigned local) {
+    const DirectRows d = direct_rows(rows, max_lr);
+    const unsigned main = st.nwaves[0] * d.full;
+    DirectWave r;
+    if (local < main) {
+        r.row0 = (local % d.full) << max_lr;
+        r.last = r.row0 + (1u << max_lr) - 1;
+        r.lr = max_lr;
+        r.w = plan[st.waves[0] + local / d.full];
+    } else {
+        r.row0 = d.full << max_lr;
+        r.last = rows - 1;
+        r.lr = d.lr;
+        r.w = plan[st.waves[max_lr - d.lr] + local - main];
+    }
+    return r;
+}
 static constexpr unsigned DIRECT_STEP_WORDS = sizeof(DirectStep) / 4;
 // an output's words: its position, three unused, then its terms: slot | sign << 31, DIRECT_NONE
 // past the last, to the step's longest sum rounded up to a multiple of the lanes

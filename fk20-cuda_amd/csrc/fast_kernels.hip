@@ -696,12 +696,6 @@ size_t direct_product_bytes(const DirectPlan &P, unsigned rows, unsigned logn, u
     return most * rows * 144;
 }
 
-// Waves that step `rec` of an item takes, one or two lanes per ladder
-static unsigned direct_waves(const DirectStep &st, unsigned rows, bool pair) {
-    if (!pair) return st.nwaves[6 - direct_row_lanes(rows)] * ((rows + 63) / 64);
-    return st.nwaves[5 - std::min(direct_row_lanes(rows), 5u)] * ((rows + 31) / 32);
-}
-
 // Estimated microseconds of the transforms of L's items, measured on MI355X: a round of generic
 // ladders takes 870 by pairs of lanes if these need at most one wave per SIMD, else 1100 when
 // each SIMD has at most one wave, 2050 per pair of waves and 1250 for an odd one after them, one
@@ -739,8 +733,8 @@ unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned
                 unsigned waves = 0, pairs = 0;
                 for (unsigned k = 0; k < L.nitems; k++) {
                     const DirectStep &st = P.rec[direct_record(L.item[k].logn2, both ? half : (unsigned)DIRECT_FFT, levels, s)];
-                    waves += direct_waves(st, L.item[k].rows, false);
-                    pairs += direct_waves(st, L.item[k].rows, true);
+                    waves += direct_waves(st, L.item[k].rows, 6);
+                    pairs += direct_waves(st, L.item[k].rows, 5);
                 }
                 t += (levels == 1 ? 190 : 110) +
                      (pairs <= DIRECT_PAIR_WAVES ? 870 : rounds(waves, 1100, 2050, 1250));
@@ -776,9 +770,9 @@ static void launch_direct(Launch &L, const DirectPlan &P, unsigned levels, unsig
             hipLaunchKernelGGL(k_direct_split, dim3(total), dim3(64), 0, s, L, P.words, pass);
             hook(add);
         }
-        total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, true); });
+        total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, 5); });
         const bool pair = total <= DIRECT_PAIR_WAVES;
-        if (!pair) total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, false); });
+        if (!pair) total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, 6); });
         hipLaunchKernelGGL(pair ? K.direct_pair : K.direct, dim3(total), dim3(64), 0, s, L, P.words, ops, index);
         hook(LK_TWIDDLE);
         total = blocks([](const Item &it, const DirectStep &st) { return ((st.nout * it.rows << st.log_lanes) + 63) / 64; });

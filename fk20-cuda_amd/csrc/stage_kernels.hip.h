@@ -160,8 +160,8 @@ __global__ void __launch_bounds__(64, OCC) k_quarter_multi(Launch L) {
     pt_store(p, x);
 }
 
-// The ladders of a direct step (direct.hip.h), record it.stage: a wave takes up to 64 >> lr
-// products of one exponent, 2^lr >= rows lanes each (more than 32 rows: one product and 64 rows).
+// The ladders of a direct step (direct.hip.h), record it.stage: a wave takes one product of 64
+// rows, or several products of one exponent of the last rows (direct_wave).
 // One round of the chip's 1024 SIMDs lasts a ladder, 1.1 ms, however few of them work.
 template <int W, int OCC>
 __global__ void __launch_bounds__(64, OCC) k_direct_products(Launch L, const uint32_t *plan, const uint32_t *ops,
@@ -169,11 +169,11 @@ __global__ void __launch_bounds__(64, OCC) k_direct_products(Launch L, const uin
     unsigned local;
     const Item &it = L.item[find_item(L, blockIdx.x, local)];
     const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
-    const unsigned rows = it.rows, rg = (rows + 63) / 64, lr = direct_row_lanes(rows);
-    const uint32_t w = plan[st.waves[6 - lr] + local / rg];
-    const unsigned sub = threadIdx.x >> lr, count = w >> 16;
-    const unsigned row = min((local % rg) * 64 + (threadIdx.x & ((1u << lr) - 1)), rows - 1);
-    const unsigned slot = (w & 0xffffu) + min(sub, count - 1);  // spare lanes repeat a product
+    const unsigned rows = it.rows;
+    const DirectWave v = direct_wave(st, plan, rows, 6, local);
+    const unsigned sub = threadIdx.x >> v.lr, count = v.w >> 16;
+    const unsigned row = min(v.row0 + (threadIdx.x & ((1u << v.lr) - 1)), v.last);
+    const unsigned slot = (v.w & 0xffffu) + min(sub, count - 1);  // spare lanes repeat a product
     const uint32_t pe = plan[st.prod + slot];
     const unsigned e = FK20_UNIFORM(pe >> 16);
     g1q x;
@@ -191,11 +191,11 @@ __global__ void __launch_bounds__(64, 1) k_direct_products_pair(Launch L, const 
     unsigned local;
     const Item &it = L.item[find_item(L, blockIdx.x, local)];
     const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
-    const unsigned rows = it.rows, rg = (rows + 31) / 32, lr = min(direct_row_lanes(rows), 5u);
-    const uint32_t w = plan[st.waves[5 - lr] + local / rg];
-    const unsigned pair = threadIdx.x >> 1, sub = pair >> lr, count = w >> 16;
-    const unsigned row = min((local % rg) * 32 + (pair & ((1u << lr) - 1)), rows - 1);
-    const unsigned slot = (w & 0xffffu) + min(sub, count - 1);  // spare lanes repeat a product
+    const unsigned rows = it.rows;
+    const DirectWave v = direct_wave(st, plan, rows, 5, local);
+    const unsigned pair = threadIdx.x >> 1, sub = pair >> v.lr, count = v.w >> 16;
+    const unsigned row = min(v.row0 + (pair & ((1u << v.lr) - 1)), v.last);
+    const unsigned slot = (v.w & 0xffffu) + min(sub, count - 1);  // spare lanes repeat a product
     const uint32_t pe = plan[st.prod + slot];
     const unsigned e = FK20_UNIFORM(pe >> 16);
     g1q x;

@@ -130,3 +130,22 @@ def test_row_lanes(plans):
     for rows in range(1, 200):
         lr = L.direct_host_row_lanes(rows)
         assert lr == min(6, (rows - 1).bit_length())
+
+
+@pytest.mark.parametrize("max_lr", [5, 6])  # two lanes per ladder, one
+def test_waves_cover_rows_and_products(plans, max_lr):
+    """Every (product, row) once or more, every wave's lanes on one exponent, nothing else."""
+    L, words = plans
+    buf = (ctypes.c_uint32 * 128)()
+    for logn, levels in ((7, 2), (8, 3), (9, 2)):
+        rec = L.direct_host_record(logn, FFT, levels, levels - 1)
+        nprod, prod = words[rec + 6], words[rec + 7]
+        for rows in (1, 2, 3, 31, 32, 33, 48, 63, 64, 65, 100, 128, 200, 256):
+            seen = set()
+            n = L.direct_host_waves(rec, rows, max_lr)
+            for local in range(n):
+                L.direct_host_wave(rec, rows, max_lr, local, buf)
+                lanes = {(buf[2 * p], buf[2 * p + 1]) for p in range(1 << max_lr)}
+                assert len({words[prod + s] >> 16 for _, s in lanes}) == 1
+                seen |= lanes
+            assert seen == {(r, s) for r in range(rows) for s in range(nprod)}
