@@ -160,6 +160,33 @@ PAIR_FN void pair_finish(pair_fq &X, pair_fq &Y, pair_fq &Z, const pair_h &P, co
     fq_mul(X, X, z);
 }
 
+// [2^n] of the homogeneous point (x : y : z) both lanes hold (coordinates < 8, z not 0): into
+// Jacobian form (X Z, Y Z^2, Z), n doublings, and back.  Any point of the curve: doublings have no
+// exception, as the curve's order is odd.  3 200 instructions for the two changes of form, 1 600
+// a doubling against 3 270 for the complete one.
+PAIR_FN void pair_dbl_n(pair_fq &x, pair_fq &y, pair_fq &z, int n) {
+    pair_h P;
+    pair_fq s, t, a, b;
+    fq_sqr(s, z);
+    pair_sel(a, x, y);
+    pair_sel(b, z, s);
+    fq_mul(s, a, b);                // X Z | Y Z^2
+    fq_add(t, s, s);
+    pair_sel(P.p, s, t);
+    P.z = z;
+#pragma unroll 1
+    for (int i = 0; i < n; i++) pair_dbl(P);
+    fq_sqr(s, P.z);
+    fq_add(t, P.z, P.z);
+    pair_sel(a, P.p, s);
+    fq_mul(s, a, t);                // 2 X Z | 2 Z^3
+    pair_swap(t, s);
+    pair_sel(x, s, t);
+    pair_sel(z, t, s);
+    pair_swap(t, P.p);
+    pair_sel(y, t, P.p);            // 2 Y
+}
+
 // The ladder's run over a table T: entry(e) gives x | 2 y of the e-th odd multiple.
 template <class Entry>
 PAIR_FN void pair_program(pair_h &acc, const uint32_t *ops, const Entry &entry) {

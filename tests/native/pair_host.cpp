@@ -26,6 +26,19 @@ void pair_host_tw_mul(uint32_t *r0, uint32_t *r1, const uint32_t *p, const uint3
     g1q_store_std(r1, g1q{X.v[1], Y.v[1], Z.v[1]});
 }
 
+// p <- [2^n] p
+void pair_host_dbl_n(uint32_t *r0, uint32_t *r1, const uint32_t *p, int n) {
+    g1q x;
+    g1q_load_std(x, p);
+    pair_fq X, Y, Z;
+    pair_both(X, x.x);
+    pair_both(Y, x.y);
+    pair_both(Z, x.z);
+    pair_dbl_n(X, Y, Z, n);
+    g1q_store_std(r0, g1q{X.v[0], Y.v[0], Z.v[0]});
+    g1q_store_std(r1, g1q{X.v[1], Y.v[1], Z.v[1]});
+}
+
 // p <- [w^128] p as the kernels' short form runs it
 void pair_host_z3(uint32_t *r0, uint32_t *r1, const uint32_t *p) {
     g1q x;

@@ -44,3 +44,19 @@ def test_programs_and_short_form(L):
     assert np.array_equal(r[0], r[1])
     bad, first = O.match_affine(r[0], want)
     assert bad == 0, exps[first]
+
+
+def test_doublings(L):
+    """[2^n] of projective points in G1 and of curve points outside it."""
+    s = S.random_fr(4, 303)
+    zs = np.array([O.fp(7 + k) for k in range(4)])
+    pts = np.concatenate([O.gen_mul_projective(s, zs), S.curve_points(4, 304)])
+    r = np.zeros((2, 18), dtype=np.uint64)
+    for p in pts:
+        for n in (0, 1, 6, 40):
+            L.pair_host_dbl_n(ptr(r[0]), ptr(r[1]), ptr(p), n)
+            want = p
+            for _ in range(n):
+                want = O.g1p_op("dbl", want)
+            assert np.array_equal(r[0], r[1])
+            assert np.array_equal(O.to_affine(r[:1]), O.to_affine(np.asarray(want).reshape(1, 18))), n
