@@ -17,8 +17,6 @@ static constexpr uint32_t FP_16P[14] = {0x1ffaaab0u, 0x1f7fffffu, 0x0ffffee7u, 0
 static constexpr uint32_t FP_32P[14] = {0x1ff55560u, 0x1effffffu, 0x1ffffdcfu, 0x1fffac54u, 0x0c483d57u, 0x0a0f6b0fu, 0x1fb39869u, 0x13ce144au, 0x0c8ee970u, 0x034bacd7u, 0x18dd3db2u, 0x1ff9a692u, 0x0223d472u, 0x000001a0u};  // 32 p
 static constexpr uint32_t FP_64P[14] = {0x1feaaac0u, 0x1dffffffu, 0x1ffffb9fu, 0x1fff58a9u, 0x18907aafu, 0x141ed61eu, 0x1f6730d2u, 0x079c2895u, 0x191dd2e1u, 0x069759aeu, 0x11ba7b64u, 0x1ff34d25u, 0x0447a8e5u, 0x00000340u};  // 64 p
 static constexpr uint32_t FP_128P[14] = {0x1fd55580u, 0x1bffffffu, 0x1ffff73fu, 0x1ffeb153u, 0x1120f55fu, 0x083dac3du, 0x1ece61a5u, 0x0f38512bu, 0x123ba5c2u, 0x0d2eb35du, 0x0374f6c8u, 0x1fe69a4bu, 0x088f51cbu, 0x00000680u};  // 128 p
-static constexpr uint32_t FP_BETA[14] = {0x1195dfebu, 0x1b04e484u, 0x06026044u, 0x086070a2u, 0x1fd68858u, 0x137e9670u, 0x06871e67u, 0x1e736664u, 0x083b24f6u, 0x08a70373u, 0x02a012fdu, 0x0112f94bu, 0x18a2733cu, 0x00000003u};  // beta (Montgomery)
-static constexpr uint32_t FP_BETA2[14] = {0x0abf79e7u, 0x194b14ebu, 0x1ceb16a6u, 0x1845cd5du, 0x0c814568u, 0x199ca109u, 0x13ee6ee1u, 0x05d123e5u, 0x0dfbdce2u, 0x010ecb54u, 0x0d9337edu, 0x1daaf4b0u, 0x146806fbu, 0x0000000cu};  // beta^2 (Montgomery)
 static constexpr uint64_t GLV_LAMBDA[2] = {0x00000000ffffffffull, 0xac45a4010001a402ull};  // z^2 - 1
 
 // ---- Fp, signed form: 13 x 30-bit digits, Montgomery radix 2^390 ----

@@ -113,7 +113,6 @@ static constexpr unsigned DIRECT_STEP_WORDS = sizeof(DirectStep) / 4;
 static constexpr unsigned DIRECT_SUM_FIRST = 4;
 // The split of radix a = 2^loga and stride 2^logb in passes of at most 32 points: pass 0 takes
 // up to 5 levels, pass 1 the rest on the sums it leaves, at the lowest 2^(loga + logb - 5) indices.
-FK20_HD unsigned direct_split_passes(unsigned loga) { return loga > 5 ? 2 : 1; }
 FK20_HD unsigned direct_split_log(unsigned loga, unsigned pass) {
     return pass == 0 ? (loga > 5 ? 5 : loga) : loga - 5;
 }

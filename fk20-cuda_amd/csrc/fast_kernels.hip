@@ -4,21 +4,21 @@
 //                      into the setup, so the G1 IFFT below runs unscaled).
 //  2. k_table_build    fixed-base signed-window tables T[b][win][d] = d * 2^(w*win) * base_b
 //                      (d = 1 .. 2^(w-1)), affine, canonical Montgomery, one per base.
-//  3. k_toeplitz_fft_T Toeplitz coefficients + NTT per (row, i), written transposed as
+//  3. k_toeplitz_fft_multi  Toeplitz coefficients + NTT per (row, i), written transposed as
 //                      tcT[j][i][row] so 64 rows of one column are contiguous.
-//  4. k_msm_comb       hext_fft[j] of every row = sum_i tc_fft[i][j] * xext_fft[i][j] by
+//  4. k_msm_multi      hext_fft[j] of every row = sum_i tc_fft[i][j] * xext_fft[i][j] by
 //                      signed fixed windows: ceil(256/w) mixed additions per term, no
-//                      doublings.  Lanes = rows of one column, so a wave gathers from the
-//                      table region of one base.  Output goes to D[bitrev(j)][row].
-//  5. k_dit_stage / k_middle / k_dif_stage / k_twiddle_multi
-//                      the G1 IFFT (DIT, bit-reversed in, natural out), the fused last IFFT
-//                      stage + zero upper half + first FFT stage, and the G1 FFT (DIF,
-//                      natural in, bit-reversed out), column-batched: a wave is one
-//                      butterfly (or, in a twiddle layer, one point) for 64 rows, so the
-//                      twiddle is wave-uniform and runs as a precomputed GLV + wNAF program
-//                      (uniform control flow, no divergence).  Radix-2^2 schedule: the
-//                      butterflies carry only w^+-128 twiddles, the point-wise layers the rest.
-//  6. k_fft_output     D[pos][row] -> h_fft[row][bitrev(pos)] in the reference ABI.
+//                      doublings.  Lanes = rows of one column (1, 4 or 16 lanes per row), so a
+//                      wave gathers from the table region of one base.  Output goes to
+//                      D[bitrev(j)][row].
+//  5. the transforms   (stage_kernels.hip.h) column-batched: the G1 IFFT (DIT, bit-reversed in,
+//                      natural out), the fused last IFFT stage + zero upper half + first FFT
+//                      stage, and the G1 FFT (DIF, natural in, bit-reversed out), radix 2^2
+//                      with point-wise twiddle layers; a wave is one butterfly or point for 64
+//                      rows, so the twiddle is wave-uniform and runs as a precomputed GLV +
+//                      wNAF program.  Small batches take the direct schedule instead
+//                      (direct.hip.h; k_direct_split, k_direct_sums).
+//  6. k_output_multi   D[pos][row] -> h_fft[row][bitrev(pos)] in the reference ABI, z = 1.
 // Same mathematics as fk20_msm.cu:23-66, g1p_fft.cu:25-330 and fk20_hext_fft2h_fft.cu:27-70;
 // the layout and algorithms are this library's own.
 #include <cstring>

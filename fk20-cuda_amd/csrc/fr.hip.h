@@ -2,9 +2,9 @@
 // canonical values in [0, r).
 //
 // Replaces the reference's standard-form Fr (fr_mul.cu:13 schoolbook + Barrett,
-// fr_addsub.cu:18, fr_add.cuh, fr_sub.cuh).  Fr work on the FK20 path is the Toeplitz
-// NTT only (well under 1% of the path's multiply-adds), so this is a plain CIOS with
-// carry chains rather than the lazy 29-bit form used for Fp.
+// fr_addsub.cu:18, fr_add.cuh, fr_sub.cuh).  This is a plain CIOS with carry chains, for the
+// element-wise operations and the programs' checks; the transforms run on the 9 signed
+// 29-bit digits of fn below.
 #pragma once
 #include <stdint.h>
 

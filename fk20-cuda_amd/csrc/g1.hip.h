@@ -3,7 +3,8 @@
 // Complete formulas of Renes, Costello and Batina (eprint 2015/1060): algorithm 7
 // (addition), 8 (mixed addition with an affine point) and 9 (doubling) for a = 0,
 // b3 = 3b = 12 -- the same formulas the reference uses (g1p_add.cu:78, g1p_dbl.cu:28,
-// g1p_multi.cu:83), written for the lazy 29-bit Fp of fp.hip.h.  The point at infinity is
+// g1p_multi.cu:83), written for the lazy 29-bit Fp of fp.hip.h.  The element-wise
+// point operations of the C ABI run them; every other kernel has g1q.hip.h.  The point at infinity is
 // (0 : 1 : 0); any (0 : y != 0 : 0) is accepted as infinity (g1.cuh:14 G1P_ANYINF).
 //
 // Value bounds (multiples of p) are annotated per step.  Inputs may be anything
@@ -121,16 +122,6 @@ FK20_HD void g1_neg(g1p &r, const g1p &p) {
     r.z = p.z;
 }
 
-// (p, q) <- (p + q, p - q)
-FK20_HD void g1_addsub(g1p &p, g1p &q) {
-    g1p nq;
-    g1_neg(nq, q);      // y < 16p: g1_add accepts inputs < 20p in practice (see bound notes)
-    g1p s;
-    g1_add(s, p, q);
-    g1_add(q, p, nq);
-    p = s;
-}
-
 // ---------------------------------------------------------------- memory forms
 
 // Standard-form g1p_t (reference ABI: 3 x 6 x u64, little endian) <-> Montgomery registers.
@@ -153,19 +144,6 @@ FK20_HD void g1_store_std(uint32_t *w, const g1p &p) {
     fe_pack(w + 12, t);
     fe_from_mont(t, p.z);
     fe_pack(w + 24, t);
-}
-
-// Packed Montgomery form (internal buffers): 36 words, values < 2^384.
-FK20_HD void g1_load_packed(g1p &p, const uint32_t *w) {
-    fe_unpack(p.x, w);
-    fe_unpack(p.y, w + 12);
-    fe_unpack(p.z, w + 24);
-}
-
-FK20_HD void g1_store_packed(uint32_t *w, const g1p &p) {
-    fe_pack(w, p.x);
-    fe_pack(w + 12, p.y);
-    fe_pack(w + 24, p.z);
 }
 
 // ---------------------------------------------------------------- scalar multiplication

@@ -120,8 +120,6 @@ def main():
     assert lam * lam + lam + 1 == R
     beta = 0x1A0111EA397FE699EC02408663D4DE85AA0D857D89759AD4897D29650FB85F9B409427EB4F49FFFD8BFD00000000AAAC
     assert pow(beta, 3, P) == 1 and beta != 1
-    out.append(carr("FP_BETA", limbs(beta * rm % P, FP_BITS, FP_N)) + "  // beta (Montgomery)")
-    out.append(carr("FP_BETA2", limbs(beta * beta * rm % P, FP_BITS, FP_N)) + "  // beta^2 (Montgomery)")
     out.append("static constexpr uint64_t GLV_LAMBDA[2] = {0x%016xull, 0x%016xull};  // z^2 - 1"
                % (lam & (2**64 - 1), lam >> 64))
     out.append("")

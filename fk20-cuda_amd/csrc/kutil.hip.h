@@ -46,13 +46,6 @@ __device__ __forceinline__ void fq_store(uint32_t *g, const fq &a) {
     st_words(g, w, 3);
 }
 
-// a coordinate of a window-table entry: canonical Montgomery, no offset
-__device__ __forceinline__ void fq_load_raw(fq &a, const uint32_t *g) {
-    uint32_t w[12];
-    ld_words(w, g, 3);
-    fq_unpack_raw(a, w);
-}
-
 // ---------------------------------------------------------------- sums across lanes
 
 __device__ __forceinline__ void shfl_point(g1q &r, const g1q &p, int lane) {
