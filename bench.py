@@ -453,8 +453,8 @@ def bench_limbs(args):
 
 
 def bench_fieldmul(args):
-    """Throughput of the Fp Montgomery multiplication itself (14 x 29-bit limbs), the unit
-    every G1 kernel is built from: Fermat inversions a^(p-2) through fk20_fp_op (one lane per
+    """Throughput of the 14 x 29-bit Fp Montgomery multiplication itself (the element-wise
+    operations' form; the G1 kernels' 13-digit one is faster): Fermat inversions a^(p-2) through fk20_fp_op (one lane per
     element, 384 squarings + one multiplication per set bit of p - 2, no memory traffic in
     the loop), on `fieldmul_count` uniform non-zero elements; a sample is checked on the host."""
     count = args.fieldmul_count
