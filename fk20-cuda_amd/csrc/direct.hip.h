@@ -60,10 +60,6 @@ FK20_HD DirectRows direct_rows(unsigned rows, unsigned max_lr) {
     return d;
 }
 
-// Two lanes per ladder (k_direct_products_pair) while such a launch gives no SIMD a second wave:
-// alone on a SIMD its waves take 0.87 ms against 1.10, but they hold half as many ladders.
-static constexpr unsigned DIRECT_PAIR_WAVES = 1024;
-
 FK20_HD unsigned direct_radix_log(unsigned logn, unsigned levels, unsigned step) {
     if (levels == 1) return logn;
     if (levels == 2) return step == 0 ? (logn == 7 ? 3u : 4u) : (logn == 9 ? 5u : 4u);

@@ -147,6 +147,9 @@ struct StageKernels {
     void (*direct_pair)(Launch, const uint32_t *, const uint32_t *, const uint32_t *) = nullptr;
     void (*plain_load)(uint32_t *, const uint32_t *, unsigned, unsigned, unsigned, const uint32_t *,
                        uint32_t *) = nullptr;
+    // two lanes per ladder (ladder_pair.hip.h); radix-2^2 variants only, as `direct`
+    void (*plain_load_pair)(uint32_t *, const uint32_t *, unsigned, unsigned, unsigned, const uint32_t *,
+                            uint32_t *) = nullptr;
     int wnaf = 0;
     bool r22 = false;
     int occupancy = 0;
@@ -156,6 +159,10 @@ const StageKernels *stage_kernels(unsigned wnaf, bool r22, unsigned occupancy);
 // The default schedule: the drop-in entry points and new contexts use it.
 static constexpr unsigned DEFAULT_OCCUPANCY = 2;
 inline const StageKernels &default_stage_kernels() { return *stage_kernels(TW_WNAF, true, DEFAULT_OCCUPANCY); }
+
+// Two lanes per ladder (ladder_pair.hip.h) while such a launch gives no SIMD a second wave: alone on
+// a SIMD its waves take 0.87 ms against 1.10 for a generic ladder, but they hold half as many.
+static constexpr unsigned PAIR_WAVES = 1024;
 
 // The direct schedule's plans on the current device: the words the kernels read, and the records
 // on the host, for the launchers.

@@ -78,6 +78,13 @@ __global__ void __launch_bounds__(64, 2) k_subgroup_groups(uint32_t *flags, cons
     subgroup_test(flags, pts, (size_t)blockIdx.x * 64 + threadIdx.x, count, per_group, slots);
 }
 
+// The same by two lanes per point (ladder_pair.hip.h), 32 points a block: 126 doublings after one
+// another are the launch's time while SIMDs idle (8 192 points 0.73 -> 0.46 ms).
+__global__ void __launch_bounds__(64, 1) k_subgroup_pair(uint32_t *flags, const uint32_t *pts, size_t count,
+                                                         size_t per_group) {
+    subgroup_test_pair(flags, pts, (size_t)blockIdx.x * 32 + threadIdx.x / 2, count, per_group);
+}
+
 // ---------------------------------------------------------------- rows outside G1
 //
 // On a point P outside the order-r subgroup, [a]P and [b]P differ whenever a != b as integers,
@@ -589,8 +596,13 @@ hipError_t launch_subgroup_groups(uint32_t *flags, const uint32_t *pts, size_t c
                                   hipStream_t s) {
     if (!count || !per_group) return hipSuccess;
     launch_clear_flags(flags, (count + per_group - 1) / per_group, s);
-    hipLaunchKernelGGL(k_subgroup_groups, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, s, flags, pts, count,
-                       per_group);
+    // two lanes per point while no SIMD gets a second wave
+    if (count <= 32 * PAIR_WAVES)
+        hipLaunchKernelGGL(k_subgroup_pair, dim3((unsigned)((count + 31) / 32)), dim3(64), 0, s, flags, pts, count,
+                           per_group);
+    else
+        hipLaunchKernelGGL(k_subgroup_groups, dim3((unsigned)((count + 63) / 64)), dim3(64), 0, s, flags, pts, count,
+                           per_group);
     return hipGetLastError();
 }
 
@@ -737,7 +749,7 @@ unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned
                     pairs += direct_waves(st, L.item[k].rows, 5);
                 }
                 t += (levels == 1 ? 190 : 110) +
-                     (pairs <= DIRECT_PAIR_WAVES ? 870 : rounds(waves, 1100, 2050, 1250));
+                     (pairs <= PAIR_WAVES ? 870 : rounds(waves, 1100, 2050, 1250));
             }
         if (t < time) time = t, best = levels;
     }
@@ -771,7 +783,7 @@ static void launch_direct(Launch &L, const DirectPlan &P, unsigned levels, unsig
             hook(add);
         }
         total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, 5); });
-        const bool pair = total <= DIRECT_PAIR_WAVES;
+        const bool pair = total <= PAIR_WAVES;
         if (!pair) total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, 6); });
         hipLaunchKernelGGL(pair ? K.direct_pair : K.direct, dim3(total), dim3(64), 0, s, L, P.words, ops, index);
         hook(LK_TWIDDLE);
@@ -960,8 +972,11 @@ hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const
     // flags[0] from the bases, which every row's MSM output combines
     auto load = [&](unsigned brev, const uint32_t *scale) {
         launch_clear_flags(flags, rows, s);
-        hipLaunchKernelGGL(K.plain_load, dim3(n * rg + (rows * n + 63) / 64), dim3(64), 0, s, D, in, rows, logn, brev,
-                           scale, flags);
+        const size_t pairs = (size_t)n * ((rows + 31) / 32) + ((size_t)rows * n + 31) / 32;
+        const bool pair = pairs <= PAIR_WAVES;
+        hipLaunchKernelGGL(pair ? K.plain_load_pair : K.plain_load,
+                           dim3(pair ? (unsigned)pairs : n * rg + (rows * n + 63) / 64), dim3(64), 0, s, D, in, rows, logn,
+                           brev, scale, flags);
     };
     auto run_direct = [&](unsigned k) {
         launch_direct(L, direct, levels, k, P.ops, P.index, K, s, LaunchHook{nullptr, nullptr});

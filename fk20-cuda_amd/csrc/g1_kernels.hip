@@ -6,7 +6,6 @@
 
 #include "common.hip.h"
 #include "kutil.hip.h"
-#include "ladder_pair.hip.h"
 
 namespace fk20 {
 

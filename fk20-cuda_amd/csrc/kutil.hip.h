@@ -3,6 +3,7 @@
 // lookup of the batched path.
 #pragma once
 #include "fast.hip.h"
+#include "ladder_pair.hip.h"
 
 namespace fk20 {
 
@@ -124,6 +125,16 @@ __device__ __forceinline__ void subgroup_test(uint32_t *flags, const uint32_t *p
     g1q_load_std(p, w);
     LdsSlot orig{slots + threadIdx.x * 25}, base{slots + 64 * 25 + threadIdx.x * 25};
     if (!g1_in_subgroup(p, orig, base)) atomicOr(flags + i / per_group, 1u);
+}
+// the same by the two lanes of a pair, 32 points a block
+__device__ __forceinline__ void subgroup_test_pair(uint32_t *flags, const uint32_t *pts, size_t i, size_t count,
+                                                   size_t per_group) {
+    if (i >= count) return;
+    uint32_t w[36];
+    ld_words(w, pts + i * G1P_WORDS, 9);
+    g1q p;
+    g1q_load_std(p, w);
+    if (!g1_in_subgroup_pair(p)) atomicOr(flags + i / per_group, 1u);
 }
 
 }  // namespace fk20

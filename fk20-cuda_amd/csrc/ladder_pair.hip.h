@@ -5,7 +5,7 @@
 // (1 630 instructions with the exchanges against 2 616), a mixed addition five products and a
 // square (3 050 against 4 020).  The values go between the lanes by DPP.  A launch of single ladders
 // takes 1.10 ms, of pairs 0.87 (one row of N = 4096: 3.09 -> 2.41 ms).  The two lanes' work
-// is a quarter more than one lane's, so it only pays on idle SIMDs (DIRECT_PAIR_WAVES, direct.hip.h).
+// is a quarter more than one lane's, so it only pays on idle SIMDs (PAIR_WAVES, fast.hip.h).
 //
 // pair_fq is a value of each lane: fq on the device, both lanes' values in the CPU tests.
 #pragma once
@@ -240,7 +240,53 @@ PAIR_FN void pair_z(pair_h &acc, const pair_fq &q) {
     }
 }
 
+// What g1_in_subgroup compares, for the point whose Jacobian (X Z | 2 Y Z^2) is `orig`: both
+// lanes' residues v are 0 and zz is not if it lies in G1.
+PAIR_FN void pair_subgroup(pair_fq &v, pair_fq &zz, const pair_fq &orig) {
+    pair_fq one, f, t, n;
+    fq k;
+    fq_one(k);
+    pair_both(one, k);
+    pair_h acc;
+    acc.p = orig;
+    zz = one;
+#pragma unroll 1
+    for (int round = 0; round < 2; round++) {
+        pair_fq base;
+        fq_mul(base, acc.p, one);   // < 30 -> < 0.6
+        pair_z(acc, base);
+        fq_mul(zz, zz, acc.z);
+    }
+    // [z^2] p = (X / zz^2, H / 2 zz^3) against -phi^2(p)
+    fq_set(k, FQ_GLV2);
+    pair_both(f, k);
+    pair_sel(f, f, one);
+    fq_mul(v, orig, f);             // beta^2 x | h
+    fq_sqr(f, zz);
+    fq_mul(t, f, zz);
+    pair_sel(f, f, t);
+    fq_mul(v, v, f);                // .. zz^2 | .. zz^3
+    fq_neg(n, acc.p);
+    pair_sel(n, n, acc.p);
+    fq_add(v, v, n);
+}
+
 #ifdef __HIPCC__
+// g1_in_subgroup by a pair of lanes that both hold p, and both get the result
+__device__ __forceinline__ bool g1_in_subgroup_pair(const g1q &p) {
+    fq px, ph, t;
+    fq_sqr(t, p.z);
+    fq_mul(px, p.x, p.z);
+    fq_mul(ph, p.y, t);
+    fq_add(ph, ph, ph);
+    pair_fq orig, v, zz;
+    pair_sel(orig, px, ph);
+    pair_subgroup(v, zz, orig);
+    const int mine = fq_is_zero(v);
+    const int other = __builtin_amdgcn_update_dpp(0, mine, 0xB1, 0xf, 0xf, true);
+    return g1q_is_inf(p) || (mine && other && !fq_is_zero(zz));
+}
+
 // tw_mul and tw_mul_z3 by a pair of lanes that both hold x, and both get the result.
 template <int W>
 __device__ __forceinline__ void tw_mul_pair(g1q &x, const uint32_t *ops) {

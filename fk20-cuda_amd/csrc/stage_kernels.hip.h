@@ -4,7 +4,6 @@
 // StageKernels table; a context picks its variant at run time (fk20_ctx_set_schedule).
 #pragma once
 #include "kutil.hip.h"
-#include "ladder_pair.hip.h"
 
 namespace fk20 {
 
@@ -295,6 +294,25 @@ __global__ void __launch_bounds__(64, OCC) k_plain_load(uint32_t *D, const uint3
     pt_store(D + ((size_t)(brev ? bitrev(j, logn) : j) * rows + row) * 36, p);
 }
 
+// The same with two lanes per row and point (PAIR_WAVES); 65 inverse transforms of 128: 0.79 -> 0.55 ms.
+template <int W>
+__global__ void __launch_bounds__(64, 1) k_plain_load_pair(uint32_t *D, const uint32_t *in, unsigned rows, unsigned logn,
+                                                           unsigned brev, const uint32_t *scale_ops, uint32_t *flags) {
+    const unsigned rg = (rows + 31) / 32, j = blockIdx.x / rg;
+    if (j >= 1u << logn) {
+        const size_t i = (size_t)(blockIdx.x - (rg << logn)) * 32 + threadIdx.x / 2;
+        subgroup_test_pair(flags, in, i, (size_t)rows << logn, (size_t)1 << logn);
+        return;
+    }
+    const unsigned row = min((blockIdx.x % rg) * 32 + threadIdx.x / 2, rows - 1);
+    uint32_t w[36];
+    ld_words(w, in + ((size_t)row * (1u << logn) + j) * G1P_WORDS, 9);
+    g1q p;
+    g1q_load_std(p, w);
+    if (scale_ops) tw_mul_pair<W>(p, scale_ops);
+    pt_store(D + ((size_t)(brev ? bitrev(j, logn) : j) * rows + row) * 36, p);
+}
+
 // The kernel table of variant (W, R22, OCC); the persistent chain (radix 2 whatever the
 // variant's butterflies) is published by the radix-2 variants only.
 template <int W, bool R22, int OCC>
@@ -309,6 +327,7 @@ constexpr StageKernels make_stage_kernels() {
     if constexpr (R22) {
         K.direct = k_direct_products<W, OCC>;
         K.direct_pair = k_direct_products_pair<W>;
+        K.plain_load_pair = k_plain_load_pair<W>;
     }
     K.plain_load = k_plain_load<W, R22, OCC>;
     K.wnaf = W;

@@ -26,6 +26,22 @@ void pair_host_tw_mul(uint32_t *r0, uint32_t *r1, const uint32_t *p, const uint3
     g1q_store_std(r1, g1q{X.v[1], Y.v[1], Z.v[1]});
 }
 
+// whether p lies in G1, by the pair's comparison
+int pair_host_in_subgroup(const uint32_t *p) {
+    g1q x;
+    g1q_load_std(x, p);
+    fq t, px, ph;
+    fq_sqr(t, x.z);
+    fq_mul(px, x.x, x.z);
+    fq_mul(ph, x.y, t);
+    fq_add(ph, ph, ph);
+    pair_fq orig, v, zz;
+    orig.v[0] = px;
+    orig.v[1] = ph;
+    pair_subgroup(v, zz, orig);
+    return g1q_is_inf(x) || (fq_is_zero(v.v[0]) && fq_is_zero(v.v[1]) && !fq_is_zero(zz.v[0]));
+}
+
 // p <- [2^n] p
 void pair_host_dbl_n(uint32_t *r0, uint32_t *r1, const uint32_t *p, int n) {
     g1q x;

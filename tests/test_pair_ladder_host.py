@@ -60,3 +60,21 @@ def test_doublings(L):
                 want = O.g1p_op("dbl", want)
             assert np.array_equal(r[0], r[1])
             assert np.array_equal(O.to_affine(r[:1]), O.to_affine(np.asarray(want).reshape(1, 18))), n
+
+
+def test_membership(L):
+    """The pair's comparison against the definition [r]P = 0: points of G1, infinity, curve points,
+    points of small order and their sums with G1 points."""
+    from test_device_arith_host import H_COF, _mul_big
+    G = O.g1p_gen()
+    curve = list(S.curve_points(3, 305))
+    pts = [G, O.g1p_inf(), O.g1p_op("mul", G, O.fr(R - 1))] + curve + [_mul_big(curve[0], H_COF)]
+    small = []
+    for q in curve:
+        rq = O.g1p_op("mul", q, O.fr(R))
+        small += [t for t in (_mul_big(rq, H_COF // m) for m in (3, 11, 121)) if not O.g1p_is_inf(t)]
+    assert small
+    pts += small + [O.g1p_op("add", G, t) for t in small[:2]]
+    for p in pts:
+        want = O.g1p_is_inf(O.g1p_op("mul", p, O.fr(R)))
+        assert L.pair_host_in_subgroup(ptr(np.ascontiguousarray(p))) == int(want)
