@@ -45,21 +45,6 @@ FK20_HD unsigned direct_row_lanes(unsigned rows) {
     return lr;
 }
 
-// How the waves of a step cover `rows` rows: `full` groups of 2^max_lr rows of one product each,
-// then waves of 2^k products whose rows are the `rest` last ones, 2^lr lanes each (max_lr = k + lr:
-// 6 with one lane per ladder, 5 with two).  Without the packing of the rest a batch of 65 rows would
-// cost as much as one of 128.
-struct DirectRows {
-    unsigned full, rest, lr;
-};
-FK20_HD DirectRows direct_rows(unsigned rows, unsigned max_lr) {
-    DirectRows d;
-    d.full = rows >> max_lr;
-    d.rest = rows - (d.full << max_lr);
-    d.lr = direct_row_lanes(d.rest);
-    return d;
-}
-
 FK20_HD unsigned direct_radix_log(unsigned logn, unsigned levels, unsigned step) {
     if (levels == 1) return logn;
     if (levels == 2) return step == 0 ? (logn == 7 ? 3u : 4u) : (logn == 9 ? 5u : 4u);
@@ -75,32 +60,69 @@ struct DirectStep {
     uint32_t nout, sums;             // outputs
     uint32_t nwaves[7], waves[7];    // for 2^k products per wave: first slot | count << 16 (k = 0..6)
 };
-// Waves of one step over `rows` rows
-FK20_HD unsigned direct_waves(const DirectStep &st, unsigned rows, unsigned max_lr) {
-    const DirectRows d = direct_rows(rows, max_lr);
-    return st.nwaves[0] * d.full + (d.rest ? st.nwaves[max_lr - d.lr] : 0);
+// How the waves of a step cover `rows` rows, 2^max_lr lanes or pairs of lanes a wave (6, or 5 with
+// two lanes per ladder): groups of 2^max_lr rows of one product each, and the rows left over in
+// parts of 2^lr rows, up to 2^(max_lr - lr) products of one exponent a wave.  `parts` has a bit for each
+// part's lr, the largest first; the last one may be partly empty.  Of 100 rows a wave takes 64 of
+// one product, 32 of two or 4 of sixteen.  With one part for all of the rest, 40 rows of N = 4096
+// took 12.4 ms, now 8.5, 40 of N = 2048 6.0 and 5.2; 72 and 100 rows are the same.
+struct DirectParts {
+    unsigned waves, parts;
+};
+// The fewest waves for `rest` rows in parts below 2^limit: one part, or the largest that is full and
+// the same for what is left (a part costs at least a wave per exponent).
+FK20_HD DirectParts direct_rest(const DirectStep &st, unsigned rest, unsigned max_lr, unsigned limit) {
+    DirectParts best{0, 0}, done{0, 0};
+    bool have = rest == 0;
+    while (rest) {
+        const unsigned lr = direct_row_lanes(rest);
+        if (lr < limit) {
+            const unsigned w = done.waves + st.nwaves[max_lr - lr];
+            if (!have || w < best.waves) best = DirectParts{w, done.parts | 1u << lr}, have = true;
+        }
+        unsigned top = lr;
+        if ((1u << top) > rest) top--;
+        done.waves += st.nwaves[max_lr - top];
+        done.parts |= 1u << top;
+        rest -= 1u << top;
+        limit = top;
+    }
+    return best;
+}
+FK20_HD DirectParts direct_parts(const DirectStep &st, unsigned rows, unsigned max_lr) {
+    const unsigned full = rows >> max_lr;
+    DirectParts d = direct_rest(st, rows - (full << max_lr), max_lr, max_lr + 1);
+    d.waves += st.nwaves[0] * full;
+    return d;
 }
 // What wave `local` of them does: row0 + the lane's index below 2^lr, product word w
 struct DirectWave {
-    unsigned row0, last, lr;  // last: the batch's last row among them
+    unsigned row0, last, lr;  // last: the last row among them
     uint32_t w;
 };
 FK20_HD DirectWave direct_wave(const DirectStep &st, const uint32_t *plan, unsigned rows, unsigned max_lr,
-                               unsigned local) {
-    const DirectRows d = direct_rows(rows, max_lr);
-    const unsigned main = st.nwaves[0] * d.full;
+                               unsigned parts, unsigned local) {
+    const unsigned full = rows >> max_lr, main = st.nwaves[0] * full;
     DirectWave r;
     if (local < main) {
-        r.row0 = (local % d.full) << max_lr;
-        r.last = r.row0 + (1u << max_lr) - 1;
         r.lr = max_lr;
-        r.w = plan[st.waves[0] + local / d.full];
+        r.row0 = (local % full) << max_lr;
+        r.w = plan[st.waves[0] + local / full];
     } else {
-        r.row0 = d.full << max_lr;
-        r.last = rows - 1;
-        r.lr = d.lr;
-        r.w = plan[st.waves[max_lr - d.lr] + local - main];
+        local -= main;
+        r.row0 = full << max_lr;
+        r.lr = max_lr;
+        while (r.lr && (!(parts >> r.lr & 1u) || local >= st.nwaves[max_lr - r.lr])) {
+            if (parts >> r.lr & 1u) {
+                local -= st.nwaves[max_lr - r.lr];
+                r.row0 += 1u << r.lr;
+            }
+            r.lr--;
+        }
+        r.w = plan[st.waves[max_lr - r.lr] + local];
     }
+    r.last = r.row0 + (1u << r.lr) - 1;
+    if (r.last >= rows) r.last = rows - 1;
     return r;
 }
 static constexpr unsigned DIRECT_STEP_WORDS = sizeof(DirectStep) / 4;

@@ -96,6 +96,7 @@ struct Item {
     const uint32_t *rowflag;
     uint32_t flag_stride;
     uint32_t *P;            // products of the direct schedule [slot][rows], dead data before
+    uint32_t parts;         // how its waves cover the rows (direct_parts), set per launch
 };
 struct Launch {
     Item item[MAX_ITEMS];

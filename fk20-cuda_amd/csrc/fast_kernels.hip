@@ -745,8 +745,8 @@ unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned
                 unsigned waves = 0, pairs = 0;
                 for (unsigned k = 0; k < L.nitems; k++) {
                     const DirectStep &st = P.rec[direct_record(L.item[k].logn2, both ? half : (unsigned)DIRECT_FFT, levels, s)];
-                    waves += direct_waves(st, L.item[k].rows, 6);
-                    pairs += direct_waves(st, L.item[k].rows, 5);
+                    waves += direct_parts(st, L.item[k].rows, 6).waves;
+                    pairs += direct_parts(st, L.item[k].rows, 5).waves;
                 }
                 t += (levels == 1 ? 190 : 110) +
                      (pairs <= PAIR_WAVES ? 870 : rounds(waves, 1100, 2050, 1250));
@@ -782,9 +782,18 @@ static void launch_direct(Launch &L, const DirectPlan &P, unsigned levels, unsig
             hipLaunchKernelGGL(k_direct_split, dim3(total), dim3(64), 0, s, L, P.words, pass);
             hook(add);
         }
-        total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, 5); });
+        unsigned max_lr = 5;
+        auto waves = [&](Item &it, const DirectStep &st) {
+            const DirectParts d = direct_parts(st, it.rows, max_lr);
+            it.parts = d.parts;
+            return d.waves;
+        };
+        total = blocks(waves);
         const bool pair = total <= PAIR_WAVES;
-        if (!pair) total = blocks([](const Item &it, const DirectStep &st) { return direct_waves(st, it.rows, 6); });
+        if (!pair) {
+            max_lr = 6;
+            total = blocks(waves);
+        }
         hipLaunchKernelGGL(pair ? K.direct_pair : K.direct, dim3(total), dim3(64), 0, s, L, P.words, ops, index);
         hook(LK_TWIDDLE);
         total = blocks([](const Item &it, const DirectStep &st) { return ((st.nout * it.rows << st.log_lanes) + 63) / 64; });

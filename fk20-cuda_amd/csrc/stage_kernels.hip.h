@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(64, OCC) k_quarter_multi(Launch L) {
 }
 
 // The ladders of a direct step (direct.hip.h), record it.stage: a wave takes one product of 64
-// rows, or several products of one exponent of the last rows (direct_wave).
+// rows, or several products of one exponent of fewer (direct_wave).
 // One round of the chip's 1024 SIMDs lasts a ladder, 1.1 ms, however few of them work.
 template <int W, int OCC>
 __global__ void __launch_bounds__(64, OCC) k_direct_products(Launch L, const uint32_t *plan, const uint32_t *ops,
@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(64, OCC) k_direct_products(Launch L, const uin
     const Item &it = L.item[find_item(L, blockIdx.x, local)];
     const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
     const unsigned rows = it.rows;
-    const DirectWave v = direct_wave(st, plan, rows, 6, local);
+    const DirectWave v = direct_wave(st, plan, rows, 6, it.parts, local);
     const unsigned sub = threadIdx.x >> v.lr, count = v.w >> 16;
     const unsigned row = min(v.row0 + (threadIdx.x & ((1u << v.lr) - 1)), v.last);
     const unsigned slot = (v.w & 0xffffu) + min(sub, count - 1);  // spare lanes repeat a product
@@ -182,8 +182,7 @@ __global__ void __launch_bounds__(64, OCC) k_direct_products(Launch L, const uin
     pt_store(it.P + ((size_t)slot * rows + row) * 36, x);
 }
 
-// The same ladders by two lanes each (ladder_pair.hip.h): 2^lr rows of up to 32 >> lr products a
-// wave, both lanes of a pair storing the result they share.
+// The same ladders by two lanes each (ladder_pair.hip.h), both lanes of a pair storing the result they share.
 template <int W>
 __global__ void __launch_bounds__(64, 1) k_direct_products_pair(Launch L, const uint32_t *plan, const uint32_t *ops,
                                                                 const uint32_t *index) {
@@ -191,7 +190,7 @@ __global__ void __launch_bounds__(64, 1) k_direct_products_pair(Launch L, const 
     const Item &it = L.item[find_item(L, blockIdx.x, local)];
     const DirectStep &st = reinterpret_cast<const DirectStep *>(plan)[it.stage];
     const unsigned rows = it.rows;
-    const DirectWave v = direct_wave(st, plan, rows, 5, local);
+    const DirectWave v = direct_wave(st, plan, rows, 5, it.parts, local);
     const unsigned pair = threadIdx.x >> 1, sub = pair >> v.lr, count = v.w >> 16;
     const unsigned row = min(v.row0 + (pair & ((1u << v.lr) - 1)), v.last);
     const unsigned slot = (v.w & 0xffffu) + min(sub, count - 1);  // spare lanes repeat a product

@@ -22,11 +22,11 @@ unsigned direct_host_record(unsigned logn, unsigned kind, unsigned levels, unsig
 }
 // waves of record `rec` (word offset) over `rows` rows, and lane `pair` of wave `local`: row, slot
 unsigned direct_host_waves(unsigned rec, unsigned rows, unsigned max_lr) {
-    return direct_waves(*reinterpret_cast<const DirectStep *>(&g_words[rec]), rows, max_lr);
+    return direct_parts(*reinterpret_cast<const DirectStep *>(&g_words[rec]), rows, max_lr).waves;
 }
 void direct_host_wave(unsigned rec, unsigned rows, unsigned max_lr, unsigned local, uint32_t *out) {
-    const DirectWave v =
-        direct_wave(*reinterpret_cast<const DirectStep *>(&g_words[rec]), g_words.data(), rows, max_lr, local);
+    const DirectStep &st = *reinterpret_cast<const DirectStep *>(&g_words[rec]);
+    const DirectWave v = direct_wave(st, g_words.data(), rows, max_lr, direct_parts(st, rows, max_lr).parts, local);
     for (unsigned p = 0; p < 1u << max_lr; p++) {
         out[2 * p] = std::min(v.row0 + (p & ((1u << v.lr) - 1)), v.last);
         out[2 * p + 1] = (v.w & 0xffffu) + std::min(p >> v.lr, (v.w >> 16) - 1);

@@ -140,7 +140,7 @@ def test_waves_cover_rows_and_products(plans, max_lr):
     for logn, levels in ((7, 2), (8, 3), (9, 2)):
         rec = L.direct_host_record(logn, FFT, levels, levels - 1)
         nprod, prod = words[rec + 6], words[rec + 7]
-        for rows in (1, 2, 3, 31, 32, 33, 48, 63, 64, 65, 100, 128, 200, 256):
+        for rows in (1, 2, 3, 7, 13, 31, 32, 33, 37, 48, 63, 64, 65, 100, 127, 128, 200, 256):
             seen = set()
             n = L.direct_host_waves(rec, rows, max_lr)
             for local in range(n):
