@@ -643,7 +643,10 @@ static CommitShape commit_shape(unsigned rows, unsigned N) {
     return best;
 }
 
-size_t commit_workspace_bytes(unsigned rows, unsigned N) { return (size_t)commit_shape(rows, N).nparts * rows * 144; }
+// never below a partial sum per 16 coefficients and per 256, the published size
+size_t commit_workspace_bytes(unsigned rows, unsigned N) {
+    return (size_t)std::max(commit_shape(rows, N).nparts, N / 16 + (N + 255) / 256) * rows * 144;
+}
 
 hipError_t launch_commit(uint32_t *out, const uint32_t *poly, const uint32_t *table, const uint32_t *inf,
                          uint32_t *work, unsigned rows, unsigned N, unsigned win_bits, hipStream_t s) {
