@@ -12,6 +12,7 @@
 #include "../../include/fk20.h"
 #include "common.hip.h"
 #include "fast.hip.h"
+#include "scratch.h"
 
 using namespace fk20;
 
@@ -59,16 +60,32 @@ unsigned log2u(unsigned n) { return 31u - (unsigned)__builtin_clz(n); }
 
 // ---------------------------------------------------------------- per-device state
 
+// The spare workspace's memory: nothing is given up for it.
+struct SpareMemory {
+    static bool alloc(void **p, size_t bytes) {
+        if (hipMalloc(p, bytes) == hipSuccess) return true;
+        (void)hipGetLastError();  // the launches after it report their own errors
+        return false;
+    }
+    static void release(void *p) { (void)hipFree(p); }
+    static bool idle() {
+        if (hipDeviceSynchronize() == hipSuccess) return true;
+        (void)hipGetLastError();
+        return false;
+    }
+};
+
 struct DeviceState {
     DevTables *tables = nullptr;            // device copy (g_tables_dev)
     Programs prog;                          // twiddle programs of the drop-in transforms
-    void *scratch = nullptr;                // workspace of the drop-in entry points
-    size_t scratch_bytes = 0;
+    Workspace<DeviceMemory> scratch;        // workspace of the drop-in entry points
+    Workspace<SpareMemory> spare;           // what only makes them faster: see Scratch
     unsigned char *noalloc = nullptr;       // this device's address of `scratch`
     DirectPlan direct;                      // plans of the direct schedule (g_direct_words)
 };
 
 std::mutex g_mu;
+std::recursive_mutex g_scratch_mu;  // the devices' scratch and spare; taken before g_mu
 // one heap-allocated entry per device, so pointers handed out stay valid when the table grows
 std::vector<std::unique_ptr<DeviceState>> g_dev;
 
@@ -184,30 +201,62 @@ int device_state(DeviceState **out) {
     return FK20_OK;
 }
 
-// Grows the library-owned scratch of the current device to at least `bytes`.  The old
-// buffer is released after the device is idle, since queued work may still use it.
-int device_scratch(DeviceState *st, size_t bytes, void **out) {
-    std::lock_guard<std::mutex> lk(g_mu);
-    if (st->scratch_bytes < bytes) {
-        if (st->scratch) {
-            FK20_TRY(hipDeviceSynchronize());
-            FK20_TRY(hipFree(st->scratch));
-            st->scratch = nullptr;
-            st->scratch_bytes = 0;
-        }
-        FK20_TRY(hipMalloc(&st->scratch, bytes));
-        st->scratch_bytes = bytes;
-    }
-    *out = st->scratch;
-    return FK20_OK;
+uint32_t *W(const void *p) { return reinterpret_cast<uint32_t *>(const_cast<void *>(p)); }
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (!s) return false;
+    if (hipStreamIsCapturing(s, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
 }
 
-uint32_t *W(const void *p) { return reinterpret_cast<uint32_t *>(const_cast<void *>(p)); }
+// The current device's workspace for one call of a drop-in entry point, which holds it until its
+// launches are enqueued.  base: what the call cannot do without, linear in its rows, so that no call
+// after a larger one allocates.  spare: room for the multiples of an MSM's bases (up to 604 MB) and
+// a small batch's products, as much as there is; the launchers choose the fastest form that fits, the
+// smallest ones in base.  It does not grow with the rows alone and may move in any call, so calls
+// under capture do without; it is also what is given back when other memory runs short.
+struct Scratch {
+    std::lock_guard<std::recursive_mutex> lk{g_scratch_mu};
+    char *base = nullptr, *spare = nullptr;
+    size_t spare_bytes = 0;
+    int get(DeviceState *st, size_t base_bytes, size_t want_spare, fk20_stream_t stream) {
+        if (st->scratch.fit(base_bytes, base_bytes) == Workspace<DeviceMemory>::FAILED) return hip_status(DeviceMemory::error);
+        base = static_cast<char *>(st->scratch.ptr());
+        if (want_spare && !capturing(S(stream))) {
+            st->spare.try_grow(want_spare);
+            spare = static_cast<char *>(st->spare.ptr());
+            spare_bytes = st->spare.bytes();
+        }
+        return FK20_OK;
+    }
+};
 
 }  // namespace
 
 namespace fk20 {
 int status_from_hip(hipError_t e) { return hip_status(e); }
+
+thread_local hipError_t DeviceMemory::error = hipSuccess;
+
+hipError_t device_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return e;
+    std::lock_guard<std::recursive_mutex> use(g_scratch_mu);
+    DeviceState *st = nullptr;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        if (dev < (int)g_dev.size()) st = g_dev[dev].get();
+    }
+    if (!st || !st->spare.give_back()) return e;
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
 
 const DevTables *current_device_tables(hipError_t *err) {
     DeviceState *st;
@@ -281,9 +330,7 @@ int fr_ift(fk20_fr_t *output, const fk20_fr_t *input, unsigned count, unsigned n
     return fr_transform(output, input, count, n, true, stream);
 }
 
-// Scratch of the drop-in transforms besides the points: one flag per row, padded, and the direct
-// schedule's products when the batch is small enough for it.
-static size_t flag_bytes(unsigned rows) { return ((size_t)rows * 4 + 255) & ~(size_t)255; }
+// The products of the direct schedule when the batch is small enough for it.
 static size_t transform_product_bytes(const DeviceState *st, unsigned rows, unsigned logn, bool both = false) {
     Launch L;
     L.nitems = 1;
@@ -302,15 +349,13 @@ static int g1_transform(fk20_g1p_t *out, const fk20_g1p_t *in, unsigned count, u
     DeviceState *st;
     int rc = device_state(&st);
     if (rc) return rc;
-    void *D;
-    const size_t d_bytes = (size_t)count * n * 144, f_bytes = flag_bytes(count);
-    const size_t p_bytes = transform_product_bytes(st, count, log2u(n));
-    rc = device_scratch(st, d_bytes + f_bytes + p_bytes, &D);
+    Scratch w;
+    const size_t d_bytes = (size_t)count * n * 144;
+    rc = w.get(st, d_bytes + (size_t)count * 4, transform_product_bytes(st, count, log2u(n)), stream);
     if (rc) return rc;
-    char *base = reinterpret_cast<char *>(D);
     return hip_status(launch_plain(inv ? PLAIN_G1_IFT : PLAIN_G1_FFT, W(out), W(in), nullptr, count, log2u(n),
-                                   W(base), nullptr, nullptr, 0, W(base + d_bytes), st->tables, st->prog, S(stream),
-                                   st->direct, W(base + d_bytes + f_bytes), p_bytes));
+                                   W(w.base), nullptr, nullptr, 0, W(w.base + d_bytes), st->tables, st->prog, S(stream),
+                                   st->direct, W(w.spare), w.spare_bytes));
 }
 
 int g1p_fft(fk20_g1p_t *output, const fk20_g1p_t *input, unsigned count, unsigned n, fk20_stream_t stream) {
@@ -330,16 +375,15 @@ int fk20_msm(fk20_g1p_t *hext_fft, const fk20_fr_t *tc_fft, const fk20_g1p_t *xe
     DeviceState *st;
     int rc = device_state(&st);
     if (rc) return rc;
-    const size_t x_bytes = (size_t)16 * n2 * 144;
-    void *scratch;
-    const size_t m_bytes = msm_plain_bytes(rows, n2);
-    rc = device_scratch(st, x_bytes + m_bytes, &scratch);
+    const size_t x_bytes = (size_t)16 * n2 * 144, m_bytes = msm_plain_min_bytes(rows, n2);
+    Scratch w;
+    rc = w.get(st, x_bytes + m_bytes, msm_plain_bytes(rows, n2), stream);
     if (rc) return rc;
-    uint32_t *xpk = reinterpret_cast<uint32_t *>(scratch);
-    void *work = reinterpret_cast<char *>(scratch) + x_bytes;
     hipStream_t s = S(stream);
-    FK20_TRY(launch_std_to_packed(xpk, W(xext_fft), (size_t)16 * n2, s));
-    return hip_status(launch_msm_plain(W(hext_fft), W(tc_fft), xpk, work, m_bytes, rows, n2, s));
+    FK20_TRY(launch_std_to_packed(W(w.base), W(xext_fft), (size_t)16 * n2, s));
+    const bool spare = w.spare_bytes > m_bytes;
+    return hip_status(launch_msm_plain(W(hext_fft), W(tc_fft), W(w.base), spare ? w.spare : w.base + x_bytes,
+                                       spare ? w.spare_bytes : m_bytes, rows, n2, s));
 }
 
 int fk20_hext2h(fk20_g1p_t *h, unsigned rows, unsigned n2, fk20_stream_t stream) {
@@ -354,15 +398,13 @@ int fk20_hext_fft2h_fft(fk20_g1p_t *h_fft, const fk20_g1p_t *hext_fft, unsigned 
     DeviceState *st;
     int rc = device_state(&st);
     if (rc) return rc;
-    void *D;
-    const size_t d_bytes = (size_t)rows * n2 * 144, f_bytes = flag_bytes(rows);
-    const size_t p_bytes = transform_product_bytes(st, rows, log2u(n2), true);
-    rc = device_scratch(st, d_bytes + f_bytes + p_bytes, &D);
+    Scratch w;
+    const size_t d_bytes = (size_t)rows * n2 * 144;
+    rc = w.get(st, d_bytes + (size_t)rows * 4, transform_product_bytes(st, rows, log2u(n2), true), stream);
     if (rc) return rc;
-    char *base = reinterpret_cast<char *>(D);
-    return hip_status(launch_plain(PLAIN_HEXT_FFT2H_FFT, W(h_fft), W(hext_fft), nullptr, rows, log2u(n2), W(base),
-                                   nullptr, nullptr, 0, W(base + d_bytes), st->tables, st->prog, S(stream), st->direct,
-                                   W(base + d_bytes + f_bytes), p_bytes));
+    return hip_status(launch_plain(PLAIN_HEXT_FFT2H_FFT, W(h_fft), W(hext_fft), nullptr, rows, log2u(n2), W(w.base),
+                                   nullptr, nullptr, 0, W(w.base + d_bytes), st->tables, st->prog, S(stream), st->direct,
+                                   W(w.spare), w.spare_bytes));
 }
 
 // fk20_poly2h_fft.cu:47-80: toeplitz -> NTT (16 per row) -> MSM -> IFFT -> zero -> FFT, with
@@ -370,28 +412,32 @@ int fk20_hext_fft2h_fft(fk20_g1p_t *h_fft, const fk20_g1p_t *hext_fft, unsigned 
 // scalar multiplication per point) and the transforms column-batched over the rows.
 // Workspace: D, the packed bases, the subgroup flag of the bases (one 256-byte slot), tcT and the
 // MSM's workspace, in that order; tcT and that workspace are dead after the MSM, and a small
-// batch's transforms keep their products there and past their end.
-static size_t poly2h_scratch_bytes(unsigned rows, unsigned n2, size_t msm_bytes) {
-    return (size_t)rows * 16 * n2 * 32 + (size_t)rows * n2 * 144 + (size_t)16 * n2 * 144 + 256 + msm_bytes;
+// batch's transforms keep their products there and past their end, or in the spare workspace.
+static size_t poly2h_scratch_bytes(unsigned rows, unsigned n2) {
+    return (size_t)rows * 16 * n2 * 32 + (size_t)rows * n2 * 144 + (size_t)16 * n2 * 144 + 256 +
+           msm_plain_min_bytes(rows, n2);
 }
 
-// bytes: all of scratch, at least poly2h_scratch_bytes with the smallest MSM workspace
-static int poly2h_fft_in(void *scratch, size_t bytes, DeviceState *st, fk20_g1p_t *h_fft, const fk20_fr_t *poly,
-                         const fk20_g1p_t *xext_fft, unsigned rows, unsigned n2, fk20_stream_t stream) {
+// bytes: all of scratch, at least poly2h_scratch_bytes
+static int poly2h_fft_in(void *scratch, size_t bytes, char *spare, size_t spare_bytes, DeviceState *st, fk20_g1p_t *h_fft,
+                         const fk20_fr_t *poly, const fk20_g1p_t *xext_fft, unsigned rows, unsigned n2,
+                         fk20_stream_t stream) {
     const size_t tc_bytes = (size_t)rows * 16 * n2 * 32;
     const size_t d_bytes = (size_t)rows * n2 * 144;
     const size_t x_bytes = (size_t)16 * n2 * 144;
     char *base = reinterpret_cast<char *>(scratch);
     uint32_t *D = W(base), *xpk = W(base + d_bytes), *flag = W(base + d_bytes + x_bytes);
     uint32_t *tcT = W(base + d_bytes + x_bytes + 256);
-    void *work = base + d_bytes + x_bytes + 256 + tc_bytes;
+    char *work = base + d_bytes + x_bytes + 256 + tc_bytes;
     const size_t rest = bytes - (d_bytes + x_bytes + 256 + tc_bytes);
+    const bool m = spare_bytes > rest, p = spare_bytes > tc_bytes + rest;  // where the spare workspace is the larger
     hipStream_t s = S(stream);
     // one flag for all rows: a base outside G1 can put every row's MSM output outside it
     FK20_TRY(launch_subgroup_groups(flag, W(xext_fft), (size_t)16 * n2, (size_t)16 * n2, s));
     FK20_TRY(launch_std_to_packed(xpk, W(xext_fft), (size_t)16 * n2, s));
-    return hip_status(launch_plain(PLAIN_POLY2H_FFT, W(h_fft), W(poly), xpk, rows, log2u(n2), D, tcT, work, rest,
-                                   flag, st->tables, st->prog, s, st->direct, tcT, tc_bytes + rest));
+    return hip_status(launch_plain(PLAIN_POLY2H_FFT, W(h_fft), W(poly), xpk, rows, log2u(n2), D, tcT, m ? spare : work,
+                                   m ? spare_bytes : rest, flag, st->tables, st->prog, s, st->direct,
+                                   p ? W(spare) : tcT, p ? spare_bytes : tc_bytes + rest));
 }
 
 int fk20_poly2h_fft(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20_g1p_t *xext_fft, unsigned rows,
@@ -402,14 +448,13 @@ int fk20_poly2h_fft(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20_g1p_t *
     DeviceState *st;
     int rc = device_state(&st);
     if (rc) return rc;
-    void *scr;
-    // the workspace past D, bases and flag holds first tcT and the MSM's, then the products
-    const size_t tc_bytes = (size_t)rows * 16 * n2 * 32, dead = tc_bytes + msm_plain_bytes(rows, n2);
-    const size_t products = transform_product_bytes(st, rows, log2u(n2), true);
-    const size_t bytes = poly2h_scratch_bytes(rows, n2, std::max(dead, products) - tc_bytes);
-    rc = device_scratch(st, bytes, &scr);
+    const size_t bytes = poly2h_scratch_bytes(rows, n2), msm_min = msm_plain_min_bytes(rows, n2);
+    const size_t msm = msm_plain_bytes(rows, n2), products = transform_product_bytes(st, rows, log2u(n2), true);
+    const size_t dead = (size_t)rows * 16 * n2 * 32 + msm_min;  // of base, when the products are made
+    Scratch w;
+    rc = w.get(st, bytes, std::max(msm > msm_min ? msm : 0, products > dead ? products : 0), stream);
     if (rc) return rc;
-    return poly2h_fft_in(scr, bytes, st, h_fft, poly, xext_fft, rows, n2, stream);
+    return poly2h_fft_in(w.base, bytes, w.spare, w.spare_bytes, st, h_fft, poly, xext_fft, rows, n2, stream);
 }
 
 // The same launch sequence with its workspace in this device's fixed `scratch` array: no
@@ -421,11 +466,11 @@ int fk20_poly2h_fft_noalloc(fk20_g1p_t *h_fft, const fk20_fr_t *poly, const fk20
     if (!valid_N(N) || (rows && (!h_fft || !poly || !xext_fft))) return FK20_EINVAL;
     if (!rows) return FK20_OK;
     const unsigned n2 = N / 8;
-    if (poly2h_scratch_bytes(rows, n2, msm_plain_min_bytes(rows, n2)) > NOALLOC_SCRATCH_BYTES) return FK20_ERANGE;
+    if (poly2h_scratch_bytes(rows, n2) > NOALLOC_SCRATCH_BYTES) return FK20_ERANGE;
     DeviceState *st;
     int rc = device_state(&st);
     if (rc) return rc;
-    return poly2h_fft_in(st->noalloc, NOALLOC_SCRATCH_BYTES, st, h_fft, poly, xext_fft, rows, n2, stream);
+    return poly2h_fft_in(st->noalloc, NOALLOC_SCRATCH_BYTES, nullptr, 0, st, h_fft, poly, xext_fft, rows, n2, stream);
 }
 
 int fk20_setup2xext_fft(fk20_g1p_t *xext_fft, const fk20_g1p_t *setup, unsigned N, fk20_stream_t stream) {
@@ -433,17 +478,15 @@ int fk20_setup2xext_fft(fk20_g1p_t *xext_fft, const fk20_g1p_t *setup, unsigned 
     DeviceState *st;
     int rc = device_state(&st);
     if (rc) return rc;
-    void *D;
-    const size_t d_bytes = (size_t)16 * (N / 8) * 144, f_bytes = flag_bytes(16);
-    const size_t p_bytes = transform_product_bytes(st, 16, log2u(N / 8));
-    rc = device_scratch(st, d_bytes + f_bytes + p_bytes, &D);
+    Scratch w;
+    const size_t d_bytes = (size_t)16 * (N / 8) * 144;
+    rc = w.get(st, d_bytes + 16 * 4, transform_product_bytes(st, 16, log2u(N / 8)), stream);
     if (rc) return rc;
-    char *base = reinterpret_cast<char *>(D);
     hipStream_t s = S(stream);
     FK20_TRY(launch_setup_gather(W(xext_fft), W(setup), N, s));
-    return hip_status(launch_plain(PLAIN_G1_FFT, W(xext_fft), W(xext_fft), nullptr, 16, log2u(N / 8), W(base), nullptr,
-                                   nullptr, 0, W(base + d_bytes), st->tables, st->prog, s, st->direct,
-                                   W(base + d_bytes + f_bytes), p_bytes));
+    return hip_status(launch_plain(PLAIN_G1_FFT, W(xext_fft), W(xext_fft), nullptr, 16, log2u(N / 8), W(w.base), nullptr,
+                                   nullptr, 0, W(w.base + d_bytes), st->tables, st->prog, s, st->direct, W(w.spare),
+                                   w.spare_bytes));
 }
 
 // ---------------------------------------------------------------- helpers
@@ -497,7 +540,7 @@ int fk20_set_device(int device) { return hip_status(hipSetDevice(device)); }
 
 int fk20_malloc(void **ptr, size_t bytes) {
     if (!ptr) return FK20_EINVAL;
-    return hip_status(hipMalloc(ptr, bytes));
+    return hip_status(device_malloc(ptr, bytes));
 }
 
 int fk20_free(void *ptr) { return hip_status(hipFree(ptr)); }

@@ -42,6 +42,18 @@ void build_host_tables(DevTables &T);
 // FK20_* status of a HIP error, recorded as the thread's last HIP error (api.cpp).
 int status_from_hip(hipError_t e);
 
+// hipMalloc; where memory is short, with what the drop-in entry points hold beyond their need (the
+// spare workspace of api.cpp) given back first.
+hipError_t device_malloc(void **p, size_t bytes);
+
+// Memory of the workspaces that calls cannot do without (Workspace, scratch.h).
+struct DeviceMemory {
+    static thread_local hipError_t error;  // of the last call that failed
+    static bool alloc(void **p, size_t bytes) { return (error = device_malloc(p, bytes)) == hipSuccess; }
+    static void release(void *p) { (void)hipFree(p); }
+    static bool idle() { return (error = hipDeviceSynchronize()) == hipSuccess; }
+};
+
 // Constant tables of the current device, built on first use (api.cpp).  Returns nullptr
 // and sets *err on failure.
 const DevTables *current_device_tables(hipError_t *err);
