@@ -9,6 +9,7 @@
 
 #include "../../include/fk20.h"
 #include "fast.hip.h"
+#include "scratch.h"
 
 using namespace fk20;
 
@@ -303,8 +304,8 @@ hipError_t fk20::build_programs(Programs &P, unsigned wnaf) {
     if (wnaf < 3 || wnaf > 5 || !all_programs_host(ops, index, P.scale_off, (int)wnaf)) return hipErrorInvalidValue;
     P.owned = true;
     P.wnaf = wnaf;
-    hipError_t err = hipMalloc(&P.ops, ops.size() * 4);
-    if (err == hipSuccess) err = hipMalloc(&P.index, index.size() * 4);
+    hipError_t err = device_malloc(reinterpret_cast<void **>(&P.ops), ops.size() * 4);
+    if (err == hipSuccess) err = device_malloc(reinterpret_cast<void **>(&P.index), index.size() * 4);
     if (err == hipSuccess) err = hipMemcpy(P.ops, ops.data(), ops.size() * 4, hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemcpy(P.index, index.data(), index.size() * 4, hipMemcpyHostToDevice);
     if (err != hipSuccess) free_programs(P);
@@ -352,8 +353,7 @@ struct fk20_ctx {
     DirectPlan direct;
     Programs prog;
     std::vector<Setup> setups;
-    void *work = nullptr;
-    size_t work_bytes = 0;
+    Workspace<DeviceMemory> work;
     bool use_graph = false;
     bool use_chain = false;  // transform stages as one persistent launch (k_chain)
     uint64_t chain_wait = CHAIN_WAIT_TICKS;
@@ -435,7 +435,7 @@ int fk20_ctx_destroy(fk20_ctx_t *c) {
         if (s.table) (void)hipFree(s.table);
         if (s.inf) (void)hipFree(s.inf);
     }
-    if (c->work) (void)hipFree(c->work);
+    c->work.drop();
     free_programs(c->prog);
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
     for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
@@ -551,8 +551,6 @@ int fk20_ctx_set_graph(fk20_ctx_t *c, int enable) {
     return FK20_OK;
 }
 
-static hipError_t grow_work(fk20_ctx *c, size_t bytes);
-
 // Window tables of nbases points (standard-form g1p_t, device), each first multiplied by the
 // standard-form scalar `scale` (device, 8 words).  Fills st.table / st.inf.  *outside: some
 // base lies outside the order-r subgroup G1; *small_order: a base of small order outside G1
@@ -568,11 +566,12 @@ static hipError_t build_tables(Setup &st, const fk20_g1p_t *points, unsigned nba
     const size_t zt_per_base = table_build_scratch_bytes(1, st.win, st.nwin);
     unsigned chunk = (unsigned)std::max<size_t>(1, ((size_t)4 << 30) / zt_per_base);
     if (chunk > nbases) chunk = nbases;
-    hipError_t e = hipMalloc(&st.table, (size_t)nbases * per_base);
+    hipError_t e = device_malloc(reinterpret_cast<void **>(&st.table), (size_t)nbases * per_base);
     // inf[0 .. nbases), then two words: outside G1, table-build error
-    if (e == hipSuccess) e = hipMalloc(&st.inf, (size_t)nbases * 4 + 8);
-    if (e == hipSuccess) e = hipMalloc(&xs, (size_t)nbases * 144);
-    if (e == hipSuccess) e = hipMalloc(&zt, table_build_scratch_bytes(chunk, st.win, st.nwin));
+    if (e == hipSuccess) e = device_malloc(reinterpret_cast<void **>(&st.inf), (size_t)nbases * 4 + 8);
+    if (e == hipSuccess) e = device_malloc(reinterpret_cast<void **>(&xs), (size_t)nbases * 144);
+    if (e == hipSuccess)
+        e = device_malloc(reinterpret_cast<void **>(&zt), table_build_scratch_bytes(chunk, st.win, st.nwin));
     uint32_t *words = st.inf ? st.inf + nbases : nullptr;
     if (e == hipSuccess) e = hipMemsetAsync(words, 0, 8, s);
     if (e == hipSuccess)
@@ -648,6 +647,16 @@ int fk20_commit_setup_load(fk20_ctx_t *c, const fk20_g1p_t *srs, unsigned N, uns
     return FK20_OK;
 }
 
+// The context's workspace for a call that cannot do without `need` bytes.
+static hipError_t fit_work(fk20_ctx *c, size_t need, size_t want) {
+    const Workspace<DeviceMemory>::Fit r = c->work.fit(need, want);
+    if (r != Workspace<DeviceMemory>::KEPT && c->gexec) {  // captured with the old address
+        (void)hipGraphExecDestroy(c->gexec);
+        c->gexec = nullptr;
+    }
+    return r == Workspace<DeviceMemory>::FAILED ? DeviceMemory::error : hipSuccess;
+}
+
 // Orders a call that uses the context workspace on stream s after the previous one.
 static hipError_t order_before(fk20_ctx *c, hipStream_t s) {
     if (!c->done_valid || c->done_stream == s) return hipSuccess;
@@ -684,11 +693,12 @@ int fk20_commit_rows(fk20_ctx_t *c, int setup_id, fk20_g1p_t *commitments, const
     if (!commitments || !polynomial) return FK20_EINVAL;
     const Setup &st = c->setups[setup_id];
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    hipError_t e = grow_work(c, commit_workspace_bytes(rows, st.N));
+    const size_t bytes = commit_workspace_bytes(rows, st.N);
+    hipError_t e = fit_work(c, bytes, bytes);
     if (e == hipSuccess) e = order_before(c, s);
     if (e == hipSuccess)
         e = launch_commit(reinterpret_cast<uint32_t *>(commitments), reinterpret_cast<const uint32_t *>(polynomial),
-                          st.table, st.inf, reinterpret_cast<uint32_t *>(c->work), rows, st.N, st.win, s);
+                          st.table, st.inf, reinterpret_cast<uint32_t *>(c->work.ptr()), rows, st.N, st.win, s);
     if (e == hipSuccess) e = order_after(c, s);
     return status_of(e);
 }
@@ -741,34 +751,28 @@ static Launch items_launch(const fk20_ctx *c, const fk20_batch_item_t *items, un
     return L;
 }
 
-static hipError_t grow_work(fk20_ctx *c, size_t bytes) {
-    if (c->work_bytes >= bytes) return hipSuccess;
-    if (c->work) {
-        hipError_t e = hipDeviceSynchronize();
-        if (e != hipSuccess) return e;
-        (void)hipFree(c->work);
-        c->work = nullptr;
-        c->work_bytes = 0;
-        if (c->gexec) {
-            (void)hipGraphExecDestroy(c->gexec);
-            c->gexec = nullptr;
-        }
-    }
-    hipError_t e = hipMalloc(&c->work, bytes);
-    if (e == hipSuccess) c->work_bytes = bytes;
-    return e;
+// Device bytes with which `rows` rows of 2^logn points, and every smaller number of them, take the
+// direct schedule in the levels they are fastest in; for a single row of any size at least.
+static size_t wanted_bytes(const fk20_ctx *c, unsigned rows, unsigned logn) {
+    size_t want = fk20_rows_workspace_bytes(rows, 8u << logn);
+    auto with_products = [&](unsigned r, unsigned lg) {
+        Launch L;
+        L.nitems = 1;
+        L.item[0].rows = r;
+        L.item[0].logn2 = lg;
+        size_t more = 0;
+        (void)direct_levels(c, L, ~(size_t)0, &more);
+        return fk20_rows_workspace_bytes(r, 8u << lg) + more;
+    };
+    for (unsigned r = 1; r <= std::min(rows, DIRECT_MAX_ROWS); r++) want = std::max(want, with_products(r, logn));
+    return rows ? std::max(want, with_products(1, 9)) : want;
 }
 
 int fk20_ctx_reserve(fk20_ctx_t *c, unsigned rows, unsigned N) {
     if (!c || !valid_N(N)) return FK20_EINVAL;
     std::lock_guard<std::mutex> lk(c->mu);
-    Launch L;
-    L.nitems = rows ? 1 : 0;
-    L.item[0].rows = rows;
-    L.item[0].logn2 = N == 1024 ? 7 : N == 2048 ? 8 : 9;
-    size_t more = 0;
-    if (rows) (void)direct_levels(c, L, ~(size_t)0, &more);
-    return status_of(grow_work(c, fk20_rows_workspace_bytes(rows, N) + more));
+    return status_of(fit_work(c, fk20_rows_workspace_bytes(rows, N),
+                              wanted_bytes(c, rows, N == 1024 ? 7 : N == 2048 ? 8 : 9)));
 }
 
 static size_t items_workspace_bytes(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n) {
@@ -848,21 +852,21 @@ static hipError_t enqueue_items(fk20_ctx *c, const fk20_batch_item_t *items, uns
     // the persistent form only on the context's own workspace (fk20_prove_batch reads its
     // error words back; the serving loop's fk20_prove_batch_ws does not wait for its batches)
     const bool chain = c->use_chain && !workspace;
-    char *w = reinterpret_cast<char *>(workspace ? workspace : c->work);
+    char *w = reinterpret_cast<char *>(workspace ? workspace : c->work.ptr());
     unsigned groups = 0;
     for (unsigned k = 0; k < n; k++) groups += (items[k].rows + 63) / 64;
-    // the context path with at least two 64-row groups, launches not timed one by one
     // small batches run unsplit in the direct schedule, with what the context's workspace has
     // beyond the items' own for its products
     unsigned levels = 0;
     const size_t base = items_workspace_bytes(c, items, n);
     if (!chain && c->sch_r22) {
         size_t bytes;
-        levels = direct_levels(c, items_launch(c, items, n), workspace ? 0 : c->work_bytes - base, &bytes);
+        levels = direct_levels(c, items_launch(c, items, n), workspace ? 0 : c->work.bytes() - base, &bytes);
     }
+    // halves: on the context path, with at least two 64-row groups, launches not timed one by one
     if (workspace || c->nsub < 2 || groups < 2 || hook.fn || levels || !worth_splitting(c, items, n, groups))
         return enqueue_launch(c, items, n, s, hook, w, chain, levels, w + base);
-    // halves: each item's rows split at a 64-row boundary (items of one group go to the first)
+    // each item's rows split at a 64-row boundary (items of one group go to the first)
     fk20_batch_item_t half[2][MAX_ITEMS];
     unsigned nh[2] = {0, 0};
     for (unsigned k = 0; k < n; k++) {
@@ -922,13 +926,16 @@ int fk20_prove_batch(fk20_ctx_t *c, const fk20_batch_item_t *items, unsigned nit
     const unsigned n = (unsigned)v.size();
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     // what is reserved is not grown for the direct schedule's products (three levels do without);
-    // a workspace that has to grow anyway takes them along
+    // a workspace that has to grow anyway takes them along, if they are to be had
     hipError_t e = hipSuccess;
     const size_t base = items_workspace_bytes(c, v.data(), n);
-    if (c->work_bytes < base) {
-        size_t more = 0;
-        (void)direct_levels(c, items_launch(c, v.data(), n), ~(size_t)0, &more);
-        e = grow_work(c, base + more);
+    if (!c->work.holds(base)) {
+        size_t want = 0;
+        (void)direct_levels(c, items_launch(c, v.data(), n), ~(size_t)0, &want);
+        want += base;
+        for (const fk20_batch_item_t &it : v)
+            want = std::max(want, wanted_bytes(c, it.rows, c->setups[it.setup_id].logn2()));
+        e = fit_work(c, base, want);
     }
     if (e == hipSuccess) e = order_before(c, s);
     if (e != hipSuccess) return status_of(e);

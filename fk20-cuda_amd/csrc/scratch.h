@@ -14,6 +14,8 @@ class Workspace {
     enum Fit { KEPT, MOVED, FAILED };
     void *ptr() const { return p_; }
     size_t bytes() const { return bytes_; }
+    // whether fit(need, ..) has nothing to do
+    bool holds(size_t need) const { return need <= need_; }
 
     // At least `need` bytes.  The buffer only moves (its old address dies) for a call that needs
     // more than every one before it, and then takes `want` bytes if they are there: a captured

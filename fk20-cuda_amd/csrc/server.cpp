@@ -291,7 +291,7 @@ int fk20_server_create(fk20_server_t **out, fk20_ctx_t *ctx, size_t budget_bytes
     srv->budget = budget_bytes;
     srv->max_batch_rows = max_batch_rows;
     hipError_t e = hipGetDevice(&srv->device);
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&srv->arena_dev), budget_bytes);
+    if (e == hipSuccess) e = fk20::device_malloc(reinterpret_cast<void **>(&srv->arena_dev), budget_bytes);
     srv->arena.reset(budget_bytes);
     srv->slots.resize(nslots);
     for (Slot &s : srv->slots) {
