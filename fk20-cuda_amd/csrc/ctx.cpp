@@ -693,12 +693,13 @@ int fk20_commit_rows(fk20_ctx_t *c, int setup_id, fk20_g1p_t *commitments, const
     if (!commitments || !polynomial) return FK20_EINVAL;
     const Setup &st = c->setups[setup_id];
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const size_t bytes = commit_workspace_bytes(rows, st.N);
-    hipError_t e = fit_work(c, bytes, bytes);
+    const size_t need = commit_workspace_bytes(rows, st.N);
+    hipError_t e = hipSuccess;
+    if (!c->work.holds(need)) e = fit_work(c, need, commit_wanted_bytes(rows, st.N));
     if (e == hipSuccess) e = order_before(c, s);
     if (e == hipSuccess)
         e = launch_commit(reinterpret_cast<uint32_t *>(commitments), reinterpret_cast<const uint32_t *>(polynomial),
-                          st.table, st.inf, reinterpret_cast<uint32_t *>(c->work.ptr()), rows, st.N, st.win, s);
+                          st.table, st.inf, reinterpret_cast<uint32_t *>(c->work.ptr()), c->work.bytes(), rows, st.N, st.win, s);
     if (e == hipSuccess) e = order_after(c, s);
     return status_of(e);
 }

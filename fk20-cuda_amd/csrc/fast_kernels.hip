@@ -624,16 +624,17 @@ hipError_t launch_table_build(uint32_t *table, uint32_t *zt, const uint32_t *xs,
 
 // Lanes per row and coefficients per lane of k_commit_partial: no idle lanes below 64 rows, then
 // the chunk with the fewest additions one after the other (20 windows per coefficient; larger
-// chunks where it does not matter, for fewer partial sums).
+// chunks where it does not matter, for fewer partial sums) of those whose partial sums fit in `bytes`.
 struct CommitShape {
     unsigned lp, chunk, nparts;
 };
-static CommitShape commit_shape(unsigned rows, unsigned N) {
+static CommitShape commit_shape(unsigned rows, unsigned N, size_t bytes) {
     CommitShape best{1, 16, N / 16};
     unsigned lp = 1, time = ~0u;
     while (lp < 64 && rows * lp * 2 <= 64) lp *= 2;
     for (unsigned chunk = 16; chunk * lp >= 4 && chunk >= 1; chunk /= 2) {
         const unsigned nparts = N / (chunk * lp), per_wave = 64 / lp;
+        if ((size_t)nparts * rows * 144 > bytes) break;
         const size_t waves = (size_t)((rows + per_wave - 1) / per_wave) * nparts;
         unsigned close = (nparts + 63) / 64 + 6;
         for (unsigned l = lp; l > 1; l /= 2) close++;
@@ -643,15 +644,25 @@ static CommitShape commit_shape(unsigned rows, unsigned N) {
     return best;
 }
 
-// never below a partial sum per 16 coefficients and per 256, the published size
-size_t commit_workspace_bytes(unsigned rows, unsigned N) {
-    return (size_t)std::max(commit_shape(rows, N).nparts, N / 16 + (N + 255) / 256) * rows * 144;
+// a partial sum per 16 coefficients and per 256
+size_t commit_workspace_bytes(unsigned rows, unsigned N) { return (size_t)(N / 16 + (N + 255) / 256) * rows * 144; }
+
+// What `rows` rows, and every smaller number of them, are fastest in: rows that share lanes or a
+// launch's waves want the same number of partial sums, so the last of each such range decides.
+size_t commit_wanted_bytes(unsigned rows, unsigned N) {
+    size_t want = commit_workspace_bytes(rows, N);
+    for (unsigned r = 1;; r = r < 64 ? r + 1 : r + 64) {
+        r = std::min(r, rows);
+        want = std::max(want, (size_t)commit_shape(r, N, ~(size_t)0).nparts * r * 144);
+        if (r >= rows) return want;
+    }
 }
 
 hipError_t launch_commit(uint32_t *out, const uint32_t *poly, const uint32_t *table, const uint32_t *inf,
-                         uint32_t *work, unsigned rows, unsigned N, unsigned win_bits, hipStream_t s) {
+                         uint32_t *work, size_t work_bytes, unsigned rows, unsigned N, unsigned win_bits,
+                         hipStream_t s) {
     if (!rows) return hipSuccess;
-    const CommitShape c = commit_shape(rows, N);
+    const CommitShape c = commit_shape(rows, N, work_bytes);
     const unsigned per_wave = 64 / c.lp, rg = (rows + per_wave - 1) / per_wave;
     hipLaunchKernelGGL(k_commit_partial, dim3(c.nparts * rg), dim3(64), 0, s, poly, table, inf, work, rows, N, win_bits,
                        c.chunk, c.lp);
