@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -214,14 +215,19 @@ bool build_programs_host(std::vector<uint32_t> &ops, std::vector<uint32_t> &inde
     build_host_tables(T);
     ops.clear();
     index.assign(2 * 512, 0);
-    for (int dir = 0; dir < 2; dir++) {
-        for (int idx = 0; idx < 512; idx++) {
-            const int e = dir == TW_FWD ? idx : (512 - idx) % 512;
-            index[dir * 512 + idx] = (uint32_t)ops.size();
-            fs expect;
-            fs_set(expect, T.tw_mont[e]);
-            if (!append_program(ops, T.tw_std[e], W, expect)) return false;
-        }
+    for (int e = 0; e < 512; e++) {
+        index[TW_FWD * 512 + e] = (uint32_t)ops.size();
+        fs expect;
+        fs_set(expect, T.tw_mont[e]);
+        if (!append_program(ops, T.tw_std[e], W, expect)) return false;
+    }
+    // w^-idx = w^(512 - idx): the same programs
+    const std::vector<uint32_t> fwd = ops;
+    for (int idx = 0; idx < 512; idx++) {
+        const int e = (512 - idx) % 512;
+        index[TW_INV * 512 + idx] = (uint32_t)ops.size();
+        const size_t end = e < 511 ? index[TW_FWD * 512 + e + 1] : fwd.size();
+        ops.insert(ops.end(), fwd.begin() + index[TW_FWD * 512 + e], fwd.begin() + end);
     }
     return true;
 }
@@ -246,7 +252,6 @@ int status_of(hipError_t e) { return status_from_hip(e); }
 }  // namespace
 
 namespace {
-// Every program (w^+-i, then 2^-j) on the host, each checked, with its index table.
 // Ladder cost of an encoded program (the units of program_cost): its doublings, its mixed
 // additions after the first entry and its endomorphism products.
 int ops_cost(const uint32_t *ops) {
@@ -283,25 +288,44 @@ bool layer_tables_host(const std::vector<uint32_t> &ops, std::vector<uint32_t> &
     return true;
 }
 
-bool all_programs_host(std::vector<uint32_t> &ops, std::vector<uint32_t> &index, uint32_t *scale_off,
-                       int W = TW_WNAF) {
-    if (!build_programs_host(ops, index, W)) return false;
-    DevTables T;
-    build_host_tables(T);
-    index.resize(TW_INDEX_SIZE);
-    for (int j = 0; j < 10; j++) {
-        index[TW_SCALE + j] = scale_off[j] = (uint32_t)ops.size();
-        fs expect;
-        fs_set(expect, T.inv2k_mont[j]);
-        if (!append_program(ops, T.inv2k_std[j], W, expect)) return false;
+// Every program (w^+-i, then 2^-j) on the host, each checked, with its index table; no ops if one fails.
+struct HostPrograms {
+    std::vector<uint32_t> ops, index;
+    uint32_t scale_off[10];
+    explicit HostPrograms(int W) {
+        if (!build(W)) ops.clear();
     }
-    return layer_tables_host(ops, index);
+    bool build(int W) {
+        if (!build_programs_host(ops, index, W)) return false;
+        DevTables T;
+        build_host_tables(T);
+        index.resize(TW_INDEX_SIZE);
+        for (int j = 0; j < 10; j++) {
+            index[TW_SCALE + j] = scale_off[j] = (uint32_t)ops.size();
+            fs expect;
+            fs_set(expect, T.inv2k_mont[j]);
+            if (!append_program(ops, T.inv2k_std[j], W, expect)) return false;
+        }
+        return layer_tables_host(ops, index);
+    }
+};
+
+// The default width's, 8 ms of host work, built once for the drop-ins, every context and the direct
+// schedule's plans: the first call of a process takes 55 ms and a context 0.1, 87 and 16 with a build
+// for each of them.
+const HostPrograms &default_programs() {
+    static const HostPrograms P(TW_WNAF);
+    return P;
 }
 }  // namespace
 
 hipError_t fk20::build_programs(Programs &P, unsigned wnaf) {
-    std::vector<uint32_t> ops, index;
-    if (wnaf < 3 || wnaf > 5 || !all_programs_host(ops, index, P.scale_off, (int)wnaf)) return hipErrorInvalidValue;
+    if (wnaf < 3 || wnaf > 5) return hipErrorInvalidValue;
+    std::unique_ptr<HostPrograms> own(wnaf == (unsigned)TW_WNAF ? nullptr : new HostPrograms((int)wnaf));
+    const HostPrograms &H = own ? *own : default_programs();
+    const std::vector<uint32_t> &ops = H.ops, &index = H.index;
+    if (ops.empty()) return hipErrorInvalidValue;
+    memcpy(P.scale_off, H.scale_off, sizeof P.scale_off);
     P.owned = true;
     P.wnaf = wnaf;
     hipError_t err = device_malloc(reinterpret_cast<void **>(&P.ops), ops.size() * 4);
@@ -313,8 +337,10 @@ hipError_t fk20::build_programs(Programs &P, unsigned wnaf) {
 }
 
 hipError_t fk20::load_programs(Programs &P, uint32_t *ops_dev, size_t ops_cap, uint32_t *index_dev) {
-    std::vector<uint32_t> ops, index;
-    if (!all_programs_host(ops, index, P.scale_off) || ops.size() > ops_cap) return hipErrorInvalidValue;
+    const HostPrograms &H = default_programs();
+    const std::vector<uint32_t> &ops = H.ops, &index = H.index;
+    if (ops.empty() || ops.size() > ops_cap) return hipErrorInvalidValue;
+    memcpy(P.scale_off, H.scale_off, sizeof P.scale_off);
     hipError_t err = hipMemcpy(ops_dev, ops.data(), ops.size() * 4, hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemcpy(index_dev, index.data(), index.size() * 4, hipMemcpyHostToDevice);
     if (err == hipSuccess) {
@@ -336,11 +362,12 @@ void fk20::free_programs(Programs &P) {
 
 const std::vector<uint32_t> &fk20::direct_plan_words() {
     static const std::vector<uint32_t> words = [] {
-        std::vector<uint32_t> w, ops, index;
-        uint32_t scale_off[10];
+        std::vector<uint32_t> w;
         int cost[256] = {};
-        if (!all_programs_host(ops, index, scale_off)) return w;
-        for (int e = 1; e < 256; e++) cost[e] = e == 128 ? 63 * COST_DBL : ops_cost(ops.data() + index[TW_FWD * 512 + e]);
+        const HostPrograms &P = default_programs();
+        if (P.ops.empty()) return w;
+        for (int e = 1; e < 256; e++)
+            cost[e] = e == 128 ? 63 * COST_DBL : ops_cost(P.ops.data() + P.index[TW_FWD * 512 + e]);
         direct_build(w, cost);
         return w;
     }();

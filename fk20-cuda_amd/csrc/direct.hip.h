@@ -157,10 +157,10 @@ inline unsigned direct_bitrev(unsigned x, unsigned bits) {
     return r;
 }
 
-// Appends one step's tables to `words` and returns its record.  cost[e]: ladder cost of w^e
-// (e < 256; 0 for e = 0), the order in which exponents are handed out.
+// Appends one step's tables to `words` and returns its record.  order: the exponents e < 256 as they
+// are handed out.  slot: DIRECT_NONE for every (position << 8 | exponent), and left so.
 inline DirectStep direct_build_step(std::vector<uint32_t> &words, unsigned logn, unsigned kind, unsigned levels,
-                                    unsigned step, const int *cost) {
+                                    unsigned step, const unsigned *order, std::vector<uint32_t> &slot) {
     const unsigned steps = levels, n = 1u << logn;
     const bool inverse = kind == DIRECT_IFFT_HALF || kind == DIRECT_IFFT;
     unsigned logdone = 0;
@@ -173,14 +173,15 @@ inline DirectStep direct_build_step(std::vector<uint32_t> &words, unsigned logn,
     const bool last = step + 1 == steps;
     r.in_map = step == 0 ? (inverse ? 1u : 0u) | (kind == DIRECT_FFT_HALF ? 2u : 0u) : 0u;
     const unsigned a = 1u << r.loga, b = 1u << r.logb, N = a * b;
-    auto position = [&](unsigned i) { return (r.in_map & 1u) ? direct_bitrev(i, logn) : i; };
+    unsigned position[512];
+    for (unsigned i = 0; i < n; i++) position[i] = (r.in_map & 1u) ? direct_bitrev(i, logn) : i;
 
     struct Out {
         unsigned pos, first, terms;  // terms in `terms`: position << 8 | exponent | sign << 31
     };
     std::vector<Out> outs;
-    std::vector<uint32_t> terms, slot((size_t)n << 8, DIRECT_NONE);  // position << 8 | exponent -> slot
-    std::vector<unsigned> keys;
+    std::vector<uint32_t> terms;
+    std::vector<unsigned> keys, of[256];  // the products, and by exponent
     for (unsigned blk = 0; blk < (1u << r.logblocks); blk++)
         for (unsigned j = 0; j < a; j++) {
             // output index of this block's Y[j][0]: the digits so far, least significant first
@@ -208,25 +209,26 @@ inline DirectStep direct_build_step(std::vector<uint32_t> &words, unsigned logn,
                     hi = a >> v;
                 }
                 for (unsigned t = lo; t < hi; t++) {
-                    unsigned e = (j * (m + b * (t - lo))) % N * (512 / N);
-                    if (inverse) e = (512 - e) % 512;
-                    const unsigned p = position(blk * N + m + b * t);
+                    unsigned e = (j * (m + b * (t - lo)) & (N - 1)) * (512 / N);
+                    if (inverse) e = (512 - e) & 511u;
+                    const unsigned p = position[blk * N + m + b * t];
                     const unsigned key = p << 8 | (e & 255u);
                     terms.push_back(key | (e >> 8) << 31);
                     if (slot[key] == DIRECT_NONE) {
                         slot[key] = 0;
-                        keys.push_back(key);
+                        of[e & 255u].push_back(key);
                     }
                 }
                 o.terms = (unsigned)terms.size() - o.first;
                 outs.push_back(o);
             }
         }
-    // slots: exponents by decreasing cost, all products of one exponent together
-    std::sort(keys.begin(), keys.end(), [&](unsigned x, unsigned y) {
-        const unsigned ex = x & 255u, ey = y & 255u;
-        return cost[ex] != cost[ey] ? cost[ex] > cost[ey] : ex != ey ? ex < ey : x < y;
-    });
+    // slots: all products of one exponent together
+    for (unsigned k = 0; k < 256; k++) {
+        std::vector<unsigned> &v = of[order[k]];
+        std::sort(v.begin(), v.end());
+        keys.insert(keys.end(), v.begin(), v.end());
+    }
     r.nprod = (uint32_t)keys.size();
     r.prod = (uint32_t)words.size();
     for (unsigned i = 0; i < keys.size(); i++) {
@@ -260,17 +262,24 @@ inline DirectStep direct_build_step(std::vector<uint32_t> &words, unsigned logn,
             words[at + DIRECT_SUM_FIRST + t] = slot[k & 0x7fffffffu] | (k & 0x80000000u);
         }
     }
+    for (unsigned k : keys) slot[k] = DIRECT_NONE;
     return r;
 }
 
-// Every plan: the record table (DIRECT_RECORDS records), then the records' tables.
+// Every plan: the record table (DIRECT_RECORDS records), then the records' tables.  cost[e]: ladder
+// cost of w^e (e < 256; 0 for e = 0); the dearest are handed out first.
 inline void direct_build(std::vector<uint32_t> &words, const int *cost) {
+    unsigned order[256];
+    for (unsigned e = 0; e < 256; e++) order[e] = e;
+    std::stable_sort(order, order + 256, [&](unsigned x, unsigned y) { return cost[x] > cost[y]; });
+    std::vector<uint32_t> slot((size_t)512 << 8, DIRECT_NONE);
+    words.reserve((size_t)3 << 19);
     words.assign((size_t)DIRECT_RECORDS * DIRECT_STEP_WORDS, 0);
     for (unsigned logn = 7; logn <= 9; logn++)
         for (unsigned kind = 0; kind < DIRECT_KINDS; kind++)
             for (unsigned levels = 1; levels <= DIRECT_MAX_STEPS; levels++)
                 for (unsigned s = 0; s < levels; s++) {
-                    const DirectStep r = direct_build_step(words, logn, kind, levels, s, cost);
+                    const DirectStep r = direct_build_step(words, logn, kind, levels, s, order, slot);
                     memcpy(&words[(size_t)direct_record(logn, kind, levels, s) * DIRECT_STEP_WORDS], &r, sizeof r);
                 }
 }
