@@ -148,8 +148,9 @@ FK20_HD void fs_from_mont(fs &z, const fs &a) {
 // Montgomery form), so there is no conversion.
 //
 // Digits: a product's are in [0, 2^29) under a signed top digit; sums and differences of up to four
-// such values (|digit| <= 2^31 - 1) may be multiplied as they are.  Values: |v| < 16 r, products in
-// (-1.2 r, 0.2 r).
+// such values (|digit| <= 2^31 - 1) may be multiplied as they are.  Values: r^2 / 2^261 = 0.0142 r, so
+// a product of |v| < 18 r is in (-1.26 r, 0.26 r); the sum of eight inputs, any 256-bit values
+// below 2.21 r each, is below 17.7 r, and eight products later passes add are below 10.1 r.
 struct fn {
     int32_t l[9];
 };
@@ -213,12 +214,12 @@ FK20_HD void fn_unpack(fn &z, const uint32_t *w) {
     }
 }
 
-// words of the canonical value of a product (|digits| as fn_mul gives them, -1.2 r < a < 0.2 r)
+// words of the canonical value of -2 r <= a < r, |digits| as fn_mul gives them (a product is well inside)
 FK20_HD void fn_canon(uint32_t *w, const fn &a) {
     fn t, u;
     int32_t c = 0;
 #pragma unroll
-    for (int i = 0; i < 9; i++) {  // a + r, in (-0.2 r, 1.2 r)
+    for (int i = 0; i < 9; i++) {  // a + r
         const int32_t v = a.l[i] - FN_RT[i] + c;
         t.l[i] = i < 8 ? (int32_t)((uint32_t)v & 0x1fffffffu) : v;
         c = v >> 29;

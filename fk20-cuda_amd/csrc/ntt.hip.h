@@ -166,7 +166,7 @@ __device__ __forceinline__ void ntt_wide(uint32_t *lds, unsigned scale, const De
         put(bitrev(e, LOGN), x);
     }
     __syncthreads();
-    // decimation in time; the left points gain at most 1.2 r a stage
+    // decimation in time; the left points gain at most 1.26 r a stage, to 13.6 r
 #pragma unroll 1
     for (unsigned st = 0; st < LOGN; st++) {
         const unsigned h = 1u << st, j = t & (h - 1), l = ((t >> st) << (st + 1)) + j, r = l + h;
