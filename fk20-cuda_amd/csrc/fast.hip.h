@@ -95,7 +95,7 @@ struct Item {
     uint32_t scale_tc;      // 1: the NTT output is scaled by 1/n2 (setups without folded 1/n2)
     int32_t stage;          // set per launch by launch_batch
     // rowflag[row * flag_stride] != 0: the row holds a point outside the order-r subgroup and
-    // is recomputed by launch_ref_rows, so the output kernel leaves it alone (nullptr: none)
+    // is recomputed by k_ref_rows, so the output kernel leaves it alone (nullptr: none)
     const uint32_t *rowflag;
     uint32_t flag_stride;
     uint32_t *P;            // products of the direct schedule [slot][rows], dead data before
@@ -147,11 +147,12 @@ struct StageKernels {
     // radix-2^2 only: the w^128 twiddles of a DIF stage, after its butterflies (k_quarter_multi)
     void (*quarter)(Launch) = nullptr;
     void (*chain)(Chain, const uint32_t *, const uint32_t *) = nullptr;
+    // radix-2^2 only: a direct step's ladders, and by two lanes each (ladder_pair.hip.h)
     void (*direct)(Launch, const uint32_t *, const uint32_t *, const uint32_t *) = nullptr;
     void (*direct_pair)(Launch, const uint32_t *, const uint32_t *, const uint32_t *) = nullptr;
+    // the default variant only: the drop-ins' load, and the same by two lanes per ladder
     void (*plain_load)(uint32_t *, const uint32_t *, unsigned, unsigned, unsigned, const uint32_t *,
                        uint32_t *) = nullptr;
-    // two lanes per ladder (ladder_pair.hip.h); radix-2^2 variants only, as `direct`
     void (*plain_load_pair)(uint32_t *, const uint32_t *, unsigned, unsigned, unsigned, const uint32_t *,
                             uint32_t *) = nullptr;
     int wnaf = 0;
@@ -216,7 +217,7 @@ enum PlainKind { PLAIN_G1_FFT = 0, PLAIN_G1_IFT = 1, PLAIN_HEXT_FFT2H_FFT = 2, P
 // few); it may overlap tcT and msm_work.
 // flags: `rows` words of workspace (one word for PLAIN_POLY2H_FFT, set by the caller with
 // launch_subgroup_groups over the bases).  Rows holding a point outside G1 are recomputed in
-// the reference's order of operations (launch_ref_rows).
+// the reference's order of operations (k_ref_rows).
 hipError_t launch_plain(PlainKind kind, uint32_t *out, const uint32_t *in, const uint32_t *xpk, unsigned rows,
                         unsigned logn, uint32_t *D, uint32_t *tcT, void *msm_work, size_t msm_bytes, uint32_t *flags,
                         const DevTables *T, const Programs &P, hipStream_t s, const DirectPlan &direct, uint32_t *products,

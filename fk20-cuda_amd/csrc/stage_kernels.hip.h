@@ -273,7 +273,7 @@ __global__ void __launch_bounds__(64, OCC) k_chain(Chain C, const uint32_t *ops,
 // test the inputs, flags[row] |= 1 for a point outside G1: 126 doublings beside the scaling ladders
 // instead of a launch before them (65 inverse transforms of 128, two launches of 0.74 and
 // 0.77 ms: 0.79 together, the call 3.34 -> 2.57).
-template <int W, bool R22, int OCC>
+template <int W, int OCC>
 __global__ void __launch_bounds__(64, OCC) k_plain_load(uint32_t *D, const uint32_t *in, unsigned rows,
                                                        unsigned logn, unsigned brev, const uint32_t *scale_ops,
                                                        uint32_t *flags) {
@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(64, 1) k_plain_load_pair(uint32_t *D, const ui
 }
 
 // The kernel table of variant (W, R22, OCC); the persistent chain (radix 2 whatever the
-// variant's butterflies) is published by the radix-2 variants only.
+// variant's butterflies) is published by the radix-2 variants only, the drop-ins' load by the default.
 template <int W, bool R22, int OCC>
 constexpr StageKernels make_stage_kernels() {
     StageKernels K{};
@@ -326,9 +326,11 @@ constexpr StageKernels make_stage_kernels() {
     if constexpr (R22) {
         K.direct = k_direct_products<W, OCC>;
         K.direct_pair = k_direct_products_pair<W>;
+    }
+    if constexpr (W == TW_WNAF && R22 && OCC == (int)DEFAULT_OCCUPANCY) {
+        K.plain_load = k_plain_load<W, OCC>;
         K.plain_load_pair = k_plain_load_pair<W>;
     }
-    K.plain_load = k_plain_load<W, R22, OCC>;
     K.wnaf = W;
     K.r22 = R22;
     K.occupancy = OCC;
