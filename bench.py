@@ -42,7 +42,6 @@ def log(msg):
 
 
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "fk20_batch_hbm_traffic.json")
-FPMUL_JSON = os.path.join(ROOT, "profiles", "fp_mul_rate.json")
 MAD_JSON = os.path.join(ROOT, "profiles", "mad_rate.json")
 # launch kind (as timed by the library) -> kernel symbol prefix in rocprofv3 output
 KIND_SYMBOL = {"k_dit_stage": "fk20::k_dit_multi<", "k_dif_stage": "fk20::k_dif_multi<",
@@ -101,6 +100,11 @@ def measured_valu(kernel, N, rows, window, avg_launch_s):
             "issue_frac": round(lane_rate / peak, 4),
             "valu_busy": round(k["valu_busy"], 4) if k.get("valu_busy") is not None else None,
             "source": os.path.relpath(VALU_JSON, ROOT)}
+
+
+def known(x, digits=4):
+    """x rounded, or None for a figure the work model does not have (NaN)."""
+    return None if x != x else round(x, digits)
 
 
 def pct(v, q):
@@ -843,12 +847,19 @@ def main():
         stages = WL.r22_layers(args.N)
     else:
         stages = [None]
-    # executed work of this kernel's algorithm per launch (mean over its launches in a step)
+    # executed work of this kernel's algorithm per launch (mean over its launches in a step); the
+    # model knows the MSM, the staged launches (they have a middle one) and the persistent chain,
+    # but not the direct schedule that small batches' transforms run in
+    modelled = bool(sch["chain"]) or "k_middle" in launches
     wl_kw = {"wnaf": sch["wnaf"], "r22": sch["radix"] == 4}
-    exe_fp = (sum(WL.executed_launch_fp_muls(args.N, dom, st, args.window, **wl_kw) for st in stages)
-              / len(stages) * args.rows)
+    exe_fp = canon = float("nan")
+    if modelled or dom == "k_msm_comb":
+        exe_fp = (sum(WL.executed_launch_fp_muls(args.N, dom, st, args.window, **wl_kw) for st in stages)
+                  / len(stages) * args.rows)
+        canon = WL.launch_mul32(args.N, dom, args.rows)
+    exe_step = (WL.executed_row_fp_muls(args.N, args.window, chain=bool(sch["chain"]), **wl_kw) * args.rows
+                if modelled else float("nan"))
     work = exe_fp * WL.FP_MUL32
-    canon = WL.launch_mul32(args.N, dom, args.rows)
     achieved = work / (avg_ms / 1e3) / 1e12
     peak = WL.PEAK_MUL32_PER_S / 1e12
     roofline = {
@@ -856,39 +867,37 @@ def main():
         "kernel": dom,
         "launches_per_step": n_launch,
         "avg_launch_ms": round(avg_ms, 4),
-        "achieved": round(achieved, 4),
+        "achieved": known(achieved),
         "peak": round(peak, 2),
         "unit": "Tmul32/s",
-        "frac": round(achieved / peak, 4),
+        "frac": known(achieved / peak),
         "traffic": None,
         "traffic_detail": None,
         "valu_counters": None,
         "work": "executed Fp muls of the kernel's algorithm x 300 mul32 (12x32-bit CIOS convention)",
         "timing": "per-launch HIP events on the launch stream, one launch sequence of all rows "
                   "(the --streams 1 layout: each launch has the GPU to itself)",
-        "fp_mul_per_s": round(exe_fp / (avg_ms / 1e3), 1),
-        "achieved_canonical": round(canon / (avg_ms / 1e3) / 1e12, 4),
+        "fp_mul_per_s": known(exe_fp / (avg_ms / 1e3), 1),
+        "achieved_canonical": known(canon / (avg_ms / 1e3) / 1e12),
         # the whole step in the benchmarked layout: executed work of every kernel / step time
-        "achieved_step": round(WL.executed_row_fp_muls(args.N, args.window, chain=bool(sch["chain"]), **wl_kw)
-                               * args.rows * WL.FP_MUL32 / (ms / 1e3) / 1e12, 4),
+        "achieved_step": known(exe_step * WL.FP_MUL32 / (ms / 1e3) / 1e12),
     }
 
     roofline["valu_counters"] = measured_valu(dom, args.N, args.rows, args.window, avg_ms / 1e3)
-    try:  # the library's own Fp multiplication rate (bench.py --workload fieldmul)
-        with open(FPMUL_JSON) as f:
-            ceil = json.load(f)["value"]
-        roofline["fp_mul_ceiling"] = {"fp_mul_per_s": ceil, "frac": round(exe_fp / (avg_ms / 1e3) / ceil, 4),
-                                      "source": os.path.relpath(FPMUL_JSON, ROOT)}
-    except (OSError, KeyError, ValueError):
-        roofline["fp_mul_ceiling"] = None
     try:  # the measured v_mad_u64_u32 issue rate (bench.py --workload madrate)
         with open(MAD_JSON) as f:
             mad = json.load(f)["value"]
         roofline["mad_probe"] = {"mad_per_s": mad, "peak_frac": round(mad / WL.PEAK_MUL32_PER_S, 4),
-                                 "achieved_frac": round(achieved * 1e12 / mad, 4),
+                                 "achieved_frac": known(achieved * 1e12 / mad),
                                  "source": os.path.relpath(MAD_JSON, ROOT)}
+        # the G1 kernels' product is 338 multiply-adds (fq.hip.h) and their square 260; executed Fp
+        # muls count a square as one product
+        ceil = mad / WL.FQ_MUL_MADS
+        roofline["fp_mul_ceiling"] = {"fp_mul_per_s": round(ceil, 1),
+                                      "frac": known(exe_fp / (avg_ms / 1e3) / ceil),
+                                      "source": os.path.relpath(MAD_JSON, ROOT)}
     except (OSError, KeyError, ValueError):
-        roofline["mad_probe"] = None
+        roofline["mad_probe"] = roofline["fp_mul_ceiling"] = None
     tr = measured_traffic(dom, args.N, args.rows, args.window)
     if tr:
         roofline["traffic"] = tr["bytes"]

@@ -16,6 +16,8 @@ import math
 
 FP_MUL32 = 2 * 12 * 12 + 12
 FR_MUL32 = 2 * 8 * 8 + 8
+# multiply-adds of the G1 kernels' own product: 13 x 13 digits, as many for the reduction
+FQ_MUL_MADS = 2 * 13 * 13
 DBL, ADD = 8, 12
 SM = 255 * DBL + 128 * ADD
 BF = SM + 2 * ADD
