@@ -867,8 +867,11 @@ static hipError_t enqueue_launch(fk20_ctx *c, const fk20_batch_item_t *items, un
 // Whether two halves on two streams beat one sequence.  The layers hand their ladders to the
 // SIMDs in decreasing cost, which two concurrent launches disturb: batches of one size are faster
 // in one sequence (rows x N: 100 x 4096 17.3 against 22.9 ms, 512 x 4096 43.9 against 46.1,
-// 200 x 2048 15.0 against 19.3, 512 x 1024 14.7 against 19.0), and so are small mixed ones
-// (150 + 75 + 301 rows 39.4 against 39.6); 512 rows of each size take 74.8 in one and 74.2 in two.
+// 200 x 2048 15.0 against 19.3, 512 x 1024 14.7 against 19.0), and so are small mixed ones (two
+// sequences against one, rows of 1024 + 2048 + 4096: 300 + 64 + 64, 7 groups of 64, 1.12;
+// 300 + 128 + 128 1.07, 400 + 200 + 64 1.02, 150 + 75 + 301 1.00, 512 + 256 + 128, 14 groups, 1.01).
+// From about 16 groups two halves are faster or the same (600 + 300 + 5 0.94, 641 + 300 + 40 0.97,
+// 400 + 400 + 200 0.97, 512 + 300 + 300 0.98, 700 + 700 + 100 1.00, 1000 of each 0.99).
 static bool worth_splitting(const fk20_ctx *c, const fk20_batch_item_t *items, unsigned n, unsigned groups) {
     bool mixed = false;
     for (unsigned k = 1; k < n; k++) mixed = mixed || c->setups[items[k].setup_id].N != c->setups[items[0].setup_id].N;

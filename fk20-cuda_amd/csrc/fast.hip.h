@@ -186,7 +186,11 @@ static constexpr unsigned DIRECT_ANY = 0xe;
 unsigned direct_choose(const Launch &L, const DirectPlan &P, bool both, unsigned allowed);
 // Bytes of P an item of `rows` transforms of 2^logn points needs at `levels`.
 size_t direct_product_bytes(const DirectPlan &P, unsigned rows, unsigned logn, unsigned levels);
-// Largest batch the direct schedule is used for, in rows of one size: workspaces are sized by it.
+// Largest batch the direct schedule is used for, in rows of one size: it bounds the products and the
+// sizes that a workspace is chosen over (wanted_bytes, ctx.cpp).  At N = 4096 and 2048 the
+// radix-2^2 launches win below it (4096 from about 130 rows, 2048 from about 200); at N = 1024 the
+// direct schedule would win up to about 350 rows (257: 10.5 against 12.6 ms, 320: 11.0 and 13.0,
+// 352: 12.7 and 13.3, 416: 14.1 and 14.2) and in whole transforms of 128 too (257: 4.5 and 5.4).
 static constexpr unsigned DIRECT_MAX_ROWS = 256;
 
 // The whole batched path for the items of `L`: Toeplitz + NTT, MSM, 2*Lmax - 1 transform

@@ -84,8 +84,11 @@ int fr_ift(fk20_fr_t *output, const fk20_fr_t *input, unsigned count, unsigned n
 
 /* count G1 FFTs of size n.  Replaces g1p_fft_wrapper (g1.cuh:96; g1p_fft.cu:337).  The G1
  * transforms (and fk20_hext_fft2h_fft, fk20_poly2h_fft, fk20_setup2xext_fft) stage their
- * points in library-owned scratch of count * n * 144 bytes (grown on demand, per device,
- * shared by these calls: not reentrant), so output may alias input. */
+ * points in library-owned scratch of count * n * 148 bytes at most (grown on demand, per device,
+ * shared by these calls: not reentrant), so output may alias input.  What only makes a call faster
+ * -- the products of a small count, the multiples of an MSM's bases, up to 604 MB -- goes to a second
+ * buffer as far as there is memory for it.  Calls under stream capture use the first one only; a
+ * graph of them stays valid until a call outgrows that one. */
 int g1p_fft(fk20_g1p_t *output, const fk20_g1p_t *input, unsigned count, unsigned n,
             fk20_stream_t stream);
 /* Inverse G1 FFT including 1/n.  Replaces g1p_ift_wrapper (g1.cuh:97; g1p_fft.cu:350). */
@@ -120,7 +123,9 @@ int fk20_poly2h_fft(fk20_g1p_t *h_fft, const fk20_fr_t *polynomial, const fk20_g
  * FK20_NOALLOC_SCRATCH_BYTES array in device memory, one per device the library runs on, held
  * until the process ends; a call needs rows * (N/8) * 1344 + (N/8) * 2304 bytes of it, so
  * rows <= 95 at N = 4096, 193 at N = 2048 and 388 at N = 1024, and larger requests return
- * FK20_ERANGE without touching the device.  Every call on a device shares that device's
+ * FK20_ERANGE without touching the device.  From 17 rows its MSM keeps the bases' multiples in that
+ * array if there is room for windows of 7 bits or more (not at N = 4096), else in LDS, as the
+ * smallest form of fk20_poly2h_fft does.  Every call on a device shares that device's
  * array: calls that overlap on one device (different streams, threads) race and must be
  * serialised by the caller.  The first call of any entry point on a device copies the
  * library's constant tables into static device memory (no allocation there either). */
@@ -219,7 +224,8 @@ int fk20_setup_unload(fk20_ctx_t *ctx, int setup_id);
 /* Workspace bytes fk20_prove_rows needs for `rows` rows of length N:
  * rows * (N/8) * 656 + ceil(rows/64) * (N/8) * 4 + 512. */
 size_t fk20_rows_workspace_bytes(unsigned rows, unsigned N);
-/* Grows the context workspace to fit `rows` rows of length N. */
+/* Grows the context workspace to fit `rows` rows of length N, and if there is memory for it the
+ * products that make smaller batches fastest (calls within what is reserved allocate nothing). */
 int fk20_ctx_reserve(fk20_ctx_t *ctx, unsigned rows, unsigned N);
 /* polynomial[rows][N] -> h_fft[rows][N/8] for the setup's N: Toeplitz + NTT, window-table
  * MSM, column-batched G1 IFFT / zero / FFT with endomorphism-split twiddles. */
@@ -237,7 +243,8 @@ typedef struct {
 int fk20_prove_batch(fk20_ctx_t *ctx, const fk20_batch_item_t *items, unsigned nitems,
                      fk20_stream_t stream);
 /* fk20_prove_batch with a caller-provided device workspace of at least the sum of
- * fk20_rows_workspace_bytes over the items (no allocation; used by the serving loop). */
+ * fk20_rows_workspace_bytes over the items (no allocation; used by the serving loop).  Small batches
+ * take the direct schedule in those steps whose products fit that size. */
 int fk20_prove_batch_ws(fk20_ctx_t *ctx, const fk20_batch_item_t *items, unsigned nitems,
                         void *workspace, size_t workspace_bytes, fk20_stream_t stream);
 /* KZG commitments of rows (the step before the path): commitments[r] = sum_{i<N}
@@ -250,6 +257,7 @@ int fk20_prove_batch_ws(fk20_ctx_t *ctx, const fk20_batch_item_t *items, unsigne
 int fk20_commit_setup_load(fk20_ctx_t *ctx, const fk20_g1p_t *srs, unsigned N, unsigned window,
                            int *setup_id, fk20_stream_t stream);
 size_t fk20_commit_setup_table_bytes(unsigned N, unsigned window);
+/* Workspace bytes fk20_commit_rows needs: rows * (N/16 + N/256) * 144. */
 size_t fk20_commit_workspace_bytes(unsigned rows, unsigned N);
 int fk20_commit_rows(fk20_ctx_t *ctx, int setup_id, fk20_g1p_t *commitments, const fk20_fr_t *polynomial,
                      unsigned rows, fk20_stream_t stream);
